@@ -4,38 +4,9 @@
 #include "plans.hpp"
 #include "stencil_bodies.hpp"
 #include "graph_bodies.hpp"
+#include "launch_tiles.hpp"
 
 namespace gp {
-
-// the three instantiations of one kernel: general dispatcher loop, no counters, fixed claims
-template <class Kernel> struct KernelSet { Kernel any, plain, fixed; };
-template <class Kernel> static KernelSet<Kernel> kernel_set(Kernel a, Kernel p, Kernel f) { return {a, p, f}; }
-#define GP_KSET(...) kernel_set(__VA_ARGS__, LOOP_ANY>, __VA_ARGS__, LOOP_PLAIN>, __VA_ARGS__, LOOP_FIXED>)
-
-template <class Kernel, class Arg>
-static int launch_tiles(KernelSet<Kernel> ks, int sx, int sy, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info, const Arg &arg, size_t lds_bytes = 0, int max_batch = 16) {
-    BlpArgs blp;
-    int grid = 0;
-    // several tiles per claim once there are far more tiles than workgroups that could hold them
-    const long tiles = (long)sx * sy;
-    const int batch = (int)std::min<long>(max_batch, std::max<long>(1, tiles / (32L * device_cus())));
-    if (lds_bytes > 48 * 1024) {
-        GP_HIP(hipFuncSetAttribute((const void *)ks.any, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
-        GP_HIP(hipFuncSetAttribute((const void *)ks.plain, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
-        GP_HIP(hipFuncSetAttribute((const void *)ks.fixed, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
-    }
-    // planned for the general form; the special ones need no more resources
-    int rc = plan_launch(ks.any, NT, lds_bytes, sx, sy, 1, ctx, &blp, &grid, info, batch, batch == 1 ? 4 : 1);
-    if (rc) return rc;
-    Kernel kern = ks.any;
-    if (batch == 1) {  // the special forms call the body once: one tile per claim only
-        if (!ctx) kern = ks.plain;
-        else if (fixed_claims(true, blp.groups, grid - blp.front, blp.total)) kern = ks.fixed;
-    }
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), lds_bytes, native(s), arg, blp);
-    GP_HIP(hipGetLastError());
-    return GP_SUCC;
-}
 
 static bool al16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 static bool is_float(int dt) { return dt == GP_F32 || dt == GP_F16 || dt == GP_BF16; }

@@ -1,0 +1,408 @@
+// The kernels the graph executors run: whole iterations of breadth-first search, single-source shortest paths and
+// PageRank, and connected components by union-find, over 32-bit adjacency in vectors of four.
+//
+// Layout.  row[v] .. row[v+1] are offsets into `ids` (and `weights`) in units of four neighbours; a list's last vector
+// is padded with the id vertex_count, whose label / cost / rank entry exists and makes every kernel pass it over.
+// Against the 64-bit lists of the files this is half the bytes, every access is an aligned 16-byte load, and a list
+// of 16 neighbours keeps four lanes busy for one load each (the 16-lane groups of graph_bodies.hpp started at a
+// 128-byte boundary and left half of their lanes without an edge).
+//
+// Split.  A wavefront owns 64 consecutive vertices: lane l reads what belongs to vertex l (coalesced), and the four
+// lanes of a quad walk the lists of the quad's four vertices one after the other, handing the offsets round with DPP
+// quad broadcasts.  The first vectors of all four lists are requested before the first is used.  A list of more than
+// kLongRow vectors is walked by the whole wavefront afterwards, so that a hub does not hold four lanes for long.
+// A tile is 256 vertices; a preemptible launch hands tiles out through tile_loop.hpp like any other kernel.
+//
+// Several iterations are queued at once: an iteration whose predecessor changed nothing (*prev_changed == 0) leaves
+// before its first claim, so the host looks at the convergence words once per batch instead of once per iteration.
+#include "launch_tiles.hpp"
+
+namespace gp {
+
+constexpr int GF_TILE = 256;
+constexpr unsigned GF_INF = 0xFFFFFFFFu;
+constexpr unsigned kLongRow = 64;
+
+template <int S> __device__ __forceinline__ unsigned quad_bcast(unsigned x) { return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, S * 0x55, 0xf, 0xf, true); }
+// sum over the four lanes of a quad, left in all of them
+__device__ __forceinline__ float quad_sum(float x) {
+    x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0xB1, 0xf, 0xf, true));  // lanes 1 0 3 2
+    x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x4E, 0xf, 0xf, true));  // lanes 2 3 0 1
+    return x;
+}
+
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+// f(index of a vector of four neighbours, its ids, the owner's payload) for every vector of the 64 lists that this
+// wavefront's lanes own; an empty range (begin == end) stands for a vertex that takes no part
+template <class F>
+__device__ __forceinline__ void gf_walk(const u32x4 *ids, unsigned begin, unsigned end, unsigned payload, F &&f) {
+    const unsigned sub = threadIdx.x & 3;
+    const bool is_long = end - begin > kLongRow;
+    const unsigned stop = is_long ? begin : end;
+    const unsigned b0 = quad_bcast<0>(begin) + sub, b1 = quad_bcast<1>(begin) + sub, b2 = quad_bcast<2>(begin) + sub, b3 = quad_bcast<3>(begin) + sub;
+    const unsigned e0 = quad_bcast<0>(stop), e1 = quad_bcast<1>(stop), e2 = quad_bcast<2>(stop), e3 = quad_bcast<3>(stop);
+    const unsigned p0 = quad_bcast<0>(payload), p1 = quad_bcast<1>(payload), p2 = quad_bcast<2>(payload), p3 = quad_bcast<3>(payload);
+    u32x4 i0{}, i1{}, i2{}, i3{};
+    if (b0 < e0) i0 = ids[b0];
+    if (b1 < e1) i1 = ids[b1];
+    if (b2 < e2) i2 = ids[b2];
+    if (b3 < e3) i3 = ids[b3];
+    if (b0 < e0) f(b0, i0, p0);
+    if (b1 < e1) f(b1, i1, p1);
+    if (b2 < e2) f(b2, i2, p2);
+    if (b3 < e3) f(b3, i3, p3);
+    for (unsigned c = b0 + 4; c < e0; c += 4) f(c, ids[c], p0);
+    for (unsigned c = b1 + 4; c < e1; c += 4) f(c, ids[c], p1);
+    for (unsigned c = b2 + 4; c < e2; c += 4) f(c, ids[c], p2);
+    for (unsigned c = b3 + 4; c < e3; c += 4) f(c, ids[c], p3);
+    for (unsigned long long m = __builtin_amdgcn_ballot_w64(is_long); m; m &= m - 1) {
+        const int l = __builtin_ctzll(m);
+        const unsigned lb = __builtin_amdgcn_readlane(begin, l), le = __builtin_amdgcn_readlane(end, l), lp = __builtin_amdgcn_readlane(payload, l);
+        for (unsigned c = lb + (threadIdx.x & 63); c < le; c += 64) f(c, ids[c], lp);
+    }
+}
+
+__device__ __forceinline__ void raise_changed(unsigned *word, bool mine) {
+    if (__builtin_amdgcn_ballot_w64(mine) && (threadIdx.x & 63) == 0) *word = 1;
+}
+
+// ---- connected components: union-find with the smaller id as the parent ---------------------------------------------
+// Parents only ever fall, so a stale read (the L2s of the eight XCDs do not see each other's stores within a launch)
+// is an older ancestor and still an ancestor; a root is only hooked by a compare-and-swap, whose answer comes from
+// memory.  Every turn replaces the larger of the two candidates by something smaller, so the loop ends.
+__device__ __forceinline__ void cc_link(unsigned *parent, unsigned u, unsigned v) {
+    unsigned a = parent[u], b = parent[v];
+    while (a != b) {
+        const unsigned hi = a > b ? a : b, lo = a > b ? b : a;
+        unsigned p = parent[hi];
+        if (p == lo) return;
+        if (p == hi) {
+            p = atomicCAS(&parent[hi], hi, lo);
+            if (p == hi || p == lo) return;
+        }
+        a = p;
+        b = lo;
+    }
+}
+__device__ __forceinline__ unsigned cc_root(const unsigned *parent, unsigned v) {
+    unsigned p = parent[v];
+    for (unsigned g; (g = parent[p]) != p; p = g) { }
+    return p;
+}
+
+// ---- PageRank -----------------------------------------------------------------------------------------------------------
+// Many vertices over the tolerance (PR): residual[v] += the shares its in-neighbours hand out this iteration, then the
+// update of the reference's pr_update on the spot.  Shares are double-buffered (0 where u has nothing to hand out).
+// The push's 16.8 million float atomics of a 2^20-vertex iteration (207 us, and 14 us for the update) become a gather
+// from an array of 4 MB: 40 us, of which 16 are the streams and the rest the 4.4 million lines asked of the L2s for
+// the gather (1.2 million of them beyond; non-temporal streams keep fewer of those but lose the vector cache's reuse
+// of a quad's line and take 52).
+// Few (PR_STEP): one launch takes in what the iteration before pushed (gained), updates, and pushes what the vertices
+// over the tolerance hand out into the next iteration's sums; the rest of the residual stays where it is, so only the
+// vertices that gained something are touched at all.
+__device__ __forceinline__ float pr_pull4(const float *share, const u32x4 &i) { return (share[i[0]] + share[i[1]]) + (share[i[2]] + share[i[3]]); }
+
+__device__ __forceinline__ float pr_share(const gp_graph_iter_params &p, unsigned v, float r) {
+    const float degree = p.degree[v];
+    return degree > 0.f ? r * p.alpha / degree : 0.f;  // a sink has nobody to hand it to
+}
+// whether anybody was over the tolerance, and how many in one tile of GP_GRAPH_SAMPLED
+__device__ __forceinline__ void pr_report(const gp_graph_iter_params &p, int tile, bool up) {
+    const unsigned long long ups = __builtin_amdgcn_ballot_w64(up);
+    if (ups == 0 || (threadIdx.x & 63) != 0) return;
+    *p.changed = 1;
+    if (tile % GP_GRAPH_SAMPLED == 0) atomicAdd(p.changed + 1, (unsigned)__builtin_popcountll(ups));
+}
+__device__ __forceinline__ void pr_push(const gp_graph_iter_params &p, const u32x4 *ids, unsigned v, float share) {
+    if (!__builtin_amdgcn_ballot_w64(share != 0.f)) return;
+    unsigned begin = 0, end = 0;
+    if (share != 0.f) { begin = p.row[v]; end = p.row[v + 1]; }
+    gf_walk(ids, begin, end, __builtin_bit_cast(unsigned, share), [&](unsigned, const u32x4 &i, unsigned from) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (i[j] < p.vertex_count) atomicAdd(&p.next_gained[i[j]], __builtin_bit_cast(float, from));
+    });
+}
+
+// What a tile is looked through for (the vertices on the frontier): read for several tiles at a time, and before the
+// claim where the claim's answer is known, so that the reads of a claim's tiles are one trip to memory.
+template <int KIND>
+__device__ __forceinline__ unsigned gf_key(const gp_graph_iter_params &p, int tile) {
+    const unsigned v = (unsigned)tile * GF_TILE + threadIdx.x;
+    if (v >= p.vertex_count) return KIND == GP_GRAPH_IT_BFS ? GF_INF : 0;
+    if constexpr (KIND == GP_GRAPH_IT_BFS) return p.label[v];
+    else if constexpr (KIND == GP_GRAPH_IT_SSSP) return p.active[v];
+    else if constexpr (KIND == GP_GRAPH_IT_PR_STEP) return __builtin_bit_cast(unsigned, p.gained[v]);
+    else return 0;
+}
+
+template <int KIND>
+__device__ __forceinline__ void gf_tile(const gp_graph_iter_params &p, int tile, unsigned key, unsigned limit) {
+    const unsigned n = p.vertex_count;
+    const unsigned v = (unsigned)tile * GF_TILE + threadIdx.x;
+    const bool in = v < n;
+    const u32x4 *ids = reinterpret_cast<const u32x4 *>(p.ids);
+    if constexpr (KIND == GP_GRAPH_IT_BFS) {
+        const bool on = key == p.level;
+        if (!__builtin_amdgcn_ballot_w64(on)) return;
+        unsigned begin = 0, end = 0;
+        if (on) { begin = p.row[v]; end = p.row[v + 1]; }
+        bool mine = false;
+        gf_walk(ids, begin, end, 0, [&](unsigned, const u32x4 &i, unsigned) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (p.label[i[j]] == GF_INF) { p.label[i[j]] = p.level + 1; mine = true; }
+        });
+        raise_changed(p.changed, mine);
+    } else if constexpr (KIND == GP_GRAPH_IT_SSSP) {
+        bool on = key != 0;
+        if (!__builtin_amdgcn_ballot_w64(on)) return;
+        bool far = false;
+        unsigned begin = 0, end = 0, cost = 0;
+        if (on) {
+            cost = p.cost[v];
+            far = cost >= limit;
+            on = !far;
+            p.active[v] = 0;
+            if (far) p.next_active[v] = 1;  // its turn comes with a later limit
+        }
+        if (on) { begin = p.row[v]; end = p.row[v + 1]; }
+        bool mine = far, near = false;
+        const u32x4 *weights = reinterpret_cast<const u32x4 *>(p.weights);
+        gf_walk(ids, begin, end, cost, [&](unsigned c, const u32x4 &i, unsigned from) {
+            const u32x4 w = weights[c];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                // (costs only fall, so a stale one is too large and never hides an improvement)
+                const unsigned via = from + w[j];
+                if (p.cost[i[j]] > via && atomicMin(&p.cost[i[j]], via) > via) {
+                    p.next_active[i[j]] = 1;
+                    mine = true;
+                    near |= via < limit;
+                }
+            }
+        });
+        raise_changed(p.changed, mine);
+        raise_changed(p.changed + 1, near);
+    } else if constexpr (KIND == GP_GRAPH_IT_PR) {
+        unsigned begin = 0, end = 0;
+        float r = 0.f;
+        if (in) { begin = p.row[v]; end = p.row[v + 1]; r = p.residual[v]; }
+        const unsigned sub = threadIdx.x & 3, none = p.row_end;
+        const bool is_long = end - begin > kLongRow;
+        const unsigned stop = is_long ? begin : end;
+        const unsigned b[4] = {quad_bcast<0>(begin) + sub, quad_bcast<1>(begin) + sub, quad_bcast<2>(begin) + sub, quad_bcast<3>(begin) + sub};
+        const unsigned e[4] = {quad_bcast<0>(stop), quad_bcast<1>(stop), quad_bcast<2>(stop), quad_bcast<3>(stop)};
+        // (no branches around these loads: a lane without a vector reads the one behind the last list, which names
+        // only the neighbour that counts nothing; two vectors per lane and list, 32 neighbours, are in flight at once)
+        const bool two = __builtin_amdgcn_ballot_w64(stop - begin > 4);
+        u32x4 i[4], k[4];
+        float g[4], h[4] = {0.f, 0.f, 0.f, 0.f}, sum[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) i[s] = ids[b[s] < e[s] ? b[s] : none];
+        if (two) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) k[s] = ids[b[s] + 4 < e[s] ? b[s] + 4 : none];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) g[s] = pr_pull4(p.share, i[s]);
+        if (two) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) h[s] = pr_pull4(p.share, k[s]);
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            sum[s] = g[s] + h[s];
+            for (unsigned c = b[s] + 8; c < e[s]; c += 4) sum[s] += pr_pull4(p.share, ids[c]);
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s) sum[s] = quad_sum(sum[s]);
+        r += sub == 0 ? sum[0] : sub == 1 ? sum[1] : sub == 2 ? sum[2] : sum[3];
+        for (unsigned long long m = __builtin_amdgcn_ballot_w64(is_long); m; m &= m - 1) {
+            const int l = __builtin_ctzll(m);
+            const unsigned lb = __builtin_amdgcn_readlane(begin, l), le = __builtin_amdgcn_readlane(end, l);
+            float x = 0.f;
+            for (unsigned c = lb + (threadIdx.x & 63); c < le; c += 64) x += pr_pull4(p.share, ids[c]);
+            for (int d = 32; d; d >>= 1) x += __shfl_xor(x, d);
+            if ((int)(threadIdx.x & 63) == l) r += x;
+        }
+        const bool up = in && r > p.tolerance;
+        if (in) {
+            __builtin_nontemporal_store(up ? pr_share(p, v, r) : 0.f, p.next_share + v);
+            __builtin_nontemporal_store(up ? 0.f : r, p.residual + v);
+        }
+        if (up) __builtin_nontemporal_store(p.value[v] + r, p.value + v);
+        pr_report(p, tile, up);
+    } else if constexpr (KIND == GP_GRAPH_IT_PR_PUSH) {
+        const float share = in ? p.share[v] : 0.f;
+        pr_push(p, ids, v, share);
+    } else if constexpr (KIND == GP_GRAPH_IT_PR_STEP) {
+        // (next_gained == nullptr: the next iteration pulls; the shares are left for it instead of pushed)
+        const float gained = __builtin_bit_cast(float, key);
+        if (p.next_gained && !__builtin_amdgcn_ballot_w64(gained != 0.f)) return;
+        bool up = false;
+        float share = 0.f;
+        if (gained != 0.f) {
+            const float r = p.residual[v] + gained;
+            p.gained[v] = 0.f;
+            up = r > p.tolerance;
+            p.residual[v] = up ? 0.f : r;
+            if (up) { p.value[v] += r; share = pr_share(p, v, r); }
+        }
+        pr_report(p, tile, up);
+        if (p.next_gained) pr_push(p, ids, v, share);
+        else if (in) p.next_share[v] = share;
+    } else if constexpr (KIND == GP_GRAPH_IT_PR_INIT) {
+        if (!in) return;
+        p.value[v] = 1.0f - p.alpha;
+        p.next_share[v] = p.degree[v] > 0.f ? (1.0f - p.alpha) * p.alpha / p.degree[v] : 0.f;
+        p.residual[v] = 0.f;
+        p.gained[v] = 0.f;
+        p.next_gained[v] = 0.f;
+    } else if constexpr (KIND == GP_GRAPH_IT_BFS_INIT) {
+        if (in) p.label[v] = v == 0 ? 0 : GF_INF;  // source = vertex 0
+    } else if constexpr (KIND == GP_GRAPH_IT_SSSP_INIT) {
+        if (!in) return;
+        p.cost[v] = v == 0 ? 0 : GF_INF;
+        p.active[v] = v == 0;
+        p.next_active[v] = 0;
+    } else if constexpr (KIND == GP_GRAPH_IT_CC_INIT) {
+        // hook every vertex to its first neighbour at once, if that is smaller (nobody reads a parent in this launch)
+        if (!in) return;
+        unsigned first = v;
+        if (p.row[v] < p.row[v + 1]) { first = p.ids[4ull * p.row[v]]; }
+        p.parent[v] = first < v ? first : v;
+    } else if constexpr (KIND == GP_GRAPH_IT_CC_FLATTEN) {
+        if (in) p.parent[v] = cc_root(p.parent, v);
+    } else if constexpr (KIND == GP_GRAPH_IT_CC_LINK) {
+        unsigned begin = 0, end = 0;
+        if (in) { begin = p.row[v]; end = p.row[v + 1]; }
+        gf_walk(ids, begin, end, v, [&](unsigned, const u32x4 &i, unsigned from) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (i[j] < n) cc_link(p.parent, from, i[j]);
+        });
+    } else {  // GP_GRAPH_IT_CC_LABEL
+        if (in) p.comp[v] = cc_root(p.parent, v);
+    }
+}
+
+// Shortest paths: an iteration relaxes the marked vertices whose cost is below a limit; the others keep their mark.  The
+// limit rises by one step whenever an iteration has left no marked vertex below it.  Vertices are then relaxed close to
+// their final cost: on the generated graphs 1.1-1.4 times per vertex, where relaxing whatever is marked takes 4-5, for
+// a fifth more iterations (weights uniform in 1..64, a step of the average weight).  The limit of the iteration before
+// and whether it improved anything below it are in that iteration's words; the first iteration's limit is one step.
+__device__ __forceinline__ unsigned sssp_limit(const gp_graph_iter_params &p) {
+    unsigned limit = p.step;
+    if (p.prev_changed) {
+        limit = p.prev_changed[2];
+        if (!p.prev_changed[1]) limit = limit + p.step < limit ? GF_INF : limit + p.step;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) p.changed[2] = limit;
+    return limit;
+}
+
+// a claim of a launch stands for `per` tiles of 256 vertices
+template <int KIND, int LOOP = LOOP_ANY>
+__global__ __launch_bounds__(GF_TILE) void graph_iter_kernel(gp_graph_iter_params p, int per, BlpArgs blp) {
+    if (p.prev_changed && *p.prev_changed == 0) return;  // converged before this iteration (the same answer for every workgroup)
+    unsigned limit = 0;
+    if constexpr (KIND == GP_GRAPH_IT_SSSP) limit = sssp_limit(p);
+    unsigned key[4];  // of the next tiles
+    auto look = [&](int first, int count) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (j < count) key[j] = gf_key<KIND>(p, first + j);
+    };
+    const int known = LOOP == LOOP_ANY || wg_id(blp) < 0 || wg_id(blp) >= blp.total ? -1 : xcd_contiguous(wg_id(blp), blp.total);
+    if (known >= 0) look(known * per, per);
+    tiles<LOOP>(blp, [&](TileIdx t) {
+#pragma unroll 1
+        for (int j = 0; j < per; ++j) {
+            if (j % 4 == 0 && (j || known < 0)) look(t.x * per + j, per - j);
+            gf_tile<KIND>(p, t.x * per + j, key[0], limit);
+            key[0] = key[1]; key[1] = key[2]; key[2] = key[3];
+        }
+    });
+}
+
+// 64-bit neighbour ids (and weights) into padded vectors of four
+__global__ __launch_bounds__(GF_TILE) void graph_pack_kernel(gp_graph_pack_params p) {
+    const unsigned v = (unsigned)blockIdx.x * (GF_TILE / 4) + threadIdx.x / 4;
+    if (v == 0) p.ids[4ull * p.row_end + (threadIdx.x & 3)] = p.vertex_count;  // behind the last list
+    if (v >= p.vertex_count) return;
+    const unsigned long long from = p.vertex_list[v], to = p.vertex_list[v + 1];
+    for (unsigned c = p.row[v] + (threadIdx.x & 3); c < p.row[v + 1]; c += 4) {
+        const unsigned long long at = from + 4ull * (c - p.row[v]);
+        for (int j = 0; j < 4; ++j) {
+            p.ids[4ull * c + j] = at + j < to ? (unsigned)p.edge_list[at + j] : p.vertex_count;
+            if (p.weights) p.weights[4ull * c + j] = at + j < to ? p.weight_list[at + j] : 0u;
+        }
+    }
+}
+
+// one wavefront hands the words of the launches to the host: the words first, then the sequence number it waits for
+__global__ void graph_report_kernel(const unsigned *words, int stride, const int *stop_index, unsigned *host, int n, unsigned seq) {
+    if ((int)threadIdx.x < n) {
+        __hip_atomic_store(host + 2 + 2 * threadIdx.x, words[threadIdx.x * stride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(host + 3 + 2 * threadIdx.x, words[threadIdx.x * stride + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    if (threadIdx.x == 0) __hip_atomic_store(host + 1, stop_index ? (unsigned)*stop_index : 0xFFFFFFFFu, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    // (the stores above have arrived when the counter is down; a system-scope release would write the L2s back as well,
+    // 12 us in front of the next iteration)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (threadIdx.x == 0) __hip_atomic_store(host, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+}  // namespace gp
+
+using namespace gp;
+
+extern "C" int gp_launch_graph_iter(const gp_graph_iter_params *p, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
+    GP_REQUIRE(p && p->row && p->ids, "null graph iteration params");
+    GP_REQUIRE(p->vertex_count > 0 && p->vertex_count < (1u << 31), "graph: vertex count out of range");
+    switch (p->kernel) {
+        case GP_GRAPH_IT_BFS: GP_REQUIRE(p->label && p->changed, "bfs: operands missing"); break;
+        case GP_GRAPH_IT_BFS_INIT: GP_REQUIRE(p->label, "bfs: label missing"); break;
+        case GP_GRAPH_IT_SSSP: GP_REQUIRE(p->weights && p->cost && p->active && p->next_active && p->active != p->next_active && p->changed, "sssp: operands missing"); break;
+        case GP_GRAPH_IT_SSSP_INIT: GP_REQUIRE(p->cost && p->active && p->next_active, "sssp: operands missing"); break;
+        case GP_GRAPH_IT_PR: GP_REQUIRE(p->share && p->next_share && p->share != p->next_share && p->residual && p->value && p->degree && p->changed, "pagerank: operands missing"); break;
+        case GP_GRAPH_IT_PR_PUSH: GP_REQUIRE(p->share && p->next_gained, "pagerank: operands missing"); break;
+        case GP_GRAPH_IT_PR_STEP: GP_REQUIRE(p->gained && p->gained != p->next_gained && (p->next_gained || p->next_share) && p->residual && p->value && p->degree && p->changed, "pagerank: operands missing"); break;
+        case GP_GRAPH_IT_PR_INIT: GP_REQUIRE(p->next_share && p->residual && p->value && p->degree && p->gained && p->next_gained, "pagerank: operands missing"); break;
+        case GP_GRAPH_IT_CC_LABEL: GP_REQUIRE(p->comp, "cc: labels missing");  // fallthrough
+        case GP_GRAPH_IT_CC_INIT: case GP_GRAPH_IT_CC_LINK: case GP_GRAPH_IT_CC_FLATTEN: GP_REQUIRE(p->parent, "cc: parents missing"); break;
+    }
+    const long tiles = ((long)p->vertex_count + GF_TILE - 1) / GF_TILE;
+    // A launch's cost besides its edges is its workgroups (a claim, a barrier: 4096 of them take 12 us): up to eight
+    // tiles per claim as long as that leaves four workgroups per compute unit.  The pull wants as many lists in flight
+    // as the chip holds and takes one tile at a time.
+    const int per = p->kernel == GP_GRAPH_IT_PR ? 1 : (int)std::min<long>(8, std::max<long>(1, tiles / (4L * device_cus())));
+    switch (p->kernel) {
+#define GP_GI(K) case K: return launch_tiles(GP_KSET(graph_iter_kernel<K), (int)((tiles + per - 1) / per), 1, ctx, s, info, *p, 0, 4, GF_TILE, per);
+        GP_GI(GP_GRAPH_IT_BFS) GP_GI(GP_GRAPH_IT_BFS_INIT) GP_GI(GP_GRAPH_IT_SSSP) GP_GI(GP_GRAPH_IT_SSSP_INIT) GP_GI(GP_GRAPH_IT_PR)
+        GP_GI(GP_GRAPH_IT_PR_PUSH) GP_GI(GP_GRAPH_IT_PR_STEP) GP_GI(GP_GRAPH_IT_PR_INIT) GP_GI(GP_GRAPH_IT_CC_INIT) GP_GI(GP_GRAPH_IT_CC_LINK)
+        GP_GI(GP_GRAPH_IT_CC_FLATTEN) GP_GI(GP_GRAPH_IT_CC_LABEL)
+#undef GP_GI
+    }
+    set_error("graph iteration kernel %d", p->kernel);
+    return GP_OUTOFRANGE;
+}
+
+extern "C" int gp_graph_pack_async(const gp_graph_pack_params *p, gp_stream s) {
+    GP_REQUIRE(p && p->vertex_list && p->row && p->ids && (p->edge_list || p->row_end == 0), "null graph pack params");
+    GP_REQUIRE(!p->weights == !p->weight_list, "graph pack: weights come together");
+    GP_REQUIRE(p->vertex_count > 0 && p->vertex_count < (1u << 31), "graph: vertex count out of range");
+    hipLaunchKernelGGL(graph_pack_kernel, dim3((p->vertex_count + GF_TILE / 4 - 1) / (GF_TILE / 4)), dim3(GF_TILE), 0, native(s), *p);
+    GP_HIP(hipGetLastError());
+    return GP_SUCC;
+}
+
+extern "C" int gp_graph_report_async(const unsigned *words, int n, int stride, const int *stop_index, unsigned *host_words, unsigned seq, gp_stream s) {
+    GP_REQUIRE(words && host_words && n >= 0 && n <= 64 && stride >= 2, "graph report: 0..64 pairs of words");
+    hipLaunchKernelGGL(graph_report_kernel, dim3(1), dim3(64), 0, native(s), words, stride, stop_index, host_words, n, seq);
+    GP_HIP(hipGetLastError());
+    return GP_SUCC;
+}

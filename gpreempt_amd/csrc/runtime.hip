@@ -190,6 +190,13 @@ extern "C" int gp_host_alloc(void **host, size_t bytes) {
     return GP_SUCC;
 }
 extern "C" int gp_host_free(void *host) { if (host) GP_HIP(hipHostFree(host)); return GP_SUCC; }
+extern "C" int gp_host_alloc_coherent(void **host, void **dev, size_t bytes) {
+    GP_REQUIRE(host && dev && bytes, "null out pointer");
+    GP_HIP(hipHostMalloc(host, bytes, hipHostMallocCoherent | hipHostMallocMapped));
+    memset(*host, 0, bytes);
+    GP_HIP(hipHostGetDevicePointer(dev, *host, 0));
+    return GP_SUCC;
+}
 extern "C" int gp_memcpy_h2d(void *dev, const void *host, size_t bytes) { GP_HIP(hipMemcpy(dev, host, bytes, hipMemcpyHostToDevice)); return GP_SUCC; }
 extern "C" int gp_memcpy_d2h(void *host, const void *dev, size_t bytes) { GP_HIP(hipMemcpy(host, dev, bytes, hipMemcpyDeviceToHost)); return GP_SUCC; }
 extern "C" int gp_memcpy_h2d_async(void *dev, const void *host, size_t bytes, gp_stream s) { GP_HIP(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, native(s))); return GP_SUCC; }

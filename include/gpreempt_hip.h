@@ -73,6 +73,8 @@ int gp_malloc(void **dev, size_t bytes);
 int gp_free(void *dev);
 int gp_host_alloc(void **host, size_t bytes); /* pinned */
 int gp_host_free(void *host);
+/* pinned, zeroed and coherent: a running kernel's stores (through *dev) are visible to a host that spins on them */
+int gp_host_alloc_coherent(void **host, void **dev, size_t bytes);
 int gp_memcpy_h2d(void *dev, const void *host, size_t bytes);
 int gp_memcpy_d2h(void *host, const void *dev, size_t bytes);
 int gp_memcpy_h2d_async(void *dev, const void *host, size_t bytes, gp_stream s);
@@ -408,6 +410,59 @@ typedef struct gp_graph_params {
     int lanes_per_vertex;                    /* edge-parallel kernels: 16, 32 or 64 lanes walk one neighbour list (0 = 64); pick ~ the average degree */
 } gp_graph_params;
 int gp_launch_graph(const gp_graph_params *p, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info);
+
+/* One iteration of a graph algorithm per launch, over 32-bit adjacency in vectors of four: row[v] .. row[v+1] are
+ * offsets into ids / weights in units of four elements, and the last vector of a list is filled up with the id
+ * vertex_count.  label, cost and share therefore have vertex_count + 1 entries, the last of them 0, and ids and
+ * weights are 16-byte aligned.  What the graph executors run; gp_launch_graph keeps the reference's kernels.
+ *   BFS(_INIT)   label[v] == level: unlabelled (0xFFFFFFFF) neighbours get level + 1
+ *   SSSP(_INIT)  active[v] and cost[v] below the limit: offers cost[v] + weight to the neighbours (atomic min) and goes
+ *                inactive; who improves is marked in next_active, and so are the active ones at or above the limit,
+ *                which starts at `step` and rises by it after an iteration that left nobody active below it
+ *   PR(_INIT)    row / ids list IN-neighbours: residual += sum of their share; above the tolerance it moves into value
+ *                and next_share = residual * alpha / degree (out-degree; 0: nothing), else next_share = 0 (INIT writes next_share)
+ *   PR_PUSH      row / ids list OUT-neighbours: share is added to every neighbour's next_gained (atomic)
+ *   PR_STEP      residual += gained (which is cleared), the update as in PR, and what a vertex over the tolerance hands
+ *                out is pushed into next_gained; with next_gained NULL it is left in next_share
+ *   CC_*         union-find: INIT hooks every vertex to its first neighbour if that is smaller, LINK joins the ends of
+ *                every edge, FLATTEN points every vertex at its root, LABEL writes the root (the smallest id of the
+ *                component) to comp
+ * *changed is set to 1 by an iteration that changed something; changed[1] counts the vertices over the tolerance in
+ * every GP_GRAPH_SAMPLED-th tile (PR, PR_STEP) or says whether anybody improved below the limit, which is changed[2]
+ * (SSSP).  prev_changed, if given, is the word of the iteration
+ * before: a launch that finds it 0 does nothing (so several iterations can be queued without a look in between). */
+#define GP_GRAPH_SAMPLED 64
+enum gp_graph_iter_kernel { GP_GRAPH_IT_BFS = 0, GP_GRAPH_IT_BFS_INIT = 1, GP_GRAPH_IT_SSSP = 2, GP_GRAPH_IT_SSSP_INIT = 3, GP_GRAPH_IT_PR = 4,
+                            GP_GRAPH_IT_PR_INIT = 5, GP_GRAPH_IT_CC_INIT = 6, GP_GRAPH_IT_CC_LINK = 7, GP_GRAPH_IT_CC_FLATTEN = 8, GP_GRAPH_IT_CC_LABEL = 9,
+                            GP_GRAPH_IT_PR_PUSH = 10, GP_GRAPH_IT_PR_STEP = 11 };
+typedef struct gp_graph_iter_params {
+    int kernel;
+    unsigned int level, vertex_count, row_end;  /* row_end = row[vertex_count] */
+    const unsigned int *row, *ids, *weights;
+    unsigned int *label, *cost, *parent;
+    unsigned char *active, *next_active;
+    unsigned long long *comp;
+    const float *share, *degree;
+    float *next_share, *residual, *value, *gained, *next_gained;
+    float alpha, tolerance;
+    unsigned int step;
+    unsigned int *changed;                   /* three words */
+    const unsigned int *prev_changed;
+} gp_graph_iter_params;
+int gp_launch_graph_iter(const gp_graph_iter_params *p, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info);
+/* fills ids (4 * row_end + 4 of them: a last vector of vertex_count lies behind the lists) and weights of that layout from
+ * 64-bit lists; row has been computed by the caller, row_end = row[vertex_count] */
+typedef struct gp_graph_pack_params {
+    unsigned int vertex_count, row_end;
+    const unsigned long long *vertex_list, *edge_list;
+    const unsigned int *weight_list;  /* may be NULL, with weights */
+    const unsigned int *row;
+    unsigned int *ids, *weights;
+} gp_graph_pack_params;
+int gp_graph_pack_async(const gp_graph_pack_params *p, gp_stream s);
+/* Stores the pairs words[i * stride], words[i * stride + 1] (i < n) and *stop_index (-1 without one) into pinned host
+ * memory (host_words[2 + 2 i], host_words[3 + 2 i] and host_words[1]), then seq into host_words[0]. */
+int gp_graph_report_async(const unsigned int *words, int n, int stride, const int *stop_index, unsigned int *host_words, unsigned int seq, gp_stream s);
 
 /* out[t,:] = tok[ids[t],:] + pos[t % seq,:] (+ seg[0,:]); ids are int64 (the reference feeds
  * BERT int64 token ids, src/tests/test-dnn.cpp:21-23). */

@@ -4,9 +4,10 @@
 // GraphComputeBlp: read_graph, copy_gpu_graph, classes CC / BFS / PageRank / SSSP with
 // compute(stream[, preempted, executed, lc_tasks, be_tasks])) and of the host loops in
 // src/workloads/graphcompute.tr.cu:142-174 (CC), :257-285 (BFS), :450-495 (PageRank), :635-675
-// (SSSP).  One class drives all four: an algorithm is a list of kernels per iteration plus a few
-// host actions, and the loop that launches, notices a stop, waits for its turn and relaunches from
-// the stopped kernel is shared (the reference repeats it with `goto resume` per algorithm).
+// (SSSP).  One class drives all four: an algorithm is a list of launches, and the loop that launches, notices a
+// stop, waits for its turn and relaunches from the stopped launch is shared (the reference repeats it with
+// `goto resume` per algorithm).  A run queues several iterations at a time (gp_launch_graph_iter); a run with a
+// preemption injected at one of the reference's kernels (a test hook) goes through those, one iteration at a time.
 #pragma once
 #include <cstdint>
 #include <functional>
@@ -24,6 +25,7 @@ struct CsrGraph {
     std::vector<uint64_t> vertexList;   // vertex_count + 1 offsets into edgeList
     std::vector<uint64_t> edgeList;     // neighbour ids
     std::vector<uint32_t> weightList;   // per edge; empty when the graph has none
+    bool symmetric = false;             // known to hold every edge in both directions
 };
 
 // Files <base>.col (offsets), <base>.dst (neighbours), <base>.val (weights, optional): each is
@@ -52,8 +54,7 @@ public:
     // kind: "cc" | "bfs" | "pagerank" | "sssp"; nullptr for anything else (or sssp without weights)
     static std::unique_ptr<Workload> create(const std::string &kind, const CsrGraph &g);
     ~Workload();
-    // Runs the algorithm to convergence on `stream` (blocking: the host reads the convergence
-    // word every iteration, as the reference does).  env == nullptr: not preemptible.
+    // Runs the algorithm to convergence on `stream` (blocking).  env == nullptr: not preemptible.
     Status compute(GPUstream stream, const PreemptEnv *env);
 
     // results: "comp" (u64 per vertex), "label" (u32 BFS level), "value" (f32 PageRank), "cost" (u32 distance)
@@ -70,6 +71,16 @@ private:
     Workload() = default;
     Status run_kernels(const std::vector<int> &kernels, GPUstream stream, const PreemptEnv *env, int iteration, bool *changed);
     Status begin(GPUstream stream);
+    Status compute_stepwise(GPUstream stream, const PreemptEnv *env);
+    // a queue of launches, kRing of them at most outstanding; launch i uses slot i % kRing of ring_
+    Status queue(const std::vector<gp_graph_iter_params> &list, int report_before_last, GPUstream stream, const PreemptEnv *env);
+    Status launch_slot(int i, bool fresh, GPUstream stream, const PreemptEnv *env);
+    Status report(GPUstream stream, const PreemptEnv *env);
+    Status await_report(int first, GPUstream stream, const PreemptEnv *env);
+    const volatile unsigned *words(int i) const { return report_ + 2 + 2 * (i % kRing); }
+    Status wait_turn(GPUstream stream, const PreemptEnv *env);
+    bool upload_packed(const CsrGraph &g, bool with_weights);
+    gp_graph_iter_params params(int kernel) const;
     std::string kind_;
     uint64_t n_ = 0, m_ = 0;
     int iterations_ = 0, preemptions_ = 0, launches_ = 0;
@@ -82,6 +93,17 @@ private:
     GPUdeviceptr delta_ = nullptr, residual_ = nullptr, value_ = nullptr, cost_ = nullptr, new_cost_ = nullptr;
     GPUdeviceptr changed_ = nullptr;
     int *host_words_ = nullptr;  // pinned: [0] stop index, [1] changed
+    // adjacency in vectors of four 32-bit ids (in-neighbours for PageRank), and what only it needs
+    GPUdeviceptr row_ = nullptr, ids_ = nullptr, weights_ = nullptr, parent_ = nullptr, share_ = nullptr, degree_ = nullptr, gained_ = nullptr;
+    uint32_t row_end_ = 0, step_ = 1;
+    bool symmetric_ = false;
+    static constexpr int kRing = 64;
+    GPUdeviceptr ring_ = nullptr;                    // device: per slot two convergence words and the claim counters, a line apart
+    size_t slot_ints_ = 0;
+    std::vector<gp_graph_iter_params> queued_;       // launches of this run by number; the last kRing of them matter
+    volatile unsigned *report_ = nullptr;            // pinned, coherent: sequence number, stop index, words of every slot
+    void *report_dev_ = nullptr;
+    unsigned report_seq_ = 0;
 };
 
 }  // namespace GraphCompute

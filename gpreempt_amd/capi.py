@@ -4,6 +4,7 @@ Fails loudly when the library is missing: there is no fallback path.
 """
 import ctypes as C
 import os
+import threading
 
 import numpy as np
 
@@ -100,7 +101,7 @@ class EmbedParams(C.Structure):
 SYMBOLS = """gp_init gp_last_error gp_device_info gp_device_clock gp_stream_create gp_stream_destroy gp_stream_sync
 gp_stream_query gp_stream_priority gp_stream_set_priority gp_stream_native gp_event_create gp_event_destroy gp_event_record
 gp_event_sync gp_event_query gp_event_elapsed_ms gp_malloc gp_free gp_host_alloc gp_host_alloc_coherent gp_host_free gp_memcpy_h2d gp_memcpy_d2h
-gp_memcpy_h2d_async gp_memcpy_d2h_async gp_memcpy_d2d_async gp_fill32_async gp_flag_create gp_flag_destroy gp_store_word_async gp_flag_relay_start
+gp_memcpy_h2d_async gp_memcpy_d2h_async gp_memcpy_d2d_async gp_fill32_async gp_fetch gp_stage_create gp_stage_destroy gp_stage_upload_async gp_flag_create gp_flag_destroy gp_store_word_async gp_flag_relay_start
 gp_launch_gemm gp_gemm_ln_supported gp_launch_gemm_noalloc gp_gemm_ckpt_bytes gp_conv_ckpt_bytes gp_ckpt_reset_async gp_launch_conv2d gp_launch_nchw_to_nhwc gp_launch_pool2d gp_launch_eltwise gp_launch_softmax
 gp_launch_layernorm gp_launch_attention gp_launch_miniweather gp_launch_graph gp_launch_graph_iter gp_graph_pack_async gp_graph_report_async gp_launch_embed gp_launch_gate gp_launch_noop gp_graph_begin gp_graph_end gp_graph_launch
 gp_graph_destroy gp_program_create gp_program_destroy gp_program_add_gemm gp_program_add_conv2d
@@ -175,6 +176,63 @@ def from_storage(raw, dtype):
     if dtype == I32:
         return raw.view(np.int32)
     raise ValueError(dtype)
+
+
+class _Pinned:
+    """Memory under an array of HostPool.empty; goes back to the pool with the last array that refers to it."""
+
+    def __init__(self, pool, ptr, room, nbytes):
+        self._pool, self._ptr, self._room = pool, ptr, room
+        self.__array_interface__ = {"shape": (nbytes,), "typestr": "|u1", "data": (ptr, False), "version": 3}
+
+    def __del__(self):
+        self._pool._give_back(self._ptr, self._room)
+
+
+class HostPool:
+    """Arrays in pinned, coherent host memory (gp_host_alloc_coherent), which the GPU writes at the speed of PCIe: a
+    copy into an ordinary new array goes through the runtime's own pinned memory and pays for its pages, 2-4 times as
+    long (4.8 MB: 92 us for 270; 84 MB: 1.5 ms for 4.8).  At most LIMIT bytes at a time, of which at most KEEP stay
+    allocated while nobody uses them; beyond LIMIT callers get ordinary arrays."""
+
+    LIMIT = 1 << 30
+    KEEP = 512 << 20
+
+    def __init__(self):
+        self._lock = threading.RLock()  # (an array may die, and call _give_back, while its own thread is in here)
+        self._free = {}
+        self._total = self._idle = 0
+
+    def empty(self, nbytes):
+        """(uint8 array of nbytes, its address if pinned or else None)"""
+        # four sizes per power of two
+        step = max(4096, 1 << max(0, nbytes.bit_length() - 3))
+        room = max(step, -(-nbytes // step) * step)
+        ptr = None
+        with self._lock:
+            if self._free.get(room):
+                ptr = self._free[room].pop()
+                self._idle -= room
+            elif self._total + room <= self.LIMIT:
+                host, dev = vp(), vp()
+                if lib().gp_host_alloc_coherent(C.byref(host), C.byref(dev), C.c_size_t(room)) == 0:
+                    ptr = host.value
+                    self._total += room
+        if ptr is None:
+            return np.empty(nbytes, np.uint8), None
+        return np.asarray(_Pinned(self, ptr, room, nbytes)), ptr
+
+    def _give_back(self, ptr, room):
+        with self._lock:
+            if self._idle + room <= self.KEEP:
+                self._free.setdefault(room, []).append(ptr)
+                self._idle += room
+                return
+            self._total -= room
+        lib().gp_host_free(vp(ptr))
+
+
+host_pool = HostPool()
 
 
 class DevBuf:

@@ -350,10 +350,8 @@ __global__ void graph_report_kernel(const unsigned *words, int stride, const int
         __hip_atomic_store(host + 3 + 2 * threadIdx.x, words[threadIdx.x * stride + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     if (threadIdx.x == 0) __hip_atomic_store(host + 1, stop_index ? (unsigned)*stop_index : 0xFFFFFFFFu, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    // (the stores above have arrived when the counter is down; a system-scope release would write the L2s back as well,
-    // 12 us in front of the next iteration)
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (threadIdx.x == 0) __hip_atomic_store(host, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __threadfence_system();
+    if (threadIdx.x == 0) __hip_atomic_store(host, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 }  // namespace gp

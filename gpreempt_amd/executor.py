@@ -12,10 +12,10 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libgpreempt_exec.so")
 vp = C.c_void_p
 
-SYMBOLS = """gpx_create gpx_destroy gpx_init gpx_set_input gpx_get_output gpx_get_data_size gpx_execute
+SYMBOLS = """gpx_create gpx_destroy gpx_init gpx_set_input gpx_get_output gpx_fetch_output gpx_get_data_size gpx_execute
 gpx_launch_kernel gpx_get_kernel_num gpx_capture_graph gpx_uses_program gpx_clear gpx_set_flag gpx_set_running gpx_resume
 gpx_get_stop_point gpx_last_stop_index gpx_inject_preempt gpx_read_counters gpx_reset_counters gpx_storage_num gpx_storage_info
-gpx_kernel_info gpx_read_storage gpx_miniweather_reductions gpx_graph_info gpx_graph_result_bytes gpx_graph_result
+gpx_kernel_info gpx_read_storage gpx_miniweather_reductions gpx_graph_info gpx_graph_result_bytes gpx_graph_result gpx_graph_fetch_result
 gpx_graph_inject_preempt gpx_set_lc_tasks gpx_set_graph_path gpx_write_synthetic_graph gpx_run_scenario gpx_preempt_probe gpx_parse_params gpx_parse_tvm_export gpx_plan_tvm_export gpx_set_priority gpx_domain_create gpx_domain_destroy gpx_get_fd gpx_domain_flag gpx_domain_flag_value
 gpx_domain_begin gpx_domain_end gpx_suspend_streams gpx_resume_streams""".split()
 
@@ -123,13 +123,23 @@ class Executor:
     # -- data
     def set_input(self, key, raw, stream=None):
         raw = np.ascontiguousarray(raw)
-        _chk(lib().gpx_set_input(self.h, key.encode(), raw.ctypes.data_as(vp), C.c_size_t(raw.nbytes), stream.h if stream else None), f"set_input({key})")
+        rc = lib().gpx_set_input(self.h, key.encode(), vp(raw.ctypes.data), C.c_size_t(raw.nbytes), stream.h if stream else None)
+        if rc:
+            _chk(rc, f"set_input({key})")
         self._keep = raw
 
     def get_output(self, key="heads", stream=None):
-        raw = np.empty(self.data_size(key), np.uint8)
-        _chk(lib().gpx_get_output(self.h, key.encode(), raw.ctypes.data_as(vp), C.c_size_t(raw.nbytes), stream.h if stream else None), f"get_output({key})")
-        capi.check(capi.lib().gp_stream_sync(stream.h if stream else None))
+        n = self.data_size(key)
+        raw, pinned = capi.host_pool.empty(n)
+        h = stream.h if stream else None
+        if pinned and n:
+            rc = lib().gpx_fetch_output(self.h, key.encode(), vp(pinned), C.c_size_t(n), h)
+        else:
+            rc = lib().gpx_get_output(self.h, key.encode(), raw.ctypes.data_as(vp), C.c_size_t(n), h)
+            if not rc:
+                capi.check(capi.lib().gp_stream_sync(h))
+        if rc:
+            _chk(rc, f"get_output({key})")
         return raw
 
     def read_storage(self, key):
@@ -145,8 +155,9 @@ class Executor:
         return dict(vertices=v[0], edges=v[1], iterations=v[2], preemptions=v[3], kernels_launched=v[4])
 
     def graph_result(self, key, np_dtype):
-        raw = np.empty(lib().gpx_graph_result_bytes(self.h, key.encode()), np.uint8)
-        _chk(lib().gpx_graph_result(self.h, key.encode(), raw.ctypes.data_as(vp), C.c_size_t(raw.nbytes)), f"graph_result({key})")
+        raw, pinned = capi.host_pool.empty(lib().gpx_graph_result_bytes(self.h, key.encode()))
+        fn = lib().gpx_graph_fetch_result if pinned else lib().gpx_graph_result
+        _chk(fn(self.h, key.encode(), raw.ctypes.data_as(vp), C.c_size_t(raw.nbytes)), f"graph_result({key})")
         return raw.view(np_dtype)
 
     def graph_inject_preempt(self, iteration, kernel, claim):

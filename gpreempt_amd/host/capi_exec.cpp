@@ -57,6 +57,7 @@ void gpx_destroy(gpx_executor e) { delete H(e); }
 int gpx_init(gpx_executor e, const char *workload) { return guarded("gpx_init", [&] { return H(e)->ex->init(workload ? workload : ""); }); }
 int gpx_set_input(gpx_executor e, const char *key, void *value, size_t len, gp_stream s) { return H(e)->ex->set_input(key, value, len, s); }
 int gpx_get_output(gpx_executor e, const char *key, void *value, size_t len, gp_stream s) { return H(e)->ex->get_output(key, value, len, s); }
+int gpx_fetch_output(gpx_executor e, const char *key, void *pinned, size_t len, gp_stream s) { return H(e)->ex->fetch_output(key, pinned, len, s); }
 size_t gpx_get_data_size(gpx_executor e, const char *key) { return H(e)->ex->get_data_size(key); }
 int gpx_execute(gpx_executor e, gp_stream s) { return guarded("gpx_execute", [&] { return H(e)->ex->execute(s); }); }
 int gpx_launch_kernel(gpx_executor e, size_t idx, gp_stream s) { return H(e)->ex->launch_kernel(idx, s); }
@@ -127,6 +128,10 @@ extern "C" size_t gpx_graph_result_bytes(gpx_executor e, const char *key) {
 extern "C" int gpx_graph_result(gpx_executor e, const char *key, void *out, size_t len) {
     GraphCompute::Workload *w = H(e)->ex->graph_workload();
     return w ? w->read_result(key, out, len) : Status::NotFound;
+}
+extern "C" int gpx_graph_fetch_result(gpx_executor e, const char *key, void *pinned, size_t len) {
+    GraphCompute::Workload *w = H(e)->ex->graph_workload();
+    return w ? w->read_result(key, pinned, len, true) : Status::NotFound;
 }
 extern "C" int gpx_graph_inject_preempt(gpx_executor e, int iteration, int kernel, int claim) {
     if (!H(e)->blp) return Status::Fail;

@@ -91,6 +91,11 @@ Status Executor::get_output(const std::string &key, void *value, size_t len, GPU
 Status Executor::get_output(const std::string &key, std::vector<float> &value, GPUstream stream) {
     return get_output(key, value.data(), value.size() * sizeof(float), stream);
 }
+Status Executor::fetch_output(const std::string &key, void *pinned, size_t len, GPUstream stream) {
+    size_t idx;
+    if (!model || model->find_storage_idx(key, idx) != Status::Succ) return Status::NotFound;
+    return model->fetch(idx, pinned, len, stream);
+}
 size_t Executor::get_data_size(const std::string &key) {
     size_t idx;
     if (!model || model->find_storage_idx(key, idx) != Status::Succ) return 0;
@@ -198,7 +203,8 @@ Status BLPExecutor::init(std::string workload) {
     std::string model_path = model_root() + "/" + workload;
     RETURN_STATUS(model->load_model(model_path + "/mod.json", model_path + "/host.json", model_path + "/mod.tr.co"));
     CUDA_RETURN_STATUS(gp_malloc(&dpStopIndex, sizeof(int)));
-    CUDA_RETURN_STATUS(gp_host_alloc((void **)&stop_host, sizeof(int)));
+    void *stop_host_dev = nullptr;
+    CUDA_RETURN_STATUS(gp_host_alloc_coherent((void **)&stop_host, &stop_host_dev, sizeof(int)));
     CUDA_RETURN_STATUS(gp_flag_create(&left_host, &left_dev));
     model->set_left_word(left_dev);
     stopIndex = -1;
@@ -281,8 +287,7 @@ void BLPExecutor::clear() {
 // reference executor.cpp:269-278
 Status BLPExecutor::getStopPoint(GPUstream stream) {
     if (graph_compute) { stopIndex = -1; return Status::Succ; }  // the workload's loop resumes itself
-    CUDA_RETURN_STATUS(gp_memcpy_d2h_async(stop_host, dpStopIndex, sizeof(int), stream));
-    CUDA_RETURN_STATUS(gp_stream_sync(stream));
+    CUDA_RETURN_STATUS(gp_fetch(stop_host, dpStopIndex, sizeof(int), stream));
     stopIndex = *stop_host;
     if (stopIndex == -1) return Status::Succ;
     CUDA_RETURN_STATUS(gp_fill32_async(dpStopIndex, 0xFFFFFFFFu, 1, stream));

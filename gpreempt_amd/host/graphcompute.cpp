@@ -527,11 +527,15 @@ size_t Workload::result_bytes(const std::string &key) const {
     return 0;
 }
 
-Status Workload::read_result(const std::string &key, void *out, size_t len) const {
+Status Workload::read_result(const std::string &key, void *out, size_t len, bool pinned) const {
     const size_t bytes = result_bytes(key);
     if (bytes == 0) return Status::NotFound;
     if (len < bytes) return Status::OutOfRange;
     GPUdeviceptr src = key == "comp" ? comp_ : key == "label" ? label_ : key == "value" ? value_ : cost_;
+    if (pinned) {
+        GC_CHECK(gp_fetch(out, src, bytes, nullptr));  // (compute() has waited for its stream)
+        return Status::Succ;
+    }
     GC_CHECK(gp_stream_sync(nullptr));
     GC_CHECK(gp_memcpy_d2h(out, src, bytes));
     return Status::Succ;

@@ -371,7 +371,15 @@ Status Model::set(size_t idx, void *value, size_t len, GPUstream stream) {
     if (idx >= storages.size()) return Status::OutOfRange;
     size_t size = storage_infos[idx].size;
     if (len < size) return Status::OutOfRange;
-    CUDA_RETURN_STATUS(gp_memcpy_h2d_async(storages[idx], value, size, stream));
+    // (through the model's own pinned ring; memory that is pinned itself would be read in place, but nothing here says so)
+    if (!stage_) CUDA_RETURN_STATUS(gp_stage_create(&stage_));
+    CUDA_RETURN_STATUS(gp_stage_upload_async(stage_, storages[idx], value, size, stream));
+    return Status::Succ;
+}
+Status Model::fetch(size_t idx, void *pinned, size_t len, GPUstream stream) {
+    if (idx >= storages.size()) return Status::OutOfRange;
+    if (len < storage_infos[idx].size) return Status::Fail;
+    CUDA_RETURN_STATUS(gp_fetch(pinned, storages[idx], storage_infos[idx].size, stream));
     return Status::Succ;
 }
 Status Model::set(const std::string &key, void *value, size_t len, GPUstream stream) {
@@ -398,6 +406,7 @@ Status Model::get_global_ptr(const std::string &name, GPUdeviceptr *ptr) {
 
 Status Model::clear() {
     if (program_) { gp_program_destroy(program_); program_ = nullptr; }
+    if (stage_) { gp_stage_destroy(stage_); stage_ = nullptr; }
     if (!loaded_) return Status::Succ;
     for (GPUdeviceptr p : storages) CUDA_RETURN_STATUS(gp_free(p));
     storage_infos.clear(); layouts.clear(); kernel_infos.clear(); storages.clear(); storages_idx.clear();

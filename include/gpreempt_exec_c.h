@@ -21,6 +21,7 @@ void gpx_destroy(gpx_executor e);
 int gpx_init(gpx_executor e, const char *workload);                 /* Executor::init */
 int gpx_set_input(gpx_executor e, const char *key, void *value, size_t len, gp_stream s);  /* Executor::set_input */
 int gpx_get_output(gpx_executor e, const char *key, void *value, size_t len, gp_stream s); /* Executor::get_output */
+int gpx_fetch_output(gpx_executor e, const char *key, void *pinned, size_t len, gp_stream s); /* Executor::fetch_output */
 size_t gpx_get_data_size(gpx_executor e, const char *key);          /* Executor::get_data_size */
 int gpx_execute(gpx_executor e, gp_stream s);                        /* Executor::execute */
 int gpx_launch_kernel(gpx_executor e, size_t idx, gp_stream s);      /* Executor::launch_kernel */
@@ -56,6 +57,7 @@ int gpx_read_storage(gpx_executor e, const char *key, void *out, size_t len); /*
  * called with counters the handle owns). */
 int gpx_graph_info(gpx_executor e, unsigned long long info[5]);
 size_t gpx_graph_result_bytes(gpx_executor e, const char *key);
+int gpx_graph_fetch_result(gpx_executor e, const char *key, void *pinned, size_t len); /* into memory of gp_host_alloc_coherent */
 int gpx_graph_result(gpx_executor e, const char *key, void *out, size_t len);
 int gpx_graph_inject_preempt(gpx_executor e, int iteration, int kernel, int claim); /* BLPExecutor::inject_preempt_graph */
 int gpx_set_lc_tasks(gpx_executor e, int n);

@@ -80,6 +80,16 @@ int gp_memcpy_d2h(void *host, const void *dev, size_t bytes);
 int gp_memcpy_h2d_async(void *dev, const void *host, size_t bytes, gp_stream s);
 int gp_memcpy_d2h_async(void *host, const void *dev, size_t bytes, gp_stream s);
 int gp_memcpy_d2d_async(void *dst, const void *src, size_t bytes, gp_stream s);
+/* Copies `bytes` from device memory to memory of gp_host_alloc_coherent and returns when they are there: a kernel
+ * writes them and then a word the host spins on, where a copy and a stream synchronisation take twice as long. */
+int gp_fetch(void *host_coherent, const void *dev, size_t bytes, gp_stream s);
+/* Uploads from ordinary host memory through a ring of pinned memory that belongs to the handle: the caller's buffer
+ * may be reused as soon as the call returns, and the copy runs in stream order.  (hipMemcpyAsync from ordinary memory
+ * takes 2-4 times as long.)  Calls on one handle are serialised. */
+typedef struct gp_stage_s *gp_stage;
+int gp_stage_create(gp_stage *out);
+int gp_stage_destroy(gp_stage st); /* waits for uploads still under way */
+int gp_stage_upload_async(gp_stage st, void *dev, const void *host, size_t bytes, gp_stream s);
 /* Fills `count` 32-bit words with `value` using a fill kernel (safe inside a captured graph). */
 int gp_fill32_async(void *dev, uint32_t value, size_t count, gp_stream s);
 

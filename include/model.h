@@ -128,6 +128,8 @@ public:
 
     Status get(size_t idx, void *out, size_t len, GPUstream stream);
     Status get(const std::string &key, void *out, size_t len, GPUstream stream);
+    // as get, into memory of gp_host_alloc_coherent; returns when the values are there
+    Status fetch(size_t idx, void *pinned, size_t len, GPUstream stream);
     Status set(size_t idx, void *value, size_t len, GPUstream stream);
     Status set(const std::string &key, void *value, size_t len, GPUstream stream);
 
@@ -190,6 +192,7 @@ public:
 private:
     bool loaded_ = false;
     gp_program program_ = nullptr;
+    gp_stage stage_ = nullptr;  // pinned ring the inputs go through; made by the first set()
     int counter_groups_ = 1;
     int poll_every_ = 0;
     std::vector<char> fresh_;

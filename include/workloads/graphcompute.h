@@ -59,7 +59,8 @@ public:
 
     // results: "comp" (u64 per vertex), "label" (u32 BFS level), "value" (f32 PageRank), "cost" (u32 distance)
     size_t result_bytes(const std::string &key) const;
-    Status read_result(const std::string &key, void *out, size_t len) const;
+    // (pinned: `out` is memory of gp_host_alloc_coherent)
+    Status read_result(const std::string &key, void *out, size_t len, bool pinned = false) const;
     const std::string &kind() const { return kind_; }
     uint64_t vertex_count() const { return n_; }
     uint64_t edge_count() const { return m_; }

@@ -1,0 +1,44 @@
+"""gp_stage_upload_async and gp_fetch: bytes arrive whole at the sizes where the copies change form (a vector of 16
+bytes, one workgroup or several, one piece of the ring or many, the copy engine), whatever ran before."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 4096, 16384, 16385, 100003, (256 << 10) + 1, (1 << 20) + 3, (5 << 20) + 7, (9 << 20) + 5])
+def test_upload_and_fetch_round_trip(gp, n):
+    rng = np.random.default_rng(n)
+    st, stream, other = C.c_void_p(), gp.Stream(), gp.Stream()
+    gp.check(gp.lib().gp_stage_create(C.byref(st)))
+    devs = [gp.DevBuf(n + 16) for _ in range(3)]
+    for r in range(8):
+        want = [rng.integers(0, 256, n, np.uint8) for _ in devs]
+        for d, w in zip(devs, want):
+            host = w.copy()
+            gp.check(gp.lib().gp_stage_upload_async(st, C.c_void_p(d.ptr), host.ctypes.data_as(C.c_void_p), C.c_size_t(n), (stream if r % 2 else other).h))
+            host[:] = 0  # the caller's buffer is free again
+        for d, w in zip(devs, want):
+            out, pinned = gp.host_pool.empty(n)
+            assert pinned
+            gp.check(gp.lib().gp_fetch(C.c_void_p(pinned), C.c_void_p(d.ptr), C.c_size_t(n), (stream if r % 2 else other).h))
+            assert np.array_equal(d.download()[:n], w), (n, r)
+            assert np.array_equal(out, w), (n, r)
+    gp.check(gp.lib().gp_stage_destroy(st))
+
+
+def test_pool_memory_comes_back_and_is_bounded(gp):
+    pool = gp.HostPool()
+    a, pa = pool.empty(1000)
+    view = a[10:20]
+    del a
+    b, pb = pool.empty(1000)
+    assert pb != pa  # still referred to
+    del view
+    c, pc = pool.empty(900)
+    assert pc == pa
+    pool.LIMIT = 1 << 20
+    d, pd = pool.empty(2 << 20)
+    assert pd is None and d.nbytes == 2 << 20

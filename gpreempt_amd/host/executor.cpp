@@ -121,6 +121,10 @@ Status Executor::execute(GPUstream stream) {
         CUDA_RETURN_STATUS(gp_graph_launch(graph_exec, stream));
         return Status::Succ;
     }
+    if (model && model->has_sweeps()) {
+        for (size_t g = 0; g * Model::kSweepKernels < get_kernel_num(); g++) RETURN_STATUS(model->launch_sweep(g, stream));
+        return Status::Succ;
+    }
     for (size_t i = 0; i < get_kernel_num(); i++) RETURN_STATUS(launch_kernel(i, stream));
     return Status::Succ;
 }
@@ -274,7 +278,15 @@ Status BLPExecutor::execute(GPUstream stream) {
         model->launched_once_more();  // (a resume relaunches kernel by kernel and has to know)
         return Status::Succ;
     }
+    // (a preemption injected at one of the kernels, a test hook, wants the kernels)
+    swept = model->has_sweeps() && inject_kernel < 0;
+    if (swept) return launch_sweeps(0, stream);
     for (size_t i = 0; i < get_kernel_num(); i++) RETURN_STATUS(launch_kernel(i, stream));
+    return Status::Succ;
+}
+
+Status BLPExecutor::launch_sweeps(size_t from_kernel, GPUstream stream) {
+    for (size_t g = from_kernel / Model::kSweepKernels; g * Model::kSweepKernels < get_kernel_num(); g++) RETURN_STATUS(model->launch_sweep(g, stream));
     return Status::Succ;
 }
 
@@ -304,6 +316,7 @@ Status BLPExecutor::resume(GPUstream stream) {
     // the program continues from its own per-layer counters; per-kernel mode relaunches one by one
     model->set_poll_every(poll_every);
     if (use_program) return model->launch_program(stream, false, inject_kernel, inject_claim);
+    if (swept) return launch_sweeps((size_t)stopIndex, stream);
     for (size_t i = (size_t)stopIndex; i < get_kernel_num(); i++) RETURN_STATUS(launch_kernel(i, stream));
     return Status::Succ;
 }
@@ -387,6 +400,7 @@ int64_t BLPExecutor::device_ticks_to_ns(unsigned long long ticks) const {
 
 Status BLPExecutor::reset_counters(GPUstream stream) {
     if (graph_compute) return Status::Succ;
+    swept = false;
     CUDA_RETURN_STATUS(gp_fill32_async(executed, 0, 2 * model->get_kernel_num() * (size_t)kCounterGroups * kCounterStride, stream));
     if (ckpt) CUDA_RETURN_STATUS(gp_ckpt_reset_async(ckpt, stream));  // a fresh run has no tile to continue
     // launches recorded into a graph are replayed with the arguments of the recording: never fresh

@@ -213,6 +213,7 @@ Status Model::allocate_and_bind() {
     }
     loaded_ = true;
     plan_fusions();
+    RETURN_STATUS(plan_sweeps());
     // seeded random initialisation of every parameter (overwritten by load_param when a file exists)
     uint64_t seed = 0x5EEDull;
     for (size_t i = 0; i < storage_infos.size(); ++i) {
@@ -258,6 +259,31 @@ void Model::plan_fusions() {
         mm.has_ln_gemm = true;
         ln.fused_away = true;
     }
+}
+
+// A list that is the miniWeather step (x, z, z, x; three stages of halo, fluxes, update) also gets its sweeps.
+Status Model::plan_sweeps() {
+    sweeps_.clear();
+    if (kernel_infos.size() != 4 * kSweepKernels) return Status::Succ;
+    for (size_t i = 0; i < kernel_infos.size(); ++i) {
+        const int dir = i / kSweepKernels == 1 || i / kSweepKernels == 2 ? GP_MW_HALO_Z : GP_MW_HALO_X;
+        if (kernel_infos[i].op != OpKind::Stencil || kernel_infos[i].p.miniweather.kernel != dir + (int)(i % 3)) return Status::Succ;
+    }
+    const gp_miniweather_params &first = kernel_infos[2].p.miniweather;  // an update: state_init = state, state_out = state_tmp
+    float *state = (float *)first.state_init, *tmp = first.state_out;
+    const size_t bytes = get_storage_size(kernel_infos[0].args_index[0]);
+    CUDA_RETURN_STATUS(gp_malloc(&sweep_state_, bytes));
+    for (size_t g = 0; g < 4; ++g) {
+        gp_mw_sweep_params p{};
+        p.dir_z = g == 1 || g == 2; p.last = g >= 2;
+        p.nx = first.nx; p.nz = first.nz; p.dx = first.dx; p.dz = first.dz;
+        for (size_t stage = 0; stage < 3; ++stage) p.dt[stage] = kernel_infos[kSweepKernels * g + 3 * stage].p.miniweather.dt;
+        p.in = g % 2 ? (const float *)sweep_state_ : state;
+        p.out = g % 2 ? state : (float *)sweep_state_;
+        p.state = state; p.state_tmp = tmp; p.flux = first.flux; p.hydro = first.hydro;
+        sweeps_.push_back(p);
+    }
+    return Status::Succ;
 }
 
 // Slot order per operator is fixed by the builders in zoo.cpp.
@@ -409,6 +435,9 @@ Status Model::clear() {
     if (stage_) { gp_stage_destroy(stage_); stage_ = nullptr; }
     if (!loaded_) return Status::Succ;
     for (GPUdeviceptr p : storages) CUDA_RETURN_STATUS(gp_free(p));
+    if (sweep_state_) CUDA_RETURN_STATUS(gp_free(sweep_state_));
+    sweep_state_ = nullptr;
+    sweeps_.clear();
     storage_infos.clear(); layouts.clear(); kernel_infos.clear(); storages.clear(); storages_idx.clear();
     loaded_ = false;
     return Status::Succ;
@@ -464,31 +493,7 @@ Status Model::launch(size_t idx, GPUstream stream, int inject_at) {
     const bool fuse = fuse_launches_;
     if (fuse && k.fused_away) return Status::Succ;  // the next kernel's prologue does this one's work
     gp_preempt_ctx ctx{};
-    const gp_preempt_ctx *pc = nullptr;
-    if (k.preemptible) {
-        size_t n = k.args_ptr.size();
-        ctx.flag = (int *)*k.args_ptr[n - 2];
-        ctx.stop_index = (int *)*k.args_ptr[n - 1];
-        ctx.executed = (int *)k.executed;
-        ctx.kernel_id = k.kernel_id;
-        ctx.inject_at = inject_at;
-        ctx.max_workgroups = 0;
-        ctx.poll_every = poll_every_;
-        ctx.counter_groups = counter_groups_;
-        ctx.fresh = idx < fresh_.size() && fresh_[idx] ? (eager_tiles_ ? 2 : 1) : 0;
-        ctx.ckpt = ckpt_;
-        ctx.ckpt_bytes = ckpt_bytes_;
-        ctx.stamps = (unsigned long long *)stamps_;
-        if (done_offset_) {
-            ctx.done = (int *)((char *)k.executed + done_offset_);
-            ctx.done_launches = idx < launches_.size() ? launches_[idx] : 0;
-        }
-        if (started_) {
-            ctx.started_host = (int *)started_;
-            ctx.started_seq = launch_seq_ + 1;
-        }
-        pc = &ctx;
-    }
+    const gp_preempt_ctx *pc = preempt_ctx(idx, inject_at, ctx) ? &ctx : nullptr;
     gp_launch_info info{};
     int rc = GP_FAIL;
     switch (k.op) {
@@ -505,14 +510,60 @@ Status Model::launch(size_t idx, GPUstream stream, int inject_at) {
         case OpKind::Nop: break;
     }
     if (idx < fresh_.size()) fresh_[idx] = 0;  // launched (or refused): from here on only its counters know
-    if (idx < launches_.size() && rc == 0) ++launches_[idx];
-    if (pc && started_ && rc == 0) ++launch_seq_;
     CUDA_RETURN_STATUS(rc);
+    launched(idx, pc != nullptr, info);
+    return Status::Succ;
+}
+
+// what the launch of a preemptible kernel is handed; false: the kernel is not preemptible
+bool Model::preempt_ctx(size_t idx, int inject_at, gp_preempt_ctx &ctx) {
+    KernelInfo &k = kernel_infos[idx];
+    if (!k.preemptible) return false;
+    size_t n = k.args_ptr.size();
+    ctx.flag = (int *)*k.args_ptr[n - 2];
+    ctx.stop_index = (int *)*k.args_ptr[n - 1];
+    ctx.executed = (int *)k.executed;
+    ctx.kernel_id = k.kernel_id;
+    ctx.inject_at = inject_at;
+    ctx.max_workgroups = 0;
+    ctx.poll_every = poll_every_;
+    ctx.counter_groups = counter_groups_;
+    ctx.fresh = idx < fresh_.size() && fresh_[idx] ? (eager_tiles_ ? 2 : 1) : 0;
+    ctx.ckpt = ckpt_;
+    ctx.ckpt_bytes = ckpt_bytes_;
+    ctx.stamps = (unsigned long long *)stamps_;
+    if (done_offset_) {
+        ctx.done = (int *)((char *)k.executed + done_offset_);
+        ctx.done_launches = idx < launches_.size() ? launches_[idx] : 0;
+    }
+    if (started_) {
+        ctx.started_host = (int *)started_;
+        ctx.started_seq = launch_seq_ + 1;
+    }
+    return true;
+}
+
+void Model::launched(size_t idx, bool preemptible, const gp_launch_info &info) {
+    KernelInfo &k = kernel_infos[idx];
+    if (idx < launches_.size()) ++launches_[idx];
+    if (preemptible && started_) ++launch_seq_;
     k.total_blocks = info.total_tiles;
     k.fixed_claims = info.fixed_claims != 0;
     k.launch_params[0] = (uint32_t)info.grid; k.launch_params[1] = 1; k.launch_params[2] = 1;
     k.front_workgroups = info.front;
     k.launch_params[3] = (uint32_t)info.block; k.launch_params[4] = 1; k.launch_params[5] = 1;
+}
+
+Status Model::launch_sweep(size_t g, GPUstream stream) {
+    if (g >= sweeps_.size()) return Status::OutOfRange;
+    const size_t idx = g * kSweepKernels;
+    gp_preempt_ctx ctx{};
+    const bool preemptible = preempt_ctx(idx, -1, ctx);
+    gp_launch_info info{};
+    const int rc = gp_launch_miniweather_sweep(&sweeps_[g], preemptible ? &ctx : nullptr, stream, &info);
+    if (idx < fresh_.size()) fresh_[idx] = 0;
+    CUDA_RETURN_STATUS(rc);
+    launched(idx, preemptible, info);
     return Status::Succ;
 }
 

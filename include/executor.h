@@ -176,6 +176,8 @@ private:
     unsigned long long cal_ticks[2] = {0, 0};   // first and latest calibration: device ticks ...
     double cal_host_ns[2] = {0, 0};             // ... and the host clock at that moment
     int inject_kernel = -1, inject_claim = -1, inject_iteration = -2;
+    bool swept = false;  // the run under way was launched as sweeps (Model::launch_sweep)
+    Status launch_sweeps(size_t from_kernel, GPUstream stream);
     std::atomic<int> *lc_tasks = nullptr;
     std::atomic<int> *be_tasks = nullptr;
 };

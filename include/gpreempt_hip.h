@@ -386,6 +386,21 @@ typedef struct gp_miniweather_params {
 } gp_miniweather_params;
 int gp_launch_miniweather(const gp_miniweather_params *p, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info);
 
+/* A direction sweep of the time step in one launch: the three Runge-Kutta stages of all nine kernels (halo, fluxes,
+ * update, three times), with the bits they leave.  Reads `in`, writes the cells of `out` (laid out like state; neither
+ * may be the other).  What the nine kernels leave elsewhere is written as far as it outlives a step of four sweeps
+ * x, z, z, x with in / out = state / other, other / state, state / other, other / state:
+ *   halo of state and of state_tmp   an x sweep: the columns; a z sweep with `last`: the rows
+ *   state_tmp (second stage), flux   an x sweep with `last`; of flux, the top row by the z sweep with `last` */
+typedef struct gp_mw_sweep_params {
+    int dir_z, last, nx, nz;
+    float dt[3], dx, dz;  /* the three stages' time steps */
+    const float *in;
+    float *out, *state, *state_tmp, *flux;
+    const float *hydro;
+} gp_mw_sweep_params;
+int gp_launch_miniweather_sweep(const gp_mw_sweep_params *p, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info);
+
 /* One kernel of the graph workloads over a CSR graph (vertex_list: vertex_count+1 offsets,
  * edge_list: neighbour ids, both 64-bit as in the reference's files; weight_list: 32-bit edge
  * weights for SSSP).  Replaces the kernels of src/workloads/graphcompute.tr.cu: cc_kernel_coalesce

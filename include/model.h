@@ -147,6 +147,12 @@ public:
     // GPULaunchKernel); preemptible kernels take their flag and stop index from the by-reference
     // arguments added with batchAddParam.  inject_at is a test hook (-1 = off).
     Status launch(size_t idx, GPUstream stream, int inject_at = -1);
+    // The miniWeather step as its four direction sweeps, one launch each (gp_launch_miniweather_sweep).  Sweep `g` stands
+    // for kernels kSweepKernels * g on and uses the first one's index, counters and stop index; a run launches either
+    // the kernels or the sweeps, and resumes with what it was launched with.
+    static constexpr size_t kSweepKernels = 9;
+    bool has_sweeps() const { return !sweeps_.empty(); }
+    Status launch_sweep(size_t g, GPUstream stream);
     void set_poll_every(int n) { poll_every_ = n; }
     // The claim counters have just been cleared (or are about to be, earlier on the same stream):
     // until its next launch every kernel is known to have made no claim (gp_preempt_ctx::fresh).
@@ -196,6 +202,11 @@ private:
     int counter_groups_ = 1;
     int poll_every_ = 0;
     std::vector<char> fresh_;
+    std::vector<gp_mw_sweep_params> sweeps_;
+    GPUdeviceptr sweep_state_ = nullptr;  // what the first and third sweep write
+    Status plan_sweeps();
+    bool preempt_ctx(size_t idx, int inject_at, gp_preempt_ctx &ctx);
+    void launched(size_t idx, bool preemptible, const gp_launch_info &info);
     std::vector<int> launches_;           // per kernel: launches since the counters were cleared (gp_preempt_ctx::done_launches)
     size_t done_offset_ = 0;              // 0: no done counters
     GPUdeviceptr left_word_ = nullptr;

@@ -228,3 +228,30 @@ def test_unknown_options_are_refused(gp, ex_mod):
     for wl in ("miniweather@nx=2,nz=8", "miniweather@spec=4", "miniweather@nx=100000,nz=100000"):
         with pytest.raises(ex_mod.StatusError):
             ex_mod.Executor(wl)
+
+
+@pytest.mark.parametrize("nx,nz", [(4, 4), (5, 116), (116, 117), (117, 5), (128, 128), (233, 6), (15, 349), (349, 233)])
+@pytest.mark.parametrize("blp", [False, True])
+def test_sweeps_leave_what_the_kernels_leave(gp, ex_mod, nx, nz, blp):
+    """execute() runs a direction's nine kernels as one launch: the same bits in the state, its halo, the second
+    stage's state and the fluxes, around the 116 cells of a wavefront's stretch and the 16 columns of a strip"""
+    wl = f"miniweather@nx={nx},nz={nz}"
+    swept, listed = ex_mod.Executor(wl, blp=blp), ex_mod.Executor(wl, blp=blp)
+    if blp:
+        flag = gp.Flag()
+        swept.set_flag(flag)
+        listed.set_flag(flag)
+    rng = np.random.default_rng(nx * 1000 + nz)
+    x = f32(swept.read_storage("state")).reshape(4, nz + 4, nx + 4)
+    x += rng.normal(0, 1e-3, x.shape).astype(np.float32) * np.array([1, 10, 10, 100], np.float32)[:, None, None]
+    for ex in (swept, listed):
+        ex.set_input("state", x)
+        ex.set_input("state_tmp", x)
+    for _ in range(2):
+        swept.execute()
+        if blp:
+            listed.reset_counters()
+        for i in range(listed.kernel_num()):
+            listed.launch_kernel(i)
+        for a, b, name in zip(_arrays(swept), _arrays(listed), ("state", "state_tmp", "flux")):
+            assert np.array_equal(a, b), name

@@ -51,6 +51,21 @@ inline void set_poll_slices(BlpArgs *blp, int grid) {
         blp->poll_n[g] = ng > 1 && g < ng ? group_slice_begin(blp->total, g + 1, ng, grid) - group_slice_begin(blp->total, g, ng, grid) : 0;
 }
 
+// hipOccupancyMaxActiveBlocksPerMultiprocessor, asked once per thread for each kernel and shape: the answer does not
+// change, and the question costs a launch half a microsecond of host time.
+inline int occupancy_of(const void *kernel, int block, size_t lds_bytes, int *per_cu) {
+    struct Entry { const void *kernel; int block, per_cu; size_t lds; };
+    static thread_local Entry cache[256] = {};
+    Entry &e = cache[(((uintptr_t)kernel >> 4) ^ ((uintptr_t)kernel >> 12) ^ (lds_bytes >> 10)) & 255];
+    if (e.kernel != kernel || e.block != block || e.lds != lds_bytes) {
+        int n = 0;
+        GP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, block, lds_bytes));
+        e = Entry{kernel, block, n < 1 ? 1 : n, lds_bytes};
+    }
+    *per_cu = e.per_cu;
+    return GP_SUCC;
+}
+
 // Resolves the launch geometry of one preemptible kernel, as Model::add_block_preemption_param
 // does in the reference (src/model.cpp:366-396): total_block = sx*sy*sz; persistent grid =
 // min(total_block, resident workgroups the device can hold); a NULL context keeps one
@@ -78,8 +93,7 @@ int plan_launch(Kernel kernel, int block, size_t lds_bytes, int sx, int sy, int 
         GP_REQUIRE((ng & (ng - 1)) == 0 && ng <= 64, "counter_groups must be a power of two <= 64");
         blp->groups = ng;
         int per_cu = 0;
-        GP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, lds_bytes));
-        if (per_cu < 1) per_cu = 1;
+        if (int rc = occupancy_of((const void *)kernel, block, lds_bytes, &per_cu)) return rc;
         long resident = (long)per_cu * device_cus();
         if (ctx->max_workgroups > 0 && resident > ctx->max_workgroups) resident = ctx->max_workgroups;
         *grid = (int)(total < resident ? total : resident);

@@ -66,12 +66,14 @@ int plan_eltwise(const gp_eltwise_params *p, EltPlan *out) {
     GP_REQUIRE(p->a_stride % vec == 0 && p->out_stride % vec == 0 && (!p->b || p->b_stride % vec == 0), "eltwise strides");
     GP_REQUIRE(al16(p->a) && al16(p->out) && al16(p->b) && al16(p->scale) && al16(p->shift), "eltwise: 16-byte alignment");
     long items = p->rows * (p->cols / vec);
-    long tiles = (items + (long)NT * ELT_PER - 1) / ((long)NT * ELT_PER);
+    // (the chip holds eight workgroups of 256 threads per compute unit)
+    const int single = items <= 8L * NT * device_cus();
+    const long per = single ? NT : (long)NT * ELT_PER, tiles = (items + per - 1) / per;
     GP_REQUIRE(items < (1L << 31), "eltwise: too large (2^31 16-byte items at most)");
     *out = EltPlan{};
     out->op = OP_ELTWISE; out->dtype = p->dtype; out->sx = (int)tiles; out->sy = 1;
     const long bytes = p->rows * p->cols * (long)dtype_size(p->dtype) * (p->b ? 3 : 2);
-    out->u.elt = EltwiseArgs{*p, items, bytes > kStreamBytes};
+    out->u.elt = EltwiseArgs{*p, items, bytes > kStreamBytes, single};
     return GP_SUCC;
 }
 

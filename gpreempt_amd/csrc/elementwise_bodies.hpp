@@ -221,14 +221,22 @@ __device__ __forceinline__ void pool_tile_block2(const PoolArgs &a, TileIdx t) {
     T *out = (T *)p.out;
     const int h_first = hb * 4 - p.pad, w_first = wb * 4 - p.pad;  // input coordinate of the patch's corner
     u32x4 f[25];
+    // (row starts and column offsets once, an addition per load: with a product per load the kernel spent more time on
+    // its 25 addresses than on the loads)
+    const T *row[5];
+    long col_at[5];
+    const T *image = in + n * p.H * p.W * p.in_pix_stride + ch * VEC;
+#pragma unroll
+    for (int r = 0; r < 5; ++r) {
+        const int hi = h_first + r, wi = w_first + r;
+        const int hc = hi < 0 ? 0 : (hi >= p.H ? p.H - 1 : hi), wc = wi < 0 ? 0 : (wi >= p.W ? p.W - 1 : wi);
+        row[r] = image + (long)hc * p.W * p.in_pix_stride;
+        col_at[r] = wc * p.in_pix_stride;
+    }
 #pragma unroll
     for (int r = 0; r < 5; ++r) {
 #pragma unroll
-        for (int s = 0; s < 5; ++s) {
-            const int hi = h_first + r, wi = w_first + s;
-            const int hc = hi < 0 ? 0 : (hi >= p.H ? p.H - 1 : hi), wc = wi < 0 ? 0 : (wi >= p.W ? p.W - 1 : wi);
-            f[r * 5 + s] = *(const u32x4 *)(in + ((n * p.H + hc) * p.W + wc) * p.in_pix_stride + ch * VEC);
-        }
+        for (int s = 0; s < 5; ++s) f[r * 5 + s] = *(const u32x4 *)(row[r] + col_at[s]);
     }
     // column maxima of the three row triples a window can take, then the windows
 #pragma unroll
@@ -271,11 +279,20 @@ __device__ __forceinline__ void pool_tile(const PoolArgs &a, TileIdx t) {
 #pragma unroll
             for (int i = 0; i < VEC; ++i) acc[i] = 0.f;
             const T *src = in + pix * p.H * p.W * p.in_pix_stride + ch * VEC;
-            for (int i = 0; i < p.H * p.W; ++i) {
-                float f[VEC];
-                VecIO<T>::load(src + (long)i * p.in_pix_stride, f);
+            // (sixteen pixels' loads in flight; they are added in order all the same)
+            constexpr int AHEAD = 16;
+            const int pixels = p.H * p.W;
+            for (int i = 0; i < pixels; i += AHEAD) {
+                out_u32x4 raw[AHEAD];
 #pragma unroll
-                for (int j = 0; j < VEC; ++j) acc[j] += f[j];
+                for (int u = 0; u < AHEAD; ++u) raw[u] = ld_raw128<false>(src + (long)(i + u < pixels ? i + u : i) * p.in_pix_stride);
+#pragma unroll
+                for (int u = 0; u < AHEAD; ++u) {
+                    float f[VEC];
+                    VecIO<T>::unpack(raw[u], f);
+#pragma unroll
+                    for (int j = 0; j < VEC; ++j) acc[j] = i + u < pixels ? acc[j] + f[j] : acc[j];
+                }
             }
             float inv = 1.f / (float)(p.H * p.W);
 #pragma unroll
@@ -298,14 +315,28 @@ __device__ __forceinline__ void pool_tile(const PoolArgs &a, TileIdx t) {
             bool in_range[R * S];
             // every tap is loaded, from a clamped coordinate when it lies outside the image, and
             // dropped afterwards: no branch sits between the loads, so all R*S are in flight at once
+            // (row starts and column offsets once: see pool_tile_block2)
+            const T *row[R], *image = in + n * p.H * p.W * p.in_pix_stride + ch * VEC;
+            long col_at[S];
+            bool row_in[R], col_in[S];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int hi = ho * p.stride - p.pad + r;
+                row_in[r] = (unsigned)hi < (unsigned)p.H;
+                row[r] = image + (long)(hi < 0 ? 0 : (hi >= p.H ? p.H - 1 : hi)) * p.W * p.in_pix_stride;
+            }
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                const int wi = wo * p.stride - p.pad + s;
+                col_in[s] = (unsigned)wi < (unsigned)p.W;
+                col_at[s] = (wi < 0 ? 0 : (wi >= p.W ? p.W - 1 : wi)) * p.in_pix_stride;
+            }
 #pragma unroll
             for (int r = 0; r < R; ++r) {
 #pragma unroll
                 for (int s = 0; s < S; ++s) {
-                    const int hi = ho * p.stride - p.pad + r, wi = wo * p.stride - p.pad + s;
-                    in_range[r * S + s] = (unsigned)hi < (unsigned)p.H && (unsigned)wi < (unsigned)p.W;
-                    const int hc = hi < 0 ? 0 : (hi >= p.H ? p.H - 1 : hi), wc = wi < 0 ? 0 : (wi >= p.W ? p.W - 1 : wi);
-                    VecIO<T>::load(in + ((n * p.H + hc) * p.W + wc) * p.in_pix_stride + ch * VEC, f[r * S + s]);
+                    in_range[r * S + s] = row_in[r] & col_in[s];
+                    VecIO<T>::load(row[r] + col_at[s], f[r * S + s]);
                 }
             }
 #pragma unroll
@@ -348,9 +379,11 @@ __global__ __launch_bounds__(NT) void pool_kernel(PoolArgs a, BlpArgs blp) {
 }
 
 // ---- elementwise ---------------------------------------------------------------------------
-// item = (row, 16-byte chunk); tile = 1024 items (4 per thread, strided by 256 for coalescing).
+// item = (row, 16-byte chunk); tile = 1024 items (4 per thread, strided by 256 for coalescing), or 256 (a.single) while
+// that many workgroups still run side by side: a small problem is one trip to memory, and what lengthens it is whatever
+// a thread does one after the other.
 constexpr int ELT_PER = 4;
-struct EltwiseArgs { gp_eltwise_params p; long items; int stream; };
+struct EltwiseArgs { gp_eltwise_params p; long items; int stream, single; };
 template <typename T>
 __device__ __forceinline__ void eltwise_finish(const gp_eltwise_params &p, int ch, float (&a)[VecIO<T>::VEC]) {
     constexpr int VEC = VecIO<T>::VEC;
@@ -405,8 +438,45 @@ __device__ __forceinline__ void eltwise_full_tile(const EltwiseArgs &a, unsigned
         st_raw128<NTH>((T *)p.out + row[u] * p.out_stride + ch[u] * VEC, VecIO<T>::pack(x));
     }
 }
+// one item per thread: operand, addend, scale and shift are requested together, and nothing branches in front of them
+// (an item beyond the end reads the last one).  784 x 1024 fp16 with scale, shift and ReLU: 2.4 us per launch; through the
+// tiles of 1024, whose bounds checks made every load wait for the one before, 4.3.
+template <typename T>
+__device__ __forceinline__ void eltwise_single_tile(const EltwiseArgs &a, unsigned base) {
+    const gp_eltwise_params &p = a.p;
+    constexpr int VEC = VecIO<T>::VEC;
+    const unsigned chunks = (unsigned)(p.cols / VEC), items = (unsigned)a.items;
+    const unsigned mine = base + threadIdx.x, item = mine < items ? mine : items - 1;
+    const unsigned row = item / chunks, ch = item - row * chunks;
+    out_u32x4 rb{}, rs{}, rt{};
+    const out_u32x4 ra = ld_raw128<false>((const T *)p.a + (long)row * p.a_stride + ch * VEC);
+    if (p.b) rb = ld_raw128<false>((const T *)p.b + (long)row * p.b_stride + ch * VEC);
+    if (p.scale) rs = ld_raw128<false>((const T *)p.scale + ch * VEC);
+    if (p.shift) rt = ld_raw128<false>((const T *)p.shift + ch * VEC);
+    float x[VEC], y[VEC];
+    VecIO<T>::unpack(ra, x);
+    if (p.b) {
+        VecIO<T>::unpack(rb, y);
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) x[j] += y[j];
+    }
+    if (p.scale) {
+        VecIO<T>::unpack(rs, y);
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) x[j] *= y[j];
+    }
+    if (p.shift) {
+        VecIO<T>::unpack(rt, y);
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) x[j] += y[j];
+    }
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) x[j] = act_f(x[j], p.act);
+    if (mine < items) st_raw128<false>((T *)p.out + (long)row * p.out_stride + ch * VEC, VecIO<T>::pack(x));
+}
 template <typename T>
 __device__ __forceinline__ void eltwise_tile(const EltwiseArgs &a, TileIdx t) {
+    if (a.single) { eltwise_single_tile<T>(a, (unsigned)t.x * NT); return; }
     const gp_eltwise_params &p = a.p;
     const long items = a.items;
     constexpr int VEC = VecIO<T>::VEC;

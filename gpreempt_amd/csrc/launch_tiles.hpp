@@ -20,9 +20,12 @@ static int launch_tiles(KernelSet<Kernel> ks, int sx, int sy, const gp_preempt_c
     const long tiles = (long)sx * sy;
     const int batch = (int)std::min<long>(max_batch, std::max<long>(1, tiles / (32L * device_cus())));
     if (lds_bytes > 48 * 1024) {
-        GP_HIP(hipFuncSetAttribute((const void *)ks.any, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
-        GP_HIP(hipFuncSetAttribute((const void *)ks.plain, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
-        GP_HIP(hipFuncSetAttribute((const void *)ks.fixed, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
+        static thread_local size_t allowed = 0;  // (of this kernel: one instantiation of this function per kernel type,
+        static thread_local const void *of = nullptr;  // and the kernels of one type share it)
+        if (of != (const void *)ks.any || allowed < lds_bytes) {
+            for (Kernel k : {ks.any, ks.plain, ks.fixed}) GP_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
+            of = (const void *)ks.any; allowed = lds_bytes;
+        }
     }
     // planned for the general form; the special ones need no more resources
     int rc = plan_launch(ks.any, block, lds_bytes, sx, sy, 1, ctx, &blp, &grid, info, batch, batch == 1 ? 4 : 1);

@@ -502,3 +502,25 @@ def test_launches_report_their_start_and_a_marker_reports_the_end(gp):
     stream.sync()
     want = np.maximum(O.gemm_bias_act(A, B, None, None, gp.ACT_NONE, b_is_nk=True) + A[:, :1], 0)
     assert rel_err(dY.download(gp.F16, (M, N)), want) < TOL["f16"]
+
+
+@pytest.mark.parametrize("dt", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("rows,chunks", [(1, 1), (1, 255), (257, 1), (8, 32), (19, 27), (4096, 128), (4097, 128)])
+def test_eltwise_at_the_edges_of_its_tiles(gp, dt, rows, chunks):
+    """one item per thread up to 2^19 items of 16 bytes, four beyond: last items of a tile, one tile, the change-over"""
+    dtype = gp.DTYPE_BY_NAME[dt]
+    cols = chunks * (4 if dt == "f32" else 8)
+    rng = np.random.default_rng(rows * chunks)
+    a, b, sc, sh = (gp.from_storage(gp.to_storage(rng.uniform(-1, 1, s).astype(np.float32), dtype), dtype) for s in ((rows, cols), (rows, cols), (cols,), (cols,)))
+    da, db, ds, dh = (gp.DevBuf.from_array(x, dtype) for x in (a, b, sc, sh))
+    do = gp.DevBuf(da.nbytes + 64)
+    do.fill32(0x55AA55AA)
+    st = gp.BlpState(1, gp.Flag(), 32)
+    for ctx in (None, st.ctx(fresh=1)):
+        gp.launch("gp_launch_eltwise", gp.EltwiseParams(dtype, rows, cols, da.ptr, cols, db.ptr, cols, ds.ptr, dh.ptr, do.ptr, cols, gp.ACT_RELU), ctx)
+        gp.check(gp.lib().gp_stream_sync(None))
+        raw = do.download()
+        got = gp.from_storage(raw[:da.nbytes].copy(), dtype).reshape(rows, cols)
+        want = np.maximum((a.astype(np.float32) + b) * sc + sh, 0)
+        assert np.abs(got - want).max() <= {"f32": 1e-6, "f16": 2e-3, "bf16": 2e-2}[dt]
+        assert (raw[da.nbytes:].view(np.uint32) == 0x55AA55AA).all()  # nothing behind the end

@@ -70,30 +70,24 @@ struct LnWideKernel {
         const int l32 = lane & 31, half = lane >> 5;
         const int m0 = t.y * BM, n0 = t.x * BN;
         const T *A = (const T *)g.A, *B = (const T *)g.B;
-        const T *zero = (const T *)g_zero_page;
         const int KT = g.K / BK;                        // blocks along K (K is a multiple of BK: checked by the planner)
         const int NS = (KT + KB - 1) / KB;              // stages of B
 
         // ---- B loader slots, as in WideKernel ---------------------------------------------------
         const int rig = lane >> 3, cpos = lane & 7;
-        const T *base[LPW];
-        bool row_ok[LPW];
-        int kc[LPW];
+        const u32x4 rsrc_b = buffer_of(B);
+        unsigned off[LPW];
 #pragma unroll
         for (int j = 0; j < LPW; ++j) {
             const int r = (wv * LPW + j) * 8 + rig;
-            kc[j] = (cpos ^ ((r >> 1) & 7)) * VEC;
-            row_ok[j] = n0 + r < g.N;
-            base[j] = B + (long)(n0 + r) * g.ldb + kc[j];
+            off[j] = n0 + r < g.N ? ((unsigned)(n0 + r) * (unsigned)g.ldb + (unsigned)(cpos ^ ((r >> 1) & 7)) * VEC) * (unsigned)sizeof(T) : kBufferEnd;
         }
         auto issue = [&](int s) {
             const int k0 = (s * KB + kb) * BK;
             const unsigned sbase = lds0 + ((unsigned)s % STAGES) * STAGE_BYTES + (unsigned)kb * B_BLK_BYTES;
 #pragma unroll
-            for (int j = 0; j < LPW; ++j) {
-                const bool ok = row_ok[j] & (k0 < g.K);   // whole blocks past the last one, when the stage is not full
-                load_lds16(ok ? base[j] + k0 : zero, sbase + (unsigned)((wv * LPW + j) * 8 * RB));
-            }
+            for (int j = 0; j < LPW; ++j)  // (whole blocks past the last one, when the stage is not full: zeros)
+                load_lds16_buffer(rsrc_b, k0 < g.K ? off[j] : kBufferEnd, (unsigned)k0 * (unsigned)sizeof(T), sbase + (unsigned)((wv * LPW + j) * 8 * RB));
         };
 
         __syncthreads();  // the previous tile of this workgroup may still be reading LDS

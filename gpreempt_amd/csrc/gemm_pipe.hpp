@@ -37,6 +37,20 @@ __device__ __forceinline__ void load_lds16(const void *gptr, unsigned lds_byte) 
                  : "memory", "m0");
 }
 
+// The same through a buffer descriptor: lane i reads 16 bytes at the descriptor's base + off + soff.  A lane whose `off`
+// is kBufferEnd reads zeros (the descriptor's range ends there, and soff is not negative).
+constexpr unsigned kBufferEnd = 0x80000000u;
+__device__ __forceinline__ u32x4 buffer_of(const void *base) {  // (a raw buffer of 2 GB: what the planners allow an operand to span)
+    const unsigned long long a = (unsigned long long)base;
+    return u32x4{(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)a), (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(a >> 32)), kBufferEnd, 0x00027000u};
+}
+__device__ __forceinline__ void load_lds16_buffer(u32x4 rsrc, unsigned off, unsigned soff, unsigned lds_byte) {
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+                 :
+                 : "v"(off), "s"(rsrc), "s"(soff), "s"(lds_byte)
+                 : "memory", "m0");
+}
+
 // Reads a word that a load-to-LDS has written.  The pointer must carry the LDS address space: through a plain
 // `volatile int *` the read is a flat load, which counts as a vector-memory operation as well, and the wait that the
 // compiler puts behind it (vmcnt 0) also waits for every operand load the wavefront has in flight.

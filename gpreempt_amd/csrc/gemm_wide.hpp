@@ -197,18 +197,23 @@ struct WideKernel {
             offa = t.z * g.stride_a; offb = t.z * g.stride_b; offc = t.z * g.stride_c;
         }
         const T *A = (const T *)g.A + offa, *B = (const T *)g.B + offb;
-        const T *zero = (const T *)g_zero_page;
 
         // ---- loader slots: every wavefront fetches LPW_A row groups of A and LPW_B of B of its block (which
         // kind a slot is is known at compile time: no branches in the stage's load sequence) ------
         // lane -> (row in the group, chunk position); the swizzle is applied on the source side:
-        // the lane at position cpos of row r fetches chunk cpos ^ ((r >> 1) & 7) of that row
+        // the lane at position cpos of row r fetches chunk cpos ^ ((r >> 1) & 7) of that row.
+        // The loads go through buffer descriptors: a lane's row and chunk are one 32-bit offset that never changes, the
+        // position in K (CONV: the tap) is a scalar, and a lane with nothing to fetch has an offset beyond the
+        // descriptor's end, which the hardware answers with zeros.  Sixteen wavefronts issue a stage's loads, four to a
+        // SIMD: with 64-bit addresses, selects and a page of zeros a stage of a 3 x 3 layer cost as much in vector
+        // instructions as its loads take.
         const int rig = lane >> 3, cpos = lane & 7;
         const int hw = CONV ? g.Ho * g.Wo : 1, ntap_rows = CONV ? g.K / (g.Cin * g.S) : 0;
         const bool small = g.M < kSmallDivLimit;
         const float rcp_hw = 1.0f / (float)hw, rcp_wo = CONV ? 1.0f / (float)g.Wo : 1.0f;
-        const T *base[LPW];    // the lane's row and chunk at k = 0 (CONV, A rows: its window's origin, which may lie outside the image)
-        bool row_ok[LPW];
+        // (CONV: offsets count from the origin of the window of output pixel (0, 0), which lies in front of the image by the padding)
+        const u32x4 rsrc_a = buffer_of(CONV ? A - (long)(g.ph * g.W + g.pw) * g.lda : A), rsrc_b = buffer_of(B);
+        unsigned off[LPW];     // the lane's row and chunk at k = 0, in bytes
         int kc[LPW];           // the lane's chunk offset in elements
         unsigned taps[CONV ? LPW : 1];  // CONV, A rows: bit t set = tap t of the row's window is inside the image
 #pragma unroll
@@ -219,22 +224,15 @@ struct WideKernel {
             kc[j] = (cpos ^ ((r >> 1) & 7)) * VEC;
             if (is_a && CONV) {
                 const int m = m0 + r;
-                row_ok[j] = m < g.M;
-                const int mm = row_ok[j] ? m : 0;
+                const bool in = m < g.M;
+                const int mm = in ? m : 0;
                 const int n = small ? small_div(mm, hw, rcp_hw) : mm / hw, rem = mm - n * hw;
                 const int ho = small ? small_div(rem, g.Wo, rcp_wo) : rem / g.Wo, wo = rem - ho * g.Wo;
-                const int h0 = ho * g.sh - g.ph, w0 = wo * g.sw - g.pw;
-                base[j] = A + (long)((n * g.H + h0) * g.W + w0) * g.lda + kc[j];  // (pixel indices fit an int: checked by the planner)
-                const unsigned mask = row_ok[j] ? window_tap_mask(h0, w0, g.H, g.W, ntap_rows, g.S) : 0u;
-                taps[CONV ? j : 0] = mask;
-            } else if (is_a) {
-                const int m = m0 + r;
-                row_ok[j] = m < g.M;
-                base[j] = A + (long)m * g.lda + kc[j];
+                off[j] = ((unsigned)((n * g.H + ho * g.sh) * g.W + wo * g.sw) * (unsigned)g.lda + (unsigned)kc[j]) * (unsigned)sizeof(T);
+                taps[CONV ? j : 0] = in ? window_tap_mask(ho * g.sh - g.ph, wo * g.sw - g.pw, g.H, g.W, ntap_rows, g.S) : 0u;
             } else {
-                const int n = n0 + r;
-                row_ok[j] = n < g.N;
-                base[j] = B + (long)n * g.ldb + kc[j];
+                const int x = (is_a ? m0 : n0) + r;
+                off[j] = x < (is_a ? g.M : g.N) ? ((unsigned)x * (unsigned)(is_a ? g.lda : g.ldb) + (unsigned)kc[j]) * (unsigned)sizeof(T) : kBufferEnd;
             }
         }
         const int KT = (g.K + BK - 1) / BK;             // blocks along K
@@ -251,19 +249,19 @@ struct WideKernel {
             const int k0 = (s * KB + kb) * BK;          // first K element of this wavefront group's block
             const unsigned sbase = lds0 + ((unsigned)s % STAGES) * STAGE_BYTES + (unsigned)kb * BLK_BYTES;
             const unsigned tap_bit = (k0 < g.K && nx_tap < 32) ? 1u << nx_tap : 0u;  // blocks past K have no tap
-            const int tap_off = (nx_r * g.W + nx_s) * (int)g.lda + nx_ci;  // elements from the window's origin
+            const unsigned tap_off = (unsigned)((nx_r * g.W + nx_s) * (int)g.lda + nx_ci) * (unsigned)sizeof(T);
+            const bool whole = k0 + BK <= g.K;          // (uniform) the block's K elements all exist
 #pragma unroll
             for (int j = 0; j < LPW; ++j) {
                 const int gi = group_of(wv, j);
                 if (CONV && j < LPW_A) {
-                    // taps outside the image, rows outside the problem and blocks past K come from the zero page
-                    const bool ok = (taps[CONV ? j : 0] & tap_bit) != 0;
-                    load_lds16(ok ? base[j] + tap_off : zero, sbase + (unsigned)(gi * 8 * RB));
+                    // taps outside the image, rows outside the problem and blocks past K have nothing to fetch
+                    load_lds16_buffer(rsrc_a, (taps[CONV ? j : 0] & tap_bit) ? off[j] : kBufferEnd, tap_off, sbase + (unsigned)(gi * 8 * RB));
                 } else {
-                    // rows outside the problem and K-chunks past K (also whole blocks past the last one,
-                    // when the stage is not full) come from the zero page
-                    const bool ok = row_ok[j] & (k0 + kc[j] < g.K);
-                    load_lds16(ok ? base[j] + k0 : zero, sbase + (unsigned)(gi * 8 * RB));
+                    // (nor have rows outside the problem and K-chunks past K, also whole blocks past the last one when
+                    // the stage is not full)
+                    const unsigned at = whole || k0 + kc[j] < g.K ? off[j] : kBufferEnd;
+                    load_lds16_buffer(j < LPW_A ? rsrc_a : rsrc_b, at, (unsigned)k0 * (unsigned)sizeof(T), sbase + (unsigned)(gi * 8 * RB));
                 }
             }
             if (CONV) {
@@ -319,17 +317,31 @@ struct WideKernel {
             }
             if (kb >= G) continue;  // (uniform) the other wavefronts only fetch
             const int stage = (int)((unsigned)s % STAGES);
+            // fp32: every block's fragments are asked for before the first is multiplied (a block is four MFMAs of 64 cycles
+            // then, in a chain that also waited for LDS once per block: 3 x 3 at 7 x 7 x 512 35.2 -> 32.5 us).  The 16-bit
+            // bodies read as they go: their blocks are one MFMA, and 128 x 768 x 3072 took 2 % longer.
+            constexpr int AHEAD = sizeof(T) == 4 ? KB : 1;
+            u32x4 fa[AHEAD][MI], fb[AHEAD][NI];
+            auto read = [&](int slot, int b) {
+#pragma unroll
+                for (int i = 0; i < MI; ++i) fa[slot][i] = frag(stage, b, 0, i * 32 + l32, wv * 2 + half);
+#pragma unroll
+                for (int j = 0; j < NI; ++j) fb[slot][j] = frag(stage, b, A_BYTES, j * 32 + l32, wv * 2 + half);
+            };
+            if constexpr (AHEAD > 1) {
+#pragma unroll
+                for (int b = 0; b < KB; ++b) read(b, b);
+            }
 #pragma unroll
             for (int b = 0; b < KB; ++b) {
                 // a block past the last one holds zeros; it is skipped, not multiplied, so that the sum
                 // has the bits of a K loop that ends at the last block
                 if (s * KB + b >= KT) break;
+                if constexpr (AHEAD == 1) read(0, b);
 #pragma unroll
                 for (int q = 0; q < BPW; ++q) {
-                    const int blk = kb + q * G, i = blk / NI, j = blk % NI;
-                    const u32x4 fa = frag(stage, b, 0, i * 32 + l32, wv * 2 + half);
-                    const u32x4 fb = frag(stage, b, A_BYTES, j * 32 + l32, wv * 2 + half);
-                    Elem<T>::mma(fa, fb, acc[q]);
+                    const int blk = kb + q * G;
+                    Elem<T>::mma(fa[AHEAD > 1 ? b : 0][blk / NI], fb[AHEAD > 1 ? b : 0][blk % NI], acc[q]);
                 }
             }
         }

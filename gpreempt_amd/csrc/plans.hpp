@@ -21,6 +21,8 @@ struct MatPlan {
     int sx, sy;        // tile grid (x over N, y over M, z = batch)
     int order;         // tile order handed to the dispatcher: 0 = x fastest, 1 = y fastest, G >= 2 = bands of G tile rows
     size_t lds_bytes;
+    int ring;          // stages of the operand ring of the 64 x 64 and 128 x 128 bodies: 2, or 0 for the body's own depth
+    int rounds;        // rounds of workgroups a preemptible launch may take with a workgroup per claim; 0: the launcher's own number
 };
 
 enum EltOp { OP_MAT = 0, OP_LAYOUT, OP_POOL, OP_ELTWISE, OP_SOFTMAX, OP_LAYERNORM, OP_EMBED, OP_COPY, OP_ATTENTION };

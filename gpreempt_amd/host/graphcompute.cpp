@@ -370,16 +370,21 @@ Status Workload::queue(const std::vector<gp_graph_iter_params> &list, int report
     return report_before_last ? Status::Succ : report(stream, env);
 }
 
+// (spinning on the word: a blocked thread wakes up tens of microseconds late, a query of the stream costs microseconds)
+Status Workload::await_word(GPUstream stream) {
+    for (unsigned spins = 1; __atomic_load_n(&report_[0], __ATOMIC_ACQUIRE) != report_seq_; ++spins) {
+        if (spins % (1u << 16)) continue;
+        int idle = 0;
+        GC_CHECK(gp_stream_query(stream, &idle));  // an error of the device ends the wait
+    }
+    return Status::Succ;
+}
+
 // Waits for the last report.  A launch that was stopped is relaunched, and the ones behind it with it (they left when
 // they found the stop recorded); `first` is the first launch the report is about.
 Status Workload::await_report(int first, GPUstream stream, const PreemptEnv *env) {
     for (;;) {
-        // (spinning on the word: a blocked thread wakes up tens of microseconds late, a query of the stream costs microseconds)
-        for (unsigned spins = 1; __atomic_load_n(&report_[0], __ATOMIC_ACQUIRE) != report_seq_; ++spins) {
-            if (spins % (1u << 16)) continue;
-            int idle = 0;
-            GC_CHECK(gp_stream_query(stream, &idle));  // an error of the device ends the wait
-        }
+        RETURN_STATUS(await_word(stream));
         const int stop = (int)report_[1];
         if (!env || stop < 0) return Status::Succ;
         RETURN_STATUS(wait_turn(stream, env));
@@ -470,7 +475,13 @@ Status Workload::compute(GPUstream stream, const PreemptEnv *env) {
         unsigned sampled = 0;
         while (iterations_ < (int)last_of.size() && last_of[iterations_] < known) {
             const volatile unsigned *w = words(last_of[iterations_++]);
-            if (w[0] == 0) return Status::Succ;
+            if (w[0] == 0) {
+                // The launches behind it find that out for themselves and leave, each by the word of the launch before
+                // it: a run that came after them on another stream would clear those words under them.  So they are
+                // waited for here, which is what a blocking call promises anyway.
+                if (tail) { RETURN_STATUS(report(stream, env)); RETURN_STATUS(await_word(stream)); }
+                return Status::Succ;
+            }
             sampled = w[1];
         }
         if (iterations_ >= max_iter) return Status::Succ;

@@ -54,7 +54,8 @@ public:
     // kind: "cc" | "bfs" | "pagerank" | "sssp"; nullptr for anything else (or sssp without weights)
     static std::unique_ptr<Workload> create(const std::string &kind, const CsrGraph &g);
     ~Workload();
-    // Runs the algorithm to convergence on `stream` (blocking).  env == nullptr: not preemptible.
+    // Runs the algorithm to convergence on `stream` (blocking: nothing of it is queued or running when this returns).
+    // env == nullptr: not preemptible.
     Status compute(GPUstream stream, const PreemptEnv *env);
 
     // results: "comp" (u64 per vertex), "label" (u32 BFS level), "value" (f32 PageRank), "cost" (u32 distance)
@@ -77,6 +78,7 @@ private:
     Status queue(const std::vector<gp_graph_iter_params> &list, int report_before_last, GPUstream stream, const PreemptEnv *env);
     Status launch_slot(int i, bool fresh, GPUstream stream, const PreemptEnv *env);
     Status report(GPUstream stream, const PreemptEnv *env);
+    Status await_word(GPUstream stream);
     Status await_report(int first, GPUstream stream, const PreemptEnv *env);
     const volatile unsigned *words(int i) const { return report_ + 2 + 2 * (i % kRing); }
     Status wait_turn(GPUstream stream, const PreemptEnv *env);

@@ -6,6 +6,7 @@
 #include <chrono>
 #include <cstdio>
 #include <cstring>
+#include <deque>
 #include <thread>
 
 #include "numeric.h"
@@ -326,7 +327,7 @@ Status Workload::run_kernels(const std::vector<int> &kernels, GPUstream stream, 
 }
 
 Status Workload::launch_slot(int i, bool fresh, GPUstream stream, const PreemptEnv *env) {
-    gp_graph_iter_params p = queued_[i];
+    gp_graph_iter_params p = queued_[i % kRing];
     int *slot = (int *)ring_ + slot_ints_ * (i % kRing);
     p.changed = (unsigned *)slot;
     if (p.prev_changed) p.prev_changed = (const unsigned *)((int *)ring_ + slot_ints_ * ((i - (int)(uintptr_t)p.prev_changed) % kRing));
@@ -358,8 +359,8 @@ Status Workload::queue(const std::vector<gp_graph_iter_params> &list, int report
         GC_CHECK(gp_malloc(&ring_, slot_ints * kRing * sizeof(int)));
         slot_ints_ = slot_ints;
     }
-    const int first = (int)queued_.size(), count = (int)list.size();
-    queued_.insert(queued_.end(), list.begin(), list.end());
+    const int first = submitted_, count = (int)list.size();
+    for (const gp_graph_iter_params &p : list) queued_[submitted_++ % kRing] = p;
     const int at = first % kRing, here = std::min(count, kRing - at);
     GC_CHECK(gp_fill32_async((int *)ring_ + slot_ints_ * at, 0, slot_ints_ * here, stream));
     GC_CHECK(gp_fill32_async(ring_, 0, slot_ints_ * (count - here), stream));
@@ -388,9 +389,9 @@ Status Workload::await_report(int first, GPUstream stream, const PreemptEnv *env
         const int stop = (int)report_[1];
         if (!env || stop < 0) return Status::Succ;
         RETURN_STATUS(wait_turn(stream, env));
-        int from = (int)queued_.size() - 1;
+        int from = submitted_ - 1;
         while (from > first && from % kRing != stop) --from;
-        for (int i = from; i < (int)queued_.size(); ++i) RETURN_STATUS(launch_slot(i, false, stream, env));
+        for (int i = from; i < submitted_; ++i) RETURN_STATUS(launch_slot(i, false, stream, env));
         RETURN_STATUS(report(stream, env));
     }
 }
@@ -418,7 +419,7 @@ gp_graph_iter_params Workload::params(int kernel) const {
 Status Workload::compute(GPUstream stream, const PreemptEnv *env) {
     if (!row_ || (env && env->inject_kernel >= 0 && env->inject_iteration >= -1)) return compute_stepwise(stream, env);
     iterations_ = 0;
-    queued_.clear();
+    submitted_ = 0;
     if (kind_ == "cc") {
         iterations_ = 3;  // the passes behind the set-up one
         RETURN_STATUS(queue({params(GP_GRAPH_IT_CC_INIT), params(GP_GRAPH_IT_CC_FLATTEN), params(GP_GRAPH_IT_CC_LINK), params(GP_GRAPH_IT_CC_LABEL)}, 0, stream, env));
@@ -427,7 +428,10 @@ Status Workload::compute(GPUstream stream, const PreemptEnv *env) {
     const bool bfs = kind_ == "bfs", pagerank = kind_ == "pagerank";
     const int max_iter = pagerank ? 100 : 1 << 30;  // graphcompute.h:82
     std::vector<gp_graph_iter_params> list{params(bfs ? GP_GRAPH_IT_BFS_INIT : pagerank ? GP_GRAPH_IT_PR_INIT : GP_GRAPH_IT_SSSP_INIT)};
-    std::vector<int> last_of;  // by iteration: its last launch, whose word says whether it changed anything
+    // of the iterations whose outcome is not known yet (iterations_ on): the last launch, whose word says whether it changed
+    // anything.  Nothing is kept of the others: a path of a million vertices takes as many iterations.
+    std::deque<int> last_of;
+    int next_first = 0;  // the launch behind the last known iteration
     GPUdeviceptr share = delta_, other = share_;
     float *gained = (float *)gained_, *next_gained = gained + (gained ? n_ : 0);
     bool push = false, pushing = false;  // wanted; the shares of the iteration before have been pushed
@@ -436,8 +440,8 @@ Status Workload::compute(GPUstream stream, const PreemptEnv *env) {
     int batch = bfs ? 8 : 16;
     const int ahead = bfs ? 1 : 2;
     for (;;) {
-        const int upto = std::min(max_iter, iterations_ + batch), first = (int)queued_.size();
-        for (int it = (int)last_of.size(); it < upto; ++it) {
+        const int upto = std::min(max_iter, iterations_ + batch), first = submitted_;
+        for (int it = iterations_ + (int)last_of.size(); it < upto; ++it) {
             gp_graph_iter_params p = params(bfs ? GP_GRAPH_IT_BFS : pagerank ? GP_GRAPH_IT_PR : GP_GRAPH_IT_SSSP);
             p.level = (unsigned)it;
             if (it & 1) std::swap(p.active, p.next_active);
@@ -470,11 +474,14 @@ Status Workload::compute(GPUstream stream, const PreemptEnv *env) {
         }
         const int tail = upto == max_iter ? 0 : std::min(ahead, (int)list.size() - 1);
         RETURN_STATUS(queue(list, tail, stream, env));
-        RETURN_STATUS(await_report(iterations_ ? last_of[iterations_ - 1] + 1 : 0, stream, env));
-        const int known = (int)queued_.size() - tail;
+        RETURN_STATUS(await_report(next_first, stream, env));
+        const int known = submitted_ - tail;
         unsigned sampled = 0;
-        while (iterations_ < (int)last_of.size() && last_of[iterations_] < known) {
-            const volatile unsigned *w = words(last_of[iterations_++]);
+        while (!last_of.empty() && last_of.front() < known) {
+            const volatile unsigned *w = words(last_of.front());
+            next_first = last_of.front() + 1;
+            last_of.pop_front();
+            ++iterations_;
             if (w[0] == 0) {
                 // The launches behind it find that out for themselves and leave, each by the word of the launch before
                 // it: a run that came after them on another stream would clear those words under them.  So they are

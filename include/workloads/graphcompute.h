@@ -103,7 +103,8 @@ private:
     static constexpr int kRing = 64;
     GPUdeviceptr ring_ = nullptr;                    // device: per slot two convergence words and the claim counters, a line apart
     size_t slot_ints_ = 0;
-    std::vector<gp_graph_iter_params> queued_;       // launches of this run by number; the last kRing of them matter
+    gp_graph_iter_params queued_[kRing];             // the last kRing launches of this run: number i is in slot i % kRing
+    int submitted_ = 0;                              // how many there have been
     volatile unsigned *report_ = nullptr;            // pinned, coherent: sequence number, stop index, words of every slot
     void *report_dev_ = nullptr;
     unsigned report_seq_ = 0;

@@ -167,9 +167,25 @@ static void check_nothing_left_behind() {
     g_delay_us = 0;
 }
 
+// a run of many iterations keeps as much as a short one
+static void check_long_run_keeps_nothing() {
+    auto w = GraphCompute::Workload::create("bfs", path_graph(64));
+    const GraphCompute::PreemptEnv env = env_of();
+    const int iterations = 100000;
+    g_ran.reserve(iterations + 64);
+    gp_stream_s s;
+    run("bfs", 100, &s, &env, *w);
+    const long before = g_live;
+    g_peak = before;
+    run("bfs", iterations - 1, &s, &env, *w);
+    // (what the fake device has queued at one time, and the loop's own lists)
+    CHECK(g_peak - before < 256 << 10, "%ld bytes more in use during %d iterations", g_peak.load() - before, iterations);
+}
+
 int main(int argc, char **argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "blocking") check_nothing_left_behind();
+    else if (what == "memory") check_long_run_keeps_nothing();
     else return 2;
     std::printf("ok %s\n", what.c_str());
 }

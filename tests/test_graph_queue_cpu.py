@@ -22,3 +22,7 @@ def check(tmp_path_factory):
 
 def test_a_run_leaves_nothing_in_its_stream(check):
     check("blocking")
+
+
+def test_a_long_run_keeps_nothing_per_launch(check):
+    check("memory")

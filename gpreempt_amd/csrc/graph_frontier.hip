@@ -68,6 +68,8 @@ __device__ __forceinline__ void raise_changed(unsigned *word, bool mine) {
 }
 
 // ---- connected components: union-find with the smaller id as the parent ---------------------------------------------
+// (Afforest, Sutton et al.: hook every vertex to a neighbour, compress, link the remaining edges, compress; the linking
+// by compare-and-swap on the larger root.)
 // Parents only ever fall, so a stale read (the L2s of the eight XCDs do not see each other's stores within a launch)
 // is an older ancestor and still an ancestor; a root is only hooked by a compare-and-swap, whose answer comes from
 // memory.  Every turn replaces the larger of the two candidates by something smaller, so the loop ends.
@@ -125,6 +127,23 @@ __device__ __forceinline__ void pr_push(const gp_graph_iter_params &p, const u32
     });
 }
 
+// ---- shortest paths: delta-stepping with one bucket (Meyer and Sanders), or the near and far piles of Davidson et al. ----
+// An iteration relaxes the marked vertices whose cost is below a limit; the others keep their mark.  The limit rises by
+// one step whenever an iteration has left no marked vertex below it.  Vertices are then relaxed close to their final
+// cost: on the generated graphs 1.1-1.4 times per vertex, where relaxing whatever is marked takes 4-5, for a fifth more
+// iterations (weights uniform in 1..64, a step of the average weight).  The first iteration's limit is one step; the
+// words of the iteration before say how it went on:
+//   [1] somebody improved below the limit   [2] the limit   [3] somebody was below it   [4] ~(lowest marked cost)
+// After an iteration that found nobody below its limit, an iteration of its own finds the lowest marked cost, and the
+// limit goes one step beyond that: a gap in the costs (one heavy edge in a light graph) takes two iterations more,
+// whatever its width, where step by step a bridge of 10^6 among unit weights took half a million.
+__device__ __forceinline__ void sssp_lowest(const gp_graph_iter_params &p, unsigned cost) {
+    for (int d = 32; d; d >>= 1) cost = min(cost, (unsigned)__shfl_xor((int)cost, d));
+    // (a look first: it may be an old one, which is a higher cost; an atomic on one address takes 40 ns of everybody's time)
+    if (cost != GF_INF && (threadIdx.x & 63) == 0 && __hip_atomic_load(p.changed + 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < ~cost)
+        atomicMax(p.changed + 4, ~cost);
+}
+
 // What a tile is looked through for (the vertices on the frontier): read for several tiles at a time, and before the
 // claim where the claim's answer is known, so that the reads of a claim's tiles are one trip to memory.
 template <int KIND>
@@ -138,7 +157,7 @@ __device__ __forceinline__ unsigned gf_key(const gp_graph_iter_params &p, int ti
 }
 
 template <int KIND>
-__device__ __forceinline__ void gf_tile(const gp_graph_iter_params &p, int tile, unsigned key, unsigned limit) {
+__device__ __forceinline__ void gf_tile(const gp_graph_iter_params &p, int tile, unsigned key, unsigned limit, bool find) {
     const unsigned n = p.vertex_count;
     const unsigned v = (unsigned)tile * GF_TILE + threadIdx.x;
     const bool in = v < n;
@@ -162,11 +181,13 @@ __device__ __forceinline__ void gf_tile(const gp_graph_iter_params &p, int tile,
         unsigned begin = 0, end = 0, cost = 0;
         if (on) {
             cost = p.cost[v];
-            far = cost >= limit;
+            far = find || cost >= limit;
             on = !far;
             p.active[v] = 0;
             if (far) p.next_active[v] = 1;  // its turn comes with a later limit
         }
+        if (find) sssp_lowest(p, far ? cost : GF_INF);
+        else raise_changed(p.changed + 3, on);
         if (on) { begin = p.row[v]; end = p.row[v + 1]; }
         bool mine = far, near = false;
         const u32x4 *weights = reinterpret_cast<const u32x4 *>(p.weights);
@@ -289,16 +310,15 @@ __device__ __forceinline__ void gf_tile(const gp_graph_iter_params &p, int tile,
     }
 }
 
-// Shortest paths: an iteration relaxes the marked vertices whose cost is below a limit; the others keep their mark.  The
-// limit rises by one step whenever an iteration has left no marked vertex below it.  Vertices are then relaxed close to
-// their final cost: on the generated graphs 1.1-1.4 times per vertex, where relaxing whatever is marked takes 4-5, for
-// a fifth more iterations (weights uniform in 1..64, a step of the average weight).  The limit of the iteration before
-// and whether it improved anything below it are in that iteration's words; the first iteration's limit is one step.
-__device__ __forceinline__ unsigned sssp_limit(const gp_graph_iter_params &p) {
+__device__ __forceinline__ unsigned sssp_limit(const gp_graph_iter_params &p, bool *find) {
     unsigned limit = p.step;
+    *find = false;
     if (p.prev_changed) {
+        auto above = [&](unsigned x) { return x + p.step < x ? GF_INF : x + p.step; };
         limit = p.prev_changed[2];
-        if (!p.prev_changed[1]) limit = limit + p.step < limit ? GF_INF : limit + p.step;
+        if (p.prev_changed[4]) limit = above(~p.prev_changed[4]);
+        else if (!p.prev_changed[1] && p.prev_changed[3]) limit = above(limit);
+        else *find = !p.prev_changed[1];
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) p.changed[2] = limit;
     return limit;
@@ -309,7 +329,8 @@ template <int KIND, int LOOP = LOOP_ANY>
 __global__ __launch_bounds__(GF_TILE) void graph_iter_kernel(gp_graph_iter_params p, int per, BlpArgs blp) {
     if (p.prev_changed && *p.prev_changed == 0) return;  // converged before this iteration (the same answer for every workgroup)
     unsigned limit = 0;
-    if constexpr (KIND == GP_GRAPH_IT_SSSP) limit = sssp_limit(p);
+    bool find = false;
+    if constexpr (KIND == GP_GRAPH_IT_SSSP) limit = sssp_limit(p, &find);
     unsigned key[4];  // of the next tiles
     auto look = [&](int first, int count) {
 #pragma unroll
@@ -322,7 +343,7 @@ __global__ __launch_bounds__(GF_TILE) void graph_iter_kernel(gp_graph_iter_param
 #pragma unroll 1
         for (int j = 0; j < per; ++j) {
             if (j % 4 == 0 && (j || known < 0)) look(t.x * per + j, per - j);
-            gf_tile<KIND>(p, t.x * per + j, key[0], limit);
+            gf_tile<KIND>(p, t.x * per + j, key[0], limit, find);
             key[0] = key[1]; key[1] = key[2]; key[2] = key[3];
         }
     });

@@ -443,7 +443,9 @@ int gp_launch_graph(const gp_graph_params *p, const gp_preempt_ctx *ctx, gp_stre
  *   BFS(_INIT)   label[v] == level: unlabelled (0xFFFFFFFF) neighbours get level + 1
  *   SSSP(_INIT)  active[v] and cost[v] below the limit: offers cost[v] + weight to the neighbours (atomic min) and goes
  *                inactive; who improves is marked in next_active, and so are the active ones at or above the limit,
- *                which starts at `step` and rises by it after an iteration that left nobody active below it
+ *                which starts at `step` and rises by it after an iteration that left nobody active below it; after one
+ *                that found nobody below it, an iteration relaxes nobody and finds the lowest active cost instead, and
+ *                the limit is `step` beyond that
  *   PR(_INIT)    row / ids list IN-neighbours: residual += sum of their share; above the tolerance it moves into value
  *                and next_share = residual * alpha / degree (out-degree; 0: nothing), else next_share = 0 (INIT writes next_share)
  *   PR_PUSH      row / ids list OUT-neighbours: share is added to every neighbour's next_gained (atomic)
@@ -454,7 +456,7 @@ int gp_launch_graph(const gp_graph_params *p, const gp_preempt_ctx *ctx, gp_stre
  *                component) to comp
  * *changed is set to 1 by an iteration that changed something; changed[1] counts the vertices over the tolerance in
  * every GP_GRAPH_SAMPLED-th tile (PR, PR_STEP) or says whether anybody improved below the limit, which is changed[2]
- * (SSSP).  prev_changed, if given, is the word of the iteration
+ * (SSSP; changed[3]: whether anybody was below it, changed[4]: ~the lowest active cost, if that was looked for).  prev_changed, if given, is the word of the iteration
  * before: a launch that finds it 0 does nothing (so several iterations can be queued without a look in between). */
 #define GP_GRAPH_SAMPLED 64
 enum gp_graph_iter_kernel { GP_GRAPH_IT_BFS = 0, GP_GRAPH_IT_BFS_INIT = 1, GP_GRAPH_IT_SSSP = 2, GP_GRAPH_IT_SSSP_INIT = 3, GP_GRAPH_IT_PR = 4,
@@ -471,7 +473,7 @@ typedef struct gp_graph_iter_params {
     float *next_share, *residual, *value, *gained, *next_gained;
     float alpha, tolerance;
     unsigned int step;
-    unsigned int *changed;                   /* three words */
+    unsigned int *changed;                   /* five words, cleared by the caller */
     const unsigned int *prev_changed;
 } gp_graph_iter_params;
 int gp_launch_graph_iter(const gp_graph_iter_params *p, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info);

@@ -306,3 +306,30 @@ def test_queued_iterations_at_the_edges_of_tiles(gp, ex_mod, tmp_path, n, m, sym
                 else:
                     want = {"bfs": lambda: G.bfs(ip, ix)[0], "sssp": lambda: G.sssp(ip, ix, w)[0], "cc": lambda: G.cc(ip, ix)[0]}[kind]()
                     assert np.array_equal(got, want), (kind, n)
+
+
+@pytest.mark.parametrize("bridge", [3, 1000, 10 ** 6, 0x70000000])
+@pytest.mark.parametrize("n", [300, 40000])
+def test_one_heavy_edge_in_a_light_graph(gp, ex_mod, tmp_path, n, bridge):
+    """the second half of the vertices hangs on the first by one edge: the iterations do not grow with its weight"""
+    rng = np.random.default_rng(n)
+    half = n // 2
+    u = np.arange(half - 1)
+    near = np.concatenate([np.stack([u, u + 1], 1)[:50], np.stack([rng.integers(0, 51, half), np.arange(half)], 1)])
+    edges = np.concatenate([near, near + half, [[half - 1, half]]])
+    base = str(tmp_path / "g")
+    _write_directed(base, n, edges, rng)
+    ip, ix, _ = G.read_graph(base, weights=True)
+    w = np.where(ix == half, bridge, 1).astype(np.uint32)  # (the bridge, and an edge or two back to its far end)
+    with open(base + ".val", "wb") as f:
+        np.array([w.size, 4], np.uint64).tofile(f)
+        w.tofile(f)
+    want = G.sssp(ip, ix, w)[0]
+    assert want[half:].min() >= bridge
+    ex = ex_mod.Executor("sssp", blp=True, graph_path=base)
+    ex.set_flag(gp.Flag())
+    for _ in range(2):
+        ex.execute()
+        assert np.array_equal(ex.graph_result("cost", np.uint32), want)
+        # at most 52 hops to either side: three iterations for each, and those of the gap
+        assert ex.graph_info()["iterations"] <= 3 * 2 * 53 + 10

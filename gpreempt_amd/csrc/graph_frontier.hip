@@ -14,7 +14,7 @@
 // A tile is 256 vertices; a preemptible launch hands tiles out through tile_loop.hpp like any other kernel.
 //
 // Several iterations are queued at once: an iteration whose predecessor changed nothing (*prev_changed == 0) leaves
-// before its first claim, so the host looks at the convergence words once per batch instead of once per iteration.
+// before its first claim.  A launch that starts says how the iteration before it went, so the host needs no look of its own.
 #include "launch_tiles.hpp"
 
 namespace gp {
@@ -324,9 +324,21 @@ __device__ __forceinline__ unsigned sssp_limit(const gp_graph_iter_params &p, bo
     return limit;
 }
 
+// The launch tells the host that it has started, and how the iteration before it went (gp_graph_iter_params::started).
+// One store to host memory that nobody waits for; the next launch is queued while this one works.
+__device__ __forceinline__ void report_start(const gp_graph_iter_params &p, const BlpArgs &blp) {
+    if (!p.started || blockIdx.x != 0 || threadIdx.x != 0) return;
+    unsigned low = GP_GRAPH_START_CHANGED;
+    if (p.prev_changed) low = p.prev_changed[0] ? GP_GRAPH_START_CHANGED | min(p.prev_changed[1], GP_GRAPH_START_COUNT) : 0u;
+    const int stop = blp.stop_index ? __hip_atomic_load(blp.stop_index, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : -1;
+    if (stop != -1) low = GP_GRAPH_START_STOPPED | (unsigned)stop;
+    __hip_atomic_store(p.started, (unsigned long long)p.seq << 32 | low, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // a claim of a launch stands for `per` tiles of 256 vertices
 template <int KIND, int LOOP = LOOP_ANY>
 __global__ __launch_bounds__(GF_TILE) void graph_iter_kernel(gp_graph_iter_params p, int per, BlpArgs blp) {
+    report_start(p, blp);
     if (p.prev_changed && *p.prev_changed == 0) return;  // converged before this iteration (the same answer for every workgroup)
     unsigned limit = 0;
     bool find = false;
@@ -366,11 +378,16 @@ __global__ __launch_bounds__(GF_TILE) void graph_pack_kernel(gp_graph_pack_param
 
 // one wavefront hands the words of the launches to the host: the words first, then the sequence number it waits for
 __global__ void graph_report_kernel(const unsigned *words, int stride, const int *stop_index, unsigned *host, int n, unsigned seq) {
+    const unsigned stop = stop_index ? (unsigned)*stop_index : 0xFFFFFFFFu;
+    if (n == 0 && ((uintptr_t)host & 7) == 0) {  // (one store needs no release in front of it, which would write this XCD's L2 back)
+        if (threadIdx.x == 0) __hip_atomic_store((unsigned long long *)host, (unsigned long long)stop << 32 | seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        return;
+    }
     if ((int)threadIdx.x < n) {
         __hip_atomic_store(host + 2 + 2 * threadIdx.x, words[threadIdx.x * stride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         __hip_atomic_store(host + 3 + 2 * threadIdx.x, words[threadIdx.x * stride + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
-    if (threadIdx.x == 0) __hip_atomic_store(host + 1, stop_index ? (unsigned)*stop_index : 0xFFFFFFFFu, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (threadIdx.x == 0) __hip_atomic_store(host + 1, stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __threadfence_system();
     if (threadIdx.x == 0) __hip_atomic_store(host, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }

@@ -167,7 +167,7 @@ std::unique_ptr<Workload> Workload::create(const std::string &kind, const CsrGra
     }
     // (beyond 32-bit offsets a graph is run one iteration at a time, on the 64-bit lists)
     if (n < (1ULL << 31) && g.edge_count / 4 + n < (1ULL << 32)) ok = ok && w->upload_packed(g, kind == "sssp");
-    ok = ok && gp_host_alloc_coherent((void **)&w->report_, &w->report_dev_, (2 + 2 * kRing) * sizeof(unsigned)) == 0;
+    ok = ok && gp_host_alloc_coherent((void **)&w->starts_, &w->starts_dev_, (kRing + 1) * sizeof(unsigned long long)) == 0;
     if (!ok) {
         std::fprintf(stderr, "graph workload: allocation failed: %s\n", gp_last_error());
         return nullptr;
@@ -179,7 +179,7 @@ Workload::~Workload() {
     for (GPUdeviceptr p : {vertex_list_, edge_list_, weight_list_, label_, active_, next_active_, comp_, delta_, residual_, value_, cost_, new_cost_, changed_,
                            row_, ids_, weights_, parent_, share_, degree_, gained_, ring_})
         if (p) gp_free(p);
-    if (report_) gp_host_free((void *)report_);
+    if (starts_) gp_host_free((void *)starts_);
     if (host_words_) gp_host_free(host_words_);
 }
 
@@ -331,6 +331,8 @@ Status Workload::launch_slot(int i, bool fresh, GPUstream stream, const PreemptE
     int *slot = (int *)ring_ + slot_ints_ * (i % kRing);
     p.changed = (unsigned *)slot;
     if (p.prev_changed) p.prev_changed = (const unsigned *)((int *)ring_ + slot_ints_ * ((i - (int)(uintptr_t)p.prev_changed) % kRing));
+    p.started = (unsigned long long *)starts_dev_ + i % kRing;
+    p.seq = seq_of_[i % kRing] = ++seq_;
     gp_preempt_ctx ctx;
     if (env) {
         std::memset(&ctx, 0, sizeof(ctx));
@@ -344,14 +346,9 @@ Status Workload::launch_slot(int i, bool fresh, GPUstream stream, const PreemptE
     return Status::Succ;
 }
 
-Status Workload::report(GPUstream stream, const PreemptEnv *env) {
-    GC_CHECK(gp_graph_report_async((const unsigned *)ring_, kRing, (int)slot_ints_, env ? (const int *)env->stop_index : nullptr, (unsigned *)report_dev_, ++report_seq_, stream));
-    return Status::Succ;
-}
-
-// Queues the launches of `list` behind those queued before.  The host is told how the run stands when all but the last
-// `report_before_last` of them are done, so that it can queue the next ones while the GPU still has work.
-Status Workload::queue(const std::vector<gp_graph_iter_params> &list, int report_before_last, GPUstream stream, const PreemptEnv *env) {
+// Queues one launch behind the others.  The words and claim counters of half the ring are cleared at a time, in stream
+// order behind the launches that used them last.
+Status Workload::submit(const gp_graph_iter_params &p, GPUstream stream, const PreemptEnv *env) {
     const size_t slot_ints = 16 + (env ? (size_t)env->counter_groups * env->counter_stride : 0);
     if (slot_ints != slot_ints_) {
         if (ring_) gp_free(ring_);
@@ -359,40 +356,72 @@ Status Workload::queue(const std::vector<gp_graph_iter_params> &list, int report
         GC_CHECK(gp_malloc(&ring_, slot_ints * kRing * sizeof(int)));
         slot_ints_ = slot_ints;
     }
-    const int first = submitted_, count = (int)list.size();
-    for (const gp_graph_iter_params &p : list) queued_[submitted_++ % kRing] = p;
-    const int at = first % kRing, here = std::min(count, kRing - at);
-    GC_CHECK(gp_fill32_async((int *)ring_ + slot_ints_ * at, 0, slot_ints_ * here, stream));
-    GC_CHECK(gp_fill32_async(ring_, 0, slot_ints_ * (count - here), stream));
-    for (int j = 0; j < count; ++j) {
-        if (j == count - report_before_last) RETURN_STATUS(report(stream, env));
-        RETURN_STATUS(launch_slot(first + j, true, stream, env));
-    }
-    return report_before_last ? Status::Succ : report(stream, env);
+    const int i = submitted_++;
+    if (i % (kRing / 2) == 0) GC_CHECK(gp_fill32_async((int *)ring_ + slot_ints_ * (i % kRing), 0, slot_ints_ * (kRing / 2), stream));
+    queued_[i % kRing] = p;
+    return launch_slot(i, true, stream, env);
 }
 
-// (spinning on the word: a blocked thread wakes up tens of microseconds late, a query of the stream costs microseconds)
-Status Workload::await_word(GPUstream stream) {
-    for (unsigned spins = 1; __atomic_load_n(&report_[0], __ATOMIC_ACQUIRE) != report_seq_; ++spins) {
-        if (spins % (1u << 16)) continue;
+// Spins until a word of host memory says so: a blocked thread wakes up tens of microseconds late, a query of the stream
+// costs microseconds.  (One is made now and then, so that an error of the device ends the wait.)
+template <class There>
+static Status spin(GPUstream stream, There &&there) {
+    for (unsigned spins = 1;; ++spins) {
         int idle = 0;
-        GC_CHECK(gp_stream_query(stream, &idle));  // an error of the device ends the wait
+        if (spins % (1u << 16) == 0) GC_CHECK(gp_stream_query(stream, &idle));
+        if (there()) return Status::Succ;
+        if (idle) {
+            std::fprintf(stderr, "graph workload: a launch did not report\n");
+            return Status::Fail;
+        }
     }
+}
+
+// Waits until everything queued has left the GPU; *stop receives the slot of the launch that was stopped, or -1.
+Status Workload::drain(GPUstream stream, const PreemptEnv *env, int *stop) {
+    GC_CHECK(gp_graph_report_async((const unsigned *)ring_, 0, (int)slot_ints_, env ? (const int *)env->stop_index : nullptr,
+                                   (unsigned *)((unsigned long long *)starts_dev_ + kRing), ++seq_, stream));
+    unsigned long long report = 0;  // the stop index and the sequence number
+    RETURN_STATUS(spin(stream, [&] { report = __atomic_load_n(starts_ + kRing, __ATOMIC_ACQUIRE); return (unsigned)report == seq_; }));
+    *stop = (int)(report >> 32);
     return Status::Succ;
 }
 
-// Waits for the last report.  A launch that was stopped is relaunched, and the ones behind it with it (they left when
-// they found the stop recorded); `first` is the first launch the report is about.
-Status Workload::await_report(int first, GPUstream stream, const PreemptEnv *env) {
+// A launch was stopped and nothing of this run is on the GPU: when it is this workload's turn again, that launch is
+// queued once more, and the ones behind it with it (they left when they found the stop recorded).
+Status Workload::restart(int stop, GPUstream stream, const PreemptEnv *env) {
+    RETURN_STATUS(wait_turn(stream, env));
+    int from = submitted_ - 1;
+    while (from > 0 && from % kRing != stop) --from;
+    for (int i = from; i < submitted_; ++i) RETURN_STATUS(launch_slot(i, false, stream, env));
+    return Status::Succ;
+}
+
+// The end of a run: everything queued is done, or had nothing to do, and has left.
+Status Workload::settle(GPUstream stream, const PreemptEnv *env) {
     for (;;) {
-        RETURN_STATUS(await_word(stream));
-        const int stop = (int)report_[1];
-        if (!env || stop < 0) return Status::Succ;
-        RETURN_STATUS(wait_turn(stream, env));
-        int from = submitted_ - 1;
-        while (from > first && from % kRing != stop) --from;
-        for (int i = from; i < submitted_; ++i) RETURN_STATUS(launch_slot(i, false, stream, env));
-        RETURN_STATUS(report(stream, env));
+        int stop = -1;
+        RETURN_STATUS(drain(stream, env, &stop));
+        if (stop < 0) return Status::Succ;
+        RETURN_STATUS(restart(stop, stream, env));
+    }
+}
+
+// Waits until launch `i` starts, i.e. until the ones before it are done.  *changed: the iteration before it changed
+// something; *count: of how many vertices over the tolerance it knows.
+Status Workload::await_start(int i, GPUstream stream, const PreemptEnv *env, bool *changed, unsigned *count) {
+    for (;;) {
+        unsigned long long word = 0;  // the sequence number and what the launch knows
+        RETURN_STATUS(spin(stream, [&] { word = __atomic_load_n(starts_ + i % kRing, __ATOMIC_ACQUIRE); return (unsigned)(word >> 32) == seq_of_[i % kRing]; }));
+        const unsigned low = (unsigned)word;
+        if (!(low & GP_GRAPH_START_STOPPED)) {
+            *changed = (low & GP_GRAPH_START_CHANGED) != 0;
+            *count = low & GP_GRAPH_START_COUNT;
+            return Status::Succ;
+        }
+        int stop = -1;
+        RETURN_STATUS(drain(stream, env, &stop));
+        RETURN_STATUS(restart(stop, stream, env));
     }
 }
 
@@ -413,39 +442,38 @@ gp_graph_iter_params Workload::params(int kernel) const {
     return p;
 }
 
-// The iterations are those of the reference's loops.  They are queued a batch at a time: the host learns afterwards
-// which was the first to change nothing (the ones behind it did nothing), and queues the next batch before the last
-// launches of this one are done.
+// The iterations are those of the reference's loops.  Launches are queued a few ahead of the GPU: a launch tells the host
+// when it starts and, since the ones before it are done then, whether the iteration before it changed anything, and the
+// host queues the next one.  (A launch takes 3-4 us at least and the host's turn, from the word to a queued launch, as
+// long; kAhead of them keep the GPU busy.  Those are what is still queued when the run converges or is stopped: each has
+// to start and leave, 3-4 us, before the run can end or the GPU is vacated.)
 Status Workload::compute(GPUstream stream, const PreemptEnv *env) {
     if (!row_ || (env && env->inject_kernel >= 0 && env->inject_iteration >= -1)) return compute_stepwise(stream, env);
-    iterations_ = 0;
-    submitted_ = 0;
+    iterations_ = submitted_ = 0;
     if (kind_ == "cc") {
         iterations_ = 3;  // the passes behind the set-up one
-        RETURN_STATUS(queue({params(GP_GRAPH_IT_CC_INIT), params(GP_GRAPH_IT_CC_FLATTEN), params(GP_GRAPH_IT_CC_LINK), params(GP_GRAPH_IT_CC_LABEL)}, 0, stream, env));
-        return await_report(0, stream, env);
+        for (int kernel : {GP_GRAPH_IT_CC_INIT, GP_GRAPH_IT_CC_FLATTEN, GP_GRAPH_IT_CC_LINK, GP_GRAPH_IT_CC_LABEL}) RETURN_STATUS(submit(params(kernel), stream, env));
+        return settle(stream, env);
     }
     const bool bfs = kind_ == "bfs", pagerank = kind_ == "pagerank";
     const int max_iter = pagerank ? 100 : 1 << 30;  // graphcompute.h:82
-    std::vector<gp_graph_iter_params> list{params(bfs ? GP_GRAPH_IT_BFS_INIT : pagerank ? GP_GRAPH_IT_PR_INIT : GP_GRAPH_IT_SSSP_INIT)};
-    // of the iterations whose outcome is not known yet (iterations_ on): the last launch, whose word says whether it changed
-    // anything.  Nothing is kept of the others: a path of a million vertices takes as many iterations.
-    std::deque<int> last_of;
-    int next_first = 0;  // the launch behind the last known iteration
+    RETURN_STATUS(submit(params(bfs ? GP_GRAPH_IT_BFS_INIT : pagerank ? GP_GRAPH_IT_PR_INIT : GP_GRAPH_IT_SSSP_INIT), stream, env));
     GPUdeviceptr share = delta_, other = share_;
     float *gained = (float *)gained_, *next_gained = gained + (gained ? n_ : 0);
     bool push = false, pushing = false;  // wanted; the shares of the iteration before have been pushed
-    // an iteration that is queued and not needed costs an empty launch (3-4 us), a batch that the host has to wait for
-    // 20 us: batches grow with what a run of the algorithm takes, and the last launches cover the host's turn
-    int batch = bfs ? 8 : 16;
-    const int ahead = bfs ? 1 : 2;
+    unsigned sampled = ~0u;              // vertices over the tolerance in the sampled tiles, of the last iteration that is known
+    int next = 0, started = 0;           // the iteration to queue next; launches that have started
+    std::deque<int> first_of;            // of the iterations queued and not started (next - 1 the last): their first launch
     for (;;) {
-        const int upto = std::min(max_iter, iterations_ + batch), first = submitted_;
-        for (int it = iterations_ + (int)last_of.size(); it < upto; ++it) {
+        while (next < max_iter && submitted_ - started <= kAhead) {
             gp_graph_iter_params p = params(bfs ? GP_GRAPH_IT_BFS : pagerank ? GP_GRAPH_IT_PR : GP_GRAPH_IT_SSSP);
-            p.level = (unsigned)it;
-            if (it & 1) std::swap(p.active, p.next_active);
-            p.prev_changed = it ? (const unsigned *)(uintptr_t)1 : nullptr;  // (how many launches back that word is; launch_slot makes it an address)
+            p.level = (unsigned)next;
+            if (next & 1) std::swap(p.active, p.next_active);
+            p.prev_changed = next ? (const unsigned *)(uintptr_t)1 : nullptr;  // (how many launches back that word is; launch_slot makes it an address)
+            first_of.push_back(submitted_);
+            // (2^20 vertices of degree 16: 45-55 us for the pull, as much for atomics from one vertex in twenty-five.  The
+            // push begins a little below that, because going over to it takes a launch.)
+            if (pagerank) push = symmetric_ && sampled < n_ / GP_GRAPH_SAMPLED / (push ? 25 : 32);
             if (pagerank && pushing) {
                 p.kernel = GP_GRAPH_IT_PR_STEP;
                 p.gained = gained;
@@ -458,9 +486,9 @@ Status Workload::compute(GPUstream stream, const PreemptEnv *env) {
                 if (push) {  // the pull's shares go out; this iteration takes them in, and pushes its own
                     p.kernel = GP_GRAPH_IT_PR_PUSH;
                     p.next_gained = gained;
-                    list.push_back(p);
+                    RETURN_STATUS(submit(p, stream, env));
                     p.kernel = GP_GRAPH_IT_PR_STEP;
-                    p.prev_changed = (const unsigned *)(uintptr_t)2;
+                    p.prev_changed = next ? (const unsigned *)(uintptr_t)2 : nullptr;
                     p.gained = gained; p.next_gained = next_gained;
                     std::swap(gained, next_gained);
                     pushing = true;
@@ -469,34 +497,23 @@ Status Workload::compute(GPUstream stream, const PreemptEnv *env) {
                     std::swap(share, other);
                 }
             }
-            list.push_back(p);
-            last_of.push_back(first + (int)list.size() - 1);
+            RETURN_STATUS(submit(p, stream, env));
+            ++next;
         }
-        const int tail = upto == max_iter ? 0 : std::min(ahead, (int)list.size() - 1);
-        RETURN_STATUS(queue(list, tail, stream, env));
-        RETURN_STATUS(await_report(next_first, stream, env));
-        const int known = submitted_ - tail;
-        unsigned sampled = 0;
-        while (!last_of.empty() && last_of.front() < known) {
-            const volatile unsigned *w = words(last_of.front());
-            next_first = last_of.front() + 1;
-            last_of.pop_front();
-            ++iterations_;
-            if (w[0] == 0) {
-                // The launches behind it find that out for themselves and leave, each by the word of the launch before
-                // it: a run that came after them on another stream would clear those words under them.  So they are
-                // waited for here, which is what a blocking call promises anyway.
-                if (tail) { RETURN_STATUS(report(stream, env)); RETURN_STATUS(await_word(stream)); }
-                return Status::Succ;
-            }
-            sampled = w[1];
+        if (started == submitted_) {  // all there may be
+            iterations_ = max_iter;
+            return settle(stream, env);
         }
-        if (iterations_ >= max_iter) return Status::Succ;
-        // (below a thirty-second of the vertices with a share the push is cheaper than the pull: 2^20 vertices of degree
-        // 16, 45-55 us for the pull, as much for atomics from one vertex in twenty-five)
-        push = pagerank && symmetric_ && sampled < n_ / GP_GRAPH_SAMPLED / 32;
-        list.clear();
-        batch = bfs ? 5 : pagerank && sampled > n_ / GP_GRAPH_SAMPLED / 2 ? 16 : 8;
+        bool changed = true;
+        unsigned count = 0;
+        RETURN_STATUS(await_start(started, stream, env, &changed, &count));
+        if (!first_of.empty() && first_of.front() == started) {  // the first launch of an iteration speaks of the iteration before
+            iterations_ = next - (int)first_of.size();
+            first_of.pop_front();
+            if (!changed) return settle(stream, env);
+            sampled = iterations_ ? count : ~0u;
+        }
+        ++started;
     }
 }
 

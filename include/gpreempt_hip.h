@@ -457,7 +457,13 @@ int gp_launch_graph(const gp_graph_params *p, const gp_preempt_ctx *ctx, gp_stre
  * *changed is set to 1 by an iteration that changed something; changed[1] counts the vertices over the tolerance in
  * every GP_GRAPH_SAMPLED-th tile (PR, PR_STEP) or says whether anybody improved below the limit, which is changed[2]
  * (SSSP; changed[3]: whether anybody was below it, changed[4]: ~the lowest active cost, if that was looked for).  prev_changed, if given, is the word of the iteration
- * before: a launch that finds it 0 does nothing (so several iterations can be queued without a look in between). */
+ * before: a launch that finds it 0 does nothing (so several iterations can be queued without a look in between).
+ * started, if given, is a device-visible word of host memory (gp_host_alloc_coherent) in which the launch stores, when it
+ * starts, seq in the upper half and in the lower one what is known then: GP_GRAPH_START_STOPPED | the stop index if a stop
+ * is recorded, else GP_GRAPH_START_CHANGED unless *prev_changed is 0, and prev_changed[1] (at most GP_GRAPH_START_COUNT). */
+#define GP_GRAPH_START_STOPPED 0x80000000u
+#define GP_GRAPH_START_CHANGED 0x40000000u
+#define GP_GRAPH_START_COUNT 0x3FFFFFFFu
 #define GP_GRAPH_SAMPLED 64
 enum gp_graph_iter_kernel { GP_GRAPH_IT_BFS = 0, GP_GRAPH_IT_BFS_INIT = 1, GP_GRAPH_IT_SSSP = 2, GP_GRAPH_IT_SSSP_INIT = 3, GP_GRAPH_IT_PR = 4,
                             GP_GRAPH_IT_PR_INIT = 5, GP_GRAPH_IT_CC_INIT = 6, GP_GRAPH_IT_CC_LINK = 7, GP_GRAPH_IT_CC_FLATTEN = 8, GP_GRAPH_IT_CC_LABEL = 9,
@@ -475,6 +481,8 @@ typedef struct gp_graph_iter_params {
     unsigned int step;
     unsigned int *changed;                   /* five words, cleared by the caller */
     const unsigned int *prev_changed;
+    unsigned long long *started;             /* may be NULL */
+    unsigned int seq;
 } gp_graph_iter_params;
 int gp_launch_graph_iter(const gp_graph_iter_params *p, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info);
 /* fills ids (4 * row_end + 4 of them: a last vector of vertex_count lies behind the lists) and weights of that layout from
@@ -488,7 +496,8 @@ typedef struct gp_graph_pack_params {
 } gp_graph_pack_params;
 int gp_graph_pack_async(const gp_graph_pack_params *p, gp_stream s);
 /* Stores the pairs words[i * stride], words[i * stride + 1] (i < n) and *stop_index (-1 without one) into pinned host
- * memory (host_words[2 + 2 i], host_words[3 + 2 i] and host_words[1]), then seq into host_words[0]. */
+ * memory (host_words[2 + 2 i], host_words[3 + 2 i] and host_words[1]), then seq into host_words[0].  With n == 0 and
+ * host_words a multiple of 8 the two words are one store, and the GPU's caches are left alone. */
 int gp_graph_report_async(const unsigned int *words, int n, int stride, const int *stop_index, unsigned int *host_words, unsigned int seq, gp_stream s);
 
 /* out[t,:] = tok[ids[t],:] + pos[t % seq,:] (+ seg[0,:]); ids are int64 (the reference feeds

@@ -6,7 +6,7 @@
 // src/workloads/graphcompute.tr.cu:142-174 (CC), :257-285 (BFS), :450-495 (PageRank), :635-675
 // (SSSP).  One class drives all four: an algorithm is a list of launches, and the loop that launches, notices a
 // stop, waits for its turn and relaunches from the stopped launch is shared (the reference repeats it with
-// `goto resume` per algorithm).  A run queues several iterations at a time (gp_launch_graph_iter); a run with a
+// `goto resume` per algorithm).  A run keeps a few iterations queued (gp_launch_graph_iter); a run with a
 // preemption injected at one of the reference's kernels (a test hook) goes through those, one iteration at a time.
 #pragma once
 #include <cstdint>
@@ -74,13 +74,13 @@ private:
     Status run_kernels(const std::vector<int> &kernels, GPUstream stream, const PreemptEnv *env, int iteration, bool *changed);
     Status begin(GPUstream stream);
     Status compute_stepwise(GPUstream stream, const PreemptEnv *env);
-    // a queue of launches, kRing of them at most outstanding; launch i uses slot i % kRing of ring_
-    Status queue(const std::vector<gp_graph_iter_params> &list, int report_before_last, GPUstream stream, const PreemptEnv *env);
+    // launches of a run, kAhead of them queued and not started; launch i uses slot i % kRing of ring_
+    Status submit(const gp_graph_iter_params &p, GPUstream stream, const PreemptEnv *env);
     Status launch_slot(int i, bool fresh, GPUstream stream, const PreemptEnv *env);
-    Status report(GPUstream stream, const PreemptEnv *env);
-    Status await_word(GPUstream stream);
-    Status await_report(int first, GPUstream stream, const PreemptEnv *env);
-    const volatile unsigned *words(int i) const { return report_ + 2 + 2 * (i % kRing); }
+    Status await_start(int i, GPUstream stream, const PreemptEnv *env, bool *changed, unsigned *count);
+    Status drain(GPUstream stream, const PreemptEnv *env, int *stop);
+    Status restart(int stop, GPUstream stream, const PreemptEnv *env);
+    Status settle(GPUstream stream, const PreemptEnv *env);
     Status wait_turn(GPUstream stream, const PreemptEnv *env);
     bool upload_packed(const CsrGraph &g, bool with_weights);
     gp_graph_iter_params params(int kernel) const;
@@ -100,14 +100,15 @@ private:
     GPUdeviceptr row_ = nullptr, ids_ = nullptr, weights_ = nullptr, parent_ = nullptr, share_ = nullptr, degree_ = nullptr, gained_ = nullptr;
     uint32_t row_end_ = 0, step_ = 1;
     bool symmetric_ = false;
-    static constexpr int kRing = 64;
-    GPUdeviceptr ring_ = nullptr;                    // device: per slot two convergence words and the claim counters, a line apart
+    static constexpr int kRing = 64, kAhead = 2;
+    GPUdeviceptr ring_ = nullptr;                    // device: per slot the convergence words and the claim counters, a line apart
     size_t slot_ints_ = 0;
     gp_graph_iter_params queued_[kRing];             // the last kRing launches of this run: number i is in slot i % kRing
+    unsigned seq_of_[kRing] = {};                    // what each of them reports its start with
     int submitted_ = 0;                              // how many there have been
-    volatile unsigned *report_ = nullptr;            // pinned, coherent: sequence number, stop index, words of every slot
-    void *report_dev_ = nullptr;
-    unsigned report_seq_ = 0;
+    volatile unsigned long long *starts_ = nullptr;  // pinned, coherent: the start of every slot's launch, and the report behind the last one
+    void *starts_dev_ = nullptr;
+    unsigned seq_ = 0;
 };
 
 }  // namespace GraphCompute

@@ -112,6 +112,11 @@ int gp_launch_graph_iter(const gp_graph_iter_params *pp, const gp_preempt_ctx *c
     ++g_in_flight;
     of(s)->submit([=] {
         struct Done { ~Done() { --g_in_flight; } } done;
+        if (p.started) {
+            unsigned low = !p.prev_changed ? GP_GRAPH_START_CHANGED : *p.prev_changed ? GP_GRAPH_START_CHANGED | p.prev_changed[1] : 0;
+            if (stop && *stop != -1) low = GP_GRAPH_START_STOPPED | (unsigned)*stop;
+            __atomic_store_n(p.started, (unsigned long long)p.seq << 32 | low, __ATOMIC_RELEASE);
+        }
         pause_us(g_delay_us);
         if (p.prev_changed && *p.prev_changed == 0) return;
         if (stop && *stop != -1) { ++g_left; return; }
@@ -167,6 +172,31 @@ static void check_nothing_left_behind() {
     g_delay_us = 0;
 }
 
+// A stop, wherever it falls: when the workload gives way, nothing of it is on the GPU any more and few launches had to
+// start and leave for that; every iteration still runs once, in order.
+static void check_stops() {
+    g_delay_us = 100;
+    for (const char *kind : {"bfs", "pagerank", "sssp"})
+        for (int last : {9, 40})
+            for (int stop_at : {0, 1, 2, 5, last - 1, last}) {
+                auto w = GraphCompute::Workload::create(kind, path_graph(64));
+                gp_stream_s s;
+                GraphCompute::PreemptEnv env = env_of();
+                int gave_way = 0;
+                g_left = 0;
+                g_stop_at_level = stop_at;
+                env.higher_priority_active = [&] {
+                    ++gave_way;
+                    CHECK(g_in_flight == 0, "%s stopped at %d: %d launches still to come", kind, stop_at, g_in_flight.load());
+                    CHECK(g_left <= 4, "%s stopped at %d: %d launches had to leave", kind, stop_at, g_left);
+                    return false;
+                };
+                run(kind, last, &s, &env, *w);
+                CHECK(gave_way == 1 && w->preemptions() == 1, "%s stopped at %d: gave way %d times", kind, stop_at, gave_way);
+            }
+    g_delay_us = 0;
+}
+
 // a run of many iterations keeps as much as a short one
 static void check_long_run_keeps_nothing() {
     auto w = GraphCompute::Workload::create("bfs", path_graph(64));
@@ -185,6 +215,7 @@ static void check_long_run_keeps_nothing() {
 int main(int argc, char **argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "blocking") check_nothing_left_behind();
+    else if (what == "stops") check_stops();
     else if (what == "memory") check_long_run_keeps_nothing();
     else return 2;
     std::printf("ok %s\n", what.c_str());

@@ -26,3 +26,7 @@ def test_a_run_leaves_nothing_in_its_stream(check):
 
 def test_a_long_run_keeps_nothing_per_launch(check):
     check("memory")
+
+
+def test_a_stop_waits_for_few_launches(check):
+    check("stops")

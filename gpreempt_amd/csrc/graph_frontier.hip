@@ -33,10 +33,68 @@ __device__ __forceinline__ float quad_sum(float x) {
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
+// Whether a stop has been recorded, looked at while a wavefront works on its tile: ask() sends a load out, told() waits for
+// it, and the work between the two covers its way.  Reads of one address come back one every 11 ns, whoever asks (every
+// wavefront asking the stop index itself made sssp at 2^20 vertices 7 % slower), so the front workgroup hands the stop on
+// in GP_GRAPH_RELAYS words, a line apart, and a workgroup asks one of those.
+struct StopLook {
+    const unsigned *relay = nullptr;  // nullptr: nobody looks
+    unsigned seen = 0;
+    __device__ __forceinline__ void ask() { if (relay) seen = __hip_atomic_load(relay, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+    __device__ __forceinline__ bool told() const { return relay && __builtin_amdgcn_readfirstlane(seen) != 0; }
+};
+static_assert(GP_GRAPH_RELAYS == 64, "a lane per word");
+constexpr unsigned kRelayStride = 32;
+
+// The front workgroup of a launch whose claims are given back: as front_workgroup of tile_loop.hpp, with three differences.
+// It hands a stop on to the wavefronts that are at work.  It stays until seven eighths of the workers have left, because
+// what a frontier gives the workers to do is uneven.  And it reads the flag every ten microseconds only: while a read of
+// host memory is under way, the loads of that XCD come back later, and kernels that walk chains of them feel every one
+// (read back to back: flattening 40 -> 178 us, bfs at 2^20 vertices 320 -> 369, sssp 1.68 -> 1.80 ms).  Bounded like
+// front_workgroup; true in a front workgroup.
+__device__ __forceinline__ bool gf_front(const BlpArgs &b, unsigned *relay) {
+    if ((int)blockIdx.x >= b.front) return false;
+    if (blockIdx.x != 0) return true;
+    __shared__ int front_leave;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x / 64;
+    if (threadIdx.x == 0) front_leave = 0;
+    __syncthreads();
+    auto told = [&] { return __hip_atomic_load(&front_leave, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0; };
+    if (wave == 0) {
+        for (int look = 0; look < (1 << 15) && !told(); ++look) {
+            int flag = 0;
+            if (lane == 0) flag = __hip_atomic_load(b.flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            if (__builtin_amdgcn_readfirstlane(flag) != 0) {
+                if (lane == 0) record_stop(b.stop_index, b.kernel_id, b.stamps);
+                break;
+            }
+            for (int us = 0; us < 8 && !told(); ++us) __builtin_amdgcn_s_sleep(36);
+        }
+    } else if (wave == 1) {
+        const int target = wg_count(b) - wg_count(b) / 8;
+        for (int look = 0; look < (1 << 18); ++look) {  // about a microsecond each
+            const int stop = __hip_atomic_load(b.stop_index, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            int n = 0;
+            for (int g = lane; g < b.groups; g += 64) n += __hip_atomic_load(b.done + g * COUNTER_STRIDE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int d = 32; d > 0; d >>= 1) n += __shfl_xor(n, d);
+            if (__builtin_amdgcn_readfirstlane(stop) != -1) {
+                __hip_atomic_store(relay + kRelayStride * lane, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                break;
+            }
+            if (__builtin_amdgcn_readfirstlane(n) >= target) break;
+            __builtin_amdgcn_s_sleep(4);
+        }
+        if (lane == 0) __hip_atomic_store(&front_leave, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    return true;
+}
+
 // f(index of a vector of four neighbours, its ids, the owner's payload) for every vector of the 64 lists that this
-// wavefront's lanes own; an empty range (begin == end) stands for a vertex that takes no part
+// wavefront's lanes own; an empty range (begin == end) stands for a vertex that takes no part.  Returns true when it
+// was left because of a stop, after some of the lists: the tile has to be walked again from the start.
 template <class F>
-__device__ __forceinline__ void gf_walk(const u32x4 *ids, unsigned begin, unsigned end, unsigned payload, F &&f) {
+__device__ __forceinline__ bool gf_walk(const u32x4 *ids, unsigned begin, unsigned end, unsigned payload, StopLook look, F &&f) {
     const unsigned sub = threadIdx.x & 3;
     const bool is_long = end - begin > kLongRow;
     const unsigned stop = is_long ? begin : end;
@@ -48,9 +106,15 @@ __device__ __forceinline__ void gf_walk(const u32x4 *ids, unsigned begin, unsign
     if (b1 < e1) i1 = ids[b1];
     if (b2 < e2) i2 = ids[b2];
     if (b3 < e3) i3 = ids[b3];
+    look.ask();
     if (b0 < e0) f(b0, i0, p0);
+    if (look.told()) return true;
+    look.ask();
     if (b1 < e1) f(b1, i1, p1);
+    if (look.told()) return true;
+    look.ask();
     if (b2 < e2) f(b2, i2, p2);
+    if (look.told()) return true;
     if (b3 < e3) f(b3, i3, p3);
     for (unsigned c = b0 + 4; c < e0; c += 4) f(c, ids[c], p0);
     for (unsigned c = b1 + 4; c < e1; c += 4) f(c, ids[c], p1);
@@ -59,8 +123,11 @@ __device__ __forceinline__ void gf_walk(const u32x4 *ids, unsigned begin, unsign
     for (unsigned long long m = __builtin_amdgcn_ballot_w64(is_long); m; m &= m - 1) {
         const int l = __builtin_ctzll(m);
         const unsigned lb = __builtin_amdgcn_readlane(begin, l), le = __builtin_amdgcn_readlane(end, l), lp = __builtin_amdgcn_readlane(payload, l);
+        look.ask();
         for (unsigned c = lb + (threadIdx.x & 63); c < le; c += 64) f(c, ids[c], lp);
+        if (look.told()) return true;
     }
+    return false;
 }
 
 __device__ __forceinline__ void raise_changed(unsigned *word, bool mine) {
@@ -120,7 +187,7 @@ __device__ __forceinline__ void pr_push(const gp_graph_iter_params &p, const u32
     if (!__builtin_amdgcn_ballot_w64(share != 0.f)) return;
     unsigned begin = 0, end = 0;
     if (share != 0.f) { begin = p.row[v]; end = p.row[v + 1]; }
-    gf_walk(ids, begin, end, __builtin_bit_cast(unsigned, share), [&](unsigned, const u32x4 &i, unsigned from) {
+    gf_walk(ids, begin, end, __builtin_bit_cast(unsigned, share), StopLook{}, [&](unsigned, const u32x4 &i, unsigned from) {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             if (i[j] < p.vertex_count) atomicAdd(&p.next_gained[i[j]], __builtin_bit_cast(float, from));
@@ -156,27 +223,37 @@ __device__ __forceinline__ unsigned gf_key(const gp_graph_iter_params &p, int ti
     else return 0;
 }
 
+// Kernels whose tiles can be left at any point and done again from the start: labels, costs and parents only fall, and a
+// second look at a neighbour finds nothing left to do.  (PR and PR_PUSH add: a tile of theirs is done once.  One of
+// PR_STEP that is done finds nothing gained when it is done again, but only if it does not leave its shares behind.)
 template <int KIND>
-__device__ __forceinline__ void gf_tile(const gp_graph_iter_params &p, int tile, unsigned key, unsigned limit, bool find) {
+__device__ __forceinline__ bool gf_repeatable(const gp_graph_iter_params &p) {
+    return KIND == GP_GRAPH_IT_BFS || KIND == GP_GRAPH_IT_SSSP || KIND == GP_GRAPH_IT_CC_LINK || (KIND == GP_GRAPH_IT_PR_STEP && p.next_gained);
+}
+
+// true: a stop is recorded and the tile was left
+template <int KIND>
+__device__ __forceinline__ bool gf_tile(const gp_graph_iter_params &p, int tile, unsigned key, unsigned limit, bool find, StopLook look) {
     const unsigned n = p.vertex_count;
     const unsigned v = (unsigned)tile * GF_TILE + threadIdx.x;
     const bool in = v < n;
     const u32x4 *ids = reinterpret_cast<const u32x4 *>(p.ids);
     if constexpr (KIND == GP_GRAPH_IT_BFS) {
         const bool on = key == p.level;
-        if (!__builtin_amdgcn_ballot_w64(on)) return;
+        if (!__builtin_amdgcn_ballot_w64(on)) return false;
         unsigned begin = 0, end = 0;
         if (on) { begin = p.row[v]; end = p.row[v + 1]; }
         bool mine = false;
-        gf_walk(ids, begin, end, 0, [&](unsigned, const u32x4 &i, unsigned) {
+        const bool left = gf_walk(ids, begin, end, 0, look, [&](unsigned, const u32x4 &i, unsigned) {
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 if (p.label[i[j]] == GF_INF) { p.label[i[j]] = p.level + 1; mine = true; }
         });
         raise_changed(p.changed, mine);
+        return left;
     } else if constexpr (KIND == GP_GRAPH_IT_SSSP) {
         bool on = key != 0;
-        if (!__builtin_amdgcn_ballot_w64(on)) return;
+        if (!__builtin_amdgcn_ballot_w64(on)) return false;
         bool far = false;
         unsigned begin = 0, end = 0, cost = 0;
         if (on) {
@@ -191,7 +268,7 @@ __device__ __forceinline__ void gf_tile(const gp_graph_iter_params &p, int tile,
         if (on) { begin = p.row[v]; end = p.row[v + 1]; }
         bool mine = far, near = false;
         const u32x4 *weights = reinterpret_cast<const u32x4 *>(p.weights);
-        gf_walk(ids, begin, end, cost, [&](unsigned c, const u32x4 &i, unsigned from) {
+        const bool left = gf_walk(ids, begin, end, cost, look, [&](unsigned c, const u32x4 &i, unsigned from) {
             const u32x4 w = weights[c];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -204,8 +281,10 @@ __device__ __forceinline__ void gf_tile(const gp_graph_iter_params &p, int tile,
                 }
             }
         });
+        if (left && on) p.active[v] = 1;  // its turn again when the tile is done again
         raise_changed(p.changed, mine);
         raise_changed(p.changed + 1, near);
+        return left;
     } else if constexpr (KIND == GP_GRAPH_IT_PR) {
         unsigned begin = 0, end = 0;
         float r = 0.f;
@@ -262,7 +341,7 @@ __device__ __forceinline__ void gf_tile(const gp_graph_iter_params &p, int tile,
     } else if constexpr (KIND == GP_GRAPH_IT_PR_STEP) {
         // (next_gained == nullptr: the next iteration pulls; the shares are left for it instead of pushed)
         const float gained = __builtin_bit_cast(float, key);
-        if (p.next_gained && !__builtin_amdgcn_ballot_w64(gained != 0.f)) return;
+        if (p.next_gained && !__builtin_amdgcn_ballot_w64(gained != 0.f)) return false;
         bool up = false;
         float share = 0.f;
         if (gained != 0.f) {
@@ -276,7 +355,7 @@ __device__ __forceinline__ void gf_tile(const gp_graph_iter_params &p, int tile,
         if (p.next_gained) pr_push(p, ids, v, share);
         else if (in) p.next_share[v] = share;
     } else if constexpr (KIND == GP_GRAPH_IT_PR_INIT) {
-        if (!in) return;
+        if (!in) return false;
         p.value[v] = 1.0f - p.alpha;
         p.next_share[v] = p.degree[v] > 0.f ? (1.0f - p.alpha) * p.alpha / p.degree[v] : 0.f;
         p.residual[v] = 0.f;
@@ -285,22 +364,34 @@ __device__ __forceinline__ void gf_tile(const gp_graph_iter_params &p, int tile,
     } else if constexpr (KIND == GP_GRAPH_IT_BFS_INIT) {
         if (in) p.label[v] = v == 0 ? 0 : GF_INF;  // source = vertex 0
     } else if constexpr (KIND == GP_GRAPH_IT_SSSP_INIT) {
-        if (!in) return;
+        if (!in) return false;
         p.cost[v] = v == 0 ? 0 : GF_INF;
         p.active[v] = v == 0;
         p.next_active[v] = 0;
     } else if constexpr (KIND == GP_GRAPH_IT_CC_INIT) {
         // hook every vertex to its first neighbour at once, if that is smaller (nobody reads a parent in this launch)
-        if (!in) return;
+        if (!in) return false;
         unsigned first = v;
         if (p.row[v] < p.row[v + 1]) { first = p.ids[4ull * p.row[v]]; }
         p.parent[v] = first < v ? first : v;
     } else if constexpr (KIND == GP_GRAPH_IT_CC_FLATTEN) {
         if (in) p.parent[v] = cc_root(p.parent, v);
     } else if constexpr (KIND == GP_GRAPH_IT_CC_LINK) {
+        // (every edge between two trees walks up to their roots, and tries to hook one that an L2 still takes for a root:
+        // linking all edges of a graph at once takes 300-570 us at 2^20 vertices of degree 16, and what is in flight when a
+        // stop comes is most of that.  So a few edges of everybody are linked first, and the trees are flattened again before
+        // the others are: then both ends have the same root already, mostly)
         unsigned begin = 0, end = 0;
         if (in) { begin = p.row[v]; end = p.row[v + 1]; }
-        gf_walk(ids, begin, end, v, [&](unsigned, const u32x4 &i, unsigned from) {
+        if (p.level && p.level < 4) {
+            for (unsigned j = 0; j < p.level; ++j) {
+                const unsigned other = begin < end ? p.ids[4ull * begin + j] : n;
+                if (other < n) cc_link(p.parent, v, other);
+            }
+            return false;
+        }
+        if (p.level) end = min(end, begin + 1);
+        return gf_walk(ids, begin, end, v, look, [&](unsigned, const u32x4 &i, unsigned from) {
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 if (i[j] < n) cc_link(p.parent, from, i[j]);
@@ -308,6 +399,7 @@ __device__ __forceinline__ void gf_tile(const gp_graph_iter_params &p, int tile,
     } else {  // GP_GRAPH_IT_CC_LABEL
         if (in) p.comp[v] = cc_root(p.parent, v);
     }
+    return false;
 }
 
 __device__ __forceinline__ unsigned sssp_limit(const gp_graph_iter_params &p, bool *find) {
@@ -335,7 +427,11 @@ __device__ __forceinline__ void report_start(const gp_graph_iter_params &p, cons
     __hip_atomic_store(p.started, (unsigned long long)p.seq << 32 | low, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// a claim of a launch stands for `per` tiles of 256 vertices
+// A claim of a launch stands for `per` tiles of 256 vertices.  In a launch of all its workgroups at once every claim is
+// made when it starts: from then on a stop waits for the whole launch, unless the workgroups give their claims back.  They
+// do where the tiles can be done again and the launch is a long one (gp_launch_graph_iter): a wavefront looks whether it
+// has to between the lists of a quad, a sixteenth of the launch apart.  Stops next to BERT's requests at 2^20 vertices, mean / p99: bfs 30 / 47 us,
+// sssp 39 / 71 (118 / 256 without), pagerank 32 / 57 (51 / 120), connected components 48 / 134 (278 / 598, linked at once).
 template <int KIND, int LOOP = LOOP_ANY>
 __global__ __launch_bounds__(GF_TILE) void graph_iter_kernel(gp_graph_iter_params p, int per, BlpArgs blp) {
     report_start(p, blp);
@@ -351,14 +447,26 @@ __global__ __launch_bounds__(GF_TILE) void graph_iter_kernel(gp_graph_iter_param
     };
     const int known = LOOP == LOOP_ANY || wg_id(blp) < 0 || wg_id(blp) >= blp.total ? -1 : xcd_contiguous(wg_id(blp), blp.total);
     if (known >= 0) look(known * per, per);
-    tiles<LOOP>(blp, [&](TileIdx t) {
+    auto claim = [&](TileIdx t, StopLook stop) {
+        bool left = false;
 #pragma unroll 1
-        for (int j = 0; j < per; ++j) {
+        for (int j = 0; j < per && !left; ++j) {
             if (j % 4 == 0 && (j || known < 0)) look(t.x * per + j, per - j);
-            gf_tile<KIND>(p, t.x * per + j, key[0], limit, find);
+            if (j) stop.ask();
+            left = gf_tile<KIND>(p, t.x * per + j, key[0], limit, find, stop) || (j && stop.told());
             key[0] = key[1]; key[1] = key[2]; key[2] = key[3];
         }
-    });
+        return left;
+    };
+    if constexpr (LOOP == LOOP_FIXED) {
+        if (blp.done && gf_front(blp, p.relay)) return;
+        tile_fixed_early(blp, [&](TileIdx t, int *) {
+            const bool looks = blp.done && gf_repeatable<KIND>(p);
+            const bool left = claim(t, StopLook{looks ? p.relay + kRelayStride * (blockIdx.x / kXcds % GP_GRAPH_RELAYS) : nullptr});
+            return looks ? __syncthreads_or(left) != 0 : false;
+        });
+    } else
+        tiles<LOOP>(blp, [&](TileIdx t) { claim(t, StopLook{}); });
 }
 
 // 64-bit neighbour ids (and weights) into padded vectors of four
@@ -374,22 +482,6 @@ __global__ __launch_bounds__(GF_TILE) void graph_pack_kernel(gp_graph_pack_param
             if (p.weights) p.weights[4ull * c + j] = at + j < to ? p.weight_list[at + j] : 0u;
         }
     }
-}
-
-// one wavefront hands the words of the launches to the host: the words first, then the sequence number it waits for
-__global__ void graph_report_kernel(const unsigned *words, int stride, const int *stop_index, unsigned *host, int n, unsigned seq) {
-    const unsigned stop = stop_index ? (unsigned)*stop_index : 0xFFFFFFFFu;
-    if (n == 0 && ((uintptr_t)host & 7) == 0) {  // (one store needs no release in front of it, which would write this XCD's L2 back)
-        if (threadIdx.x == 0) __hip_atomic_store((unsigned long long *)host, (unsigned long long)stop << 32 | seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        return;
-    }
-    if ((int)threadIdx.x < n) {
-        __hip_atomic_store(host + 2 + 2 * threadIdx.x, words[threadIdx.x * stride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        __hip_atomic_store(host + 3 + 2 * threadIdx.x, words[threadIdx.x * stride + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-    if (threadIdx.x == 0) __hip_atomic_store(host + 1, stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    __threadfence_system();
-    if (threadIdx.x == 0) __hip_atomic_store(host, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 }  // namespace gp
@@ -415,9 +507,20 @@ extern "C" int gp_launch_graph_iter(const gp_graph_iter_params *p, const gp_pree
     // A launch's cost besides its edges is its workgroups (a claim, a barrier: 4096 of them take 12 us): up to eight
     // tiles per claim as long as that leaves four workgroups per compute unit.  The pull wants as many lists in flight
     // as the chip holds and takes one tile at a time.
-    const int per = p->kernel == GP_GRAPH_IT_PR ? 1 : (int)std::min<long>(8, std::max<long>(1, tiles / (4L * device_cus())));
+    int per = p->kernel == GP_GRAPH_IT_PR ? 1 : (int)std::min<long>(8, std::max<long>(1, tiles / (4L * device_cus())));
+    // A preemptible launch that may walk a million edges (20 us) is one whose claims are given back behind a stop.  Where
+    // they cannot be (no counters for it, or more claims than a launch with fixed claims takes), they are as small as they
+    // get.  (The other kernels are done in 40 us at 2^20 vertices.)
+    const bool walks = p->kernel == GP_GRAPH_IT_BFS || p->kernel == GP_GRAPH_IT_SSSP || p->kernel == GP_GRAPH_IT_CC_LINK || p->kernel == GP_GRAPH_IT_PR || p->kernel == GP_GRAPH_IT_PR_STEP;
+    const bool far = ctx && walks && p->row_end >= (1u << 18);
+    const bool gives_back = far && ctx->done && p->relay && ctx->counter_groups > 1 && ctx->poll_every != 1 && tiles / per <= 32L * device_cus();
+    if (far && !gives_back) per = 1;
+    auto launch = [&](auto kernels) {
+        kernels.long_tiles = gives_back;
+        return launch_tiles(kernels, (int)((tiles + per - 1) / per), 1, ctx, s, info, *p, 0, far ? 1 : 4, GF_TILE, per);
+    };
     switch (p->kernel) {
-#define GP_GI(K) case K: return launch_tiles(GP_KSET(graph_iter_kernel<K), (int)((tiles + per - 1) / per), 1, ctx, s, info, *p, 0, 4, GF_TILE, per);
+#define GP_GI(K) case K: return launch(GP_KSET(graph_iter_kernel<K));
         GP_GI(GP_GRAPH_IT_BFS) GP_GI(GP_GRAPH_IT_BFS_INIT) GP_GI(GP_GRAPH_IT_SSSP) GP_GI(GP_GRAPH_IT_SSSP_INIT) GP_GI(GP_GRAPH_IT_PR)
         GP_GI(GP_GRAPH_IT_PR_PUSH) GP_GI(GP_GRAPH_IT_PR_STEP) GP_GI(GP_GRAPH_IT_PR_INIT) GP_GI(GP_GRAPH_IT_CC_INIT) GP_GI(GP_GRAPH_IT_CC_LINK)
         GP_GI(GP_GRAPH_IT_CC_FLATTEN) GP_GI(GP_GRAPH_IT_CC_LABEL)
@@ -432,13 +535,6 @@ extern "C" int gp_graph_pack_async(const gp_graph_pack_params *p, gp_stream s) {
     GP_REQUIRE(!p->weights == !p->weight_list, "graph pack: weights come together");
     GP_REQUIRE(p->vertex_count > 0 && p->vertex_count < (1u << 31), "graph: vertex count out of range");
     hipLaunchKernelGGL(graph_pack_kernel, dim3((p->vertex_count + GF_TILE / 4 - 1) / (GF_TILE / 4)), dim3(GF_TILE), 0, native(s), *p);
-    GP_HIP(hipGetLastError());
-    return GP_SUCC;
-}
-
-extern "C" int gp_graph_report_async(const unsigned *words, int n, int stride, const int *stop_index, unsigned *host_words, unsigned seq, gp_stream s) {
-    GP_REQUIRE(words && host_words && n >= 0 && n <= 64 && stride >= 2, "graph report: 0..64 pairs of words");
-    hipLaunchKernelGGL(graph_report_kernel, dim3(1), dim3(64), 0, native(s), words, stride, stop_index, host_words, n, seq);
     GP_HIP(hipGetLastError());
     return GP_SUCC;
 }

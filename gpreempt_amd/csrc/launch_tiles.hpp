@@ -7,8 +7,8 @@
 namespace gp {
 
 // the three instantiations of one kernel: general dispatcher loop, no counters, fixed claims
-template <class Kernel> struct KernelSet { Kernel any, plain, fixed; };
-template <class Kernel> static KernelSet<Kernel> kernel_set(Kernel a, Kernel p, Kernel f) { return {a, p, f}; }
+template <class Kernel> struct KernelSet { Kernel any, plain, fixed; bool long_tiles = false; };  // (long_tiles: see plan_launch)
+template <class Kernel> static KernelSet<Kernel> kernel_set(Kernel a, Kernel p, Kernel f) { return {a, p, f, false}; }
 #define GP_KSET(...) kernel_set(__VA_ARGS__, LOOP_ANY>, __VA_ARGS__, LOOP_PLAIN>, __VA_ARGS__, LOOP_FIXED>)
 
 // `more`: kernel arguments between the operator's parameters and the dispatcher's
@@ -28,7 +28,7 @@ static int launch_tiles(KernelSet<Kernel> ks, int sx, int sy, const gp_preempt_c
         }
     }
     // planned for the general form; the special ones need no more resources
-    int rc = plan_launch(ks.any, block, lds_bytes, sx, sy, 1, ctx, &blp, &grid, info, batch, batch == 1 ? 4 : 1);
+    int rc = plan_launch(ks.any, block, lds_bytes, sx, sy, 1, ctx, &blp, &grid, info, batch, batch == 1 ? 4 : 1, ks.long_tiles && batch == 1);
     if (rc) return rc;
     Kernel kern = ks.any;
     if (batch == 1) {  // the special forms call the body once: one tile per claim only

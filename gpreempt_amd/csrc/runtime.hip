@@ -76,6 +76,14 @@ __global__ __launch_bounds__(256) void host_copy_kernel(unsigned char *dst, cons
     __hip_atomic_store(done, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// hands the stop index to a host that spins on the word: one store, so nothing has to be released in front of it, which
+// would write an XCD's L2 back under whoever has the GPU by now
+__global__ void report_stop_kernel(const int *stop_index, unsigned long long *host_word, unsigned seq) {
+    if (threadIdx.x != 0) return;
+    const int stop = stop_index ? __hip_atomic_load(stop_index, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : -1;
+    __hip_atomic_store(host_word, (unsigned long long)(unsigned)stop << 32 | seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // stores the device's constant-rate clock where the host can see it
 __global__ void clock_probe_kernel(unsigned long long *host_word) {
     if (threadIdx.x == 0) __hip_atomic_store(host_word, (unsigned long long)wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -441,6 +449,13 @@ extern "C" int gp_device_clock(gp_stream s, int rounds, double *tick_ns, double 
 extern "C" int gp_store_word_async(gp_stream s, int *word_dev, int value) {
     GP_REQUIRE(word_dev != nullptr, "gp_store_word_async: null word");
     hipLaunchKernelGGL(store_word_kernel, dim3(1), dim3(64), 0, native(s), word_dev, value);
+    GP_HIP(hipGetLastError());
+    return GP_SUCC;
+}
+
+extern "C" int gp_report_stop_async(const int *stop_index, unsigned long long *word_dev, unsigned seq, gp_stream s) {
+    GP_REQUIRE(word_dev != nullptr && ((uintptr_t)word_dev & 7) == 0, "gp_report_stop_async: an aligned 64-bit word");
+    hipLaunchKernelGGL(report_stop_kernel, dim3(1), dim3(64), 0, native(s), stop_index, word_dev, seq);
     GP_HIP(hipGetLastError());
     return GP_SUCC;
 }

@@ -326,6 +326,11 @@ Status Workload::run_kernels(const std::vector<int> &kernels, GPUstream stream, 
     return Status::Succ;
 }
 
+// A launch's slot: its words, the claim counters and as many counters of the workgroups that have left it
+// (gp_preempt_ctx::done).  Behind the slots, gp_graph_iter_params::relay.
+static size_t per_kernel_ints(const PreemptEnv *env) { return (size_t)env->counter_groups * env->counter_stride; }
+constexpr size_t kWords = 16, kRelayInts = GP_GRAPH_RELAYS * 32;
+
 Status Workload::launch_slot(int i, bool fresh, GPUstream stream, const PreemptEnv *env) {
     gp_graph_iter_params p = queued_[i % kRing];
     int *slot = (int *)ring_ + slot_ints_ * (i % kRing);
@@ -337,9 +342,11 @@ Status Workload::launch_slot(int i, bool fresh, GPUstream stream, const PreemptE
     if (env) {
         std::memset(&ctx, 0, sizeof(ctx));
         ctx.flag = (int *)env->flag; ctx.stop_index = (int *)env->stop_index;
-        ctx.executed = slot + 16;
+        ctx.executed = slot + kWords;
         ctx.kernel_id = i % kRing; ctx.inject_at = -1; ctx.fresh = fresh;
         ctx.poll_every = env->poll_every; ctx.counter_groups = env->counter_groups;
+        ctx.done = slot + kWords + per_kernel_ints(env);
+        p.relay = (unsigned *)ring_ + slot_ints_ * kRing;
     }
     GC_CHECK(gp_launch_graph_iter(&p, env ? &ctx : nullptr, stream, nullptr));
     ++launches_;
@@ -349,12 +356,13 @@ Status Workload::launch_slot(int i, bool fresh, GPUstream stream, const PreemptE
 // Queues one launch behind the others.  The words and claim counters of half the ring are cleared at a time, in stream
 // order behind the launches that used them last.
 Status Workload::submit(const gp_graph_iter_params &p, GPUstream stream, const PreemptEnv *env) {
-    const size_t slot_ints = 16 + (env ? (size_t)env->counter_groups * env->counter_stride : 0);
+    const size_t slot_ints = kWords + (env ? 2 * per_kernel_ints(env) : 0);
     if (slot_ints != slot_ints_) {
         if (ring_) gp_free(ring_);
         ring_ = nullptr; slot_ints_ = 0;
-        GC_CHECK(gp_malloc(&ring_, slot_ints * kRing * sizeof(int)));
+        GC_CHECK(gp_malloc(&ring_, (slot_ints * kRing + kRelayInts) * sizeof(int)));
         slot_ints_ = slot_ints;
+        GC_CHECK(gp_fill32_async((int *)ring_ + slot_ints * kRing, 0, kRelayInts, stream));
     }
     const int i = submitted_++;
     if (i % (kRing / 2) == 0) GC_CHECK(gp_fill32_async((int *)ring_ + slot_ints_ * (i % kRing), 0, slot_ints_ * (kRing / 2), stream));
@@ -362,38 +370,27 @@ Status Workload::submit(const gp_graph_iter_params &p, GPUstream stream, const P
     return launch_slot(i, true, stream, env);
 }
 
-// Spins until a word of host memory says so: a blocked thread wakes up tens of microseconds late, a query of the stream
-// costs microseconds.  (One is made now and then, so that an error of the device ends the wait.)
-template <class There>
-static Status spin(GPUstream stream, There &&there) {
-    for (unsigned spins = 1;; ++spins) {
-        int idle = 0;
-        if (spins % (1u << 16) == 0) GC_CHECK(gp_stream_query(stream, &idle));
-        if (there()) return Status::Succ;
-        if (idle) {
-            std::fprintf(stderr, "graph workload: a launch did not report\n");
-            return Status::Fail;
-        }
-    }
-}
-
 // Waits until everything queued has left the GPU; *stop receives the slot of the launch that was stopped, or -1.
 Status Workload::drain(GPUstream stream, const PreemptEnv *env, int *stop) {
-    GC_CHECK(gp_graph_report_async((const unsigned *)ring_, 0, (int)slot_ints_, env ? (const int *)env->stop_index : nullptr,
-                                   (unsigned *)((unsigned long long *)starts_dev_ + kRing), ++seq_, stream));
-    unsigned long long report = 0;  // the stop index and the sequence number
-    RETURN_STATUS(spin(stream, [&] { report = __atomic_load_n(starts_ + kRing, __ATOMIC_ACQUIRE); return (unsigned)report == seq_; }));
+    GC_CHECK(gp_report_stop_async(env ? (const int *)env->stop_index : nullptr, (unsigned long long *)starts_dev_ + kRing, ++seq_, stream));
+    unsigned long long report = 0;
+    RETURN_STATUS(spin_until(stream, [&] { report = __atomic_load_n(starts_ + kRing, __ATOMIC_ACQUIRE); return (unsigned)report == seq_; }));
     *stop = (int)(report >> 32);
     return Status::Succ;
 }
 
-// A launch was stopped and nothing of this run is on the GPU: when it is this workload's turn again, that launch is
+// A launch was stopped and this run has left the GPU: when it is this workload's turn again, that launch is
 // queued once more, and the ones behind it with it (they left when they found the stop recorded).
 Status Workload::restart(int stop, GPUstream stream, const PreemptEnv *env) {
     RETURN_STATUS(wait_turn(stream, env));
     int from = submitted_ - 1;
     while (from > 0 && from % kRing != stop) --from;
-    for (int i = from; i < submitted_; ++i) RETURN_STATUS(launch_slot(i, false, stream, env));
+    GC_CHECK(gp_fill32_async((int *)ring_ + slot_ints_ * kRing, 0, kRelayInts, stream));
+    for (int i = from; i < submitted_; ++i) {
+        // (a launch that left in front of its first claim counted nobody: the count of leavers starts again)
+        GC_CHECK(gp_fill32_async((int *)ring_ + slot_ints_ * (i % kRing) + kWords + per_kernel_ints(env), 0, per_kernel_ints(env), stream));
+        RETURN_STATUS(launch_slot(i, false, stream, env));
+    }
     return Status::Succ;
 }
 
@@ -410,18 +407,27 @@ Status Workload::settle(GPUstream stream, const PreemptEnv *env) {
 // Waits until launch `i` starts, i.e. until the ones before it are done.  *changed: the iteration before it changed
 // something; *count: of how many vertices over the tolerance it knows.
 Status Workload::await_start(int i, GPUstream stream, const PreemptEnv *env, bool *changed, unsigned *count) {
+    auto start_of = [&](int k, unsigned *low) {
+        return spin_until(stream, [&] {
+            const unsigned long long word = __atomic_load_n(starts_ + k % kRing, __ATOMIC_ACQUIRE);
+            *low = (unsigned)word;
+            return (unsigned)(word >> 32) == seq_of_[k % kRing];
+        });
+    };
     for (;;) {
-        unsigned long long word = 0;  // the sequence number and what the launch knows
-        RETURN_STATUS(spin(stream, [&] { word = __atomic_load_n(starts_ + i % kRing, __ATOMIC_ACQUIRE); return (unsigned)(word >> 32) == seq_of_[i % kRing]; }));
-        const unsigned low = (unsigned)word;
+        unsigned low = 0;
+        RETURN_STATUS(start_of(i, &low));
         if (!(low & GP_GRAPH_START_STOPPED)) {
             *changed = (low & GP_GRAPH_START_CHANGED) != 0;
             *count = low & GP_GRAPH_START_COUNT;
             return Status::Succ;
         }
-        int stop = -1;
-        RETURN_STATUS(drain(stream, env, &stop));
-        RETURN_STATUS(restart(stop, stream, env));
+        // A stop is recorded.  The GPU is vacated when the last launch queued has started, as it finds nothing to do.  (That
+        // is known from what is in the queue already: a report submitted now can come to stand behind the work of whoever
+        // raised the flag, where the two streams share a hardware queue.)
+        unsigned other = 0;
+        for (int k = i + 1; k < submitted_; ++k) RETURN_STATUS(start_of(k, &other));
+        RETURN_STATUS(restart((int)(low & ~GP_GRAPH_START_STOPPED), stream, env));
     }
 }
 
@@ -451,8 +457,19 @@ Status Workload::compute(GPUstream stream, const PreemptEnv *env) {
     if (!row_ || (env && env->inject_kernel >= 0 && env->inject_iteration >= -1)) return compute_stepwise(stream, env);
     iterations_ = submitted_ = 0;
     if (kind_ == "cc") {
-        iterations_ = 3;  // the passes behind the set-up one
-        for (int kernel : {GP_GRAPH_IT_CC_INIT, GP_GRAPH_IT_CC_FLATTEN, GP_GRAPH_IT_CC_LINK, GP_GRAPH_IT_CC_LABEL}) RETURN_STATUS(submit(params(kernel), stream, env));
+        iterations_ = 3;  // (linking, flattening, labels)
+        // (a graph of a million edges and more in three steps, by the first two neighbours, the first four and all of them:
+        // 2^20 vertices of degree 16 take 290 us, at once 500-600, of which a stop waited for half; on a small graph the
+        // launches more cost 8 us)
+        RETURN_STATUS(submit(params(GP_GRAPH_IT_CC_INIT), stream, env));
+        for (unsigned neighbours : {2u, 4u, 0u}) {
+            if (neighbours && row_end_ < (1u << 18)) continue;
+            RETURN_STATUS(submit(params(GP_GRAPH_IT_CC_FLATTEN), stream, env));
+            gp_graph_iter_params link = params(GP_GRAPH_IT_CC_LINK);
+            link.level = neighbours;
+            RETURN_STATUS(submit(link, stream, env));
+        }
+        RETURN_STATUS(submit(params(GP_GRAPH_IT_CC_LABEL), stream, env));
         return settle(stream, env);
     }
     const bool bfs = kind_ == "bfs", pagerank = kind_ == "pagerank";

@@ -105,6 +105,9 @@ int gp_flag_destroy(volatile int *host_ptr);
  * "has my stream drained" (src/cuda-clients/blpclient.cpp:189-195 spins on a counter for the same purpose) uses
  * instead of stream queries, which cost 3-5 us apiece once the stream's last command is a kernel. */
 int gp_store_word_async(gp_stream s, int *word_dev, int value);
+/* The same with the stop index along (gp_preempt_ctx::stop_index; NULL counts as -1): stores (stop index << 32 | seq) in
+ * an aligned 64-bit word of gp_host_alloc_coherent. */
+int gp_report_stop_async(const int *stop_index, unsigned long long *word_dev, unsigned int seq, gp_stream s);
 /* Flag relay: one small resident kernel copies n host flag words (device-visible addresses of
  * gp_flag_create flags, flags_dev[i]) into device memory (mirror[i]) whenever they change, so
  * that kernels can poll a device address on every claim instead of crossing PCIe; a host store
@@ -452,7 +455,7 @@ int gp_launch_graph(const gp_graph_params *p, const gp_preempt_ctx *ctx, gp_stre
  *   PR_STEP      residual += gained (which is cleared), the update as in PR, and what a vertex over the tolerance hands
  *                out is pushed into next_gained; with next_gained NULL it is left in next_share
  *   CC_*         union-find: INIT hooks every vertex to its first neighbour if that is smaller, LINK joins the ends of
- *                every edge, FLATTEN points every vertex at its root, LABEL writes the root (the smallest id of the
+ *                every edge, or with level = 1 .. 4 those to everybody's first neighbours, FLATTEN points every vertex at its root, LABEL writes the root (the smallest id of the
  *                component) to comp
  * *changed is set to 1 by an iteration that changed something; changed[1] counts the vertices over the tolerance in
  * every GP_GRAPH_SAMPLED-th tile (PR, PR_STEP) or says whether anybody improved below the limit, which is changed[2]
@@ -460,7 +463,12 @@ int gp_launch_graph(const gp_graph_params *p, const gp_preempt_ctx *ctx, gp_stre
  * before: a launch that finds it 0 does nothing (so several iterations can be queued without a look in between).
  * started, if given, is a device-visible word of host memory (gp_host_alloc_coherent) in which the launch stores, when it
  * starts, seq in the upper half and in the lower one what is known then: GP_GRAPH_START_STOPPED | the stop index if a stop
- * is recorded, else GP_GRAPH_START_CHANGED unless *prev_changed is 0, and prev_changed[1] (at most GP_GRAPH_START_COUNT). */
+ * is recorded, else GP_GRAPH_START_CHANGED unless *prev_changed is 0, and prev_changed[1] (at most GP_GRAPH_START_COUNT).
+ * A preemptible launch over a million edges and more that comes with gp_preempt_ctx::done counters (done_launches 0: cleared
+ * before every launch) and with relay (GP_GRAPH_RELAYS words 128 bytes apart, cleared before the launch that follows a
+ * stop) gives the claims back that it is in when a stop is recorded, where the kernel allows it (BFS, SSSP, CC_LINK,
+ * PR_STEP with next_gained); the relaunch does them again. */
+#define GP_GRAPH_RELAYS 64
 #define GP_GRAPH_START_STOPPED 0x80000000u
 #define GP_GRAPH_START_CHANGED 0x40000000u
 #define GP_GRAPH_START_COUNT 0x3FFFFFFFu
@@ -483,6 +491,7 @@ typedef struct gp_graph_iter_params {
     const unsigned int *prev_changed;
     unsigned long long *started;             /* may be NULL */
     unsigned int seq;
+    unsigned int *relay;                     /* may be NULL */
 } gp_graph_iter_params;
 int gp_launch_graph_iter(const gp_graph_iter_params *p, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info);
 /* fills ids (4 * row_end + 4 of them: a last vector of vertex_count lies behind the lists) and weights of that layout from
@@ -495,10 +504,6 @@ typedef struct gp_graph_pack_params {
     unsigned int *ids, *weights;
 } gp_graph_pack_params;
 int gp_graph_pack_async(const gp_graph_pack_params *p, gp_stream s);
-/* Stores the pairs words[i * stride], words[i * stride + 1] (i < n) and *stop_index (-1 without one) into pinned host
- * memory (host_words[2 + 2 i], host_words[3 + 2 i] and host_words[1]), then seq into host_words[0].  With n == 0 and
- * host_words a multiple of 8 the two words are one store, and the GPU's caches are left alone. */
-int gp_graph_report_async(const unsigned int *words, int n, int stride, const int *stop_index, unsigned int *host_words, unsigned int seq, gp_stream s);
 
 /* out[t,:] = tok[ids[t],:] + pos[t % seq,:] (+ seg[0,:]); ids are int64 (the reference feeds
  * BERT int64 token ids, src/tests/test-dnn.cpp:21-23). */

@@ -60,6 +60,21 @@ namespace util {
 // (reference src/util/gpu_util.cpp:14-25).
 void init_cuda();
 
+// Spins until a word of host memory that the stream's work stores says so: a blocked thread wakes up tens of microseconds
+// late, a query of the stream costs microseconds.  (One is made now and then, so that an error of the device ends the wait.)
+template <class There>
+Status spin_until(GPUstream stream, There &&there) {
+    for (unsigned spins = 1;; ++spins) {
+        int idle = 0;
+        if (spins % (1u << 16) == 0) CUDA_RETURN_STATUS(gp_stream_query(stream, &idle));
+        if (there()) return Status::Succ;
+        if (idle) {
+            std::fprintf(stderr, "the stream is idle and a word is missing\n");
+            return Status::Fail;
+        }
+    }
+}
+
 class SizedGPUBuffer {
 public:
     explicit SizedGPUBuffer(size_t size);

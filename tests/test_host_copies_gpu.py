@@ -44,6 +44,22 @@ def test_pool_memory_comes_back_and_is_bounded(gp):
     assert pd is None and d.nbytes == 2 << 20
 
 
+def test_sizes_mixed_on_one_handle(gp):
+    """the count of arrivals goes on from copy to copy, whatever number of workgroups each of them has"""
+    rng = np.random.default_rng(5)
+    st, stream = C.c_void_p(), gp.Stream()
+    gp.check(gp.lib().gp_stage_create(C.byref(st)))
+    dev = gp.DevBuf(3 << 20)
+    for r in range(40):
+        n = int(rng.choice([1, 5000, 40000, 70001, 300000, 1 << 20, 3 << 20]))
+        want = rng.integers(0, 256, n, np.uint8)
+        gp.check(gp.lib().gp_stage_upload_async(st, C.c_void_p(dev.ptr), want.ctypes.data_as(C.c_void_p), C.c_size_t(n), stream.h))
+        out, pinned = gp.host_pool.empty(n)
+        gp.check(gp.lib().gp_fetch(C.c_void_p(pinned), C.c_void_p(dev.ptr), C.c_size_t(n), stream.h))
+        assert np.array_equal(out, want), (n, r)
+    gp.check(gp.lib().gp_stage_destroy(st))
+
+
 @pytest.mark.parametrize("stop", [None, -1, 0, 37, 0x7FFFFFFF])
 def test_stop_index_is_reported_with_its_number(gp, stop):
     host, dev = C.c_void_p(), C.c_void_p()

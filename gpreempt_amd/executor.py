@@ -12,7 +12,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libgpreempt_exec.so")
 vp = C.c_void_p
 
-SYMBOLS = """gpx_create gpx_destroy gpx_init gpx_set_input gpx_get_output gpx_fetch_output gpx_get_data_size gpx_execute
+SYMBOLS = """gpx_create gpx_destroy gpx_init gpx_set_input gpx_set_input_pinned gpx_get_output gpx_fetch_output gpx_get_data_size gpx_execute
 gpx_launch_kernel gpx_get_kernel_num gpx_capture_graph gpx_uses_program gpx_clear gpx_set_flag gpx_set_running gpx_resume
 gpx_get_stop_point gpx_last_stop_index gpx_inject_preempt gpx_read_counters gpx_reset_counters gpx_storage_num gpx_storage_info
 gpx_kernel_info gpx_read_storage gpx_miniweather_reductions gpx_graph_info gpx_graph_result_bytes gpx_graph_result gpx_graph_fetch_result

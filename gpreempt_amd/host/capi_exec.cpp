@@ -56,6 +56,7 @@ gpx_executor gpx_create(int blp) {
 void gpx_destroy(gpx_executor e) { delete H(e); }
 int gpx_init(gpx_executor e, const char *workload) { return guarded("gpx_init", [&] { return H(e)->ex->init(workload ? workload : ""); }); }
 int gpx_set_input(gpx_executor e, const char *key, void *value, size_t len, gp_stream s) { return H(e)->ex->set_input(key, value, len, s); }
+int gpx_set_input_pinned(gpx_executor e, const char *key, const void *pinned, size_t len, gp_stream s) { return H(e)->ex->set_input_pinned(key, pinned, len, s); }
 int gpx_get_output(gpx_executor e, const char *key, void *value, size_t len, gp_stream s) { return H(e)->ex->get_output(key, value, len, s); }
 int gpx_fetch_output(gpx_executor e, const char *key, void *pinned, size_t len, gp_stream s) { return H(e)->ex->fetch_output(key, pinned, len, s); }
 size_t gpx_get_data_size(gpx_executor e, const char *key) { return H(e)->ex->get_data_size(key); }

@@ -83,6 +83,11 @@ Status Executor::set_input(const std::string &key, void *value, size_t len, GPUs
 Status Executor::set_input(const std::string &key, std::vector<float> &value, GPUstream stream) {
     return set_input(key, value.data(), value.size() * sizeof(float), stream);
 }
+Status Executor::set_input_pinned(const std::string &key, const void *pinned, size_t len, GPUstream stream) {
+    size_t idx;
+    if (!model || model->find_storage_idx(key, idx) != Status::Succ) return Status::NotFound;
+    return model->set_pinned(idx, pinned, len, stream);
+}
 Status Executor::get_output(const std::string &key, void *value, size_t len, GPUstream stream) {
     size_t idx;
     if (!model || model->find_storage_idx(key, idx) != Status::Succ) return Status::NotFound;

@@ -731,7 +731,7 @@ Status infer_once(Tenant &t, Shared &sh, double *total_us, double *infer_us) {
     // "resident_io": operands stay in device memory (a 8192^2 matrix is 134 MB: copied per
     // request it would be the whole request); the input is uploaded once, the output never read back
     if (t.input_size && (!t.resident_io || !t.input_resident)) {
-        RETURN_STATUS(t.ex->set_input("data", t.input, t.input_size, t.stream));
+        RETURN_STATUS(t.ex->set_input_pinned("data", t.input, t.input_size, t.stream));
         CUDA_RETURN_STATUS(gp_stream_sync(t.stream));
         t.input_resident = true;
     }

@@ -397,9 +397,15 @@ Status Model::set(size_t idx, void *value, size_t len, GPUstream stream) {
     if (idx >= storages.size()) return Status::OutOfRange;
     size_t size = storage_infos[idx].size;
     if (len < size) return Status::OutOfRange;
-    // (through the model's own pinned ring; memory that is pinned itself would be read in place, but nothing here says so)
+    // (through the model's own pinned ring: the value may be gone when this returns)
     if (!stage_) CUDA_RETURN_STATUS(gp_stage_create(&stage_));
     CUDA_RETURN_STATUS(gp_stage_upload_async(stage_, storages[idx], value, size, stream));
+    return Status::Succ;
+}
+Status Model::set_pinned(size_t idx, const void *value, size_t len, GPUstream stream) {
+    if (idx >= storages.size()) return Status::OutOfRange;
+    if (len < storage_infos[idx].size) return Status::OutOfRange;
+    CUDA_RETURN_STATUS(gp_memcpy_h2d_async(storages[idx], value, storage_infos[idx].size, stream));
     return Status::Succ;
 }
 Status Model::fetch(size_t idx, void *pinned, size_t len, GPUstream stream) {

@@ -36,6 +36,8 @@ public:
     virtual Status set_input(const std::string &key, std::vector<float> &value, GPUstream stream);
     virtual Status get_output(const std::string &key, void *value, size_t len, GPUstream stream);
     virtual Status get_output(const std::string &key, std::vector<float> &value, GPUstream stream);
+    // as set_input, from memory of gp_host_alloc or gp_host_alloc_coherent that stays as it is until the stream has read it
+    Status set_input_pinned(const std::string &key, const void *pinned, size_t len, GPUstream stream);
     // as get_output, into memory of gp_host_alloc_coherent; returns when the values are there
     Status fetch_output(const std::string &key, void *pinned, size_t len, GPUstream stream);
     virtual size_t get_data_size(const std::string &key);

@@ -20,6 +20,7 @@ gpx_executor gpx_create(int block_level_preemptible); /* 0: foo::BaseExecutor, 1
 void gpx_destroy(gpx_executor e);
 int gpx_init(gpx_executor e, const char *workload);                 /* Executor::init */
 int gpx_set_input(gpx_executor e, const char *key, void *value, size_t len, gp_stream s);  /* Executor::set_input */
+int gpx_set_input_pinned(gpx_executor e, const char *key, const void *pinned, size_t len, gp_stream s); /* Executor::set_input_pinned */
 int gpx_get_output(gpx_executor e, const char *key, void *value, size_t len, gp_stream s); /* Executor::get_output */
 int gpx_fetch_output(gpx_executor e, const char *key, void *pinned, size_t len, gp_stream s); /* Executor::fetch_output */
 size_t gpx_get_data_size(gpx_executor e, const char *key);          /* Executor::get_data_size */

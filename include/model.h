@@ -132,6 +132,9 @@ public:
     Status fetch(size_t idx, void *pinned, size_t len, GPUstream stream);
     Status set(size_t idx, void *value, size_t len, GPUstream stream);
     Status set(const std::string &key, void *value, size_t len, GPUstream stream);
+    // as set, from memory of gp_host_alloc or gp_host_alloc_coherent, which is read in place: it stays as it is until the
+    // stream has got there.  One transfer by the copy engine, which a tenant next door does not feel, and never a wait.
+    Status set_pinned(size_t idx, const void *value, size_t len, GPUstream stream);
 
     static size_t get_stype_size(std::string &stype);
     Status find_storage_idx(const std::string &name, size_t &idx);

@@ -75,3 +75,41 @@ def test_stop_index_is_reported_with_its_number(gp, stop):
     gp.check(gp.lib().gp_host_free(host))
     with pytest.raises(gp.GpError):
         gp.check(gp.lib().gp_report_stop_async(None, None, C.c_uint(1), stream.h))
+
+
+class ClosedGate:
+    """A gate kernel at the head of a stream: what is submitted behind it waits until open() (about a second at most)."""
+
+    def __init__(self, gp, stream):
+        self.gp, self.flag, self.gave_up = gp, gp.Flag(), gp.DevBuf(4)
+        self.gave_up.fill32(0)
+        gp.check(gp.lib().gp_launch_gate(C.c_void_p(self.flag.dev), C.c_ulonglong(1 << 22), C.c_void_p(self.gave_up.ptr), stream.h))
+
+    def open(self):
+        self.flag.set(1)
+
+    def was_open_early(self):
+        return bool(self.gave_up.download(np_dtype=np.int32)[0])
+
+
+def test_pinned_input_is_read_in_place_and_without_a_wait(gp):
+    """set_input_pinned: one transfer in stream order; the call returns while the stream is held up"""
+    from gpreempt_amd import executor as gx
+    rows, cols = 1024, 4096  # 16 MB
+    ex = gx.Executor("toy@rows=%d,cols=%d,n=1,dtype=f32" % (rows, cols))
+    n = rows * cols * 4
+    host, dev = C.c_void_p(), C.c_void_p()
+    gp.check(gp.lib().gp_host_alloc_coherent(C.byref(host), C.byref(dev), C.c_size_t(n)))
+    x = np.frombuffer((C.c_char * n).from_address(host.value), np.float32)
+    x[:] = np.random.default_rng(1).standard_normal(x.size, np.float32)
+    stream = gp.Stream()
+    gate = ClosedGate(gp, stream)
+    assert gx.lib().gpx_set_input_pinned(ex.h, b"data", host, C.c_size_t(n), stream.h) == 0
+    assert not stream.idle()
+    gate.open()
+    stream.sync()
+    assert not gate.was_open_early()
+    assert np.array_equal(ex.read_storage("data").view(np.float32), x)
+    assert gx.lib().gpx_set_input_pinned(ex.h, b"data", host, C.c_size_t(n - 1), stream.h) == 4  # OutOfRange, as set_input
+    assert gx.lib().gpx_set_input_pinned(ex.h, b"nothing", host, C.c_size_t(n), stream.h) == 3   # NotFound
+    gp.check(gp.lib().gp_host_free(host))

@@ -398,7 +398,10 @@ Status Model::set(size_t idx, void *value, size_t len, GPUstream stream) {
     size_t size = storage_infos[idx].size;
     if (len < size) return Status::OutOfRange;
     // (through the model's own pinned ring: the value may be gone when this returns)
-    if (!stage_) CUDA_RETURN_STATUS(gp_stage_create(&stage_));
+    {
+        std::lock_guard<std::mutex> lock(stage_mu_);
+        if (!stage_) CUDA_RETURN_STATUS(gp_stage_create(&stage_));
+    }
     CUDA_RETURN_STATUS(gp_stage_upload_async(stage_, storages[idx], value, size, stream));
     return Status::Succ;
 }

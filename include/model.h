@@ -7,6 +7,7 @@
 #pragma once
 #include <cstdint>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <unordered_map>
 #include <vector>
@@ -201,7 +202,8 @@ public:
 private:
     bool loaded_ = false;
     gp_program program_ = nullptr;
-    gp_stage stage_ = nullptr;  // pinned ring the inputs go through; made by the first set()
+    gp_stage stage_ = nullptr;  // pinned ring the inputs go through; made by the first set(), whichever thread that is
+    std::mutex stage_mu_;
     int counter_groups_ = 1;
     int poll_every_ = 0;
     std::vector<char> fresh_;

@@ -268,10 +268,10 @@ struct CopyDone {
         if (arrived) hipFree(arrived);
     }
     bool reached(unsigned s) const { return (int)(__atomic_load_n(word, __ATOMIC_ACQUIRE) - s) >= 0; }
-    int wait(unsigned s, hipStream_t stream) const {
+    int wait(unsigned s) const {
         for (unsigned spins = 1; !reached(s); ++spins) {
             if (spins % (1u << 16)) continue;
-            const hipError_t e = hipStreamQuery(stream);  // an error of the device ends the wait
+            const hipError_t e = hipStreamQuery(nullptr);  // an error of the device ends the wait (the copy's own stream may be gone by now)
             if (e != hipSuccess && e != hipErrorNotReady) { set_error("host copy: %s", hipGetErrorString(e)); return GP_FAIL; }
         }
         return GP_SUCC;
@@ -305,67 +305,94 @@ extern "C" int gp_fetch(void *host, const void *dev, size_t bytes, gp_stream s) 
     }
     int rc = c.word ? GP_SUCC : c.create();
     if (rc == GP_SUCC) rc = c.launch<true>(host, dev, bytes, native(s));
-    if (rc == GP_SUCC) rc = c.wait(c.seq, native(s));
+    if (rc == GP_SUCC) rc = c.wait(c.seq);
     if (rc) return rc;  // (a copy that may still be under way keeps its words)
     std::lock_guard<std::mutex> lock(g_copies_mu);
     g_copies.push_back(c);
     return GP_SUCC;
 }
 
+// A ring whose pieces report for themselves: a piece is free again when its own copy has read it, whatever stream that was
+// on and whatever the others do.  It starts with eight pieces and grows while its streams are held up (behind a gate, a
+// suspended tenant), up to kMost bytes; from there on an upload waits for the piece that has been in use longest.
 struct gp_stage_s {
-    static constexpr size_t kPiece = 1u << 20;
-    static constexpr int kPieces = 8;
+    static constexpr size_t kPiece = 1u << 20, kMost = 64u << 20;
+    static constexpr int kPerBlock = 8;
+    struct Piece { unsigned char *host, *dev; size_t room; CopyDone done; unsigned long long turn; };
+    struct Block { void *host; void *arrived; };
     std::mutex mu;
-    CopyDone done;
-    unsigned char *ring = nullptr, *ring_dev = nullptr;
-    size_t piece = 0;                 // bytes per piece of the ring
-    unsigned used[kPieces] = {};      // the copy that last read the piece; 0: none
-    unsigned next = 0;
-    hipStream_t last = nullptr;
+    std::vector<Piece> pieces;
+    std::vector<Block> blocks;
+    size_t total = 0;
+    unsigned long long turns = 0;
+
+    // eight pieces of `room` bytes, with the words they report through (the counters are cleared here and now: the stream that
+    // asks may be held up while another one takes the next piece)
+    int grow(size_t room) {
+        Block b{};
+        unsigned char *dev = nullptr;
+        const size_t words = kPerBlock * 64;
+        if (int rc = gp_host_alloc_coherent(&b.host, (void **)&dev, room * kPerBlock + words)) return rc;
+        int rc = gp_malloc(&b.arrived, kPerBlock * 64);
+        if (rc == GP_SUCC) rc = gp_fill32_async(b.arrived, 0, kPerBlock * 16, nullptr) || gp_stream_sync(nullptr) ? GP_FAIL : GP_SUCC;
+        if (rc != GP_SUCC) { hipHostFree(b.host); if (b.arrived) hipFree(b.arrived); return rc; }
+        for (int k = 0; k < kPerBlock; ++k) {
+            Piece p{(unsigned char *)b.host + words + k * room, dev + words + k * room, room, {}, 0};
+            p.done.word = (unsigned *)((unsigned char *)b.host + 64 * k);
+            p.done.word_dev = (unsigned *)(dev + 64 * k);
+            p.done.arrived = (unsigned *)b.arrived + 16 * k;
+            pieces.push_back(p);
+        }
+        blocks.push_back(b);
+        total += room * kPerBlock;
+        return GP_SUCC;
+    }
+    // a piece for `want` bytes or, when there is nothing else to do, for fewer
+    int piece_for(size_t want, Piece **out) {
+        Piece *longest = nullptr;
+        for (Piece &p : pieces) {
+            if (p.room >= want && p.done.reached(p.done.seq)) { *out = &p; return GP_SUCC; }
+            if (!longest || p.turn < longest->turn) longest = &p;
+        }
+        if (total + want * kPerBlock <= kMost || !longest) {
+            if (int rc = grow(want)) return rc;
+            *out = &pieces[pieces.size() - kPerBlock];
+            return GP_SUCC;
+        }
+        *out = longest;
+        return longest->done.wait(longest->done.seq);
+    }
 };
 extern "C" int gp_stage_create(gp_stage *out) {
     GP_REQUIRE(out != nullptr, "null stage out");
-    gp_stage_s *st = new gp_stage_s();
-    const int rc = st->done.create();
-    if (rc) { st->done.destroy(); delete st; return rc; }
-    *out = st;
+    *out = new gp_stage_s();
     return GP_SUCC;
 }
 extern "C" int gp_stage_destroy(gp_stage st) {
     if (!st) return GP_SUCC;
-    int rc = st->done.seq ? st->done.wait(st->done.seq, st->last) : GP_SUCC;
-    if (rc == GP_SUCC) { st->done.destroy(); if (st->ring) hipHostFree(st->ring); }
+    int rc = GP_SUCC;
+    for (auto &p : st->pieces)
+        if (rc == GP_SUCC) rc = p.done.wait(p.done.seq);
+    if (rc == GP_SUCC)
+        for (auto &b : st->blocks) { hipHostFree(b.host); hipFree(b.arrived); }
     delete st;
     return rc;
 }
 extern "C" int gp_stage_upload_async(gp_stage st, void *dev, const void *host, size_t bytes, gp_stream s) {
     GP_REQUIRE(st && dev && host, "gp_stage_upload_async: null pointer");
-    if (bytes == 0) return GP_SUCC;
     std::lock_guard<std::mutex> lock(st->mu);
-    // (copies of one handle share a counter and report in order: another stream's wait for them)
-    if (st->last != native(s) && st->done.seq) { int rc = st->done.wait(st->done.seq, st->last); if (rc) return rc; }
-    st->last = native(s);
     // four pieces of a large input are copied to the ring while the one before is on its way; a small one is one piece
     size_t want = bytes <= (256u << 10) ? bytes : (bytes + 3) / 4;
     want = want > gp_stage_s::kPiece ? gp_stage_s::kPiece : (want + 4095) / 4096 * 4096;
-    if (want > st->piece) {
-        if (st->done.seq) { int rc = st->done.wait(st->done.seq, st->last); if (rc) return rc; }
-        if (st->ring) GP_HIP(hipHostFree(st->ring));
-        st->ring = nullptr; st->piece = 0;
-        int rc = gp_host_alloc_coherent((void **)&st->ring, (void **)&st->ring_dev, want * gp_stage_s::kPieces);
-        if (rc) return rc;
-        st->piece = want;
-        memset(st->used, 0, sizeof(st->used));
-    }
-    for (size_t at = 0; at < bytes; at += want) {
-        const size_t n = bytes - at < want ? bytes - at : want;
-        const int k = (int)(st->next++ % gp_stage_s::kPieces);
-        int rc = st->used[k] ? st->done.wait(st->used[k], st->last) : GP_SUCC;
-        if (rc) return rc;
-        memcpy(st->ring + k * st->piece, (const char *)host + at, n);
-        rc = st->done.launch<false>((char *)dev + at, st->ring_dev + k * st->piece, n, native(s));
-        if (rc) return rc;
-        st->used[k] = st->done.seq;
+    for (size_t at = 0; at < bytes;) {
+        gp_stage_s::Piece *p = nullptr;
+        if (int rc = st->piece_for(want, &p)) return rc;
+        size_t n = bytes - at < want ? bytes - at : want;
+        if (n > p->room) n = p->room;
+        memcpy(p->host, (const char *)host + at, n);
+        if (int rc = p->done.launch<false>((char *)dev + at, p->dev, n, native(s))) return rc;
+        p->turn = ++st->turns;
+        at += n;
     }
     return GP_SUCC;
 }

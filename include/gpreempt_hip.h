@@ -85,7 +85,8 @@ int gp_memcpy_d2d_async(void *dst, const void *src, size_t bytes, gp_stream s);
 int gp_fetch(void *host_coherent, const void *dev, size_t bytes, gp_stream s);
 /* Uploads from ordinary host memory through a ring of pinned memory that belongs to the handle: the caller's buffer
  * may be reused as soon as the call returns, and the copy runs in stream order.  (hipMemcpyAsync from ordinary memory
- * takes 2-4 times as long.)  Calls on one handle are serialised. */
+ * takes 2-4 times as long.)  Calls on one handle are serialised; they wait for the GPU only when copies of 64 MB are
+ * queued on it already. */
 typedef struct gp_stage_s *gp_stage;
 int gp_stage_create(gp_stage *out);
 int gp_stage_destroy(gp_stage st); /* waits for uploads still under way */

@@ -113,3 +113,40 @@ def test_pinned_input_is_read_in_place_and_without_a_wait(gp):
     assert gx.lib().gpx_set_input_pinned(ex.h, b"data", host, C.c_size_t(n - 1), stream.h) == 4  # OutOfRange, as set_input
     assert gx.lib().gpx_set_input_pinned(ex.h, b"nothing", host, C.c_size_t(n), stream.h) == 3   # NotFound
     gp.check(gp.lib().gp_host_free(host))
+
+
+def test_ordinary_input_does_not_wait_for_a_stream_that_is_held_up(gp):
+    """uploads of more than eight pieces, and on a second stream, behind a closed gate: each returns, the second stream's
+    arrives, and the first one's when the gate opens"""
+    rng = np.random.default_rng(8)
+    st, held, free = C.c_void_p(), gp.Stream(), gp.Stream()
+    gp.check(gp.lib().gp_stage_create(C.byref(st)))
+    sizes = [20 << 20, 3, 5 << 20, 70000, 1 << 20]
+    want = [rng.integers(0, 256, n, np.uint8) for n in sizes]
+    devs = [[gp.DevBuf(n) for n in sizes] for _ in range(2)]
+    gate = ClosedGate(gp, held)
+
+    def upload(d, w, stream):
+        host = w.copy()
+        gp.check(gp.lib().gp_stage_upload_async(st, C.c_void_p(d.ptr), host.ctypes.data_as(C.c_void_p), C.c_size_t(w.size), stream.h))
+        host[:] = 0
+    for d, w in zip(devs[0], want):
+        upload(d, w, held)
+    assert not held.idle()
+    for d, w in zip(devs[1], want):
+        upload(d, w, free)
+    free.sync()
+    assert not held.idle()
+    gate.open()
+    held.sync()
+    assert not gate.was_open_early()
+    for side in devs:
+        for d, w in zip(side, want):
+            assert np.array_equal(d.download(), w)
+    # more than the ring may hold: the pieces come round again
+    big = rng.integers(0, 256, (150 << 20) + 17, np.uint8)
+    d = gp.DevBuf(big.size)
+    upload(d, big, free)
+    free.sync()
+    assert np.array_equal(d.download(), big)
+    gp.check(gp.lib().gp_stage_destroy(st))

@@ -192,16 +192,24 @@ class _Pinned:
 class HostPool:
     """Arrays in pinned, coherent host memory (gp_host_alloc_coherent), which the GPU writes at the speed of PCIe: a
     copy into an ordinary new array goes through the runtime's own pinned memory and pays for its pages, 2-4 times as
-    long (4.8 MB: 92 us for 270; 84 MB: 1.5 ms for 4.8).  At most LIMIT bytes at a time, of which at most KEEP stay
-    allocated while nobody uses them; beyond LIMIT callers get ordinary arrays."""
+    long (4.8 MB: 92 us for 270; 84 MB: 1.5 ms for 4.8).  Memory is allocated while a caller goes through its first few
+    arrays of a size and used again from then on; one that keeps what it gets is given ordinary arrays after that.  At
+    most LIMIT bytes; what nobody uses stays allocated until trim()."""
 
-    LIMIT = 1 << 30
-    KEEP = 512 << 20
+    LIMIT = 512 << 20
+    KEEP = 64 << 20
 
     def __init__(self):
         self._lock = threading.RLock()  # (an array may die, and call _give_back, while its own thread is in here)
         self._free = {}
+        self._made = {}
         self._total = self._idle = 0
+
+    @staticmethod
+    def blocks_of(room):
+        """How many arrays of a size are in pinned memory at one time: a loop that drops its output when the next one is
+        there needs two.  (More of small ones, a megabyte of them: many models have outputs of a few KB.)"""
+        return max(4, min(64, (1 << 20) // room))
 
     def empty(self, nbytes):
         """(uint8 array of nbytes, its address if pinned or else None)"""
@@ -213,23 +221,35 @@ class HostPool:
             if self._free.get(room):
                 ptr = self._free[room].pop()
                 self._idle -= room
-            elif self._total + room <= self.LIMIT:
+            elif self._made.get(room, 0) < self.blocks_of(room) and self._total + room <= self.LIMIT:
                 host, dev = vp(), vp()
                 if lib().gp_host_alloc_coherent(C.byref(host), C.byref(dev), C.c_size_t(room)) == 0:
                     ptr = host.value
                     self._total += room
+                    self._made[room] = self._made.get(room, 0) + 1
         if ptr is None:
             return np.empty(nbytes, np.uint8), None
         return np.asarray(_Pinned(self, ptr, room, nbytes)), ptr
 
     def _give_back(self, ptr, room):
+        """(called by the garbage collector, wherever that is: nothing is freed here, which waits for the GPU)"""
         with self._lock:
-            if self._idle + room <= self.KEEP:
-                self._free.setdefault(room, []).append(ptr)
-                self._idle += room
-                return
-            self._total -= room
-        lib().gp_host_free(vp(ptr))
+            self._free.setdefault(room, []).append(ptr)
+            self._idle += room
+
+    def trim(self, keep=None):
+        """Frees what nobody uses, the largest blocks first, down to `keep` bytes (KEEP).  Waits for the GPU, as freeing
+        does: Executor.destroy calls it, which frees device memory anyway."""
+        keep, gone = self.KEEP if keep is None else keep, []
+        with self._lock:
+            for room in sorted(self._free, reverse=True):
+                while self._idle > keep and self._free[room]:
+                    gone.append(self._free[room].pop())
+                    self._made[room] -= 1
+                    self._idle -= room
+                    self._total -= room
+        for ptr in gone:
+            lib().gp_host_free(vp(ptr))
 
 
 host_pool = HostPool()

@@ -219,6 +219,7 @@ class Executor:
             lib().gpx_clear(self.h)
             lib().gpx_destroy(self.h)
             self.h = None
+            capi.host_pool.trim()
 
     def __del__(self):
         try:

@@ -285,23 +285,25 @@ extern "C" int gp_launch_conv2d(const gp_conv_params *p, const gp_preempt_ctx *c
     MatPlan pl;
     int rc = plan_conv2d(p, &pl);
     if (rc) return rc;
-    // A preemptible launch without counters of leavers (gp_preempt_ctx::done) finishes the tiles it holds before it
-    // leaves, so a tenant's preemption latency is its longest tile.  A 128 x 128 tile of a deep layer runs 45-65 us
-    // (VGG-16 b16: K = 2304 at 56 x 56, K = 4608 at 28 x 28); four 64 x 64 tiles in its place finish one by one; same
-    // summation per element, so the bits do not change.  With the counters such a tile is given up when a stop is
-    // recorded, and the larger tiles, which are 8 (K = 2304) and 24 % (K = 4608) faster, stay.  Not when the caller
-    // chose the tile, and not when it brought a checkpoint workspace (then long tiles are left between two K-steps).
-    if (ctx && !ctx->done && pl.body == MB_PIPE128 && pl.g.K >= 2304 && p->tile_m == 0 && p->variant == 0 && !(ctx->ckpt && ctx->ckpt_bytes >= plan_ckpt_bytes(pl))) {
+    // A preemptible launch that cannot give its tiles up finishes the ones it holds before it leaves, so a tenant's
+    // preemption latency is its longest tile.  A 128 x 128 tile of a deep layer runs 45-65 us (VGG-16 b16: K = 2304 at
+    // 56 x 56, K = 4608 at 28 x 28); four 64 x 64 tiles in its place finish one by one; same summation per element, so
+    // the bits do not change.  Where plan_launch finds that the tiles can be given up (counters of leavers, several
+    // claim counters, a flag that is not read at every claim, at most eight rounds of workgroups), the larger ones, which are 8 (K =
+    // 2304) and 24 % (K = 4608) faster, stay.  Not when the caller chose the tile, and not when it brought a checkpoint
+    // workspace (then long tiles are left between two K-steps).
+    pl.or_smaller = ctx && ctx->flag && pl.body == MB_PIPE128 && pl.g.K >= 2304 && p->tile_m == 0 && p->variant == 0 && !(ctx->ckpt && ctx->ckpt_bytes >= plan_ckpt_bytes(pl));
+    rc = launch_mat_plan(pl, ctx, s, info);
+    if (rc == kTileTooLong) {
         gp_conv_params q = *p;
         q.tile_m = q.tile_n = 64;
         q.variant = GP_MAT_PIPE;
-        MatPlan small;
-        if (plan_conv2d(&q, &small) == GP_SUCC) {
-            small.ring = (long)small.sx * small.sy > 2 * device_cus() ? 2 : 0;
-            pl = small;
-        }
+        rc = plan_conv2d(&q, &pl);
+        if (rc) return rc;
+        pl.ring = (long)pl.sx * pl.sy > 2 * device_cus() ? 2 : 0;
+        rc = launch_mat_plan(pl, ctx, s, info);
     }
-    return launch_mat_plan(pl, ctx, s, info);
+    return rc;
 }
 
 #ifdef GP_TILE_PROF

@@ -95,6 +95,7 @@ static int launch_mat(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s,
     const bool long_tiles = K::can_look && (double)K::bm * K::bn * pl.g.K * (pl.dtype == GP_F32 ? 8.0 : 1.0) >= long_macs;
     int rc = plan_launch(kern, K::NT, K::LDS_BYTES, pl.sx, pl.sy, pl.batch, ctx, &blp, &grid, info, 1, pl.rounds ? pl.rounds : K::LDS_BYTES <= 32 * 1024 ? 2 : K::LDS_BYTES <= 64 * 1024 ? 4 : 1, long_tiles);
     if (rc) return rc;
+    if (pl.or_smaller && ctx && !blp.done) return kTileTooLong;
     blp.order = pl.order;
     if constexpr (K_is_ckpt<K>::value) {
         if (info) info->fixed_claims = 0;  // tile_loop_ckpt always claims through the counters

@@ -524,3 +524,33 @@ def test_eltwise_at_the_edges_of_its_tiles(gp, dt, rows, chunks):
         want = np.maximum((a.astype(np.float32) + b) * sc + sh, 0)
         assert np.abs(got - want).max() <= {"f32": 1e-6, "f16": 2e-3, "bf16": 2e-2}[dt]
         assert (raw[da.nbytes:].view(np.uint32) == 0x55AA55AA).all()  # nothing behind the end
+
+
+@pytest.mark.parametrize("images,how,large", [(8, "", True), (8, "single counter", False), (8, "poll every claim", False), (8, "no counters of leavers", False),
+                                              (8, "no flag", True), (84, "", False)])
+def test_large_tiles_of_a_deep_convolution_only_where_they_can_be_given_up(gp, images, how, large):
+    """3 x 3 at 56 x 56 x 256: 128 x 128 tiles in a launch that gives them up behind a stop, tiles of a quarter in one that
+    would finish them (one claim counter, a flag read at every claim, nobody counting the leavers, more than
+    eight rounds of workgroups); the same bits either way"""
+    H, Cin, Cout = 56, 256, 256
+    rng = np.random.default_rng(images)
+    x = gp.DevBuf.from_array(rng.random((images, H, H, Cin), np.float32).astype(np.float16) - np.float16(0.5), gp.F16)
+    w = gp.DevBuf.from_array(((rng.random((Cout, 3, 3, Cin), np.float32) - 0.5) * 0.1).astype(np.float16), gp.F16)
+    out = gp.DevBuf(images * H * H * Cout * 2)
+    p = gp.ConvParams(dtype=gp.F16, N=images, H=H, W=H, Cin=Cin, Cout=Cout, R=3, S=3, stride_h=1, stride_w=1, pad_h=1, pad_w=1, in_=x.ptr, in_pix_stride=Cin,
+                      weight=w.ptr, out=out.ptr, out_pix_stride=Cout, act=gp.ACT_RELU)
+    plain = gp.launch("gp_launch_conv2d", p)
+    sync(gp)
+    assert plain.total_tiles == -(-images * H * H // 128) * (Cout // 128)
+    want = out.download()
+    out.fill32(0x7E007E00)
+    st = gp.BlpState(1, gp.Flag(), 1 if how == "single counter" else 32)
+    if how != "no counters of leavers":
+        st.enable_done_counters()
+    ctx = st.ctx(fresh=1, poll_every=1 if how == "poll every claim" else 0)
+    if how == "no flag":
+        ctx.flag = None
+    info = gp.launch("gp_launch_conv2d", p, ctx)
+    sync(gp)
+    assert info.total_tiles == (plain.total_tiles if large else -(-images * H * H // 64) * (Cout // 64)), (how, info.total_tiles)
+    assert np.array_equal(out.download(), want)

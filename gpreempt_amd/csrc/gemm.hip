@@ -83,7 +83,8 @@ static int wide_pick(const MatArgs &g, int batch, long cus, int dtype) {
     return -1;
 }
 
-// The wide bodies address their operands by 32-bit offsets in buffers of 2 GB.
+// The wide bodies address their operands by 32-bit offsets in buffers of 2 GB.  (Beyond, the four-wavefront split-K bodies
+// of gemm_pipe.hpp stand in for them: pointers of 64 bits, the same sums in the same order.)
 static bool buffer_ok(const MatArgs &g, bool conv, int dtype) {
     const double limit = 2147483648.0 / (double)dtype_size(dtype);
     const double pixels = conv ? (double)(g.M / ((long)g.Ho * g.Wo)) * g.H * g.W + (double)(g.ph + g.K / (g.Cin * g.S)) * (g.W + g.S) : (double)g.M;
@@ -97,7 +98,8 @@ static int choose_body(MatPlan *pl, int tile, int tile_n, int variant) {
     // both operands K-contiguous; a convolution, whose A operand is gathered, when a K-block never straddles
     // two filter taps and a bit per tap fits a word
     const int wide_bk = pl->dtype == GP_F32 ? 32 : 64;
-    const bool wide_ok = !pl->b_kn && (!pl->conv || (g.Cin % wide_bk == 0 && g.K / g.Cin <= 32 && g.S < 32)) && buffer_ok(g, pl->conv, pl->dtype);
+    const bool wide_shape = !pl->b_kn && (!pl->conv || (g.Cin % wide_bk == 0 && g.K / g.Cin <= 32 && g.S < 32));
+    const bool wide_ok = wide_shape && buffer_ok(g, pl->conv, pl->dtype);
     int body = -1;
     if (g.ln_gamma) body = MB_LNWIDE32x64_16;  // (plan_gemm has checked that the shape fits)
     else if (pl->b_kn || variant == GP_MAT_STAGED) {
@@ -110,11 +112,11 @@ static int choose_body(MatPlan *pl, int tile, int tile_n, int variant) {
         int tm = tile ? tile : (tiles(64) >= cus / 2 ? 64 : 32);
         body = tm == 64 ? MB_PIPE64_SK : tm == 32 ? MB_PIPE32_SK : -1;
     } else if (variant == GP_MAT_WIDE || variant == GP_MAT_WIDE8) {
-        if (wide_ok) {
+        if (wide_shape) {
             const int tn = tile_n ? tile_n : tile;
-            if (tile == 32 && tn == 32) body = variant == GP_MAT_WIDE ? MB_WIDE32x32_16 : MB_WIDE32x32_8;
-            else if (tile == 64 && tn == 32) body = MB_WIDE64x32_16;
-            else if (tile == 64 && tn == 64) body = MB_WIDE64x64_8;
+            if (tile == 32 && tn == 32) body = !wide_ok ? MB_PIPE32_SK : variant == GP_MAT_WIDE ? MB_WIDE32x32_16 : MB_WIDE32x32_8;
+            else if (tile == 64 && tn == 32) body = wide_ok ? MB_WIDE64x32_16 : MB_PIPE32_SK;
+            else if (tile == 64 && tn == 64) body = wide_ok ? MB_WIDE64x64_8 : MB_PIPE64_SK;
         }
     } else if (variant == GP_MAT_AUTO) {
         // a tile wider than the problem multiplies zero columns: N <= 64 never takes the larger tiles
@@ -172,7 +174,7 @@ static bool ln_shape_ok(const gp_gemm_params *p) {
     // one round of workgroups: every workgroup normalises its own 32 rows, which pays while that hides
     // behind the fetch of B and not when a compute unit does it twice
     const long tiles = (long)((p->M + 31) / 32) * ((p->N + 63) / 64);
-    return tiles <= device_cus() && (double)p->N * p->ldb < 1073741824.0;  // (B in a buffer of 2 GB)
+    return tiles <= device_cus() && (double)p->ldb < 16777216.0;  // (a tile's 64 rows of B in a buffer of 2 GB)
 }
 int plan_gemm(const gp_gemm_params *p, MatPlan *out);
 // ... and the body the launcher would pick for the plain GEMM sums K in the prologue body's order (K-steps

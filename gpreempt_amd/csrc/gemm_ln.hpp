@@ -75,12 +75,12 @@ struct LnWideKernel {
 
         // ---- B loader slots, as in WideKernel ---------------------------------------------------
         const int rig = lane >> 3, cpos = lane & 7;
-        const u32x4 rsrc_b = buffer_of(B);
+        const u32x4 rsrc_b = buffer_of(B + (long)n0 * g.ldb);  // (from the tile's first row: the planner bounds 64 rows, not all of B)
         unsigned off[LPW];
 #pragma unroll
         for (int j = 0; j < LPW; ++j) {
             const int r = (wv * LPW + j) * 8 + rig;
-            off[j] = n0 + r < g.N ? ((unsigned)(n0 + r) * (unsigned)g.ldb + (unsigned)(cpos ^ ((r >> 1) & 7)) * VEC) * (unsigned)sizeof(T) : kBufferEnd;
+            off[j] = n0 + r < g.N ? ((unsigned)r * (unsigned)g.ldb + (unsigned)(cpos ^ ((r >> 1) & 7)) * VEC) * (unsigned)sizeof(T) : kBufferEnd;
         }
         auto issue = [&](int s) {
             const int k0 = (s * KB + kb) * BK;

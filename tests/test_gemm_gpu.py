@@ -1051,3 +1051,84 @@ def test_looks_at_every_count_of_k_steps(gp):
     out = subprocess.run([sys.executable, "-c", _LOOKS_SWEEP, root], capture_output=True, text=True, timeout=110,
                          env={**os.environ, "GPREEMPT_LONG_TILE_MACS": "1"})
     assert out.returncode == 0 and out.stdout.strip().startswith("OK 19"), (out.stdout[-300:], out.stderr[-1500:])
+
+
+def _put(gp, ptr, a):
+    gp.check(gp.lib().gp_memcpy_h2d(C.c_void_p(ptr), a.ctypes.data_as(C.c_void_p), C.c_size_t(a.nbytes)))
+
+
+@pytest.mark.parametrize("dt", ["f16", "f32"])
+@pytest.mark.parametrize("which", ["a", "b"])
+@pytest.mark.parametrize("tm,tn,variant", [(32, 32, 4), (32, 32, 5), (64, 32, 4), (64, 64, 5)])
+def test_wide_gemm_on_operands_around_two_gigabytes(gp, dt, which, tm, tn, variant):
+    """64 rows so far apart that the operand spans a little less than the 2 GB of a buffer descriptor, and a little more"""
+    dtype, es, M, N, K = gp.DTYPE_BY_NAME[dt], gp.DTYPE_SIZE[gp.DTYPE_BY_NAME[dt]], 64, 64, 520
+    rng = np.random.default_rng(variant)
+    a, b = (gp.to_storage(rng.uniform(-1, 1, (64, K)).astype(np.float32), dtype) for _ in range(2))
+    small = [gp.DevBuf(x.nbytes) for x in (a, b)]
+    for d, x in zip(small, (a, b)):
+        d.upload(x)
+    far = gp.DevBuf((2 << 30) + (1 << 20))
+    out = gp.DevBuf(M * N * es)
+    got = []
+    for ld in (K, (2 << 30) // es // 64 - 16, (2 << 30) // es // 64):
+        ptrs, lds = [small[0].ptr, small[1].ptr], [K, K]
+        if ld > K:
+            side = 0 if which == "a" else 1
+            for r in range(64):
+                _put(gp, far.ptr + r * ld * es, (a, b)[side][r])
+            ptrs[side], lds[side] = far.ptr, ld
+        out.fill32(0x7E007E00)
+        info = gp.launch("gp_launch_gemm", gp.GemmParams(dtype=dtype, M=M, N=N, K=K, A=ptrs[0], lda=lds[0], B=ptrs[1], ldb=lds[1], b_is_nk=1, C=out.ptr, ldc=N,
+                                                       alpha=1.0, act=gp.ACT_NONE, batch=1, tile_m=tm, tile_n=tn, variant=variant))
+        gp.check(gp.lib().gp_stream_sync(None))
+        got.append(out.download().copy())
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+    assert rel_err(gp.from_storage(got[0], dtype).reshape(M, N), gp.from_storage(a, dtype) @ gp.from_storage(b, dtype).T) < TOL[dt]
+
+
+@pytest.mark.parametrize("tm,tn,variant", [(32, 32, 4), (64, 64, 5)])
+def test_wide_convolution_on_images_around_two_gigabytes(gp, tm, tn, variant):
+    """pixels 2048 channels apart, of which a 3 x 3 reads 64: the last image ends a little before and a little beyond 2 GB"""
+    H, pix, Cin, Cout = 56, 2048, 64, 32
+    image = H * H * pix * 2
+    rng = np.random.default_rng(3)
+    x = np.zeros((H, H, pix), np.float16)
+    x[:, :, :Cin] = rng.uniform(-1, 1, (H, H, Cin))
+    w = gp.DevBuf.from_array((rng.uniform(-1, 1, (Cout, 3, 3, Cin)) * 0.1).astype(np.float16), gp.F16)
+    most = (2 << 30) // image
+    dev, out = gp.DevBuf((most + 1) * image), gp.DevBuf((most + 1) * H * H * Cout * 2)
+    dev.fill32(0)
+    got = []
+    for images in (1, most - 1, most + 1):
+        _put(gp, dev.ptr + (images - 1) * image, x)
+        p = gp.ConvParams(dtype=gp.F16, N=images, H=H, W=H, Cin=Cin, Cout=Cout, R=3, S=3, stride_h=1, stride_w=1, pad_h=1, pad_w=1, in_=dev.ptr, in_pix_stride=pix,
+                          weight=w.ptr, out=out.ptr, out_pix_stride=Cout, act=gp.ACT_NONE, tile_m=tm, tile_n=tn, variant=variant)
+        out.fill32(0x7E007E00)
+        gp.launch("gp_launch_conv2d", p)
+        gp.check(gp.lib().gp_stream_sync(None))
+        whole = out.download(np_dtype=np.uint16)[: images * H * H * Cout].reshape(images, -1)
+        got.append(whole[-1].copy())
+        assert images == 1 or not whole[1:-1].any()  # (the images between are zeros; the first one is the first run's)
+        _put(gp, dev.ptr + (images - 1) * image, np.zeros_like(x))
+    assert got[0].any() and np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+
+
+def test_layernorm_prologue_with_rows_of_b_far_apart(gp):
+    """B's rows 16 MB apart, 2.1 GB in all: the bits of the compact operand"""
+    M, N, K, ldb = 100, 128, 768, (1 << 23) + 8
+    rng = np.random.default_rng(9)
+    x, w, gamma, beta = (gp.to_storage(rng.uniform(-1, 1, s).astype(np.float32), gp.F16) for s in ((M, K), (N, K), (K,), (K,)))
+    dx, dw, dg, db = (gp.DevBuf.from_array(v, gp.F16) for v in (x, w, gamma, beta))
+    far = gp.DevBuf(N * ldb * 2)
+    for r in range(N):
+        _put(gp, far.ptr + r * ldb * 2, w[r])
+    dn, dc = gp.DevBuf(M * K * 2), gp.DevBuf(M * N * 2)
+    got = []
+    for ptr, ld in ((dw.ptr, K), (far.ptr, ldb)):
+        dc.fill32(0x7E007E00)
+        gp.launch("gp_launch_gemm", gp.GemmParams(dtype=gp.F16, M=M, N=N, K=K, A=dx.ptr, lda=K, B=ptr, ldb=ld, b_is_nk=1, C=dc.ptr, ldc=N, alpha=1.0, act=gp.ACT_NONE,
+                                                  batch=1, ln_gamma=dg.ptr, ln_beta=db.ptr, ln_out=dn.ptr, ln_eps=1e-5))
+        gp.check(gp.lib().gp_stream_sync(None))
+        got.append(dc.download().copy())
+    assert np.array_equal(got[0], got[1]) and got[0].any()

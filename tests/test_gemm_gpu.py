@@ -1053,6 +1053,59 @@ def test_looks_at_every_count_of_k_steps(gp):
     assert out.returncode == 0 and out.stdout.strip().startswith("OK 19"), (out.stdout[-300:], out.stderr[-1500:])
 
 
+_RINGS = [(4096, 2048, 2048), (4096, 1920, 1152), (2048, 1600, 4608), (2000, 1580, 4640)]
+
+
+@pytest.mark.parametrize("dt,M,N,K", [(dt, *s) for s in _RINGS for dt in ("f16", "f32")] + [("f16", 6000 * 64, 64, 576), ("f16", 300001, 40, 64)])
+def test_auto_ring_depths_stopped_and_resumed(gp, dt, M, N, K):
+    """What the launcher picks by itself: rings of two stages under 128 x 128 and 64 x 64 tiles, with looks (the first
+    four; whole tiles and ragged ones), and a workgroup per claim over sixteen rounds.  The bits of the plain launch and
+    of the body at its full depth, through stops at three depths."""
+    import time
+    dtype = gp.DTYPE_BY_NAME[dt]
+    rng = np.random.default_rng(M + K)
+    A = (rng.random((M, K), np.float32) - 0.5).astype(np.float32 if dt == "f32" else np.float16)
+    B = ((rng.random((N, K), np.float32) - 0.5) * 0.1).astype(A.dtype)
+    dA, dB, dC = gp.DevBuf.from_array(A, dtype), gp.DevBuf.from_array(B, dtype), gp.DevBuf(M * N * A.itemsize)
+    p = gp.GemmParams(dtype=dtype, M=M, N=N, K=K, A=dA.ptr, lda=K, B=dB.ptr, ldb=K, b_is_nk=1, C=dC.ptr, ldc=N, alpha=1.0, act=gp.ACT_RELU, batch=1)
+    plain = gp.launch("gp_launch_gemm", p)
+    gp.check(gp.lib().gp_stream_sync(None))
+    base = dC.download().copy()
+    rows = rng.integers(0, M, 16)
+    assert rel_err(dC.download(dtype, (M, N))[rows], O.gemm_bias_act(A[rows].astype(np.float32), B.astype(np.float32), None, None, gp.ACT_RELU, b_is_nk=True)) < TOL[dt]
+    tile = 128 if plain.total_tiles == -(-M // 128) * -(-N // 128) else 64
+    assert plain.total_tiles == -(-M // tile) * -(-N // tile) and tile == (128 if M == 4096 else 64)
+    p.tile_m = p.tile_n = tile
+    p.variant = gp.MAT_PIPE
+    dC.fill32(0)
+    gp.launch("gp_launch_gemm", p)
+    gp.check(gp.lib().gp_stream_sync(None))
+    assert np.array_equal(dC.download(), base)  # (the ring's depth changes no sum)
+    p.tile_m = p.tile_n = p.variant = 0
+    flag, stream = gp.Flag(), gp.Stream(1)
+    st = gp.BlpState(1, flag, 32)
+    st.enable_done_counters()
+    for wait in (0.0, 20e-6, 60e-6):
+        st.reset(); st.clear_stop(); flag.set(0)
+        dC.fill32(0x7E007E00)
+        info = gp.launch("gp_launch_gemm", p, st.ctx(fresh=1), stream)
+        t0 = time.perf_counter()
+        while time.perf_counter() - t0 < wait:
+            pass
+        flag.set(1)
+        stream.sync()
+        assert info.total_tiles == plain.total_tiles
+        if K >= 1152:
+            assert info.fixed_claims == 1 and info.front == 8  # (long tiles: these give them up)
+        made = int(st.counters().reshape(32, 16)[:, 0].sum())
+        assert made <= info.total_tiles and (st.stop_index() == 0 or made == info.total_tiles)
+        flag.set(0)
+        st.clear_stop()
+        gp.launch("gp_launch_gemm", p, st.ctx(done_launches=1), stream)
+        stream.sync()
+        assert np.array_equal(dC.download(), base), wait
+
+
 def _put(gp, ptr, a):
     gp.check(gp.lib().gp_memcpy_h2d(C.c_void_p(ptr), a.ctypes.data_as(C.c_void_p), C.c_size_t(a.nbytes)))
 

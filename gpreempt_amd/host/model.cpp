@@ -213,7 +213,7 @@ Status Model::allocate_and_bind() {
     }
     loaded_ = true;
     plan_fusions();
-    RETURN_STATUS(plan_sweeps());
+    plan_sweeps();
     // seeded random initialisation of every parameter (overwritten by load_param when a file exists)
     uint64_t seed = 0x5EEDull;
     for (size_t i = 0; i < storage_infos.size(); ++i) {
@@ -261,29 +261,25 @@ void Model::plan_fusions() {
     }
 }
 
-// A list that is the miniWeather step (x, z, z, x; three stages of halo, fluxes, update) also gets its sweeps.
-Status Model::plan_sweeps() {
+// A list that is the miniWeather step (x, z, z, x; three stages of halo, fluxes, update) also gets its sweeps.  The state
+// between two sweeps of a pair (82 MB at 3200 x 1600) is allocated by the first of them that is launched.
+void Model::plan_sweeps() {
     sweeps_.clear();
-    if (kernel_infos.size() != 4 * kSweepKernels) return Status::Succ;
+    if (kernel_infos.size() != 4 * kSweepKernels) return;
     for (size_t i = 0; i < kernel_infos.size(); ++i) {
         const int dir = i / kSweepKernels == 1 || i / kSweepKernels == 2 ? GP_MW_HALO_Z : GP_MW_HALO_X;
-        if (kernel_infos[i].op != OpKind::Stencil || kernel_infos[i].p.miniweather.kernel != dir + (int)(i % 3)) return Status::Succ;
+        if (kernel_infos[i].op != OpKind::Stencil || kernel_infos[i].p.miniweather.kernel != dir + (int)(i % 3)) return;
     }
     const gp_miniweather_params &first = kernel_infos[2].p.miniweather;  // an update: state_init = state, state_out = state_tmp
     float *state = (float *)first.state_init, *tmp = first.state_out;
-    const size_t bytes = get_storage_size(kernel_infos[0].args_index[0]);
-    CUDA_RETURN_STATUS(gp_malloc(&sweep_state_, bytes));
     for (size_t g = 0; g < 4; ++g) {
         gp_mw_sweep_params p{};
         p.dir_z = g == 1 || g == 2; p.last = g >= 2;
         p.nx = first.nx; p.nz = first.nz; p.dx = first.dx; p.dz = first.dz;
         for (size_t stage = 0; stage < 3; ++stage) p.dt[stage] = kernel_infos[kSweepKernels * g + 3 * stage].p.miniweather.dt;
-        p.in = g % 2 ? (const float *)sweep_state_ : state;
-        p.out = g % 2 ? state : (float *)sweep_state_;
         p.state = state; p.state_tmp = tmp; p.flux = first.flux; p.hydro = first.hydro;
         sweeps_.push_back(p);
     }
-    return Status::Succ;
 }
 
 // Slot order per operator is fixed by the builders in zoo.cpp.
@@ -565,11 +561,15 @@ void Model::launched(size_t idx, bool preemptible, const gp_launch_info &info) {
 
 Status Model::launch_sweep(size_t g, GPUstream stream) {
     if (g >= sweeps_.size()) return Status::OutOfRange;
+    if (!sweep_state_) CUDA_RETURN_STATUS(gp_malloc(&sweep_state_, get_storage_size(kernel_infos[0].args_index[0])));
+    gp_mw_sweep_params &p = sweeps_[g];
+    p.in = g % 2 ? (const float *)sweep_state_ : p.state;
+    p.out = g % 2 ? p.state : (float *)sweep_state_;
     const size_t idx = g * kSweepKernels;
     gp_preempt_ctx ctx{};
     const bool preemptible = preempt_ctx(idx, -1, ctx);
     gp_launch_info info{};
-    const int rc = gp_launch_miniweather_sweep(&sweeps_[g], preemptible ? &ctx : nullptr, stream, &info);
+    const int rc = gp_launch_miniweather_sweep(&p, preemptible ? &ctx : nullptr, stream, &info);
     if (idx < fresh_.size()) fresh_[idx] = 0;
     CUDA_RETURN_STATUS(rc);
     launched(idx, preemptible, info);

@@ -208,8 +208,8 @@ private:
     int poll_every_ = 0;
     std::vector<char> fresh_;
     std::vector<gp_mw_sweep_params> sweeps_;
-    GPUdeviceptr sweep_state_ = nullptr;  // what the first and third sweep write
-    Status plan_sweeps();
+    GPUdeviceptr sweep_state_ = nullptr;  // what the first and third sweep write; made by the first launch_sweep()
+    void plan_sweeps();
     bool preempt_ctx(size_t idx, int inject_at, gp_preempt_ctx &ctx);
     void launched(size_t idx, bool preemptible, const gp_launch_info &info);
     std::vector<int> launches_;           // per kernel: launches since the counters were cleared (gp_preempt_ctx::done_launches)

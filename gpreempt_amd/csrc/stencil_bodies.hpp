@@ -193,6 +193,10 @@ __device__ __forceinline__ double mw_rcp(double a) {
 // a polynomial of degree 15 (interpolated at Chebyshev nodes; good to 1.4 10^-15 with the rounding of its evaluation)
 // and 2^(gamma e) comes from a table: 22 instructions, where a series for the logarithm and one for the exponential
 // (to 10^-14) took 45.
+// (An infinity does not get here, where the polynomial would make -inf of it: reconstruction divides by 12 by a corrected
+// product, which makes NaN of infinities, and leaves at most a twelfth of fp32's range.)  The table and the coefficients
+// are checked against the power itself in tests/test_pow_table_cpu.py.
+static_assert(MW_GAMMA == 1.40027894002789400278940027894f, "mw_pow2_gamma and the polynomial of mw_pow_gamma are for this exponent, rounded to fp32");
 constexpr int MW_POW_E0 = -149;
 static __constant__ double mw_pow2_gamma[278] = {
     1.5582319697246894e-63, 4.1129939375444373e-63, 1.08563548040066e-62, 2.865563174178731e-62, 7.563728759287419e-62, 1.9964659393861715e-61,

@@ -66,6 +66,10 @@ inline int occupancy_of(const void *kernel, int block, size_t lds_bytes, int *pe
     return GP_SUCC;
 }
 
+// Whether a front workgroup, which keeps one of the places that a device has for a kernel's workgroups, costs a launch
+// a round of its own
+inline bool front_costs_a_round(long total, long resident) { return (total + resident - 2) / (resident - 1) != (total + resident - 1) / resident; }
+
 // Resolves the launch geometry of one preemptible kernel, as Model::add_block_preemption_param
 // does in the reference (src/model.cpp:366-396): total_block = sx*sy*sz; persistent grid =
 // min(total_block, resident workgroups the device can hold); a NULL context keeps one
@@ -106,7 +110,7 @@ int plan_launch(Kernel kernel, int block, size_t lds_bytes, int sx, int sy, int 
         // the launch ends, would cost a round of its own: a compute unit holds one workgroup of the kernel and the
         // rounds are full.)
         bool long_ok = long_tiles && ctx->done && ctx->flag && blp->poll_mask != 0 && ng > 1;
-        if (long_ok && per_cu < 2 && total > resident && (ctx->max_workgroups != 0 || (total + resident - 2) / (resident - 1) != (total + resident - 1) / resident))
+        if (long_ok && per_cu < 2 && total > resident && (ctx->max_workgroups != 0 || front_costs_a_round(total, resident)))
             long_ok = false;
         if (long_ok && waves < 8) waves = 8;
         if (ng > 1 && ctx->max_workgroups == 0 && total > resident && total <= (long)waves * resident && total + 8 <= (long)ng * kFixedClaimBits)

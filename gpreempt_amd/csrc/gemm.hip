@@ -121,10 +121,11 @@ static int choose_body(MatPlan *pl, int tile, int tile_n, int variant) {
     } else if (variant == GP_MAT_AUTO) {
         // a tile wider than the problem multiplies zero columns: N <= 64 never takes the larger tiles
         if (!pl->conv && (tile == 256 || (tile == 0 && tiles(256) >= cus && g.N > 128 && g.M > 128))) body = MB_PIPE256;
-        // (a problem of one or two K-steps is all epilogue, i.e. memory-bound: the 128 x 128 body runs one workgroup
-        // per CU, too few threads for that; 25088 x 256 x 64 with a residual: 19.8 us on 128 x 128, 15.0 on 64 x 64)
+        // (a problem of one or two K-steps is all epilogue, i.e. memory-bound: the 128 x 128 body runs one or two
+        // workgroups per CU, too few threads for that; 25088 x 256 x 64 with a residual: 19.8 us on 128 x 128, 15.0 on 64 x 64)
         // (... and with hardly more tiles than compute units a shallow one is better cut into tiles of 64 x 64, several
-        // to a compute unit: 4096 x 1024 x 1024 17.1 -> 14.6 us; 2048^3 25.4 on 128 x 128, 26.2 on 64 x 64)
+        // to a compute unit: 4096 x 1024 x 1024 17.1 -> 14.6 us; 2048^3 25.4 on 128 x 128, 26.2 on 64 x 64; in fp32
+        // 5000 x 1000 x 768 105 -> 78, 3000 x 1500 x 256 42 -> 30, 4096 x 1024 x 1024 77 -> 81 but 149 -> 101 preemptible)
         else if (tile == 128 || (tile == 0 && tiles(128) >= (g.K <= 1024 ? cus + cus / 2 : cus) && g.N > 64 && g.M > 64 && g.K > 128)) body = MB_PIPE128;
         else if (tile == 0 && wide_ok && wide_pick(g, pl->batch, cus, pl->dtype) >= 0) body = wide_pick(g, pl->batch, cus, pl->dtype);
         else if (tile == 64 || (tile == 0 && (tiles(64) >= cus || g.K < 512))) body = MB_PIPE64;
@@ -147,9 +148,10 @@ static int choose_body(MatPlan *pl, int tile, int tile_n, int variant) {
     if (tile == 0 && variant == GP_MAT_AUTO && ((body == MB_PIPE128 && tiles(128) > cus) || (body == MB_PIPE64 && tiles(64) > 2 * cus))) pl->ring = 2;
     // Tiles of a few microseconds: claimed through the counters, a tile waits 1-2 us for its claim, and the kernel around
     // the general loop fits a compute unit three times where the others fit four or five times.  With a workgroup per claim a 3 x 3 layer
-    // of 12544 tiles at 224 x 224 x 64 takes 131 us instead of 172 (plain launch 119); behind a stop its workgroups
-    // still have to start and leave, about a microsecond per thousand.
-    if (tile == 0 && variant == GP_MAT_AUTO && body == MB_PIPE64 && g.K <= 640) pl->rounds = 16;
+    // of 12544 tiles at 224 x 224 x 64, seventeen rounds of them, takes 152 us instead of 182 (plain launch 136); behind
+    // a stop its workgroups still have to start and leave, about a microsecond per thousand.  (fp32, whose tiles take eight times as long and
+    // wait no longer: 3136 tiles there 150 us either way.)
+    if (tile == 0 && variant == GP_MAT_AUTO && body == MB_PIPE64 && g.K <= 640) pl->rounds = 20;
     // Each XCD works on a contiguous eighth of the tile order (util/slice_map.h).  With x fastest
     // that is a band of tile rows: every XCD fetches its share of A and all of B; with y fastest
     // it is a band of tile columns: all of A and a share of B.  Take the cheaper one.

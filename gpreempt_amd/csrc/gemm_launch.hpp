@@ -96,6 +96,12 @@ static int launch_mat(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s,
     int rc = plan_launch(kern, K::NT, K::LDS_BYTES, pl.sx, pl.sy, pl.batch, ctx, &blp, &grid, info, 1, pl.rounds ? pl.rounds : K::LDS_BYTES <= 32 * 1024 ? 2 : K::LDS_BYTES <= 64 * 1024 ? 4 : 1, long_tiles);
     if (rc) return rc;
     if (pl.or_smaller && ctx && !blp.done) return kTileTooLong;
+    if (pl.or_deeper && ctx && blp.done) {
+        int per_cu = 0;
+        rc = occupancy_of((const void *)kern, K::NT, K::LDS_BYTES, &per_cu);
+        if (rc) return rc;
+        if (front_costs_a_round(blp.total, (long)per_cu * device_cus())) return kFrontCostsARound;
+    }
     blp.order = pl.order;
     if constexpr (K_is_ckpt<K>::value) {
         if (info) info->fixed_claims = 0;  // tile_loop_ckpt always claims through the counters
@@ -174,8 +180,17 @@ int launch_typed(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, gp_l
         // 128 x 128: 3 x 3 at 56 x 56 x 256 batch 16 126 -> 83 us, at 28 x 28 x 512 110 -> 75; 64 x 64: at 224 x 224 x 64
         // 176 -> 119 us, 4096 x 1024 x 1024 17.3 -> 14.6.  A launch that fits at once keeps the depth: 3 x 3 at 14 x 14 x
         // 512 (392 tiles of 64 x 64) 33 us against 44, 2048^3 (256 of 128 x 128) 25 against 33 (choose_body has the line).
+        // fp32 the same way: 3 x 3 at 56 x 56 x 256 650 -> 591 us, at 28 x 28 x 512 634 -> 586, at 224 x 224 x 64 batch 4 176 ->
+        // 150 preemptible, 4096 x 2048 x 1024 150 -> 138.  Not where tiles fill the device to the last place and a
+        // preemptible launch's front workgroup makes a round for one of them: 4096 x 2048 x 2048, 512 tiles, 77 us for 62 in fp16 and 344 for
+        // 289 in fp32.
         case MB_PIPE128:
-            if (pl.ring == 2 && !(ctx && ctx->ckpt && ctx->ckpt_bytes >= plan_ckpt_bytes(pl))) return pipe_case<T, 128, 2, false>(pl, ctx, s, info);
+            if (pl.ring == 2 && !(ctx && ctx->ckpt && ctx->ckpt_bytes >= plan_ckpt_bytes(pl))) {
+                MatPlan shallow = pl;
+                shallow.or_deeper = true;
+                const int rc = pipe_case<T, 128, 2, false>(shallow, ctx, s, info);
+                if (rc != kFrontCostsARound) return rc;
+            }
             return pipe_case_ckpt<T, 128, GP_S128>(pl, ctx, s, info);
         case MB_PIPE64:
             // A layer of at most four K-steps is all prologue and epilogue: two stages for any number of tiles.

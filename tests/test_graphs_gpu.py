@@ -84,7 +84,8 @@ def test_synthetic_default_and_bad_names(gp, ex_mod):
         ex_mod.Executor("bfs", graph_path="/nonexistent/graph")
 
 
-# (iteration, kernel, claim): -1 = PageRank's set-up kernel
+# (iteration, kernel, claim): -1 = PageRank's set-up kernel.  An injected stop is the stepwise loop's; the launches that a
+# run queues are stopped in test_queued_launches_stopped_again_and_again.
 INJECT = {"bfs": [(0, 0, 0), (2, 0, 900), (4, 0, 1500)],
           "cc": [(-1, 0, 5), (0, 0, 1500), (1, 0, 10), (2, 0, 1800)],
           "sssp": [(1, 0, 100), (3, 1, 60), (6, 0, 1700)],
@@ -374,3 +375,29 @@ def test_queued_launches_stopped_again_and_again(gp, ex_mod, kind, n, deg):
             assert np.array_equal(got, want), pause
         if pause >= 150e-6 and n == 1 << 20:
             assert ex.graph_info()["preemptions"] > before, pause
+
+
+@pytest.mark.parametrize("n,deg", [(300, 3), (4099, 8), (30000, 5), (200000, 16)])
+@pytest.mark.parametrize("blp", [False, True])
+def test_pagerank_of_a_generated_graph_pushes(gp, ex_mod, tmp_path, n, deg, blp):
+    """A generated graph has every edge both ways, so that the last iterations push along the edges out where a file's
+    graph pulls along those in.  A run ends with residuals between nothing and the tolerance t everywhere: the values
+    are low by (I - alpha P^T)^-1 of these, which is t / (1 - alpha) times the solution x at most, vertex by vertex.
+    (1e-5: some forty fp32 additions per vertex.)"""
+    base = str(tmp_path / "g")
+    assert ex_mod.lib().gpx_write_synthetic_graph(base.encode(), C.c_ulonglong(n), deg, C.c_ulonglong(13)) == 0
+    x = G.pagerank_exact(*G.read_graph(base)[:2])
+    launches = []
+    for wl, path in ((f"pagerank@n={n},deg={deg},seed=13", None), ("pagerank", base)):
+        ex = ex_mod.Executor(wl, blp=blp, graph_path=path)
+        if blp:
+            ex.set_flag(gp.Flag())
+        for _ in range(2):
+            before = ex.graph_info()["kernels_launched"]
+            ex.execute()
+            got = ex.graph_result("value", np.float32)
+            assert (got <= x * (1 + 1e-5)).all() and (got >= x * (1 - 0.001 / 0.15 - 1e-5)).all(), wl
+            info = ex.graph_info()
+            launches.append(info["kernels_launched"] - before - info["iterations"])
+    if n >= 30000:  # (going over to the push takes a launch; a small graph's sample of its vertices may miss the moment)
+        assert min(launches[:2]) > max(launches[2:]), launches

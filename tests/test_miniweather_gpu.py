@@ -8,6 +8,7 @@ implementations differ in the last bit, so they are compared to 1e-6 (fp64 pow, 
 fp32) and 2e-5 (fp32 powf on pressures that nearly cancel against the background) of the field's
 magnitude; whole time steps to 1e-4 of each field's magnitude."""
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -131,6 +132,7 @@ INJECTIONS = [(0, 0), (1, 700), (8, 3000), (14, 5000), (17, 1234), (22, 10), (35
 
 
 def test_preempt_resume_is_bit_exact(gp, ex_mod):
+    # (an injected stop is the listed kernels'; the sweeps are stopped in test_sweeps_stopped_and_resumed_leave_the_same_bits)
     wl = "miniweather@nx=1024,nz=512"
     base = ex_mod.Executor(wl)
     ex = ex_mod.Executor(wl, blp=True)
@@ -255,3 +257,38 @@ def test_sweeps_leave_what_the_kernels_leave(gp, ex_mod, nx, nz, blp):
             listed.launch_kernel(i)
         for a, b, name in zip(_arrays(swept), _arrays(listed), ("state", "state_tmp", "flux")):
             assert np.array_equal(a, b), name
+
+
+@pytest.mark.parametrize("nx,nz", [(3200, 1600), (1203, 2001)])
+def test_sweeps_stopped_and_resumed_leave_the_same_bits(gp, ex_mod, nx, nz):
+    """A sweep writes what the next one reads: claims run twice, or left out, show in the bits.  The host raises the flag
+    at several moments of a step, and twice in some."""
+    wl = f"miniweather@nx={nx},nz={nz}"
+    base, ex = ex_mod.Executor(wl), ex_mod.Executor(wl, blp=True)
+    flag, stream = gp.Flag(), gp.Stream(1)
+    ex.set_flag(flag)
+    ex.set_running(True)
+
+    def wait(us):
+        until = time.perf_counter() + us * 1e-6
+        while time.perf_counter() < until:
+            pass
+
+    amid = set()
+    for delays in ((0,), (15,), (40,), (65,), (90, 30), (120,), (150, 20), (190,), (230, 0), (280,)):
+        base.execute()
+        ex.execute(stream)
+        for delay in delays:
+            wait(delay)
+            flag.set(1)
+            stream.sync()
+            counters = ex.counters()
+            flag.set(0)
+            ex.resume(stream)
+            at = ex.last_stop_index()
+            if at != -1 and counters[at] > 0:
+                amid.add(at // 9)
+        stream.sync()
+        for a, b, name in zip(_arrays(base), _arrays(ex), ("state", "state_tmp", "flux")):
+            assert np.array_equal(a, b), (delays, name)
+    assert len(amid) >= 2, amid  # (of the four sweeps: stopped with some of its claims taken)

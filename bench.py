@@ -1,13 +1,14 @@
 #!/usr/bin/env python3
-"""Headline benchmark: BASELINE.json config 3 on one MI355X.
+"""Headline benchmark on one MI355X: a high-priority BERT over a best-effort ResNet-152.
 
 High-priority tenant: BERT-base fp16, batch 1, seq 128, Poisson arrivals at 200 req/s.
 Best-effort tenant: ResNet-152 fp16, batch 8, 224x224, back to back, block-level preemptible.
 A "step" is one high-priority request served while the best-effort tenant co-runs; inputs are
 synthetic and resident before the timed region; weights are seeded random-init.
 
-Prints ONE JSON line.  `value` = co-run p99 latency of the high-priority tenant / its isolated
-p99 (the first figure of BASELINE.json's metric); the other two (preemption latency, best-effort
+Prints ONE JSON line, short enough for a log that keeps the last few kilobytes (`--details FILE`
+writes everything that was measured).  `value` = co-run p99 latency of the high-priority tenant / its
+isolated p99; the metric's other two figures (preemption latency, best-effort
 throughput kept) and the absolute latencies ride along in the same line, together with
   roofline      the dominant kernel (MFMA implicit-GEMM convolution of the best-effort model),
                 timed live with HIP events on the stream it is launched on
@@ -69,7 +70,7 @@ def run_config(cfg):
 
 
 def config_leg(name, seconds):
-    """One of the scenario files under gpreempt_amd/config/ (BASELINE configs 4 and 5) for a bounded time:
+    """One of the scenario files under gpreempt_amd/config/ for a bounded time:
     high-priority p99 against isolated, preemption latency, and what every lower level kept."""
     with open(os.path.join(ROOT, "gpreempt_amd", "config", name)) as f:
         cfg = json.load(f)
@@ -122,7 +123,7 @@ def summarize(rep):
 
 
 def probe(workload, trials, mode=2):
-    """per-kernel preemption / resume latency of one best-effort model, stopped at random
+    """Per-kernel preemption / resume latency of one best-effort model, stopped at random
     instants by the host.  mode 2: kernel by kernel with a bounded queue (how a tenant is fed); 1: the whole model
     as one persistent program."""
     from gpreempt_amd import executor as gx
@@ -215,7 +216,7 @@ def _time_gemm(gp, p, stream, st, iters):
 
 
 def config1_gemm1024(iters=20):
-    """BASELINE config 1: C = relu(A B + bias), 1024^3 fp32, as a plain and as a preemptible launch
+    """C = relu(A B + bias), 1024^3 fp32, as a plain and as a preemptible launch
     (the difference is what the dispatcher costs: the same kernel with and without claim counters, flag never raised)."""
     import numpy as np
     from gpreempt_amd import capi as gp
@@ -242,7 +243,7 @@ def config1_gemm1024(iters=20):
 
 
 def gemm_roofline(iters=10, operands="random"):
-    """BASELINE config 5's best-effort tenant alone: bf16 8192^3 GEMM (fp32 accumulate): launched
+    """The best-effort tenant of config5_bert384_gemm8192.json alone: bf16 8192^3 GEMM (fp32 accumulate): launched
     plainly, preemptibly (tiles are finished), and preemptibly with the checkpoint workspace that
     lets a 256 x 256 tile be left between two K-steps.  operands = "const" fills both matrices with
     1.0 instead (fewer bits toggle in the matrix cores: the same instruction stream at lower power)."""
@@ -358,9 +359,11 @@ def hbm_ops(iters=20):
 
 
 def miniweather(steps=50):
-    """The reference's non-DNN workload at its own size (3200 x 1600 cells): one execute() = 36
-    preemptible kernels = two time steps.  Achieved bandwidth = algorithmic bytes of the kernel
-    list / HIP-event time, against the 8 TB/s HBM peak; mass / energy drift over the run is the
+    """The reference's non-DNN workload at its own size (3200 x 1600 cells): one execute() = four
+    preemptible launches, the direction sweeps x, z, z, x that stand for the list's 36 kernels.  Achieved bandwidth = algorithmic bytes of
+    the sweeps / HIP-event time, against the 8 TB/s HBM peak: each reads the state and writes the next, and the
+    step leaves the second stage's state and the fluxes once.  (The kernels of the list would move six times
+    as much; the sweeps are bound by their arithmetic instead.)  Mass / energy drift over the run is the
     workload's own self-check; the CPU figure is the oracle on a 400 x 200 grid scaled by cells."""
     from gpreempt_amd import capi as gp, executor as E
     from oracle import miniweather as MW
@@ -378,7 +381,8 @@ def miniweather(steps=50):
     b.sync()
     ms = a.elapsed_ms(b) / steps
     m1, e1 = ex.miniweather_reductions()
-    nbytes = sum(k["bytes"] for k in ex.kernels())
+    nbytes = 4 * 2 * ex.data_size("state") + ex.data_size("state_tmp") + ex.data_size("flux")
+    listed = sum(k["bytes"] for k in ex.kernels())
     sim = MW.Sim(400, 200)
     sim.timestep()
     t0 = time.perf_counter()
@@ -386,8 +390,8 @@ def miniweather(steps=50):
         sim.timestep()
     cpu_ms = (time.perf_counter() - t0) / 5 * 1e3 * (3200 * 1600) / (400 * 200)
     ex.destroy()
-    return {"workload": "miniweather 3200x1600 fp32, collision test case, 36 kernels per execute", "ms_per_execute": ms,
-            "algorithmic_MB": nbytes / 1e6, "achieved_GBps": nbytes / ms / 1e6, "frac_of_hbm_peak": nbytes / ms / 1e6 / 8000.0,
+    return {"workload": "miniweather 3200x1600 fp32, collision test case, four direction sweeps per execute", "ms_per_execute": ms,
+            "algorithmic_MB": nbytes / 1e6, "listed_kernels_MB": listed / 1e6, "achieved_GBps": nbytes / ms / 1e6, "frac_of_hbm_peak": nbytes / ms / 1e6 / 8000.0,
             "mass_drift": abs(m1 - m0) / m0, "energy_drift": abs(e1 - e0) / e0, "executes": steps + 3,
             "cpu_oracle_ms_per_execute_scaled": cpu_ms, "cpu_cores": 1,
             "cpu_unit": "ms per execute on 1 core (numpy oracle on a 400 x 200 grid, scaled by cells)"}
@@ -396,9 +400,8 @@ def miniweather(steps=50):
 def graph_workloads(runs=5):
     """The reference's graph workloads on a seeded random graph (2^20 vertices, 16.8 M directed
     edges; the reference's dataset does not ship with it): wall time of one execute() to
-    convergence, preemptible launches; bytes = per iteration, every edge id (8 B) and its
-    endpoint's word once, an upper bound that frontier-driven iterations stay well below, so the
-    bandwidth figure is indicative only.  CPU figure: the numpy oracle on a 2^16-vertex graph of the
+    convergence, preemptible launches; edge visits = every edge in every iteration, an upper bound that
+    frontier-driven iterations stay well below.  CPU figure: the numpy oracle on a 2^16-vertex graph of the
     same degree, scaled by edges."""
     import ctypes as C
     import os
@@ -435,7 +438,7 @@ def graph_workloads(runs=5):
 
 def vendor_gemm(operands="random", iters=20):
     """For scale only (never part of the default run or of `value`): the vendor library's GEMM through
-    torch.matmul at config 5's size and operand layout (A [M,K] times the transpose of B [N,K])."""
+    torch.matmul at the size of config5_bert384_gemm8192.json and operand layout (A [M,K] times the transpose of B [N,K])."""
     import torch
     n = 8192
     if operands == "random":
@@ -574,8 +577,7 @@ def summary_of(out):
                       "req_s": {k: r2(v["req_s"]) for k, v in c["levels"].items() if v["priority"] > 0},
                       "gpu_drain_us_mean_p99": [r2(c["device_stamps_us"]["flagStore_to_lastWorkgroupExit"][q]) for q in ("mean", "p99")] if c.get("device_stamps_us") else None}
             if tag == "config2":
-                # the high-priority tenant of this scenario is a 53 us probe request that is only there to preempt (BASELINE
-                # config 2 asks for preemption latency and a bit-exact resume): its own latency in microseconds, not a ratio
+                # the high-priority tenant of this scenario is a 53 us probe request that is only there to preempt: its own latency in microseconds, not a ratio
                 probe = [v for v in c["levels"].values() if v["priority"] == 0]
                 del s[tag]["hp_p99_vs_isolated"]
                 if probe:
@@ -603,6 +605,30 @@ def summary_of(out):
     return s
 
 
+def extract(out):
+    """What the printed line holds of a whole run: the headline, the roofline and the CPU figures, the rest in the
+    summary's numbers; floats to six digits."""
+    keep = dict(out)
+    for k in ("config2_resnet50_fp32_b1", "config2_resnet50_fp32_b1_as_one_program", "config2_resnet50_fp32_b1_preempted", "config4_three_tenants",
+              "config5_bert384_over_gemm8192", "device_stamps", "headline_600", "hp_first_corun_latencies_ms"):
+        keep.pop(k, None)  # (in the summary)
+    keep["other_policies"] = {p: {k: r[k] for k in ("hp_p99_vs_isolated", "be_throughput_kept")} | {"preempt_us_p99": r["preemption_latency_us"]["p99"]}
+                              for p, r in out.get("other_policies", {}).items()}
+    if "config1_gemm1024_f32" in out:
+        keep["config1_gemm1024_f32"] = {k: out["config1_gemm1024_f32"][k] for k in ("plain_us", "preemptible_us", "achieved", "frac")}
+    keep["hbm_bound_ops"] = {k: {"us": v["us"], "frac": v["frac"]} for k, v in out.get("hbm_bound_ops", {}).items()}
+    keep["graph_workloads"] = {k: {"ms": v["ms_per_execute"], "iterations": v["iterations"], "cpu_1_core_ms": v["cpu_oracle_ms_scaled"]} if isinstance(v, dict) else v
+                               for k, v in out.get("graph_workloads", {}).items()}
+
+    def digits(v):
+        if isinstance(v, float):
+            return float(f"{v:.6g}")
+        if isinstance(v, dict):
+            return {k: digits(x) for k, x in v.items()}
+        return [digits(x) for x in v] if isinstance(v, list) else v
+    return digits(keep)
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -614,7 +640,8 @@ def main():
     ap.add_argument("--be-model", default="resnet152")
     ap.add_argument("--only", default="", help="run one leg only: scenario | roofline | gemm | hbm | miniweather | graphs | cpu | copycal | vendor | hp")
     ap.add_argument("--cpu-requests", type=int, default=10, help="timed submissions per graph in the cpu_baseline leg")
-    ap.add_argument("--config-seconds", type=float, default=5.0, help="co-run time of each of the config 2, 4 and 5 scenario legs")
+    ap.add_argument("--config-seconds", type=float, default=5.0, help="co-run time of each leg that runs a scenario file")
+    ap.add_argument("--details", default="", help="write everything that was measured to this file (the printed line is an extract)")
     ap.add_argument("--gemm-operands", default="random", choices=("random", "const"), help="operands of the 8192^3 GEMM leg (--only gemm)")
     args = ap.parse_args()
     if args.gpus != 1:
@@ -629,7 +656,7 @@ def main():
     out = {"metric": "HP p99 latency vs isolated (co-run p99 / isolated p99); preemption latency (us); BE throughput kept",
            "unit": "x (ratio)", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup, "higher_is_better": False,
            "scaling": "weak", "vs_baseline": None, "dtype": "f16", "data": "synthetic (seeded random-init weights, N(0,1) images, uniform token ids)",
-           "config": {"workload": "BASELINE config 3: HP BERT-base fp16 b1 s128 Poisson %g req/s + BE ResNet-152 fp16 b8 224x224 back-to-back" % args.hp_rate,
+           "config": {"workload": "HP BERT-base fp16 b1 s128 Poisson %g req/s + BE ResNet-152 fp16 b8 224x224 back-to-back" % args.hp_rate,
                       "policy": args.policy, "hp_model": args.hp_model, "be_model": args.be_model}}
     if args.only in ("", "scenario"):
         rep = summarize(scenario(args.steps, args.warmup, args.policy, args.hp_rate, args.be_model, args.hp_model))
@@ -656,9 +683,9 @@ def main():
             alone = scenario(max(200, args.steps // 2), args.warmup, "lco", args.hp_rate, args.be_model, args.hp_model)["tasks"]["hp"]
             out["hp_alone_same_arrivals_ms"] = {k: alone["totalLatency(us)"][k] / 1e3 for k in ("mean", "p50", "p99")}
             out["hp_p99_vs_alone_same_arrivals"] = out["hp_corun_ms"]["p99"] / out["hp_alone_same_arrivals_ms"]["p99"]
-            # BASELINE configs 4 and 5 for a few seconds each, and the headline scenario with device time stamps
-            # config 2's tenant as the default policy runs a best-effort tenant (per-kernel launches, two chunks ahead),
-            # stopped at random instants by a high-priority tenant that does next to nothing
+            # three scenario files for a few seconds each, and the headline scenario with device time stamps
+            # (ResNet-50 as the default policy runs a best-effort tenant (per-kernel launches, two chunks ahead),
+            # stopped at random instants by a high-priority tenant that does next to nothing)
             out["config2_resnet50_fp32_b1_preempted"] = config_leg("config2_resnet50_fp32_preempted.json", args.config_seconds)
             out["config4_three_tenants"] = config_leg("config4_bert_densenet201_vgg16.json", args.config_seconds)
             out["config5_bert384_over_gemm8192"] = config_leg("config5_bert384_gemm8192.json", args.config_seconds)
@@ -682,7 +709,10 @@ def main():
         out["cpu_baseline"] = cpu_baseline(args.cpu_requests)
     if not args.only:
         out["summary"] = summary_of(out)  # last on purpose: whoever keeps only the end of the line keeps this
-    print(json.dumps(out))
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump(out, f, indent=1)
+    print(json.dumps(out if args.only else extract(out), separators=(",", ":")))
 
 
 if __name__ == "__main__":

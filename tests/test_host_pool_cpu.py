@@ -63,9 +63,22 @@ def test_a_loop_allocates_twice_and_the_garbage_collector_frees_nothing(counting
     assert (a == 7).all()
 
 
+def test_a_new_executor_finds_the_blocks_of_the_last_one(counting):
+    pool = capi.HostPool()
+    out = pool.empty(84 << 20)
+    out = pool.empty(84 << 20)
+    pool.trim()  # (the executor goes first, its last output afterwards)
+    del out
+    pool.trim()
+    for _ in range(3):
+        assert pool.empty(84 << 20)[1] is not None
+        pool.trim()
+    assert counting.allocated == 2 and counting.freed == 0
+
+
 def test_trim_keeps_the_small_blocks(counting):
     pool = capi.HostPool()
-    arrays = [pool.empty(n) for n in (4096, 4096, 1 << 20, 40 << 20, 100 << 20)]
+    arrays = [pool.empty(n) for n in (4096, 4096, 1 << 20, 100 << 20, 200 << 20)]
     pool.trim(0)
     assert counting.freed == 0  # all of them are in use
     del arrays

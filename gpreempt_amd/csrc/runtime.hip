@@ -224,6 +224,13 @@ extern "C" int gp_malloc(void **dev, size_t bytes) {
     GP_HIP(hipMalloc(dev, bytes ? bytes : 1));
     return GP_SUCC;
 }
+extern "C" int gp_malloc_capturing(void **dev, size_t bytes) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    GP_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+    const int rc = gp_malloc(dev, bytes);
+    GP_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+    return rc;
+}
 extern "C" int gp_free(void *dev) { if (dev) GP_HIP(hipFree(dev)); return GP_SUCC; }
 extern "C" int gp_host_alloc(void **host, size_t bytes) {
     GP_REQUIRE(host != nullptr, "null out pointer");

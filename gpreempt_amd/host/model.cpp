@@ -561,7 +561,7 @@ void Model::launched(size_t idx, bool preemptible, const gp_launch_info &info) {
 
 Status Model::launch_sweep(size_t g, GPUstream stream) {
     if (g >= sweeps_.size()) return Status::OutOfRange;
-    if (!sweep_state_) CUDA_RETURN_STATUS(gp_malloc(&sweep_state_, get_storage_size(kernel_infos[0].args_index[0])));
+    if (!sweep_state_) CUDA_RETURN_STATUS(gp_malloc_capturing(&sweep_state_, get_storage_size(kernel_infos[0].args_index[0])));
     gp_mw_sweep_params &p = sweeps_[g];
     p.in = g % 2 ? (const float *)sweep_state_ : p.state;
     p.out = g % 2 ? p.state : (float *)sweep_state_;

@@ -70,6 +70,7 @@ int gp_event_elapsed_ms(gp_event start, gp_event stop, float *ms);
  * Replaces GPUMemAlloc / GPUMemFree / GPUMemcpy* / GPUMemsetAsync / GPUMemHostAlloc
  * (include/util/gpu_util.h:74-139; uses in src/model.cpp:101-113,268-279,296-327). */
 int gp_malloc(void **dev, size_t bytes);
+int gp_malloc_capturing(void **dev, size_t bytes);  /* also while this thread captures a stream (gp_graph_begin); not a node of the graph */
 int gp_free(void *dev);
 int gp_host_alloc(void **host, size_t bytes); /* pinned */
 int gp_host_free(void *host);

@@ -15,6 +15,7 @@ static long g_allocated = 0, g_blocks = 0;
 // (these take the place of the library's: the executable's symbols come first)
 extern "C" {
 int gp_malloc(void **p, size_t n) { *p = std::calloc(1, n ? n : 1); g_allocated += (long)n; ++g_blocks; return 0; }
+int gp_malloc_capturing(void **p, size_t n) { return gp_malloc(p, n); }
 int gp_free(void *p) { if (p) --g_blocks; std::free(p); return 0; }
 int gp_memcpy_h2d(void *d, const void *h, size_t n) { std::memcpy(d, h, n); return 0; }
 int gp_fill32_async(void *, uint32_t, size_t, gp_stream) { return 0; }

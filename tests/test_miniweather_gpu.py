@@ -292,3 +292,24 @@ def test_sweeps_stopped_and_resumed_leave_the_same_bits(gp, ex_mod, nx, nz):
         for a, b, name in zip(_arrays(base), _arrays(ex), ("state", "state_tmp", "flux")):
             assert np.array_equal(a, b), (delays, name)
     assert len(amid) >= 2, amid  # (of the four sweeps: stopped with some of its claims taken)
+
+
+def test_first_sweeps_may_be_captured(gp, ex_mod):
+    """The state between two sweeps is allocated by the first of them, also where a stream is being captured: the graph
+    is replayed between eager steps of the same executor and leaves what those leave"""
+    wl = "miniweather@nx=233,nz=150"
+    base, ex = ex_mod.Executor(wl), ex_mod.Executor(wl)
+    stream, graph = gp.Stream(1), C.c_void_p()
+    gp.check(gp.lib().gp_graph_begin(stream.h))
+    ex.execute(stream)
+    gp.check(gp.lib().gp_graph_end(stream.h, C.byref(graph)))
+    for step in range(6):
+        base.execute()
+        if step % 3 == 2:
+            ex.execute(stream)
+        else:
+            gp.check(gp.lib().gp_graph_launch(graph, stream.h))
+        stream.sync()
+        for a, b, name in zip(_arrays(base), _arrays(ex), ("state", "state_tmp", "flux")):
+            assert np.array_equal(a, b), (step, name)
+    gp.check(gp.lib().gp_graph_destroy(graph))

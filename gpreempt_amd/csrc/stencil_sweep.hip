@@ -1,13 +1,13 @@
 // A direction sweep of miniWeather in one launch.
 //
 // Kernel by kernel a sweep reads and writes the 82 MB state (3200 x 1600 cells) eight times per Runge-Kutta stage and
-// is bound by that: 390 us per sweep.  But a sweep couples cells along its own direction only, and a stage reaches two
+// is bound by that: 280 us per sweep.  But a sweep couples cells along its own direction only, and a stage reaches two
 // cells to either side.  So a wavefront takes a stretch of 64 * CELLS consecutive cells along the sweep, six of them at
 // either end belonging to its neighbours, and carries them through the three stages in registers: lane l holds cells
 // CELLS * l .. CELLS * l + CELLS - 1, the cells and fluxes of the next lanes come by DPP wave shifts, and the state is
 // read and written once.  What bounds it now is the arithmetic: 145 vector instructions per cell and stage, for an
-// eighth more cells than there are.  88 us per sweep, 106 (x) and 96 (z) for the two that also leave state_tmp and the
-// fluxes; two cells per lane, since four take 140-200 registers (x 100-130 us, z 154-175).
+// eighth more cells than there are.  86 us per preemptible sweep, 101 (x) and 90 (z) for the two that also leave state_tmp
+// and the fluxes; two cells per lane, since four take 140-200 registers (x 100-130 us, z 154-175).
 //
 // x: rows are contiguous, a wavefront loads and stores its stretch itself.  z: a workgroup brings 16 columns of a
 // stretch in through LDS (64-byte runs of every row; a column is contiguous there), and its wavefronts take a column

@@ -165,6 +165,8 @@ int plan_launch(Kernel kernel, int block, size_t lds_bytes, int sx, int sy, int 
         for (int g = 0; g < 4; ++g) blp->poll_n[g] = 0;
         *grid = (int)total;
     }
+    blp->grid = *grid;
+    blp->inv_sx = inverse_of(sx, tiles); blp->inv_sy = inverse_of(sy, tiles);
     if (info) {
         info->total_tiles = (int)total; info->shape[0] = sx; info->shape[1] = sy; info->shape[2] = sz;
         info->grid = *grid; info->block = block;

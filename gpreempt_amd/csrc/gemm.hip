@@ -271,6 +271,7 @@ int plan_conv2d(const gp_conv_params *p, MatPlan *out) {
     g.alpha = 1.f; g.act = p->act; g.batch_inner = 0;
     g.H = p->H; g.W = p->W; g.Cin = p->Cin; g.S = p->S; g.Ho = Ho; g.Wo = Wo;
     g.sh = p->stride_h; g.sw = p->stride_w; g.ph = p->pad_h; g.pw = p->pad_w;
+    g.R = p->R; g.rcp_hw = 1.0f / (float)(Ho * Wo); g.rcp_wo = 1.0f / (float)Wo;
     pl.dtype = p->dtype; pl.conv = 1; pl.b_kn = 0; pl.batch = 1;
     return choose_body(&pl, p->tile_m, p->tile_n, p->variant);
 }

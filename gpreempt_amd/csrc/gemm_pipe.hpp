@@ -119,6 +119,7 @@ template <typename T, int BM, int BN, int STAGES, bool CONV, bool SPLITK, bool C
 struct PipeKernel {
     using elem = T;
     static constexpr int bm = BM, bn = BN;
+    static constexpr bool conv = CONV;
     static constexpr int VEC = Elem<T>::VEC;
     static constexpr int WAVES = NWAVES, NT = WAVES * 64;
     static constexpr int RB = 128;                        // row bytes in LDS
@@ -207,13 +208,12 @@ struct PipeKernel {
         if (CONV) {
             const int hw = g.Ho * g.Wo;
             const bool small = g.M < kSmallDivLimit;
-            const float rcp_hw = 1.0f / (float)hw, rcp_wo = 1.0f / (float)g.Wo;
 #pragma unroll
             for (int j = 0; j < A_PW; ++j) {
                 int m = a_row0 + j * 8;
                 int mm = m < g.M ? m : 0;
-                int n = small ? small_div(mm, hw, rcp_hw) : mm / hw, rem = mm - n * hw;
-                int ho = small ? small_div(rem, g.Wo, rcp_wo) : rem / g.Wo, wo = rem - ho * g.Wo;
+                int n = small ? small_div(mm, hw, g.rcp_hw) : mm / hw, rem = mm - n * hw;
+                int ho = small ? small_div(rem, g.Wo, g.rcp_wo) : rem / g.Wo, wo = rem - ho * g.Wo;
                 a_h0[j] = ho * g.sh - g.ph; a_w0[j] = wo * g.sw - g.pw;
                 a_org[j] = A + ((long)n * g.H * g.W + (long)a_h0[j] * g.W + a_w0[j]) * g.lda;
             }

@@ -132,6 +132,7 @@ template <typename T, int BM, int BN, int WAVES, int STAGES, bool CONV = false>
 struct WideKernel {
     using elem = T;
     static constexpr int bm = BM, bn = BN;
+    static constexpr bool conv = CONV;
     static constexpr int VEC = Elem<T>::VEC;
     static constexpr int NT = WAVES * 64;
     static constexpr int RB = 128;                         // row bytes of a block in LDS
@@ -208,9 +209,19 @@ struct WideKernel {
         // SIMD: with 64-bit addresses, selects and a page of zeros a stage of a 3 x 3 layer cost as much in vector
         // instructions as its loads take.
         const int rig = lane >> 3, cpos = lane & 7;
-        const int hw = CONV ? g.Ho * g.Wo : 1, ntap_rows = CONV ? g.K / (g.Cin * g.S) : 0;
-        const bool small = g.M < kSmallDivLimit;
-        const float rcp_hw = 1.0f / (float)hw, rcp_wo = CONV ? 1.0f / (float)g.Wo : 1.0f;
+        // CONV: where a row's window lies and which of its taps are inside the image, worked out by one lane per row (eight lanes of
+        // each of the KB wavefront groups need it; every one for itself, that was some hundred vector instructions in front of the first
+        // load, four wavefronts to a SIMD)
+        __shared__ unsigned row_off[CONV ? BM : 1], row_taps[CONV ? BM : 1];
+        if (CONV && tid < BM) {
+            const int m = m0 + tid, hw = g.Ho * g.Wo;
+            const bool in = m < g.M, small = g.M < kSmallDivLimit;
+            const int mm = in ? m : 0;
+            const int n = small ? small_div(mm, hw, g.rcp_hw) : mm / hw, rem = mm - n * hw;
+            const int ho = small ? small_div(rem, g.Wo, g.rcp_wo) : rem / g.Wo, wo = rem - ho * g.Wo;
+            row_off[CONV ? tid : 0] = (unsigned)((n * g.H + ho * g.sh) * g.W + wo * g.sw) * (unsigned)g.lda;
+            row_taps[CONV ? tid : 0] = in ? window_tap_mask(ho * g.sh - g.ph, wo * g.sw - g.pw, g.H, g.W, g.R, g.S) : 0u;
+        }
         // (CONV: offsets count from the origin of the window of output pixel (0, 0), which lies in front of the image by the padding)
         const u32x4 rsrc_a = buffer_of(CONV ? A - (long)(g.ph * g.W + g.pw) * g.lda : A), rsrc_b = buffer_of(B);
         unsigned off[LPW];     // the lane's row and chunk at k = 0, in bytes
@@ -222,15 +233,7 @@ struct WideKernel {
             const bool is_a = j < LPW_A;
             const int r = (is_a ? gi : gi - BM / 8) * 8 + rig;   // row in its region
             kc[j] = (cpos ^ ((r >> 1) & 7)) * VEC;
-            if (is_a && CONV) {
-                const int m = m0 + r;
-                const bool in = m < g.M;
-                const int mm = in ? m : 0;
-                const int n = small ? small_div(mm, hw, rcp_hw) : mm / hw, rem = mm - n * hw;
-                const int ho = small ? small_div(rem, g.Wo, rcp_wo) : rem / g.Wo, wo = rem - ho * g.Wo;
-                off[j] = ((unsigned)((n * g.H + ho * g.sh) * g.W + wo * g.sw) * (unsigned)g.lda + (unsigned)kc[j]) * (unsigned)sizeof(T);
-                taps[CONV ? j : 0] = in ? window_tap_mask(ho * g.sh - g.ph, wo * g.sw - g.pw, g.H, g.W, ntap_rows, g.S) : 0u;
-            } else {
+            if (!is_a || !CONV) {
                 const int x = (is_a ? m0 : n0) + r;
                 off[j] = x < (is_a ? g.M : g.N) ? ((unsigned)x * (unsigned)(is_a ? g.lda : g.ldb) + (unsigned)kc[j]) * (unsigned)sizeof(T) : kBufferEnd;
             }
@@ -239,12 +242,15 @@ struct WideKernel {
         const int NS = (KT + KB - 1) / KB;              // stages
         // CONV: tap and channel of the block this wavefront group fetches next (stages are issued in order)
         int nx_tap = 0, nx_r = 0, nx_s = 0, nx_ci = 0;
-        if (CONV) {
-            nx_tap = kb * BK / g.Cin;
-            nx_ci = kb * BK - nx_tap * g.Cin;
-            nx_r = nx_tap / g.S;
-            nx_s = nx_tap - nx_r * g.S;
-        }
+        auto advance = [&](int elems) {
+            nx_ci += elems;
+            while (nx_ci >= g.Cin) {
+                nx_ci -= g.Cin;
+                ++nx_tap;
+                if (++nx_s == g.S) { nx_s = 0; ++nx_r; }
+            }
+        };
+        if (CONV) advance(kb * BK);
         auto issue = [&](int s) {
             const int k0 = (s * KB + kb) * BK;          // first K element of this wavefront group's block
             const unsigned sbase = lds0 + ((unsigned)s % STAGES) * STAGE_BYTES + (unsigned)kb * BLK_BYTES;
@@ -264,14 +270,7 @@ struct WideKernel {
                     load_lds16_buffer(j < LPW_A ? rsrc_a : rsrc_b, at, (unsigned)k0 * (unsigned)sizeof(T), sbase + (unsigned)(gi * 8 * RB));
                 }
             }
-            if (CONV) {
-                nx_ci += KB * BK;
-                while (nx_ci >= g.Cin) {
-                    nx_ci -= g.Cin;
-                    ++nx_tap;
-                    if (++nx_s == g.S) { nx_s = 0; ++nx_r; }
-                }
-            }
+            if (CONV) advance(KB * BK);
         };
 
         f32x16 acc[BPW];
@@ -287,6 +286,14 @@ struct WideKernel {
         // ---- main loop ------------------------------------------------------------------------
         GP_PROBE(1);
         __syncthreads();  // the previous tile of this workgroup may still be reading LDS
+        if (CONV) {
+#pragma unroll
+            for (int j = 0; j < LPW_A; ++j) {
+                const int r = group_of(wv, j) * 8 + rig;
+                off[j] = (row_off[CONV ? r : 0] + (unsigned)kc[j]) * (unsigned)sizeof(T);
+                taps[CONV ? j : 0] = row_taps[CONV ? r : 0];
+            }
+        }
 #pragma unroll
         for (int s = 0; s < PRE; ++s) {
             if (s < NS) issue(s);

@@ -67,6 +67,8 @@ struct MatArgs {
     int batch_inner;
     // convolution geometry (CONV only)
     int H, W, Cin, S, Ho, Wo, sh, sw, ph, pw;
+    int R;                 // window rows (K = R * S * Cin)
+    float rcp_hw, rcp_wo;  // 1 / (Ho * Wo), 1 / Wo: see small_div
     // layer-norm prologue (gemm_ln.hpp; ln_gamma == nullptr: none): the rows of A are normalised over
     // their K elements before they are multiplied, and written to ln_out (M x K)
     const void *ln_gamma, *ln_beta;

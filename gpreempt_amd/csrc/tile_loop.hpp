@@ -67,6 +67,8 @@ struct BlpArgs {
     int done_target;
     int *started;     // nullptr, or a word in host memory in which the first workgroup stores started_seq when it starts
     int started_seq;  // (gp_preempt_ctx::started_host: the host's flow control when it submits kernel by kernel)
+    int grid;         // gridDim.x (which the compiler reads from a line of its own behind the arguments, one more trip to memory)
+    unsigned inv_sx, inv_sy;  // inverse_of(sx), inverse_of(sy), see util/slice_map.h
 };
 
 // The first workgroup tells the host that this launch has reached the GPU, i.e. that everything submitted before it on
@@ -77,7 +79,7 @@ __device__ __forceinline__ void announce_start(const BlpArgs &b, bool leader) {
 
 // a worker's number among the workers of the launch, and how many there are
 __device__ __forceinline__ int wg_id(const BlpArgs &b) { return (int)blockIdx.x - b.front; }
-__device__ __forceinline__ int wg_count(const BlpArgs &b) { return (int)gridDim.x - b.front; }
+__device__ __forceinline__ int wg_count(const BlpArgs &b) { return b.grid - b.front; }
 
 // Device-scope atomics on ONE address complete at about one per 40 ns on MI355X: a kernel of a
 // few hundred tiles claimed from a single counter spends 10-20 us on claims alone.  A caller may
@@ -88,7 +90,9 @@ constexpr int COUNTER_STRIDE = 16;  // ints
 
 struct TileIdx { int x, y, z; };
 
-__device__ __forceinline__ TileIdx decode_tile(int idx, int sx, int sy, int order = 0) {
+// (inv_sx, inv_sy: the divisions by sx and sy as one multiplication each; 0: as divisions, some sixty instructions in front
+// of a tile's first load)
+__device__ __forceinline__ TileIdx decode_tile(int idx, int sx, int sy, int order = 0, unsigned inv_sx = 0, unsigned inv_sy = 0) {
     // x = idx % sx; y = (idx / sx) % sy; z = idx / (sx*sy)   (convert_to_blp.py:52-54);
     // order 1 swaps the roles of x and y, so that consecutive indices share a tile column
     // order G >= 2: bands of G tile rows, y fastest inside a band, so that consecutive indices
@@ -106,14 +110,14 @@ __device__ __forceinline__ TileIdx decode_tile(int idx, int sx, int sy, int orde
         t.x = local / rows;
         t.y = first_y + (local - t.x * rows);
     } else if (order == 0) {
-        int q = idx / sx;
+        int q = divide_by(idx, sx, inv_sx);
         t.x = idx - q * sx;
-        t.z = q / sy;
+        t.z = divide_by(q, sy, inv_sy);
         t.y = q - t.z * sy;
     } else {
-        int q = idx / sy;
+        int q = divide_by(idx, sy, inv_sy);
         t.y = idx - q * sy;
-        t.z = q / sx;
+        t.z = divide_by(q, sx, inv_sx);
         t.x = q - t.z * sx;
     }
     return t;
@@ -240,7 +244,7 @@ __device__ __forceinline__ int claim_fixed(const BlpArgs &b, int grp) {
 // leaves.  The read of host memory (1-2 us) then delays nobody's tile, where a poll after the
 // first claims made four workgroups, and with them the kernel, finish that much later.
 __device__ __forceinline__ bool spare_workgroup(const BlpArgs &b, bool fixed, bool leader) {
-    if (!fixed || b.spare == 0 || (int)blockIdx.x < (int)gridDim.x - b.spare) return false;
+    if (!fixed || b.spare == 0 || (int)blockIdx.x < b.grid - b.spare) return false;
     if (leader && b.flag && __hip_atomic_load(b.flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0 &&
         __hip_atomic_load(b.stop_index, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == -1)
         record_stop(b.stop_index, b.kernel_id, b.stamps);
@@ -317,7 +321,7 @@ __device__ __forceinline__ int *done_counter(const BlpArgs &b) { return b.done +
 // the front workgroup; the measurement mode stamps the moment.
 __device__ __forceinline__ void leave_stamped(const BlpArgs &b, bool count = true) {
     if (!b.executed || (!b.stamps && !b.done)) return;
-    if (wg_id(b) < 0 || (int)blockIdx.x >= (int)gridDim.x - b.spare) return;  // front and spare workgroups are no workers
+    if (wg_id(b) < 0 || (int)blockIdx.x >= b.grid - b.spare) return;  // front and spare workgroups are no workers
     const bool leader = (threadIdx.x == 0) & (threadIdx.y == 0) & (threadIdx.z == 0);
     if (b.stamps) {
         __syncthreads();
@@ -369,7 +373,7 @@ __device__ __forceinline__ void tile_loop(const BlpArgs &b, Body &&body) {
         // Streaming kernels have tiles of a few KB; handing them out several at a time keeps the
         // claim (an atomic and a barrier, 1-2 us) off their critical path.
         const int first = idx * b.batch, last = first + b.batch < b.tiles ? first + b.batch : b.tiles;
-        for (int tile = first; tile < last; ++tile) body(decode_tile(tile, b.sx, b.sy, b.order));
+        for (int tile = first; tile < last; ++tile) body(decode_tile(tile, b.sx, b.sy, b.order, b.inv_sx, b.inv_sy));
         if (single) { leave_stamped(b); return; }
     }
 }
@@ -390,7 +394,7 @@ __device__ __forceinline__ void tile_loop(const BlpArgs &b, Body &&body) {
 template <class Body>
 __device__ __forceinline__ void tile_plain(const BlpArgs &b, Body &&body) {
     if ((int)blockIdx.x >= b.total) return;
-    body(decode_tile(xcd_contiguous((int)blockIdx.x, b.total), b.sx, b.sy, b.order));
+    body(decode_tile(xcd_contiguous((int)blockIdx.x, b.total), b.sx, b.sy, b.order, b.inv_sx, b.inv_sy));
 }
 
 // the claim of a workgroup of a launch with fixed claims, for all its threads; -1: leave
@@ -448,7 +452,7 @@ __device__ __forceinline__ void tile_fixed_early(const BlpArgs &b, Body &&body) 
     }
     if (idx < 0) { leave_stamped(b); return; }
     int *word = (eager || b.spare || b.front) ? b.stop_index : nullptr;
-    const bool left = body(decode_tile(idx, b.sx, b.sy, b.order), word);
+    const bool left = body(decode_tile(idx, b.sx, b.sy, b.order, b.inv_sx, b.inv_sy), word);
     if (left && threadIdx.x == 0) unclaim_fixed(b);
     leave_stamped(b, !(ANNOUNCES && word != nullptr && !left));
 }
@@ -457,7 +461,7 @@ template <class Body>
 __device__ __forceinline__ void tile_fixed(const BlpArgs &b, Body &&body) {
     const int idx = fixed_claim_of_workgroup(b);
     if (idx < 0) { leave_stamped(b); return; }
-    body(decode_tile(idx, b.sx, b.sy, b.order));
+    body(decode_tile(idx, b.sx, b.sy, b.order, b.inv_sx, b.inv_sy));
     leave_stamped(b);
 }
 
@@ -550,8 +554,8 @@ __device__ __forceinline__ void tile_loop_ckpt(const BlpArgs &b, Body &&body) {
     const bool dynamic = b.executed != nullptr;
     const bool leader = (threadIdx.x == 0) & (threadIdx.y == 0) & (threadIdx.z == 0);
     const int grp = wg_group((int)blockIdx.x, b.groups);
-    const int slice_lo = b.groups > 1 ? group_slice_begin(b.total, grp, b.groups, (int)gridDim.x) : 0;
-    const int slice_n = (b.groups > 1 ? group_slice_begin(b.total, grp + 1, b.groups, (int)gridDim.x) : b.total) - slice_lo;
+    const int slice_lo = b.groups > 1 ? group_slice_begin(b.total, grp, b.groups, b.grid) : 0;
+    const int slice_n = (b.groups > 1 ? group_slice_begin(b.total, grp + 1, b.groups, b.grid) : b.total) - slice_lo;
     announce_start(b, leader);
     for (int it = 0;; ++it) {
         int idx, kt0 = 0;
@@ -588,10 +592,10 @@ __device__ __forceinline__ void tile_loop_ckpt(const BlpArgs &b, Body &&body) {
             kt0 = __builtin_amdgcn_readfirstlane(mailbox[it & 1][1]);  // K position stay scalar
         }
         if (idx < 0) { leave_stamped(b); return; }
-        if (body(decode_tile(idx, b.sx, b.sy, b.order), idx, kt0)) { leave_stamped(b); return; }
+        if (body(decode_tile(idx, b.sx, b.sy, b.order, b.inv_sx, b.inv_sy), idx, kt0)) { leave_stamped(b); return; }
         // one claim per workgroup at most (see tile_loop); a relaunch may continue a stored tile and
         // then still owe its slice a claim, so the shortcut holds on the fresh path only
-        if ((int)gridDim.x >= b.total && kt0 == 0 && !(it == 0 && b.ckpt)) { leave_stamped(b); return; }
+        if (b.grid >= b.total && kt0 == 0 && !(it == 0 && b.ckpt)) { leave_stamped(b); return; }
     }
 }
 

@@ -73,6 +73,14 @@ GP_HD bool fixed_claims(bool counters, int groups, int grid, int total) {
     return counters && groups > 1 && grid >= total && grid <= groups * kFixedClaimBits;
 }
 
+// n / d as one multiplication: floor((n + 1) * floor((2^32 - 1) / d) / 2^32), exact while (n + 1) * d <= 2^32 (with r = 2^32 - d *
+// floor((2^32 - 1) / d) in 1 .. d and n = q * d + s the product is q + (s + 1 - (n + 1) * r / 2^32) / d, and the bracket lies in
+// 0 .. d).  inverse_of() is 0 where that does not hold for every n up to n_max; divide_by() then divides.
+GP_HD unsigned inverse_of(int d, long n_max) { return d > 0 && (n_max + 1) * (long)d <= 0x100000000l ? 0xFFFFFFFFu / (unsigned)d : 0u; }
+GP_HD int divide_by(int n, int d, unsigned inverse) {
+    return inverse ? (int)(((unsigned long long)(unsigned)(n + 1) * inverse) >> 32) : n / d;
+}
+
 // Launches without claim counters (one workgroup per tile): workgroup b takes tile order index
 // xcd_contiguous(b, total), which gives XCD k the contiguous range of the tile order that its
 // workgroups b = k, k+8, ... cover.

@@ -1,5 +1,6 @@
 // CPU check of include/util/slice_map.h: the slices partition the tile order, their sizes follow
 // the number of workgroups that serve them, and the static mapping is a bijection.
+#include <algorithm>
 #include <cstdio>
 #include <vector>
 #include "util/slice_map.h"
@@ -75,6 +76,17 @@ int main() {
             }
             ++cases;
         }
+    // division by multiplication: every dividend around the multiples of the divisor up to the largest that inverse_of() takes
+    // for it ((n_max + 1) * d <= 2^32), and no inverse beyond
+    for (long d : {1l, 2l, 3l, 7l, 8l, 25l, 64l, 127l, 128l, 129l, 1000l, 4095l, 65535l, 65536l, 65537l, 1l << 20, (1l << 31) - 1}) {
+        const long n_max = std::min(0x100000000l / d - 1, (1l << 31) - 2);
+        const unsigned inv = gp::inverse_of((int)d, n_max);
+        if (!inv || (0x100000000l / d <= (1l << 31) - 2 && gp::inverse_of((int)d, n_max + 1))) { printf("inverse_of(%ld, %ld)\n", d, n_max); return 1; }
+        for (long q = 0; q * d <= n_max; q += 1 + q / 4096)
+            for (long n : {q * d - 1, q * d, q * d + 1, q * d + d - 1, n_max - q})
+                if (n >= 0 && n <= n_max && (gp::divide_by((int)n, (int)d, inv) != n / d || gp::divide_by((int)n, (int)d, 0) != n / d)) { printf("%ld / %ld\n", n, d); return 1; }
+        ++cases;
+    }
     printf("ok %ld cases\n", cases);
     return 0;
 }

@@ -27,13 +27,15 @@ __global__ __launch_bounds__(TK::NT) void mat_kernel(MatArgs g, BlpArgs blp) {
     auto *lds = reinterpret_cast<typename TK::elem *>(lds_raw);
     if constexpr (LOOP != LOOP_ANY) read_args<TK::conv>(g, blp);
     if constexpr (LOOP == LOOP_LOOKS)  // long tiles: fixed claims, and the body looks at the stop word every few K-stages
-        tile_fixed_early<true>(blp, [&](TileIdx t, int *stop) {
+        tile_fixed_early<TK::NT, true>(blp, [&](TileIdx t, int *stop) {
             CkptCtx cc{stop, nullptr, nullptr, 0};
             if (stop && blp.done) cc.announce = done_counter(blp);
-            return TK::template run<true>(g, t, lds, cc);
+            return TK::template run<true, true>(g, t, lds, cc, [&] { late_claim<TK::NT>(blp); });
         });
     else if constexpr (LOOP == LOOP_FIXED && TK::early_stop)
-        tile_fixed_early(blp, [&](TileIdx t, int *stop) { return TK::run(g, t, lds, CkptCtx{stop, nullptr, nullptr, 0}); });
+        tile_fixed_early<TK::NT>(blp, [&](TileIdx t, int *stop) { return TK::template run<false, true>(g, t, lds, CkptCtx{stop, nullptr, nullptr, 0}, [&] { late_claim<TK::NT>(blp); }); });
+    else if constexpr (LOOP == LOOP_PLAIN && TK::early_stop)
+        tile_plain(blp, [&](TileIdx t) { TK::template run<false, true>(g, t, lds); });
     else
         tiles<LOOP>(blp, [&](TileIdx t) { TK::run(g, t, lds); });
 }
@@ -44,7 +46,7 @@ __global__ __launch_bounds__(TK::NT) void mat_kernel_ckpt(MatArgs g, BlpArgs blp
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
     auto *lds = reinterpret_cast<typename TK::elem *>(lds_raw);
     const CkptCtx cc = {blp.executed && blp.ckpt ? blp.stop_index : nullptr, blp.flag, blp.ckpt, blp.kernel_id, blp.stamps};
-    tile_loop_ckpt(blp, [&](TileIdx t, int tile_index, int kt0) { return TK::run(g, t, lds, cc, tile_index, kt0); });
+    tile_loop_ckpt(blp, [&](TileIdx t, int tile_index, int kt0) { return TK::run(g, t, lds, cc, NoneAsked{}, tile_index, kt0); });
 }
 
 template <typename T, int BM, int BN, int BK, int WGM, int WGN, bool CONV, bool B_KN>

@@ -58,7 +58,8 @@ struct LnWideKernel {
     static_assert(STAGES >= 2 && STAGES <= 4 && (STAGES - 1) * LPW < 64, "pipeline depth");
     static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
 
-    static __device__ __forceinline__ bool run(const MatArgs &g, TileIdx t, T *lds_t, CkptCtx cc = CkptCtx{nullptr, nullptr, nullptr, 0}) {
+    template <bool LOOKS = false, bool SINGLE = false, class Asked = NoneAsked>  // (as in PipeKernel)
+    static __device__ __forceinline__ bool run(const MatArgs &g, TileIdx t, T *lds_t, CkptCtx cc = CkptCtx{nullptr, nullptr, nullptr, 0}, Asked &&asked = Asked{}) {
         GP_PROBE(0);
         __shared__ int early_slot[64];
         const bool early = __builtin_amdgcn_readfirstlane((int)(cc.stop_index != nullptr)) != 0;
@@ -91,7 +92,7 @@ struct LnWideKernel {
                 load_lds16_buffer(rsrc_b, k0 < g.K ? off[j] : kBufferEnd, (unsigned)k0 * (unsigned)sizeof(T), sbase + (unsigned)((wv * LPW + j) * 8 * RB));
         };
 
-        __syncthreads();  // the previous tile of this workgroup may still be reading LDS
+        if (!SINGLE) __syncthreads();  // the previous tile of this workgroup may still be reading LDS
 
         // ---- the rows of A: normalise, keep in LDS, store once -------------------------------------
         // wavefront w takes rows w, w + WAVES, ...; lane l holds chunks l and l + 64 of a row.  The rows are
@@ -135,6 +136,7 @@ struct LnWideKernel {
                 if (s < NS) issue(s);
                 if (s == 0 && early && wave == 0) load_lds4(cc.stop_index, (unsigned)(size_t)(__attribute__((address_space(3))) void *)early_slot);
             }
+            asked();
             float v[RPW][MAXC][VEC];
 #pragma unroll
             for (int q = 0; q < RPW; ++q)

@@ -112,6 +112,9 @@ struct CkptCtx {       // what a checkpointing body needs from the dispatcher, p
                                            // top of the last K-step of a tile that it finishes
 };
 
+// what a body does once it has asked for the first stages of its operands: nothing, or the claim (late_claim in tile_loop.hpp)
+struct NoneAsked { __device__ __forceinline__ void operator()() const {} };
+
 // NWAVES: wavefronts per workgroup.  With eight (two per SIMD, 128 accumulator registers each) the
 // second wavefront of a SIMD covers the first one's barrier, vmcnt and LDS waits, and each wavefront
 // issues half of a stage's loads: measured 5-8 % faster than four on the 256 x 256 tile.
@@ -156,9 +159,10 @@ struct PipeKernel {
     // all claim at once while a few spare workgroups read the host flag (tile_loop.hpp): the flag
     // read takes 1-2 us, so without the second look a kernel launched just after the flag went up
     // would still run to its end.
-    template <bool LOOKS = false>
+    // SINGLE: the workgroup's only tile, so that nothing of an earlier one has to be waited for before LDS is written.
+    template <bool LOOKS = false, bool SINGLE = false, class Asked = NoneAsked>
     static __device__ __forceinline__ bool run(const MatArgs &g, TileIdx t, T *lds_t, CkptCtx cc = CkptCtx{nullptr, nullptr, nullptr, 0},
-                                               int tile_index = 0, int kt0 = 0) {
+                                               Asked &&asked = Asked{}, int tile_index = 0, int kt0 = 0) {
         GP_PROBE(0);
         __shared__ int early_slot[LOOKS ? 192 : 64];  // landing places of the stop word (lane 0's dword of each 64): the early look's, then two that the later looks take in turn
         // (made wave-uniform by force: handed over in a vector register, the word would make the compiler treat every branch
@@ -521,7 +525,7 @@ struct PipeKernel {
 
         // ---- main loop ------------------------------------------------------------------------
         GP_PROBE(1);
-        __syncthreads();  // the previous tile of this workgroup may still be reading LDS
+        if (!SINGLE) __syncthreads();  // the previous tile of this workgroup may still be reading LDS
 #pragma unroll
         for (int s = 0; s < STAGES - 1; ++s) {
             if (kt0 + s < KT) issue(kt0 + s);
@@ -530,6 +534,7 @@ struct PipeKernel {
             if (!CKPT && s == 0 && early && wave == 0)
                 load_lds4(cc.stop_index, (unsigned)(size_t)(__attribute__((address_space(3))) void *)early_slot);
         }
+        asked();
         int kt = kt0, stopped = 0;
         // Later looks: after the first K-step the tile goes on in runs of LOOK_EVERY K-steps, as many as fit in front
         // of the last STAGES-1 K-steps.  Wavefront 0 fetches the word in front of a run, everybody reads it behind

@@ -169,8 +169,8 @@ struct WideKernel {
     static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
 
     // Returns true when the early look found a stop recorded: the tile was not run.
-    template <bool LOOKS = false>
-    static __device__ __forceinline__ bool run(const MatArgs &g, TileIdx t, T *lds_t, CkptCtx cc = CkptCtx{nullptr, nullptr, nullptr, 0}) {
+    template <bool LOOKS = false, bool SINGLE = false, class Asked = NoneAsked>  // (as in PipeKernel)
+    static __device__ __forceinline__ bool run(const MatArgs &g, TileIdx t, T *lds_t, CkptCtx cc = CkptCtx{nullptr, nullptr, nullptr, 0}, Asked &&asked = Asked{}) {
         GP_PROBE(0);
         __shared__ int early_slot[64];
         const bool early = __builtin_amdgcn_readfirstlane((int)(cc.stop_index != nullptr)) != 0;
@@ -251,14 +251,14 @@ struct WideKernel {
             }
         };
         if (CONV) advance(kb * BK);
-        auto issue = [&](int s) {
+        auto issue_part = [&](int s, auto first, auto last) {  // the loads first..last-1 of the wavefront's LPW for stage s
             const int k0 = (s * KB + kb) * BK;          // first K element of this wavefront group's block
             const unsigned sbase = lds0 + ((unsigned)s % STAGES) * STAGE_BYTES + (unsigned)kb * BLK_BYTES;
             const unsigned tap_bit = (k0 < g.K && nx_tap < 32) ? 1u << nx_tap : 0u;  // blocks past K have no tap
             const unsigned tap_off = (unsigned)((nx_r * g.W + nx_s) * (int)g.lda + nx_ci) * (unsigned)sizeof(T);
             const bool whole = k0 + BK <= g.K;          // (uniform) the block's K elements all exist
 #pragma unroll
-            for (int j = 0; j < LPW; ++j) {
+            for (int j = first; j < last; ++j) {
                 const int gi = group_of(wv, j);
                 if (CONV && j < LPW_A) {
                     // taps outside the image, rows outside the problem and blocks past K have nothing to fetch
@@ -270,8 +270,11 @@ struct WideKernel {
                     load_lds16_buffer(j < LPW_A ? rsrc_a : rsrc_b, at, (unsigned)k0 * (unsigned)sizeof(T), sbase + (unsigned)(gi * 8 * RB));
                 }
             }
-            if (CONV) advance(KB * BK);
+            if (CONV && last == LPW_A) advance(KB * BK);
         };
+        auto issue_a = [&](int s) { issue_part(s, IntC<0>{}, IntC<LPW_A>{}); };
+        auto issue_b = [&](int s) { issue_part(s, IntC<LPW_A>{}, IntC<LPW>{}); };
+        auto issue = [&](int s) { issue_b(s); issue_a(s); };
 
         f32x16 acc[BPW];
 #pragma unroll
@@ -285,7 +288,10 @@ struct WideKernel {
 
         // ---- main loop ------------------------------------------------------------------------
         GP_PROBE(1);
-        __syncthreads();  // the previous tile of this workgroup may still be reading LDS
+        // (the weights of the first stage need no row table)
+        constexpr bool B_FIRST = SINGLE && CONV;
+        if (B_FIRST) issue_b(0);
+        if (CONV || !SINGLE) __syncthreads();  // the row table; the previous tile of this workgroup may still be reading LDS
         if (CONV) {
 #pragma unroll
             for (int j = 0; j < LPW_A; ++j) {
@@ -296,9 +302,11 @@ struct WideKernel {
         }
 #pragma unroll
         for (int s = 0; s < PRE; ++s) {
-            if (s < NS) issue(s);
+            if (B_FIRST && s == 0) issue_a(s);
+            else if (s < NS) issue(s);
             if (s == 0 && early && wave == 0) load_lds4(cc.stop_index, (unsigned)(size_t)(__attribute__((address_space(3))) void *)early_slot);
         }
+        asked();
         for (int s = 0; s < NS; ++s) {
             // stage s has landed once at most the loads of the younger stages in flight remain
             if (s == 0) wait_stages<LPW>((NS < PRE ? NS : PRE) - 1);

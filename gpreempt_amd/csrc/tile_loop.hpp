@@ -425,7 +425,9 @@ __device__ __forceinline__ void unclaim_fixed(const BlpArgs &b) {
 // workgroup's number, its bit cannot be set yet, and the body's look at the stop word, which travels
 // with the first operands, stands in for the look in front of the claim.  The bit and the count go
 // out without waiting for their old values and are withdrawn like any claim if the body finds the
-// stop recorded.  A launch saves the wait for the stop index that way (0.2 us of a 10 us
+// stop recorded.  They go out behind the body's first loads (late_claim), from the last wavefront: the claim's code is 0.4 us that
+// stood in front of the first load of every launch, and in the bodies whose first four wavefronts multiply, the last one only
+// fetches.  One thread makes the claim and withdraws it, so that the two cannot pass each other.  A launch saves the wait for the stop index that way (0.2 us of a 10 us
 // convolution); a kernel queued behind a stop leaves a first operand fetch later than it would
 // have, which adds 4 us to the drain of a chunk of launches.  That trade is the caller's.
 // Everything the body is handed is computed from kernel arguments and the workgroup's number alone:
@@ -436,7 +438,12 @@ __device__ __forceinline__ void unclaim_fixed(const BlpArgs &b) {
 // tile that it finishes, a microsecond or two before it leaves (so that the front workgroup is gone by the time the
 // workers are: the launch lasts until the last workgroup has left, and the front one needs a microsecond or two to notice
 // and to get its read of the flag back).
-template <bool ANNOUNCES = false, class Body>
+// THREADS: of the workgroup; the body calls late_claim<THREADS>(b) once it has asked for its first operands.  0: it does not, the
+// claim is made in front of it by the first thread.
+template <int THREADS> __device__ __forceinline__ void late_claim(const BlpArgs &b) {
+    if (b.fresh > 1 && threadIdx.x == THREADS - 64) claim_fixed<false>(b, wg_group(wg_id(b), b.groups));
+}
+template <int THREADS = 0, bool ANNOUNCES = false, class Body>
 __device__ __forceinline__ void tile_fixed_early(const BlpArgs &b, Body &&body) {
     const bool eager = b.fresh > 1;
     int idx;
@@ -445,7 +452,7 @@ __device__ __forceinline__ void tile_fixed_early(const BlpArgs &b, Body &&body) 
         if (front_workgroup(b, leader)) return;
         if (spare_workgroup(b, true, leader)) return;
         if (wg_id(b) >= b.total) { leave_stamped(b); return; }
-        if (leader) claim_fixed<false>(b, wg_group(wg_id(b), b.groups));
+        if (THREADS == 0 && leader) claim_fixed<false>(b, wg_group(wg_id(b), b.groups));
         idx = xcd_contiguous(wg_id(b), b.total);
     } else {
         idx = fixed_claim_of_workgroup(b);
@@ -453,7 +460,7 @@ __device__ __forceinline__ void tile_fixed_early(const BlpArgs &b, Body &&body) 
     if (idx < 0) { leave_stamped(b); return; }
     int *word = (eager || b.spare || b.front) ? b.stop_index : nullptr;
     const bool left = body(decode_tile(idx, b.sx, b.sy, b.order, b.inv_sx, b.inv_sy), word);
-    if (left && threadIdx.x == 0) unclaim_fixed(b);
+    if (left && (int)threadIdx.x == (THREADS && eager ? THREADS - 64 : 0)) unclaim_fixed(b);
     leave_stamped(b, !(ANNOUNCES && word != nullptr && !left));
 }
 

@@ -276,9 +276,43 @@ int plan_conv2d(const gp_conv_params *p, MatPlan *out) {
     return choose_body(&pl, p->tile_m, p->tile_n, p->variant);
 }
 
+// The bodies that take a scale, shift and ReLU on A: those that a pointwise layer of a batch of a few images gets.
+static bool takes_pre(const MatPlan &pl) { return !pl.conv && !pl.b_kn && (pl.body == MB_PIPE64 || is_wide_body(pl.body)); }
+
+// An element-wise layer and the pointwise convolution that reads its output, as one launch of the body (and with the sums, so
+// that no bit changes) that the convolution alone would get.
+int plan_eltwise_conv2d(const gp_eltwise_params *e, const gp_conv_params *c, MatPlan *out) {
+    EltPlan elt;
+    if (int rc = plan_eltwise(e, &elt)) return rc;
+    if (int rc = plan_conv2d(c, out)) return rc;
+    GP_REQUIRE(e->scale && e->shift && !e->b && (e->act == GP_ACT_NONE || e->act == GP_ACT_RELU), "eltwise + conv: a scale, a shift and possibly a ReLU");
+    GP_REQUIRE(e->dtype == c->dtype && c->in == e->out && c->in_pix_stride == e->out_stride && c->Cin == e->cols && (long)c->N * c->H * c->W == e->rows, "eltwise + conv: the convolution does not read the layer's output");
+    GP_REQUIRE(c->out != e->a && c->residual != e->out, "eltwise + conv: overlapping operands");
+    MatPlan &pl = *out;
+    MatArgs alone = pl.g;
+    alone.A = e->a; alone.lda = e->a_stride;
+    GP_REQUIRE(c->tile_m == 0 && c->variant == 0 && takes_pre(pl) && (pl.body == MB_PIPE64 || buffer_ok(alone, false, pl.dtype)) &&
+                   pl.lds_bytes + pre_table_bytes(alone.K, (unsigned)dtype_size(pl.dtype)) <= pre_max_lds(pl.lds_bytes),
+               "eltwise + conv: no matrix body that takes a scale and shift for this shape");
+    pl.g = alone;
+    pl.g.pre_scale = e->scale; pl.g.pre_shift = e->shift; pl.g.pre_relu = e->act == GP_ACT_RELU;
+    pl.pre = true;
+    return GP_SUCC;
+}
+
 }  // namespace gp
 
 using namespace gp;
+
+extern "C" int gp_eltwise_conv2d_supported(const gp_eltwise_params *e, const gp_conv_params *c) {
+    MatPlan pl;
+    return plan_eltwise_conv2d(e, c, &pl) == GP_SUCC ? 1 : 0;
+}
+extern "C" int gp_launch_eltwise_conv2d(const gp_eltwise_params *e, const gp_conv_params *c, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
+    MatPlan pl;
+    int rc = plan_eltwise_conv2d(e, c, &pl);
+    return rc ? rc : launch_mat_plan(pl, ctx, s, info);
+}
 
 extern "C" int gp_launch_gemm(const gp_gemm_params *p, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
     MatPlan pl;

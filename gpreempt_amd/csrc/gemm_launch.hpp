@@ -81,13 +81,15 @@ static int launch_mat(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s,
     BlpArgs blp;
     int grid = 0;
     auto kern = KernelOf<K>::fn;  // the launch is planned for the general form; the others need no more resources
-    if (K::LDS_BYTES > 48 * 1024) {
+    const size_t lds_bytes = K::LDS_BYTES + (K::pre ? pre_table_bytes(pl.g.K, (unsigned)sizeof(typename K::elem)) : 0);
+    constexpr size_t max_lds = K::pre ? pre_max_lds(K::LDS_BYTES) : K::LDS_BYTES;
+    if (max_lds > 48 * 1024) {
         // several tenant threads launch concurrently: the attribute is set by exactly one of them
         static std::once_flag once;
         static hipError_t once_rc = hipSuccess;
         std::call_once(once, [] {
             for (const void *f : {(const void *)KernelOf<K>::fn, (const void *)KernelOf<K>::plain, (const void *)KernelOf<K>::fixed, (const void *)KernelOf<K>::looks}) {
-                hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)K::LDS_BYTES);
+                hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_lds);
                 if (e != hipSuccess) once_rc = e;
             }
         });
@@ -104,12 +106,12 @@ static int launch_mat(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s,
     // few scalar ones).  GPREEMPT_LONG_TILE_MACS overrides it.
     static const double long_macs = [] { const char *e = getenv("GPREEMPT_LONG_TILE_MACS"); return e && atof(e) > 0 ? atof(e) : 1.8e7; }();
     const bool long_tiles = K::can_look && (double)K::bm * K::bn * pl.g.K * (pl.dtype == GP_F32 ? 8.0 : 1.0) >= long_macs;
-    int rc = plan_launch(kern, K::NT, K::LDS_BYTES, pl.sx, pl.sy, pl.batch, ctx, &blp, &grid, info, 1, pl.rounds ? pl.rounds : K::LDS_BYTES <= 32 * 1024 ? 2 : K::LDS_BYTES <= 64 * 1024 ? 4 : 1, long_tiles);
+    int rc = plan_launch(kern, K::NT, lds_bytes, pl.sx, pl.sy, pl.batch, ctx, &blp, &grid, info, 1, pl.rounds ? pl.rounds : K::LDS_BYTES <= 32 * 1024 ? 2 : K::LDS_BYTES <= 64 * 1024 ? 4 : 1, long_tiles);
     if (rc) return rc;
     if (pl.or_smaller && ctx && !blp.done) return kTileTooLong;
     if (pl.or_deeper && ctx && blp.done) {
         int per_cu = 0;
-        rc = occupancy_of((const void *)kern, K::NT, K::LDS_BYTES, &per_cu);
+        rc = occupancy_of((const void *)kern, K::NT, lds_bytes, &per_cu);
         if (rc) return rc;
         if (front_costs_a_round(blp.total, (long)per_cu * device_cus())) return kFrontCostsARound;
     }
@@ -123,7 +125,7 @@ static int launch_mat(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s,
     // one tile per claim here (plan_launch's default), which is what the two special forms assume
     if (!ctx) kern = KernelOf<K>::plain;
     else if (fixed_claims(true, blp.groups, grid - blp.front, blp.total)) kern = blp.done ? KernelOf<K>::looks : KernelOf<K>::fixed;  // (not for checkpointing bodies: theirs is fn)
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(K::NT), K::LDS_BYTES, native(s), pl.g, blp);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(K::NT), lds_bytes, native(s), pl.g, blp);
     GP_HIP(hipGetLastError());
     return GP_SUCC;
 }
@@ -151,6 +153,8 @@ static int launch_mat(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s,
 template <typename T, bool CK> using BigPipe = PipeKernel<T, GP_BIG_BM, GP_BIG_BN, GP_BIG_STAGES, false, false, CK, GP_W256>;
 template <typename T, int TILE, int STAGES, bool SPLITK>
 static int pipe_case(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
+    if constexpr (TILE == 64 && !SPLITK)
+        if (pl.pre) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, false, false, false, 4, true>>(pl, ctx, s, info);
     if (pl.conv) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, true, SPLITK>>(pl, ctx, s, info);
     return launch_mat<PipeKernel<T, TILE, TILE, STAGES, false, SPLITK>>(pl, ctx, s, info);
 }
@@ -174,6 +178,7 @@ using WideK = WideKernel<T, BM, BN, WAVES, wide_stages(BM, BN, WAVES, CONV), CON
 
 template <typename T, int BM, int BN, int WAVES>
 static int wide_case(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
+    if (pl.pre) return launch_mat<WideKernel<T, BM, BN, WAVES, wide_stages(BM, BN, WAVES, false), false, true>>(pl, ctx, s, info);
     if (pl.conv) return launch_mat<WideK<T, BM, BN, WAVES, true>>(pl, ctx, s, info);
     return launch_mat<WideK<T, BM, BN, WAVES, false>>(pl, ctx, s, info);
 }

@@ -17,6 +17,7 @@
 //                 This quarters the length of the serial K loop for small, deep problems
 //                 without making the result depend on scheduling.
 #pragma once
+#include "gemm_pre.hpp"
 #include "mma.hpp"
 #include "../../include/util/conv_addr.h"
 
@@ -40,15 +41,30 @@ __device__ __forceinline__ void load_lds16(const void *gptr, unsigned lds_byte) 
 // The same through a buffer descriptor: lane i reads 16 bytes at the descriptor's base + off + soff.  A lane whose `off`
 // is kBufferEnd reads zeros (the descriptor's range ends there, and soff is not negative).
 constexpr unsigned kBufferEnd = 0x80000000u;
-__device__ __forceinline__ u32x4 buffer_of(const void *base) {  // (a raw buffer of 2 GB: what the planners allow an operand to span)
+__device__ __forceinline__ u32x4 buffer_of(const void *base, unsigned bytes = kBufferEnd) {  // (a raw buffer of 2 GB: what the planners allow an operand to span)
     const unsigned long long a = (unsigned long long)base;
-    return u32x4{(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)a), (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(a >> 32)), kBufferEnd, 0x00027000u};
+    return u32x4{(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)a), (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(a >> 32)), bytes, 0x00027000u};
 }
 __device__ __forceinline__ void load_lds16_buffer(u32x4 rsrc, unsigned off, unsigned soff, unsigned lds_byte) {
     asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
                  :
                  : "v"(off), "s"(rsrc), "s"(soff), "s"(lds_byte)
                  : "memory", "m0");
+}
+
+// PRE (gemm_pre.hpp): asks for the scales and shifts of all K channels, a kilobyte per instruction, to lie at LDS offset `table`
+// (zeros behind the last channel), and transforms 16 bytes of channels k .. at `at`.
+template <typename T, int WAVES> __device__ __forceinline__ void pre_fetch_table(const MatArgs &g, unsigned table, int wave, int lane) {
+    const unsigned bytes = (unsigned)g.K * (unsigned)sizeof(T), half = pre_table_bytes(g.K, sizeof(T)) / 2;
+    const u32x4 rs = buffer_of(g.pre_scale, bytes), rt = buffer_of(g.pre_shift, bytes);
+    for (unsigned at = (unsigned)wave * 1024u; at < half; at += WAVES * 1024u) {
+        load_lds16_buffer(rs, (unsigned)lane * 16u, at, table + at);
+        load_lds16_buffer(rt, (unsigned)lane * 16u, at, table + half + at);
+    }
+}
+template <typename T> __device__ __forceinline__ void pre_apply(const MatArgs &g, char *at, const char *table, int k) {
+    const char *s = table + (unsigned)k * (unsigned)sizeof(T), *t = s + pre_table_bytes(g.K, sizeof(T)) / 2;
+    *(out_u32x4 *)at = pre_chunk<T>(*(const out_u32x4 *)at, *(const out_u32x4 *)s, *(const out_u32x4 *)t, g.pre_relu != 0);
 }
 
 // Reads a word that a load-to-LDS has written.  The pointer must carry the LDS address space: through a plain
@@ -118,11 +134,13 @@ struct NoneAsked { __device__ __forceinline__ void operator()() const {} };
 // NWAVES: wavefronts per workgroup.  With eight (two per SIMD, 128 accumulator registers each) the
 // second wavefront of a SIMD covers the first one's barrier, vmcnt and LDS waits, and each wavefront
 // issues half of a stage's loads: measured 5-8 % faster than four on the 256 x 256 tile.
-template <typename T, int BM, int BN, int STAGES, bool CONV, bool SPLITK, bool CKPT = false, int NWAVES = 4>
+// PRE: the rows of A go through a scale, shift and ReLU first (gemm_pre.hpp).
+template <typename T, int BM, int BN, int STAGES, bool CONV, bool SPLITK, bool CKPT = false, int NWAVES = 4, bool PRE = false>
 struct PipeKernel {
     using elem = T;
     static constexpr int bm = BM, bn = BN;
-    static constexpr bool conv = CONV;
+    static constexpr bool conv = CONV, pre = PRE;
+    static_assert(!PRE || (!CONV && !CKPT), "GEMM rows only");
     static constexpr int VEC = Elem<T>::VEC;
     static constexpr int WAVES = NWAVES, NT = WAVES * 64;
     static constexpr int RB = 128;                        // row bytes in LDS
@@ -453,6 +471,12 @@ struct PipeKernel {
             if (!tail) wait_vmcnt<(STAGES - 2) * NLOADS>();
             else wait_vmcnt<0>();
             int stop_word = -1, flag_word = 0;
+            if constexpr (PRE) {
+                if (kt == kt0) __syncthreads();  // everyone's part of the table
+                char *mine = (char *)lds_t + (size_t)((unsigned)kt % STAGES) * STAGE_BYTES + (size_t)wave * A_PW * 8 * RB + lane * 16;
+#pragma unroll
+                for (int j = 0; j < A_PW; ++j) pre_apply<T>(g, mine + j * 8 * RB, lds_c + LDS_BYTES, kt * BK + chunk_of(wave * A_PW + j) * VEC);
+            }
             __syncthreads();  // everyone's part of stage kt is visible; stage kt-1's buffer is free
             if (kt == 0) GP_PROBE(2);
             if constexpr (LOOKS && !ISSUE)
@@ -526,6 +550,7 @@ struct PipeKernel {
         // ---- main loop ------------------------------------------------------------------------
         GP_PROBE(1);
         if (!SINGLE) __syncthreads();  // the previous tile of this workgroup may still be reading LDS
+        if constexpr (PRE) pre_fetch_table<T, WAVES>(g, lds0 + (unsigned)LDS_BYTES, wave, lane);  // (older than the first stage: the wait for that covers it)
 #pragma unroll
         for (int s = 0; s < STAGES - 1; ++s) {
             if (kt0 + s < KT) issue(kt0 + s);

@@ -128,11 +128,12 @@ __device__ __forceinline__ void wide_reduce_store(const MatArgs &g, float *red, 
     }
 }
 
-template <typename T, int BM, int BN, int WAVES, int STAGES, bool CONV = false>
+template <typename T, int BM, int BN, int WAVES, int STAGES, bool CONV = false, bool SCALED = false>  // (SCALED: PRE of PipeKernel)
 struct WideKernel {
     using elem = T;
     static constexpr int bm = BM, bn = BN;
-    static constexpr bool conv = CONV;
+    static constexpr bool conv = CONV, pre = SCALED;
+    static_assert(!SCALED || !CONV, "GEMM rows only");
     static constexpr int VEC = Elem<T>::VEC;
     static constexpr int NT = WAVES * 64;
     static constexpr int RB = 128;                         // row bytes of a block in LDS
@@ -292,6 +293,7 @@ struct WideKernel {
         constexpr bool B_FIRST = SINGLE && CONV;
         if (B_FIRST) issue_b(0);
         if (CONV || !SINGLE) __syncthreads();  // the row table; the previous tile of this workgroup may still be reading LDS
+        if constexpr (SCALED) pre_fetch_table<T, WAVES>(g, lds0 + (unsigned)LDS_BYTES, wave, lane);
         if (CONV) {
 #pragma unroll
             for (int j = 0; j < LPW_A; ++j) {
@@ -312,6 +314,15 @@ struct WideKernel {
             if (s == 0) wait_stages<LPW>((NS < PRE ? NS : PRE) - 1);
             else if (s + STAGES - 2 < NS) wait_vmcnt<(STAGES - 2) * LPW>();
             else wait_vmcnt<0>();
+            if constexpr (SCALED) {
+                if (s == 0) __syncthreads();  // everyone's part of the table
+                const int k0 = (s * KB + kb) * BK;
+                char *blk = (char *)lds_t + (size_t)((unsigned)s % STAGES) * STAGE_BYTES + (size_t)kb * BLK_BYTES + lane * 16;
+                if (k0 < g.K) {
+#pragma unroll
+                    for (int j = 0; j < LPW_A; ++j) pre_apply<T>(g, blk + group_of(wv, j) * 8 * RB, lds_c + LDS_BYTES, k0 + kc[j]);
+                }
+            }
             __syncthreads();  // everyone's part of stage s is visible; the buffer of stage s-1 is free
             if (s == 0) GP_PROBE(2);
             if (((s == 0 && early) || (looking && s > 0 && (s & (LOOK_EVERY - 1)) == 0)) && __builtin_amdgcn_readfirstlane(read_lds_word(early_slot)) != -1) {

@@ -74,6 +74,9 @@ struct MatArgs {
     const void *ln_gamma, *ln_beta;
     void *ln_out;
     float ln_eps;
+    // scale, shift and ReLU of the channels of A (gemm_pre.hpp; the bodies with PRE)
+    const void *pre_scale, *pre_shift;
+    int pre_relu;
 };
 
 }  // namespace gp

@@ -24,6 +24,7 @@ struct MatPlan {
     int ring;          // stages of the operand ring of the 64 x 64 and 128 x 128 bodies: 2, or 0 for the body's own depth
     bool or_smaller;   // a preemptible launch that could not give its tiles up is refused with kTileTooLong: the caller has a plan with smaller ones
     bool or_deeper;    // ... and one whose front workgroup would cost a round of its own with kFrontCostsARound: there is a body with another rhythm
+    bool pre;          // the rows of A go through g.pre_* first
     int rounds;        // rounds of workgroups a preemptible launch may take with a workgroup per claim; 0: the launcher's own number
 };
 
@@ -48,6 +49,7 @@ struct EltPlan {
 constexpr int kTileTooLong = -1, kFrontCostsARound = -2;  // launch_mat_plan: see MatPlan; nothing has been launched
 int plan_gemm(const gp_gemm_params *p, MatPlan *out);
 int plan_conv2d(const gp_conv_params *p, MatPlan *out);
+int plan_eltwise_conv2d(const gp_eltwise_params *e, const gp_conv_params *c, MatPlan *out);
 int launch_mat_plan(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info);
 
 int plan_layout(const gp_layout_params *p, EltPlan *out);

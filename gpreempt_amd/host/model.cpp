@@ -259,6 +259,29 @@ void Model::plan_fusions() {
         mm.has_ln_gemm = true;
         ln.fused_away = true;
     }
+    // scale-shift -> pointwise convolution, where nobody else reads (or writes) what lies between the two
+    unread_.assign(storage_infos.size(), SIZE_MAX);
+    for (size_t i = 0; i + 1 < kernel_infos.size(); ++i) {
+        KernelInfo &el = kernel_infos[i], &cv = kernel_infos[i + 1];
+        cv.has_pre = false;
+        if (el.op != OpKind::Eltwise || cv.op != OpKind::Conv) continue;
+        const size_t between = el.args_index[4], from = el.args_index[0];
+        bool alone = between != from && between != cv.args_index[4] && from != cv.args_index[4] && storage_infos[between].name != "heads";
+        for (size_t k = 0; k < kernel_infos.size() && alone; ++k)
+            for (size_t st : kernel_infos[k].args_index) alone = alone && (st != between || k == i || k == i + 1);
+        if (!alone || gp_eltwise_conv2d_supported(&el.p.eltwise, &cv.p.conv) != 1) continue;
+        cv.pre = el.p.eltwise;
+        cv.has_pre = true;
+        el.fused_away = true;
+        unread_[between] = i;
+    }
+}
+
+// The output of a layer that its reader's launch does itself (plan_fusions): computed for a caller that wants to see it.
+Status Model::compute_unread(size_t idx, GPUstream stream) {
+    if (!fuse_launches_ || idx >= unread_.size() || unread_[idx] == SIZE_MAX) return Status::Succ;
+    CUDA_RETURN_STATUS(gp_launch_eltwise(&kernel_infos[unread_[idx]].p.eltwise, nullptr, stream, nullptr));
+    return Status::Succ;
 }
 
 // A list that is the miniWeather step (x, z, z, x; three stages of halo, fluxes, update) also gets its sweeps.  The state
@@ -380,6 +403,7 @@ Status Model::get(size_t idx, void *out, size_t len, GPUstream stream) {
     if (idx >= storages.size()) return Status::OutOfRange;
     size_t size = storage_infos[idx].size;
     if (len < size) return Status::Fail;
+    RETURN_STATUS(compute_unread(idx, stream));
     CUDA_RETURN_STATUS(gp_memcpy_d2h_async(out, storages[idx], size, stream));
     return Status::Succ;
 }
@@ -410,6 +434,7 @@ Status Model::set_pinned(size_t idx, const void *value, size_t len, GPUstream st
 Status Model::fetch(size_t idx, void *pinned, size_t len, GPUstream stream) {
     if (idx >= storages.size()) return Status::OutOfRange;
     if (len < storage_infos[idx].size) return Status::Fail;
+    RETURN_STATUS(compute_unread(idx, stream));
     CUDA_RETURN_STATUS(gp_fetch(pinned, storages[idx], storage_infos[idx].size, stream));
     return Status::Succ;
 }
@@ -503,7 +528,7 @@ Status Model::launch(size_t idx, GPUstream stream, int inject_at) {
     int rc = GP_FAIL;
     switch (k.op) {
         case OpKind::Gemm: rc = gp_launch_gemm(fuse && k.has_ln_gemm ? &k.ln_gemm : &k.p.gemm, pc, stream, &info); break;
-        case OpKind::Conv: rc = gp_launch_conv2d(&k.p.conv, pc, stream, &info); break;
+        case OpKind::Conv: rc = fuse && k.has_pre ? gp_launch_eltwise_conv2d(&k.pre, &k.p.conv, pc, stream, &info) : gp_launch_conv2d(&k.p.conv, pc, stream, &info); break;
         case OpKind::Layout: rc = gp_launch_nchw_to_nhwc(&k.p.layout, pc, stream, &info); break;
         case OpKind::Pool: rc = gp_launch_pool2d(&k.p.pool, pc, stream, &info); break;
         case OpKind::Eltwise: rc = gp_launch_eltwise(&k.p.eltwise, pc, stream, &info); break;

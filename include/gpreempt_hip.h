@@ -333,6 +333,14 @@ typedef struct gp_eltwise_params {
     int act;
 } gp_eltwise_params;
 int gp_launch_eltwise(const gp_eltwise_params *p, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info);
+/* No counterpart in the reference's runtime (TVM fuses an element-wise operator into the convolution BEHIND it never):
+ * out = act(conv(relu?(a * scale + shift))) in one launch, where `e` is a per-channel scale and shift with an optional
+ * ReLU (no addend) and `c` a pointwise convolution (1 x 1, stride 1) of its output.  e->out is not written.  The result has
+ * the bits of gp_launch_eltwise followed by gp_launch_conv2d.  Only for what gp_eltwise_conv2d_supported accepts (1): the
+ * convolution reads exactly the layer's output, and a matrix body that takes a scale and shift serves its shape;
+ * c->out must not overlap e->a. */
+int gp_eltwise_conv2d_supported(const gp_eltwise_params *e, const gp_conv_params *c);
+int gp_launch_eltwise_conv2d(const gp_eltwise_params *e, const gp_conv_params *c, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info);
 
 /* Row softmax over the last axis: out = softmax(scale * x). */
 typedef struct gp_softmax_params {

@@ -84,6 +84,11 @@ public:
     bool fused_away = false;
     bool has_ln_gemm = false;
     gp_gemm_params ln_gemm;
+    // ... and likewise a scale-shift(-ReLU) layer whose output only the pointwise convolution behind it reads: that one's launch
+    // (gp_launch_eltwise_conv2d) does both, and the layer's output is not written; Model::get and fetch compute it for
+    // whoever asks for it.
+    bool has_pre = false;
+    gp_eltwise_params pre;
 };
 
 class Model {
@@ -231,6 +236,8 @@ private:
 
     Status allocate_and_bind();
     void plan_fusions();
+    Status compute_unread(size_t idx, GPUstream stream);
+    std::vector<size_t> unread_;  // per storage: the kernel that would write it, where plan_fusions found a launch that needs no such storage
     bool fuse_launches_ = true;  // GPREEMPT_FUSE_LN=0 in the environment keeps every launch of the kernel list
     bool eager_tiles_ = true;    // first launches start their tiles before the stop index has come back (gp_preempt_ctx::fresh = 2); GPREEMPT_EAGER_TILES=0 makes them wait for it
     Status upload_param(size_t idx, const float *disk, size_t n);

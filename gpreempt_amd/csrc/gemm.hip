@@ -43,6 +43,8 @@ static size_t body_lds_bytes(int body, int dtype) {
         case MB_WIDE32x32_8: return WideK<_Float16, 32, 32, 8>::LDS_BYTES;
         case MB_WIDE64x32_16: return WideK<_Float16, 64, 32, 16>::LDS_BYTES;
         case MB_WIDE64x64_8: return WideK<_Float16, 64, 64, 8>::LDS_BYTES;
+        case MB_NARROW16x16: return NarrowKernel<16, 3>::LDS_BYTES;
+        case MB_NARROW32x16: return NarrowKernel<32, 3>::LDS_BYTES;
         case MB_LNWIDE32x64_16: return LnWideKernel<_Float16, 32, 64, 16, 3>::LDS_BYTES;
         case MB_STAGED128: return (128 + 128) * ((es == 4 ? 16 : 32) + (es == 4 ? 4 : 8)) * es;
         case MB_STAGED64: return (64 + 64) * ((es == 4 ? 16 : 32) + (es == 4 ? 4 : 8)) * es;
@@ -56,7 +58,9 @@ static size_t body_lds_bytes(int body, int dtype) {
 // serial K loop shrinks instead.
 // the wide split-K bodies (gemm_wide.hpp) and their tiles
 struct WideChoice { int body, bm, bn, waves; size_t lds; };
-static const WideChoice kWide[4] = {
+static const WideChoice kWide[6] = {
+    {MB_NARROW16x16, 16, 16, 16, NarrowKernel<16, 3>::LDS_BYTES},
+    {MB_NARROW32x16, 32, 16, 16, NarrowKernel<32, 3>::LDS_BYTES},
     {MB_WIDE32x32_16, 32, 32, 16, WideK<_Float16, 32, 32, 16>::LDS_BYTES},
     {MB_WIDE32x32_8, 32, 32, 8, WideK<_Float16, 32, 32, 8>::LDS_BYTES},
     {MB_WIDE64x32_16, 64, 32, 16, WideK<_Float16, 64, 32, 16>::LDS_BYTES},
@@ -76,6 +80,10 @@ static int wide_pick(const MatArgs &g, int batch, long cus, int dtype) {
     // tiles as there are compute units to take them (ResNet-50 b1 fp32, launch to launch: 7 x 7 x 512 -> 2048
     // 13.1 -> 6.7 us, 3 x 3 at 56 x 56 x 64 16.2 -> 9.1 us; these tiles are also what a preempted tenant
     // finishes before it leaves)
+    // (deep ones in tiles of a quarter and a half while those still run side by side, gemm_narrow.hpp: ResNet-50 b1 735 -> 584 us a pass,
+    // DenseNet-201 b1 2458 -> 1907, Inception-v3 b2 1303 -> 1130, BERT b1 s64 871 -> 758; K from 128 or 256 on: level)
+    if (dtype == GP_F32 && g.K >= 512 && tiles(16, 16) <= cus) return MB_NARROW16x16;
+    if (dtype == GP_F32 && g.K >= 512 && tiles(32, 16) <= cus) return MB_NARROW32x16;
     if (dtype == GP_F32 && tiles(32, 32) <= cus) return g.K >= 768 ? MB_WIDE32x32_16 : MB_WIDE32x32_8;
     if (g.K >= 768 && tiles(32, 32) <= cus) return MB_WIDE32x32_16;
     if (g.K >= 768 && tiles(64, 32) <= cus) return MB_WIDE64x32_16;

@@ -7,6 +7,7 @@
 #include "gemm_pipe.hpp"
 #include "gemm_wide.hpp"
 #include "gemm_ln.hpp"
+#include "gemm_narrow.hpp"
 #include "plans.hpp"
 
 namespace gp {
@@ -183,6 +184,13 @@ static int wide_case(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, 
     return launch_mat<WideK<T, BM, BN, WAVES, false>>(pl, ctx, s, info);
 }
 
+template <int BM>
+static int narrow_case(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
+    if (pl.pre) return launch_mat<NarrowKernel<BM, 3, false, true>>(pl, ctx, s, info);
+    if (pl.conv) return launch_mat<NarrowKernel<BM, 3, true>>(pl, ctx, s, info);
+    return launch_mat<NarrowKernel<BM, 3, false>>(pl, ctx, s, info);
+}
+
 template <typename T>
 int launch_typed(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
     constexpr int SBK = sizeof(T) == 4 ? 16 : 32;
@@ -220,6 +228,12 @@ int launch_typed(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, gp_l
         case MB_WIDE32x32_8: return wide_case<T, 32, 32, 8>(pl, ctx, s, info);
         case MB_WIDE64x32_16: return wide_case<T, 64, 32, 16>(pl, ctx, s, info);
         case MB_WIDE64x64_8: return wide_case<T, 64, 64, 8>(pl, ctx, s, info);
+        case MB_NARROW16x16:
+            if constexpr (sizeof(T) == 4) return narrow_case<16>(pl, ctx, s, info);
+            break;
+        case MB_NARROW32x16:
+            if constexpr (sizeof(T) == 4) return narrow_case<32>(pl, ctx, s, info);
+            break;
         case MB_LNWIDE32x64_16:
             if constexpr (sizeof(T) == 2) return launch_mat<LnWideKernel<T, 32, 64, 16, 3>>(pl, ctx, s, info);
             break;

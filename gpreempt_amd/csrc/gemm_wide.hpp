@@ -50,38 +50,22 @@ template <int LPW> __device__ __forceinline__ void wait_stages(int stages) {
     else wait_vmcnt<0>();
 }
 
-// The end of a tile of the wide bodies: the partial tiles of wavefronts 0..3 are summed through LDS in
-// wavefront order and the epilogue (alpha, bias, residual, activation) is applied on the way out.
-template <typename T, int BM, int BN, int NT, int G>
-__device__ __forceinline__ void wide_reduce_store(const MatArgs &g, float *red, const f32x16 (&acc)[(BM / 32) * (BN / 32) / G], int m0, int n0, long offc,
-                                                  int tid, int wv, int lane, int kb) {
-    constexpr int MI = BM / 32, NI = BN / 32, SLICES = MI * NI * 16, BPW = MI * NI / G;
-    // ---- reduction and epilogue -------------------------------------------------------------
-    // partial tiles of wavefronts 0..3 -> LDS as [wavefront][slice][lane], slice = (i*NI + j)*16 + v,
-    // which is row 8*(v/4) + 4*(lane/32) + v%4, column 32*j + lane%32 of 32 x 32 block (i, j).
-    // The first BM*BN/4 threads then finish four consecutive columns of one row each, adding the
-    // partials in wavefront order.
+// The end of a tile of the wide bodies: the partial tiles of wavefronts 0..3, PART floats each in LDS, are summed in wavefront
+// order and the epilogue (alpha, bias, residual, activation) is applied on the way out.  The first BM * BN / 4 threads finish four
+// consecutive columns of one row each; at(row, column) is where a partial tile has those four.
+template <typename T, int BM, int BN, int NT, int PART, class At>
+__device__ __forceinline__ void wide_finish(const MatArgs &g, const float *red, int m0, int n0, long offc, int tid, At &&at) {
     T *C = (T *)g.C + offc;
     const T *R = g.residual ? (const T *)g.residual + offc : nullptr;
     const T *bias = (const T *)g.bias;
     const bool vec_ok = (g.N % 4 == 0) && (g.ldc % 4 == 0) && (offc % 4 == 0) && ((size_t)g.C % 16 == 0) &&
                         (!R || (g.ldr % 4 == 0 && (size_t)g.residual % 16 == 0)) && (!bias || (size_t)bias % 16 == 0);
-    __syncthreads();  // all wavefronts are done reading the stage buffers
-    if (kb < G) {  // wavefront (kb, wv) holds k-step wv of the 32 x 32 blocks kb, kb + G, ...
-#pragma unroll
-        for (int q = 0; q < BPW; ++q)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) red[((size_t)wv * SLICES + (kb + q * G) * 16 + v) * 64 + lane] = acc[q][v];
-    }
-    __syncthreads();
-    GP_PROBE(4);
     constexpr int L4 = BN / 4;                        // threads per output row
     constexpr int FIN = BM * L4 < NT ? BM * L4 : NT;  // threads that finish
     constexpr int RPP = FIN / L4, PASSES = BM / RPP;
     if (tid < FIN) {
-        const int c4 = tid % L4, r_in = tid / L4;
-        const int j = c4 >> 3, col = (c4 & 7) * 4;
-        const int n = n0 + j * 32 + col;
+        const int col = tid % L4 * 4, r_in = tid / L4;
+        const int n = n0 + col;
         float bq[4] = {0.f, 0.f, 0.f, 0.f};
         if (bias && n < g.N) {
             if (vec_ok) {
@@ -97,12 +81,10 @@ __device__ __forceinline__ void wide_reduce_store(const MatArgs &g, float *red, 
 #pragma unroll
         for (int p = 0; p < PASSES; ++p) {
             const int row = p * RPP + r_in, m = m0 + row;
-            const int i = row >> 5, r = row & 31;
-            const int v = 4 * (r >> 3) + (r & 3), hf = (r >> 2) & 1;
-            const size_t o = ((size_t)(i * NI + j) * 16 + v) * 64 + hf * 32 + col;
+            const size_t o = at(row, col);
             f32x4 a = *(const f32x4 *)(red + o);
 #pragma unroll
-            for (int w = 1; w < 4; ++w) a += *(const f32x4 *)(red + (size_t)w * SLICES * 64 + o);
+            for (int w = 1; w < 4; ++w) a += *(const f32x4 *)(red + (size_t)w * PART + o);
             if (m >= g.M || n >= g.N) continue;
             if (vec_ok) {
                 Vec4<T> rv;
@@ -126,6 +108,28 @@ __device__ __forceinline__ void wide_reduce_store(const MatArgs &g, float *red, 
             }
         }
     }
+}
+
+// ... of the bodies whose wavefronts hold 32 x 32 blocks: partial tiles of wavefronts 0..3 -> LDS as [wavefront][slice][lane], slice = (i*NI +
+// j)*16 + v, which is row 8*(v/4) + 4*(lane/32) + v%4, column 32*j + lane%32 of block (i, j).
+template <typename T, int BM, int BN, int NT, int G>
+__device__ __forceinline__ void wide_reduce_store(const MatArgs &g, float *red, const f32x16 (&acc)[(BM / 32) * (BN / 32) / G], int m0, int n0, long offc,
+                                                  int tid, int wv, int lane, int kb) {
+    constexpr int MI = BM / 32, NI = BN / 32, SLICES = MI * NI * 16, BPW = MI * NI / G;
+    __syncthreads();  // all wavefronts are done reading the stage buffers
+    if (kb < G) {  // wavefront (kb, wv) holds k-step wv of the 32 x 32 blocks kb, kb + G, ...
+#pragma unroll
+        for (int q = 0; q < BPW; ++q)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) red[((size_t)wv * SLICES + (kb + q * G) * 16 + v) * 64 + lane] = acc[q][v];
+    }
+    __syncthreads();
+    GP_PROBE(4);
+    wide_finish<T, BM, BN, NT, SLICES * 64>(g, red, m0, n0, offc, tid, [&](int row, int column) {
+        const int i = row >> 5, r = row & 31, j = column >> 5;
+        const int v = 4 * (r >> 3) + (r & 3), hf = (r >> 2) & 1;
+        return ((size_t)(i * NI + j) * 16 + v) * 64 + hf * 32 + (column & 31);
+    });
 }
 
 template <typename T, int BM, int BN, int WAVES, int STAGES, bool CONV = false, bool SCALED = false>  // (SCALED: PRE of PipeKernel)

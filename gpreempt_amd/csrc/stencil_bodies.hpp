@@ -70,10 +70,12 @@ struct MwCursor {
 };
 
 // fourth-order interface value and (scaled) third difference from four cell averages
+// (Here and in the fluxes a product and the sum it goes into are one fused operation, written out so that the kernels and the sweeps
+// round alike: a rounding less each, and 24 of a face's 129 vector instructions, which is what these kernels' time goes by.)
 __device__ __forceinline__ void mw_reconstruct(const float (&s)[4], float hv_coef, float &val, float &d3) {
 #pragma clang fp contract(off)
-    val = mw_div12(-s[0] + 7 * (s[1] + s[2]) - s[3]);
-    d3 = (-s[0] + 3 * (s[1] - s[2]) + s[3]) * hv_coef;
+    val = mw_div12(__builtin_fmaf(7.0f, s[1] + s[2], -s[0]) - s[3]);
+    d3 = (__builtin_fmaf(3.0f, s[1] - s[2], -s[0]) + s[3]) * hv_coef;
 }
 
 // Pointers into the hydrostatic background buffer: cell density, cell density*theta (nz+4 each),
@@ -304,10 +306,11 @@ __device__ __forceinline__ void mw_flux_x_point(const float (&s)[MW_VARS][4], fl
     const double w = vals[MW_WMOM] * r_inv;
     const double th = (vals[MW_RHOT] + h1) * r_inv;
     const double pr = MW_C0 * mw_pow_gamma(r * th);
-    f[MW_DENS] = (float)(r * u - d3[MW_DENS]);
-    f[MW_UMOM] = (float)(r * u * u + pr - d3[MW_UMOM]);
-    f[MW_WMOM] = (float)(r * u * w - d3[MW_WMOM]);
-    f[MW_RHOT] = (float)(r * u * th - d3[MW_RHOT]);
+    const double ru = r * u;
+    f[MW_DENS] = (float)(ru - d3[MW_DENS]);
+    f[MW_UMOM] = (float)(__builtin_fma(ru, u, pr) - d3[MW_UMOM]);
+    f[MW_WMOM] = (float)__builtin_fma(ru, w, -(double)d3[MW_WMOM]);
+    f[MW_RHOT] = (float)__builtin_fma(ru, th, -(double)d3[MW_RHOT]);
 }
 __device__ __forceinline__ void mw_finish(const gp_miniweather_params &p, const MwOperands<GP_MW_FLUX_X> &o) {
     const MwView v{p.nx, p.nz};
@@ -354,10 +357,11 @@ __device__ __forceinline__ void mw_flux_z_point(const float (&s)[MW_VARS][4], fl
         w = 0.f;
         d3[MW_DENS] = 0.f;
     }
-    f[MW_DENS] = r * w - d3[MW_DENS];
-    f[MW_UMOM] = r * w * u - d3[MW_UMOM];
-    f[MW_WMOM] = r * w * w + pr - d3[MW_WMOM];
-    f[MW_RHOT] = r * w * th - d3[MW_RHOT];
+    const float rw = r * w;
+    f[MW_DENS] = rw - d3[MW_DENS];
+    f[MW_UMOM] = __builtin_fmaf(rw, u, -d3[MW_UMOM]);
+    f[MW_WMOM] = __builtin_fmaf(rw, w, pr) - d3[MW_WMOM];
+    f[MW_RHOT] = __builtin_fmaf(rw, th, -d3[MW_RHOT]);
 }
 __device__ __forceinline__ void mw_finish(const gp_miniweather_params &p, const MwOperands<GP_MW_FLUX_Z> &o) {
     float f[MW_VARS];

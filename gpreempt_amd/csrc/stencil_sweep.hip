@@ -5,9 +5,11 @@
 // cells to either side.  So a wavefront takes a stretch of 64 * CELLS consecutive cells along the sweep, six of them at
 // either end belonging to its neighbours, and carries them through the three stages in registers: lane l holds cells
 // CELLS * l .. CELLS * l + CELLS - 1, the cells and fluxes of the next lanes come by DPP wave shifts, and the state is
-// read and written once.  What bounds it now is the arithmetic: 145 vector instructions per cell and stage, for an
-// eighth more cells than there are.  86 us per preemptible sweep, 101 (x) and 90 (z) for the two that also leave state_tmp
-// and the fluxes; two cells per lane, since four take 140-200 registers (x 100-130 us, z 154-175).
+// read and written once.  What bounds it now is the arithmetic: 125 vector instructions per cell and stage, for an
+// eighth more cells than there are.  82 us per preemptible sweep, 100 (x) and 88 (z) for the two that also leave state_tmp
+// and the fluxes (86, 109 and 93 before products and sums were fused and the viscosity's division went to the host); two cells per
+// lane, since four take 140-200 registers (x 100-130 us, z 154-175).  More wavefronts by fewer registers (five to a SIMD for
+// four): spills, 8260 -> 8570 us for twenty steps and their output; a workgroup per claim for the x sweeps' 11200 tiles: level.
 //
 // x: rows are contiguous, a wavefront loads and stores its stretch itself.  z: a workgroup brings 16 columns of a
 // stretch in through LDS (64-byte runs of every row; a column is contiguous there), and its wavefronts take a column
@@ -18,6 +20,11 @@
 namespace gp {
 
 constexpr int SW_HALO = 6;  // three stages of two cells
+
+// the sweep's parameters, and what a stage takes from its length and the cell's: divisions made once on the host
+struct SweepArgs : gp_mw_sweep_params {
+    float hv_coef[3];  // -MW_HV_BETA * d / (16 * dt[stage])
+};
 
 // the value of the lane below / above (lane 0 / 63: 0; those cells are the neighbours' anyway)
 __device__ __forceinline__ float from_below(float x) { return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x138, 0xf, 0xf, true)); }
@@ -58,7 +65,7 @@ typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
 constexpr int SX_CELLS = 2, SX_OUT = 64 * SX_CELLS - 2 * SW_HALO;
 
 template <bool LAST>
-__device__ __forceinline__ void sweep_x(const gp_mw_sweep_params &p, int item) {
+__device__ __forceinline__ void sweep_x(const SweepArgs &p, int item) {
 #pragma clang fp contract(off)
     const int nx = p.nx, nz = p.nz, pieces = (nx + SX_OUT - 1) / SX_OUT;
     const int lane = threadIdx.x & 63;
@@ -108,7 +115,7 @@ __device__ __forceinline__ void sweep_x(const gp_mw_sweep_params &p, int item) {
     const float dx_inv = 1.0f / p.dx, h0 = p.hydro[k + MW_HS], h1 = p.hydro[nz + 2 * MW_HS + k + MW_HS];
 #pragma unroll 1
     for (int stage = 0; stage < 3; ++stage) {
-        const float dt = p.dt[stage], hv_coef = -MW_HV_BETA * p.dx / (16 * dt);
+        const float dt = p.dt[stage], hv_coef = p.hv_coef[stage];
         sweep_fluxes<SX_CELLS>(cur, f, [&](int, const float (&s)[MW_VARS][4], float (&out)[MW_VARS]) { mw_flux_x_point(s, h0, h1, hv_coef, out); });
         if (LAST && stage == 2) {  // the faces below the cells, and the row's last one
             const unsigned fplane = (unsigned)(nz + 1) * (unsigned)(nx + 1), frow = (unsigned)k * (unsigned)(nx + 1);
@@ -161,7 +168,7 @@ constexpr int SZ_STRIDE = SZ_ROWS + 4;  // of a column in LDS: 16 columns of 4 r
 constexpr size_t SZ_LDS = sizeof(float) * MW_VARS * SZ_COLS * SZ_STRIDE;
 
 template <bool LAST>
-__device__ __forceinline__ void sweep_z(const gp_mw_sweep_params &p, int tile, float *lds) {
+__device__ __forceinline__ void sweep_z(const SweepArgs &p, int tile, float *lds) {
 #pragma clang fp contract(off)
     const int nx = p.nx, nz = p.nz, strips = (nx + SZ_COLS - 1) / SZ_COLS, pieces = (nz + SZ_OUT - 1) / SZ_OUT;
     const int piece = tile / strips, col0 = (tile - piece * strips) * SZ_COLS;
@@ -227,7 +234,7 @@ __device__ __forceinline__ void sweep_z(const gp_mw_sweep_params &p, int tile, f
         };
 #pragma unroll 1
         for (int stage = 0; stage < 3; ++stage) {
-            const float dt = p.dt[stage], hv_coef = -MW_HV_BETA * p.dz / (16 * dt);
+            const float dt = p.dt[stage], hv_coef = p.hv_coef[stage];
             if (bottom || top) walls(!LAST || stage == 1 ? nullptr : stage == 0 ? p.state : p.state_tmp);
             sweep_fluxes<SZ_CELLS>(cur, f, [&](int j, const float (&s)[MW_VARS][4], float (&out)[MW_VARS]) {
                 mw_flux_z_point(s, h0[j], h1[j], h2[j], hv_coef, first + j == 0 || first + j == nz, out);
@@ -283,7 +290,7 @@ __device__ __forceinline__ void sweep_z(const gp_mw_sweep_params &p, int tile, f
 }
 
 template <bool Z, bool LAST, int LOOP = LOOP_ANY>
-__global__ __launch_bounds__(MW_TILE) void miniweather_sweep_kernel(gp_mw_sweep_params p, BlpArgs blp) {
+__global__ __launch_bounds__(MW_TILE) void miniweather_sweep_kernel(SweepArgs p, BlpArgs blp) {
     extern __shared__ __attribute__((aligned(16))) float sweep_lds[];
     tiles<LOOP>(blp, [&](TileIdx t) {
         if constexpr (Z) sweep_z<LAST>(p, t.x, sweep_lds);
@@ -299,13 +306,16 @@ extern "C" int gp_launch_miniweather_sweep(const gp_mw_sweep_params *p, const gp
     GP_REQUIRE(p && p->in && p->out && p->in != p->out && p->state && p->state_tmp && p->flux && p->hydro, "miniweather sweep: operands missing");
     GP_REQUIRE(p->nx >= 4 && p->nz >= 4 && (long)p->nx * p->nz <= (1L << 27), "miniweather grid %d x %d", p->nx, p->nz);
     GP_REQUIRE(p->dt[0] > 0 && p->dt[1] > 0 && p->dt[2] > 0 && p->dx > 0 && p->dz > 0, "miniweather steps must be positive");
+    SweepArgs args;
+    static_cast<gp_mw_sweep_params &>(args) = *p;
+    for (int stage = 0; stage < 3; ++stage) args.hv_coef[stage] = -MW_HV_BETA * (p->dir_z ? p->dz : p->dx) / (16 * p->dt[stage]);
     if (p->dir_z) {
         const int tiles = (p->nx + SZ_COLS - 1) / SZ_COLS * ((p->nz + SZ_OUT - 1) / SZ_OUT);
-        return p->last ? launch_tiles(GP_KSET(miniweather_sweep_kernel<true, true), tiles, 1, ctx, s, info, *p, SZ_LDS, 1)
-                       : launch_tiles(GP_KSET(miniweather_sweep_kernel<true, false), tiles, 1, ctx, s, info, *p, SZ_LDS, 1);
+        return p->last ? launch_tiles(GP_KSET(miniweather_sweep_kernel<true, true), tiles, 1, ctx, s, info, args, SZ_LDS, 1)
+                       : launch_tiles(GP_KSET(miniweather_sweep_kernel<true, false), tiles, 1, ctx, s, info, args, SZ_LDS, 1);
     }
     const long waves = (long)p->nz * ((p->nx + SX_OUT - 1) / SX_OUT);
     const int tiles = (int)((waves + MW_TILE / 64 - 1) / (MW_TILE / 64));
-    return p->last ? launch_tiles(GP_KSET(miniweather_sweep_kernel<false, true), tiles, 1, ctx, s, info, *p, 0, 1)
-                   : launch_tiles(GP_KSET(miniweather_sweep_kernel<false, false), tiles, 1, ctx, s, info, *p, 0, 1);
+    return p->last ? launch_tiles(GP_KSET(miniweather_sweep_kernel<false, true), tiles, 1, ctx, s, info, args, 0, 1)
+                   : launch_tiles(GP_KSET(miniweather_sweep_kernel<false, false), tiles, 1, ctx, s, info, args, 0, 1);
 }

@@ -106,8 +106,10 @@ static int choose_body(MatPlan *pl, int tile, int tile_n, int variant) {
     // both operands K-contiguous; a convolution, whose A operand is gathered, when a K-block never straddles
     // two filter taps and a bit per tap fits a word
     const int wide_bk = pl->dtype == GP_F32 ? 32 : 64;
-    const bool wide_shape = !pl->b_kn && (!pl->conv || (g.Cin % wide_bk == 0 && g.K / g.Cin <= 32 && g.S < 32));
-    const bool wide_ok = wide_shape && buffer_ok(g, pl->conv, pl->dtype);
+    // (a caller that asks for a wide body gets one only where no block straddles two taps, as ever)
+    const bool wide_taps = !pl->conv || (g.K / g.Cin <= 32 && g.S < 32 && g.inv_cin && g.inv_s);
+    const bool wide_shape = !pl->b_kn && wide_taps && (!pl->conv || g.Cin % wide_bk == 0);
+    const bool wide_ok = !pl->b_kn && wide_taps && buffer_ok(g, pl->conv, pl->dtype);
     int body = -1;
     if (g.ln_gamma) body = MB_LNWIDE32x64_16;  // (plan_gemm has checked that the shape fits)
     else if (pl->b_kn || variant == GP_MAT_STAGED) {
@@ -279,7 +281,8 @@ int plan_conv2d(const gp_conv_params *p, MatPlan *out) {
     g.alpha = 1.f; g.act = p->act; g.batch_inner = 0;
     g.H = p->H; g.W = p->W; g.Cin = p->Cin; g.S = p->S; g.Ho = Ho; g.Wo = Wo;
     g.sh = p->stride_h; g.sw = p->stride_w; g.ph = p->pad_h; g.pw = p->pad_w;
-    g.R = p->R; g.rcp_hw = 1.0f / (float)(Ho * Wo); g.rcp_wo = 1.0f / (float)Wo;
+    g.R = p->R; g.inv_cin = inverse_of(g.Cin, g.K); g.inv_s = inverse_of(g.S, g.K / g.Cin);
+    g.rcp_hw = 1.0f / (float)(Ho * Wo); g.rcp_wo = 1.0f / (float)Wo;
     pl.dtype = p->dtype; pl.conv = 1; pl.b_kn = 0; pl.batch = 1;
     return choose_body(&pl, p->tile_m, p->tile_n, p->variant);
 }

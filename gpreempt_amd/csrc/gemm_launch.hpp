@@ -174,21 +174,25 @@ static int pipe_case_ckpt(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_strea
 // convolution chain of ResNet-152 1 us per launch (10.2 -> 11.2), and so did two stages instead of three for
 // the convolution form (10.05 -> 10.98).
 constexpr int wide_stages(int bm, int bn, int waves, bool conv) { return (!conv && bm == 32 && bn == 32 && waves == 16) ? 4 : 3; }
-template <typename T, int BM, int BN, int WAVES, bool CONV = false>
-using WideK = WideKernel<T, BM, BN, WAVES, wide_stages(BM, BN, WAVES, CONV), CONV>;
+template <typename T, int BM, int BN, int WAVES, int CONV = 0>
+using WideK = WideKernel<T, BM, BN, WAVES, wide_stages(BM, BN, WAVES, CONV != 0), CONV>;
+// whether a convolution's K-blocks (128 bytes) straddle filter taps
+template <typename T> static bool straddles_taps(const MatPlan &pl) { return pl.g.Cin % (128 / (int)sizeof(T)) != 0; }
 
 template <typename T, int BM, int BN, int WAVES>
 static int wide_case(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
-    if (pl.pre) return launch_mat<WideKernel<T, BM, BN, WAVES, wide_stages(BM, BN, WAVES, false), false, true>>(pl, ctx, s, info);
-    if (pl.conv) return launch_mat<WideK<T, BM, BN, WAVES, true>>(pl, ctx, s, info);
-    return launch_mat<WideK<T, BM, BN, WAVES, false>>(pl, ctx, s, info);
+    if (pl.pre) return launch_mat<WideKernel<T, BM, BN, WAVES, wide_stages(BM, BN, WAVES, false), 0, true>>(pl, ctx, s, info);
+    if (pl.conv && straddles_taps<T>(pl)) return launch_mat<WideK<T, BM, BN, WAVES, 2>>(pl, ctx, s, info);
+    if (pl.conv) return launch_mat<WideK<T, BM, BN, WAVES, 1>>(pl, ctx, s, info);
+    return launch_mat<WideK<T, BM, BN, WAVES, 0>>(pl, ctx, s, info);
 }
 
 template <int BM>
 static int narrow_case(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
-    if (pl.pre) return launch_mat<NarrowKernel<BM, 3, false, true>>(pl, ctx, s, info);
-    if (pl.conv) return launch_mat<NarrowKernel<BM, 3, true>>(pl, ctx, s, info);
-    return launch_mat<NarrowKernel<BM, 3, false>>(pl, ctx, s, info);
+    if (pl.pre) return launch_mat<NarrowKernel<BM, 3, 0, true>>(pl, ctx, s, info);
+    if (pl.conv && straddles_taps<float>(pl)) return launch_mat<NarrowKernel<BM, 3, 2>>(pl, ctx, s, info);
+    if (pl.conv) return launch_mat<NarrowKernel<BM, 3, 1>>(pl, ctx, s, info);
+    return launch_mat<NarrowKernel<BM, 3, 0>>(pl, ctx, s, info);
 }
 
 template <typename T>

@@ -14,13 +14,13 @@
 
 namespace gp {
 
-template <int BM, int STAGES, bool CONV = false, bool SCALED = false>
+template <int BM, int STAGES, int CONV = 0, bool SCALED = false>  // (as WideKernel)
 struct NarrowKernel {
     using T = float;
     using elem = float;
     static constexpr int BN = 16, WAVES = 16;
     static constexpr int bm = BM, bn = BN;
-    static constexpr bool conv = CONV, pre = SCALED;
+    static constexpr bool conv = CONV != 0, pre = SCALED;
     static_assert(!SCALED || !CONV, "GEMM rows only");
     static constexpr int VEC = 4, NT = WAVES * 64, RB = 128, BK = RB / 4;
     static constexpr int KB = WAVES / 2;                   // blocks per stage
@@ -75,7 +75,7 @@ struct NarrowKernel {
         }
         const u32x4 rsrc_a = buffer_of(CONV ? A - (long)(g.ph * g.W + g.pw) * g.lda : A), rsrc_b = buffer_of(B);
         auto group_of = [&](int j) { return j < LPW_A ? member + 2 * j : BM / 8 + member; };
-        unsigned off[LPW], taps[CONV ? LPW_A : 1];
+        unsigned off[LPW], taps[CONV ? LPW_A : 1], row[CONV ? LPW_A : 1];
         int kc[LPW];
 #pragma unroll
         for (int j = 0; j < LPW; ++j) {
@@ -99,6 +99,7 @@ struct NarrowKernel {
             }
         };
         if (CONV) advance(kb * BK);
+        constexpr bool straddles = CONV == 2;
         auto issue_part = [&](int s, auto first, auto last) {
             const int k0 = (s * KB + kb) * BK;
             const unsigned sbase = lds0 + ((unsigned)s % STAGES) * STAGE_BYTES + (unsigned)kb * BLK_BYTES;
@@ -108,7 +109,11 @@ struct NarrowKernel {
 #pragma unroll
             for (int j = first; j < last; ++j) {
                 const unsigned to = sbase + (unsigned)(group_of(j) * 8 * RB);
-                if (CONV && j < LPW_A) load_lds16_buffer(rsrc_a, (taps[CONV ? j : 0] & tap_bit) ? off[j] : kBufferEnd, tap_off, to);
+                if (CONV && j < LPW_A && straddles) {
+                    const int k = k0 + kc[j], tap = (int)__umulhi((unsigned)k + 1u, g.inv_cin), ci = k - tap * g.Cin, r = (int)__umulhi((unsigned)tap + 1u, g.inv_s), s2 = tap - r * g.S;
+                    const unsigned at = row[CONV ? j : 0] + (unsigned)((r * g.W + s2) * (int)g.lda + ci) * 4u;
+                    load_lds16_buffer(rsrc_a, k < g.K && (taps[CONV ? j : 0] >> tap & 1u) ? at : kBufferEnd, 0u, to);
+                } else if (CONV && j < LPW_A) load_lds16_buffer(rsrc_a, (taps[CONV ? j : 0] & tap_bit) ? off[j] : kBufferEnd, tap_off, to);
                 else load_lds16_buffer(j < LPW_A ? rsrc_a : rsrc_b, whole || k0 + kc[j] < g.K ? off[j] : kBufferEnd, (unsigned)k0 * 4u, to);
             }
             if (CONV && last == LPW_A) advance(KB * BK);
@@ -140,7 +145,8 @@ struct NarrowKernel {
 #pragma unroll
             for (int j = 0; j < LPW_A; ++j) {
                 const int r = group_of(j) * 8 + rig;
-                off[j] = (row_off[CONV ? r : 0] + (unsigned)kc[j]) * 4u;
+                row[CONV ? j : 0] = row_off[CONV ? r : 0] * 4u;
+                off[j] = row[CONV ? j : 0] + (unsigned)kc[j] * 4u;
                 taps[CONV ? j : 0] = row_taps[CONV ? r : 0];
             }
         }

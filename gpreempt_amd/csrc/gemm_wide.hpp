@@ -26,11 +26,12 @@
 // longer wait for the first, larger stage costs what the faster stream saves.
 //
 // CONV = true: the A operand is gathered (implicit GEMM over NHWC pixels): row m is output pixel
-// (n, ho, wo), K element k is filter tap k / Cin, channel k % Cin.  Needs Cin to be a multiple of
-// BK (a block never straddles two taps) and at most 32 taps: which taps of a pixel's window lie
+// (n, ho, wo), K element k is filter tap k / Cin, channel k % Cin.  Needs at most 32 taps: which taps of a pixel's window lie
 // inside the image is worked out once per tile, as one bit per tap, so that a stage's loads cost a
 // shift, a select and an add per lane; the tap and channel of a wavefront group's next block
-// advance incrementally.
+// advance incrementally.  Where Cin is no multiple of BK a block straddles taps, and a lane works out the tap and channel of its
+// chunk for itself, with two multiplications for the divisions (Inception-v3 b1, 1 x 7 over 160 channels: 10.3 -> 8.4 us a launch against the
+// four-wavefront body, which divided).
 #pragma once
 #include "gemm_pipe.hpp"
 
@@ -132,11 +133,13 @@ __device__ __forceinline__ void wide_reduce_store(const MatArgs &g, float *red, 
     });
 }
 
-template <typename T, int BM, int BN, int WAVES, int STAGES, bool CONV = false, bool SCALED = false>  // (SCALED: PRE of PipeKernel)
+// CONV: 0 a GEMM, 1 a convolution, 2 one whose blocks straddle taps (as a run-time switch, the test cost the others 1 % of a ResNet-152 pass).
+// SCALED: PRE of PipeKernel.
+template <typename T, int BM, int BN, int WAVES, int STAGES, int CONV = 0, bool SCALED = false>
 struct WideKernel {
     using elem = T;
     static constexpr int bm = BM, bn = BN;
-    static constexpr bool conv = CONV, pre = SCALED;
+    static constexpr bool conv = CONV != 0, pre = SCALED;
     static_assert(!SCALED || !CONV, "GEMM rows only");
     static constexpr int VEC = Elem<T>::VEC;
     static constexpr int NT = WAVES * 64;
@@ -232,6 +235,7 @@ struct WideKernel {
         unsigned off[LPW];     // the lane's row and chunk at k = 0, in bytes
         int kc[LPW];           // the lane's chunk offset in elements
         unsigned taps[CONV ? LPW : 1];  // CONV, A rows: bit t set = tap t of the row's window is inside the image
+        unsigned row[CONV ? LPW : 1];   // CONV, A rows: the row's window origin, in bytes
 #pragma unroll
         for (int j = 0; j < LPW; ++j) {
             const int gi = group_of(wv, j);           // group index in the block
@@ -256,6 +260,7 @@ struct WideKernel {
             }
         };
         if (CONV) advance(kb * BK);
+        constexpr bool straddles = CONV == 2;
         auto issue_part = [&](int s, auto first, auto last) {  // the loads first..last-1 of the wavefront's LPW for stage s
             const int k0 = (s * KB + kb) * BK;          // first K element of this wavefront group's block
             const unsigned sbase = lds0 + ((unsigned)s % STAGES) * STAGE_BYTES + (unsigned)kb * BLK_BYTES;
@@ -265,7 +270,11 @@ struct WideKernel {
 #pragma unroll
             for (int j = first; j < last; ++j) {
                 const int gi = group_of(wv, j);
-                if (CONV && j < LPW_A) {
+                if (CONV && j < LPW_A && straddles) {
+                    const int k = k0 + kc[j], tap = (int)__umulhi((unsigned)k + 1u, g.inv_cin), ci = k - tap * g.Cin, r = (int)__umulhi((unsigned)tap + 1u, g.inv_s), s2 = tap - r * g.S;
+                    const unsigned at = row[CONV ? j : 0] + (unsigned)((r * g.W + s2) * (int)g.lda + ci) * (unsigned)sizeof(T);
+                    load_lds16_buffer(rsrc_a, k < g.K && (taps[CONV ? j : 0] >> tap & 1u) ? at : kBufferEnd, 0u, sbase + (unsigned)(gi * 8 * RB));
+                } else if (CONV && j < LPW_A) {
                     // taps outside the image, rows outside the problem and blocks past K have nothing to fetch
                     load_lds16_buffer(rsrc_a, (taps[CONV ? j : 0] & tap_bit) ? off[j] : kBufferEnd, tap_off, sbase + (unsigned)(gi * 8 * RB));
                 } else {
@@ -302,7 +311,8 @@ struct WideKernel {
 #pragma unroll
             for (int j = 0; j < LPW_A; ++j) {
                 const int r = group_of(wv, j) * 8 + rig;
-                off[j] = (row_off[CONV ? r : 0] + (unsigned)kc[j]) * (unsigned)sizeof(T);
+                row[CONV ? j : 0] = row_off[CONV ? r : 0] * (unsigned)sizeof(T);
+                off[j] = row[CONV ? j : 0] + (unsigned)kc[j] * (unsigned)sizeof(T);
                 taps[CONV ? j : 0] = row_taps[CONV ? r : 0];
             }
         }

@@ -68,6 +68,7 @@ struct MatArgs {
     // convolution geometry (CONV only)
     int H, W, Cin, S, Ho, Wo, sh, sw, ph, pw;
     int R;                 // window rows (K = R * S * Cin)
+    unsigned inv_cin, inv_s;  // inverse_of(Cin), inverse_of(S): see util/slice_map.h
     float rcp_hw, rcp_wo;  // 1 / (Ho * Wo), 1 / Wo: see small_div
     // layer-norm prologue (gemm_ln.hpp; ln_gamma == nullptr: none): the rows of A are normalised over
     // their K elements before they are multiplied, and written to ln_out (M x K)

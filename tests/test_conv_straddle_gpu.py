@@ -1,0 +1,55 @@
+"""Convolutions whose K-blocks straddle filter taps (channels no multiple of a block) on the wide and narrow bodies: the bits of the
+four-wavefront split-K body, which divides for every chunk, plain, preempted and resumed."""
+import numpy as np
+import pytest
+
+from helpers import sync
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("N,H,W,Cin,Cout,R,S,stride,ph,pw", [
+    (1, 17, 17, 160, 160, 1, 7, 1, 0, 3),   # Inception-v3's factorised layers
+    (1, 17, 17, 160, 192, 7, 1, 1, 3, 0),
+    (1, 35, 35, 48, 64, 5, 5, 1, 2, 2),
+    (2, 35, 35, 96, 96, 3, 3, 1, 1, 1),
+    (1, 35, 35, 288, 384, 3, 3, 2, 0, 0),
+    (1, 9, 7, 24, 33, 5, 6, 1, 2, 3),       # a stage covers ten taps, rows and columns ragged, thirty taps
+    (3, 6, 6, 200, 40, 3, 3, 1, 2, 2),      # more padding than the window needs
+    (1, 8, 8, 72, 24, 4, 8, 2, 3, 4),       # the last of 32 taps
+    (8, 14, 14, 104, 136, 3, 3, 1, 1, 1),   # tiles of 64 x 32 or 64 x 64
+])
+def test_blocks_that_straddle_taps(gp, dt, N, H, W, Cin, Cout, R, S, stride, ph, pw):
+    dtype = gp.DTYPE_BY_NAME[dt]
+    rng = np.random.default_rng(H + Cin + Cout)
+    Ho, Wo = (H + 2 * ph - R) // stride + 1, (W + 2 * pw - S) // stride + 1
+    x, w = rng.uniform(-1, 1, (N, H, W, Cin + 16)).astype(np.float32), rng.uniform(-1, 1, (Cout, R, S, Cin)).astype(np.float32)
+    dx, dw, db = (gp.DevBuf.from_array(v, dtype) for v in (x, w, rng.uniform(-1, 1, Cout).astype(np.float32)))
+    out = gp.DevBuf((N * Ho * Wo * Cout * gp.DTYPE_SIZE[dtype] + 3) // 4 * 4)
+    p = gp.ConvParams(dtype=dtype, N=N, H=H, W=W, Cin=Cin, Cout=Cout, R=R, S=S, stride_h=stride, stride_w=stride, pad_h=ph, pad_w=pw, in_=dx.ptr, in_pix_stride=Cin + 16,
+                      weight=dw.ptr, bias=db.ptr, out=out.ptr, out_pix_stride=Cout, act=gp.ACT_RELU, tile_m=32, tile_n=32, variant=gp.MAT_PIPE_SPLITK)
+    out.fill32(0x7E007E00)
+    gp.launch("gp_launch_conv2d", p)
+    sync(gp)
+    want = out.download().copy()
+    p.tile_m = p.tile_n = p.variant = 0
+    flag = gp.Flag()
+    for ctx_of in (None, lambda st: st.ctx(fresh=2), lambda st: st.ctx(inject_at=0)):
+        st = gp.BlpState(1, flag, 32)
+        out.fill32(0x7E007E00)
+        info = gp.launch("gp_launch_conv2d", p, ctx_of(st) if ctx_of else None)
+        sync(gp)
+        assert info.block in (512, 1024), "not a wide body"
+        flag.set(0)
+        st.stop.upload(np.array([-1], np.int32))
+        if ctx_of:
+            gp.launch("gp_launch_conv2d", p, st.ctx())
+            sync(gp)
+        assert np.array_equal(out.download(), want)
+    for variant in (gp.MAT_WIDE, gp.MAT_WIDE8):  # asked for by name, a wide body is refused here as it always was
+        if Cin % (32 if dt == "f32" else 64):
+            p.tile_m = p.tile_n = 32
+            p.variant = variant
+            with pytest.raises(gp.GpError):
+                gp.launch("gp_launch_conv2d", p)

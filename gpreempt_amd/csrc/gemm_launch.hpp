@@ -11,6 +11,12 @@
 #include "plans.hpp"
 
 namespace gp {
+// whether a convolution's K-blocks (128 bytes) straddle filter taps
+template <typename T> static bool straddles_taps(const MatPlan &pl) { return pl.g.Cin % (128 / (int)sizeof(T)) != 0; }
+}  // namespace gp
+#include "gemm_group.hpp"
+
+namespace gp {
 
 // Asks for the arguments that stand in front of a tile's first load, and for those of its epilogue, in one go.  Left to itself
 // the compiler reads them where they are used, in four or five batches one behind the other, each a trip of 0.2 us.
@@ -176,8 +182,6 @@ static int pipe_case_ckpt(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_strea
 constexpr int wide_stages(int bm, int bn, int waves, bool conv) { return (!conv && bm == 32 && bn == 32 && waves == 16) ? 4 : 3; }
 template <typename T, int BM, int BN, int WAVES, int CONV = 0>
 using WideK = WideKernel<T, BM, BN, WAVES, wide_stages(BM, BN, WAVES, CONV != 0), CONV>;
-// whether a convolution's K-blocks (128 bytes) straddle filter taps
-template <typename T> static bool straddles_taps(const MatPlan &pl) { return pl.g.Cin % (128 / (int)sizeof(T)) != 0; }
 
 template <typename T, int BM, int BN, int WAVES>
 static int wide_case(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
@@ -251,6 +255,19 @@ int launch_typed(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, gp_l
                            : launch_mat<TK<T, 64, 64, SBK, 2, 2, false, false>>(pl, ctx, s, info);
     }
     set_error("unknown matrix kernel body %d", pl.body);
+    return GP_FAIL;
+}
+
+template <typename T>
+int launch_group_typed(const MatPlan *pl, int n, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
+    if constexpr (sizeof(T) == 4) {
+        if (pl[0].body == MB_NARROW16x16) return launch_group<NarrowKernel<16, 3, 0>, NarrowKernel<16, 3, 1>, NarrowKernel<16, 3, 2>>(pl, n, ctx, s, info);
+        if (pl[0].body == MB_NARROW32x16) return launch_group<NarrowKernel<32, 3, 0>, NarrowKernel<32, 3, 1>, NarrowKernel<32, 3, 2>>(pl, n, ctx, s, info);
+    } else {
+        if (pl[0].body == MB_WIDE32x32_16) return launch_group<WideK<T, 32, 32, 16, 0>, WideK<T, 32, 32, 16, 1>, WideK<T, 32, 32, 16, 2>>(pl, n, ctx, s, info);
+        if (pl[0].body == MB_WIDE64x32_16) return launch_group<WideK<T, 64, 32, 16, 0>, WideK<T, 64, 32, 16, 1>, WideK<T, 64, 32, 16, 2>>(pl, n, ctx, s, info);
+    }
+    set_error("matrix kernel body %d does not run in groups", pl[0].body);
     return GP_FAIL;
 }
 

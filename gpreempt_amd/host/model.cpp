@@ -275,6 +275,39 @@ void Model::plan_fusions() {
         el.fused_away = true;
         unread_[between] = i;
     }
+    // convolutions side by side
+    for (size_t i = 0; i < kernel_infos.size(); ++i) {
+        KernelInfo &first = kernel_infos[i];
+        first.group.clear();
+        if (first.op != OpKind::Conv || first.fused_away || first.has_pre) continue;
+        std::vector<gp_conv_params> group = {first.p.conv};
+        size_t end = i + 1;
+        for (; end < kernel_infos.size(); ++end) {
+            const KernelInfo &k = kernel_infos[end];
+            bool apart = k.op == OpKind::Conv && !k.has_pre;
+            for (size_t m = i; m < end && apart; ++m) apart = run_side_by_side(kernel_infos[m], k);
+            if (!apart) break;
+            group.push_back(k.p.conv);
+            if (gp_conv2d_group_supported(group.data(), (int)group.size()) != 1) { group.pop_back(); break; }
+        }
+        if (group.size() < 2) continue;
+        for (size_t m = i + 1; m < end; ++m) kernel_infos[m].fused_away = true;
+        first.group = std::move(group);
+        i = end - 1;
+    }
+}
+
+// Whether convolution b (a kernel behind a in the list) can run beside a: neither reads what the other writes, and what they write
+// does not overlap (the same buffer only in channel slices that lie apart).
+bool Model::run_side_by_side(const KernelInfo &a, const KernelInfo &b) {
+    const size_t oa = a.args_index[4], ob = b.args_index[4];
+    for (size_t slot = 0; slot < 4; ++slot)
+        if (a.args_index[slot] == ob || b.args_index[slot] == oa) return false;
+    if (oa != ob) return true;
+    const gp_conv_params &p = a.p.conv, &q = b.p.conv;
+    const long es = (long)get_stype_size(storage_infos[oa].stype);
+    const long pa = ((char *)p.out - (char *)storages[oa]) / es, pb = ((char *)q.out - (char *)storages[ob]) / es;
+    return p.out_pix_stride == q.out_pix_stride && pa + p.Cout <= p.out_pix_stride && pb + q.Cout <= q.out_pix_stride && (pa + p.Cout <= pb || pb + q.Cout <= pa);
 }
 
 // The output of a layer that its reader's launch does itself (plan_fusions): computed for a caller that wants to see it.
@@ -528,7 +561,7 @@ Status Model::launch(size_t idx, GPUstream stream, int inject_at) {
     int rc = GP_FAIL;
     switch (k.op) {
         case OpKind::Gemm: rc = gp_launch_gemm(fuse && k.has_ln_gemm ? &k.ln_gemm : &k.p.gemm, pc, stream, &info); break;
-        case OpKind::Conv: rc = fuse && k.has_pre ? gp_launch_eltwise_conv2d(&k.pre, &k.p.conv, pc, stream, &info) : gp_launch_conv2d(&k.p.conv, pc, stream, &info); break;
+        case OpKind::Conv: rc = fuse && !k.group.empty() ? gp_launch_conv2d_group(k.group.data(), (int)k.group.size(), pc, stream, &info) : fuse && k.has_pre ? gp_launch_eltwise_conv2d(&k.pre, &k.p.conv, pc, stream, &info) : gp_launch_conv2d(&k.p.conv, pc, stream, &info); break;
         case OpKind::Layout: rc = gp_launch_nchw_to_nhwc(&k.p.layout, pc, stream, &info); break;
         case OpKind::Pool: rc = gp_launch_pool2d(&k.p.pool, pc, stream, &info); break;
         case OpKind::Eltwise: rc = gp_launch_eltwise(&k.p.eltwise, pc, stream, &info); break;

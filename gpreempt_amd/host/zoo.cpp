@@ -7,6 +7,7 @@
 #include "graph_builder.h"
 #include "workloads/scicomput.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <map>
@@ -69,6 +70,26 @@ Status build_gemm(Model &m, const Options &o, int M, int N, int K, const std::st
     p.dtype = g.gp_dtype(); p.M = M; p.N = N; p.K = K; p.lda = K; p.ldb = K; p.b_is_nk = 1; p.ldc = N; p.alpha = 1.f; p.act = act; p.batch = 1;
     p.tile_m = p.tile_n = tile;
     return Status::Succ;
+}
+
+// Orders the kernel list by level, a level being the kernels whose inputs are all written by the levels before; within one the order of
+// the builder stays.  What could run side by side then stands side by side (Model::plan_fusions).  For graphs in which every
+// storage is written before it is read, slices of one by several kernels; a kernel's last slot is its output.
+void order_by_level(Model &m) {
+    std::vector<size_t> written(m.get_storage_num(), 0);  // by which level, + 1
+    std::vector<std::pair<size_t, size_t>> order;          // (level, position)
+    for (size_t i = 0; i < m.get_kernel_num(); ++i) {
+        const std::vector<ArgRef> &refs = m.get_kernel_info(i).refs;
+        size_t level = 0;
+        for (size_t r = 0; r + 1 < refs.size(); ++r)
+            if (refs[r].storage != SIZE_MAX) level = std::max(level, written[refs[r].storage]);
+        written[refs.back().storage] = std::max(written[refs.back().storage], level + 1);
+        order.emplace_back(level, i);
+    }
+    std::stable_sort(order.begin(), order.end(), [](const std::pair<size_t, size_t> &a, const std::pair<size_t, size_t> &b) { return a.first < b.first; });
+    std::vector<KernelInfo> sorted;
+    for (const auto &o : order) sorted.push_back(m.get_kernel_info(o.second));
+    for (size_t i = 0; i < sorted.size(); ++i) m.get_kernel_info(i) = sorted[i];
 }
 
 // ---- Inception-v3 ------------------------------------------------------------------------------
@@ -180,6 +201,7 @@ Status build_inception_v3(Model &m, const Options &o) {
     g.dense("fc1", gap.st, 0, N, gap.C, gap.C, classes, GP_ACT_NONE, SIZE_MAX, logits, 0, classes, 0.01f);
     size_t heads = g.add_storage("heads", (size_t)N * classes, g.stype_);
     g.softmax(logits, heads, N, classes, 1.f);
+    order_by_level(m);
     return Status::Succ;
 }
 

@@ -298,6 +298,12 @@ typedef struct gp_conv_params {
     int variant;
 } gp_conv_params;
 int gp_launch_conv2d(const gp_conv_params *p, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info);
+/* No counterpart in the reference (TVM launches operators one by one): n convolutions, two to four, as one launch, with one set of claim
+ * counters.  None may read or overwrite what another writes.  The results have the bits of n launches.  Only for what
+ * gp_conv2d_group_supported accepts (1): each would get the same one of the sixteen-wavefront bodies alone (layers of few
+ * tiles), and together they have at most one tile per compute unit. */
+int gp_conv2d_group_supported(const gp_conv_params *p, int n);
+int gp_launch_conv2d_group(const gp_conv_params *p, int n, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info);
 /* As gp_gemm_ckpt_bytes, for a convolution (0 unless it runs on the 128 x 128 body). */
 int gp_conv_ckpt_bytes(const gp_conv_params *p, size_t *bytes);
 

@@ -87,6 +87,9 @@ public:
     // ... and likewise a scale-shift(-ReLU) layer whose output only the pointwise convolution behind it reads: that one's launch
     // (gp_launch_eltwise_conv2d) does both, and the layer's output is not written; Model::get and fetch compute it for
     // whoever asks for it.
+    // ... and convolutions that follow each other in the list without reading each other run as one launch
+    // (gp_launch_conv2d_group) under the first one's index.
+    std::vector<gp_conv_params> group;
     bool has_pre = false;
     gp_eltwise_params pre;
 };
@@ -236,6 +239,7 @@ private:
 
     Status allocate_and_bind();
     void plan_fusions();
+    bool run_side_by_side(const KernelInfo &a, const KernelInfo &b);
     Status compute_unread(size_t idx, GPUstream stream);
     std::vector<size_t> unread_;  // per storage: the kernel that would write it, where plan_fusions found a launch that needs no such storage
     bool fuse_launches_ = true;  // GPREEMPT_FUSE_LN=0 in the environment keeps every launch of the kernel list

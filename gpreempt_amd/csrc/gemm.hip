@@ -158,6 +158,11 @@ static int choose_body(MatPlan *pl, int tile, int tile_n, int variant) {
     pl->sx = (g.N + tn - 1) / tn;
     pl->sy = (g.M + t - 1) / t;
     pl->lds_bytes = body_lds_bytes(body, pl->dtype);
+    // A convolution whose tiles' input windows are runs of consecutive pixels that fit in LDS fetches them once (gemm_window.hpp; where the
+    // launcher picks the body itself; 16-bit, fp32 being bound by its arithmetic; 32 x 32 tiles: with 64 x 32 the four multiplying wavefronts,
+    // which work out where a lane's row lies, are what a stage waits for, 0.76 us for the gather's 0.53, ResNet-152 b8 1530 -> 1560).
+    pl->window = pl->conv && variant == GP_MAT_AUTO && tile == 0 && pl->dtype != GP_F32 && body == MB_WIDE32x32_16 && g.Cin % 64 == 0 && g.sh == 1 && g.sw == 1 &&
+                 g.Ho == g.H && g.Wo == g.W && WindowKernel<_Float16, 32, 32, 4>::LDS_BYTES + window_bytes(g, 32, 2) <= kWindowMaxLds;
     // (a caller that names the tile gets that body at its own depth)
     if (tile == 0 && variant == GP_MAT_AUTO && ((body == MB_PIPE128 && tiles(128) > cus) || (body == MB_PIPE64 && tiles(64) > 2 * cus))) pl->ring = 2;
     // Tiles of a few microseconds: claimed through the counters, a tile waits 1-2 us for its claim, and the kernel around

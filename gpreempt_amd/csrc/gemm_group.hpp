@@ -4,18 +4,19 @@
 // whatever it computes; run side by side they cost that once.  Inception-v3 has 94 convolutions in 52 levels.
 //
 // Structure: the tiles of the members stand one behind the other in the launch's tile order; a workgroup finds the member its tile
-// belongs to and runs that member's own body (one of the three forms, GEMM, convolution, convolution whose blocks straddle
-// taps, of one wide or narrow tile shape, which is all a kernel can hold), so sums and bits are those of launches of their own.
+// belongs to and runs that member's own body (one of the forms, GEMM, convolution, convolution whose blocks straddle taps,
+// convolution with its window in LDS, of one wide or narrow tile shape, which is all a kernel can hold), so sums and bits are those of launches of their own.
 // Claims, claim counters and the kernel index are the launch's: a stop inside it resumes there.
 #pragma once
 #include "gemm_narrow.hpp"
+#include "gemm_window.hpp"
 
 namespace gp {
 
 constexpr int kGroupMax = 4;
 struct GroupMember {
     MatArgs g;
-    int first, sx, sy, order, form;  // first tile in the launch's order, tile grid, order and body form (0, 1, 2: WideKernel's CONV)
+    int first, sx, sy, order, form;  // first tile in the launch's order, tile grid, order and body form (0, 1, 2: WideKernel's CONV, 3: WindowKernel)
     unsigned inv_sx, inv_sy;
 };
 struct GroupArgs {
@@ -23,8 +24,8 @@ struct GroupArgs {
     int first[kGroupMax];  // as in m; beyond the last member: no tile is that far
 };
 
-// Forms: the bodies of forms 0, 1 and 2
-template <int LOOP, class F0, class F1, class F2>
+// F0 .. F3: the bodies of the forms; F3 == F1: there is no form 3
+template <int LOOP, class F0, class F1, class F2, class F3>
 __global__ __launch_bounds__(F0::NT) void group_kernel(GroupArgs a, BlpArgs blp) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
     using T = typename F0::elem;
@@ -49,6 +50,8 @@ __global__ __launch_bounds__(F0::NT) void group_kernel(GroupArgs a, BlpArgs blp)
         const CkptCtx cc{stop, nullptr, nullptr, 0};
         const int form = m->form;
         if (form == 0) return F0::template run<false, SINGLE>(g, t, lds, cc, asked);
+        if constexpr (F3::window)
+            if (form == 3) return F3::template run<false, SINGLE>(g, t, lds, cc, asked);
         if (form == 1) return F1::template run<false, SINGLE>(g, t, lds, cc, asked);
         return F2::template run<false, SINGLE>(g, t, lds, cc, asked);
     };
@@ -56,16 +59,17 @@ __global__ __launch_bounds__(F0::NT) void group_kernel(GroupArgs a, BlpArgs blp)
     else tiles<LOOP>(blp, [&](TileIdx t) { tile(t, nullptr, NoneAsked{}); });
 }
 
-template <class F0, class F1, class F2>
+template <class F0, class F1, class F2, class F3 = F1>
 static int launch_group(const MatPlan *pl, int n, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
-    static_assert(F0::NT == F1::NT && F0::NT == F2::NT, "one kernel");
-    constexpr size_t LDS = std::max(F0::LDS_BYTES, std::max(F1::LDS_BYTES, F2::LDS_BYTES));
-    constexpr auto any = group_kernel<LOOP_ANY, F0, F1, F2>, plain = group_kernel<LOOP_PLAIN, F0, F1, F2>, fixed = group_kernel<LOOP_FIXED, F0, F1, F2>;
+    static_assert(F0::NT == F1::NT && F0::NT == F2::NT && F0::NT == F3::NT, "one kernel");
+    constexpr size_t rings = std::max(F0::LDS_BYTES, std::max(F1::LDS_BYTES, F2::LDS_BYTES)), most = F3::window ? std::max(rings, kWindowMaxLds) : rings;
+    size_t lds = rings;
+    constexpr auto any = group_kernel<LOOP_ANY, F0, F1, F2, F3>, plain = group_kernel<LOOP_PLAIN, F0, F1, F2, F3>, fixed = group_kernel<LOOP_FIXED, F0, F1, F2, F3>;
     static std::once_flag once;
     static hipError_t once_rc = hipSuccess;
     std::call_once(once, [] {
         for (const void *f : {(const void *)any, (const void *)plain, (const void *)fixed}) {
-            hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS);
+            hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most);
             if (e != hipSuccess) once_rc = e;
         }
     });
@@ -79,16 +83,17 @@ static int launch_group(const MatPlan *pl, int n, const gp_preempt_ctx *ctx, gp_
         const int tiles = pl[i].sx * pl[i].sy;
         m.g = pl[i].g;
         m.first = total; m.sx = pl[i].sx; m.sy = pl[i].sy; m.order = pl[i].order;
-        m.form = !pl[i].conv ? 0 : straddles_taps<typename F0::elem>(pl[i]) ? 2 : 1;
+        m.form = !pl[i].conv ? 0 : F3::window && pl[i].window ? 3 : straddles_taps<typename F0::elem>(pl[i]) ? 2 : 1;
+        if (m.form == 3) lds = std::max(lds, F3::LDS_BYTES + window_bytes(m.g, F3::bm, (int)sizeof(typename F0::elem)));
         m.inv_sx = inverse_of(m.sx, tiles); m.inv_sy = inverse_of(m.sy, tiles);
         total += tiles;
     }
     BlpArgs blp;
     int grid = 0;
-    int rc = plan_launch(any, F0::NT, LDS, total, 1, 1, ctx, &blp, &grid, info, 1, 2);
+    int rc = plan_launch(any, F0::NT, lds, total, 1, 1, ctx, &blp, &grid, info, 1, 2);
     if (rc) return rc;
     auto kern = !ctx ? plain : fixed_claims(true, blp.groups, grid - blp.front, blp.total) ? fixed : any;
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(F0::NT), LDS, native(s), a, blp);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(F0::NT), lds, native(s), a, blp);
     GP_HIP(hipGetLastError());
     return GP_SUCC;
 }

@@ -88,8 +88,9 @@ static int launch_mat(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s,
     BlpArgs blp;
     int grid = 0;
     auto kern = KernelOf<K>::fn;  // the launch is planned for the general form; the others need no more resources
-    const size_t lds_bytes = K::LDS_BYTES + (K::pre ? pre_table_bytes(pl.g.K, (unsigned)sizeof(typename K::elem)) : 0);
-    constexpr size_t max_lds = K::pre ? pre_max_lds(K::LDS_BYTES) : K::LDS_BYTES;
+    constexpr int es = (int)sizeof(typename K::elem);
+    const size_t lds_bytes = K::LDS_BYTES + (K::pre ? pre_table_bytes(pl.g.K, es) : 0) + (K::window ? window_bytes(pl.g, K::bm, es) : 0);
+    constexpr size_t max_lds = K::pre ? pre_max_lds(K::LDS_BYTES) : K::window ? kWindowMaxLds : K::LDS_BYTES;
     if (max_lds > 48 * 1024) {
         // several tenant threads launch concurrently: the attribute is set by exactly one of them
         static std::once_flag once;
@@ -185,6 +186,8 @@ using WideK = WideKernel<T, BM, BN, WAVES, wide_stages(BM, BN, WAVES, CONV != 0)
 
 template <typename T, int BM, int BN, int WAVES>
 static int wide_case(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
+    if constexpr (sizeof(T) == 2 && BM == 32 && WAVES == 16)
+        if (pl.window) return launch_mat<WindowKernel<T, BM, BN, 4>>(pl, ctx, s, info);
     if (pl.pre) return launch_mat<WideKernel<T, BM, BN, WAVES, wide_stages(BM, BN, WAVES, false), 0, true>>(pl, ctx, s, info);
     if (pl.conv && straddles_taps<T>(pl)) return launch_mat<WideK<T, BM, BN, WAVES, 2>>(pl, ctx, s, info);
     if (pl.conv) return launch_mat<WideK<T, BM, BN, WAVES, 1>>(pl, ctx, s, info);
@@ -264,7 +267,7 @@ int launch_group_typed(const MatPlan *pl, int n, const gp_preempt_ctx *ctx, gp_s
         if (pl[0].body == MB_NARROW16x16) return launch_group<NarrowKernel<16, 3, 0>, NarrowKernel<16, 3, 1>, NarrowKernel<16, 3, 2>>(pl, n, ctx, s, info);
         if (pl[0].body == MB_NARROW32x16) return launch_group<NarrowKernel<32, 3, 0>, NarrowKernel<32, 3, 1>, NarrowKernel<32, 3, 2>>(pl, n, ctx, s, info);
     } else {
-        if (pl[0].body == MB_WIDE32x32_16) return launch_group<WideK<T, 32, 32, 16, 0>, WideK<T, 32, 32, 16, 1>, WideK<T, 32, 32, 16, 2>>(pl, n, ctx, s, info);
+        if (pl[0].body == MB_WIDE32x32_16) return launch_group<WideK<T, 32, 32, 16, 0>, WideK<T, 32, 32, 16, 1>, WideK<T, 32, 32, 16, 2>, WindowKernel<T, 32, 32, 4>>(pl, n, ctx, s, info);
         if (pl[0].body == MB_WIDE64x32_16) return launch_group<WideK<T, 64, 32, 16, 0>, WideK<T, 64, 32, 16, 1>, WideK<T, 64, 32, 16, 2>>(pl, n, ctx, s, info);
     }
     set_error("matrix kernel body %d does not run in groups", pl[0].body);

@@ -25,7 +25,7 @@ template <typename T, int BM, int BN, int WAVES, int STAGES>
 struct LnWideKernel {
     using elem = T;
     static constexpr int bm = BM, bn = BN;
-    static constexpr bool conv = false, pre = false;
+    static constexpr bool conv = false, pre = false, window = false;
     static constexpr int VEC = Elem<T>::VEC;
     static constexpr int NT = WAVES * 64;
     static constexpr int RB = 128;                         // row bytes of a block in LDS

@@ -20,7 +20,7 @@ struct NarrowKernel {
     using elem = float;
     static constexpr int BN = 16, WAVES = 16;
     static constexpr int bm = BM, bn = BN;
-    static constexpr bool conv = CONV != 0, pre = SCALED;
+    static constexpr bool conv = CONV != 0, pre = SCALED, window = false;
     static_assert(!SCALED || !CONV, "GEMM rows only");
     static constexpr int VEC = 4, NT = WAVES * 64, RB = 128, BK = RB / 4;
     static constexpr int KB = WAVES / 2;                   // blocks per stage

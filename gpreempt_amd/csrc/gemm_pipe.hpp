@@ -139,7 +139,7 @@ template <typename T, int BM, int BN, int STAGES, bool CONV, bool SPLITK, bool C
 struct PipeKernel {
     using elem = T;
     static constexpr int bm = BM, bn = BN;
-    static constexpr bool conv = CONV, pre = PRE;
+    static constexpr bool conv = CONV, pre = PRE, window = false;
     static_assert(!PRE || (!CONV && !CKPT), "GEMM rows only");
     static constexpr int VEC = Elem<T>::VEC;
     static constexpr int WAVES = NWAVES, NT = WAVES * 64;

@@ -10,7 +10,7 @@ template <typename T, int BM, int BN, int BK, int WGM, int WGN, bool CONV, bool 
 struct TileKernel {
     using elem = T;
     static constexpr int bm = BM, bn = BN;
-    static constexpr bool conv = CONV, pre = false;
+    static constexpr bool conv = CONV, pre = false, window = false;
     static constexpr int VEC = Elem<T>::VEC;
     static constexpr int NT = WGM * WGN * 64;
     static constexpr int LDK = BK + VEC;           // LDS row stride in elements (16-byte pad)

@@ -139,7 +139,7 @@ template <typename T, int BM, int BN, int WAVES, int STAGES, int CONV = 0, bool 
 struct WideKernel {
     using elem = T;
     static constexpr int bm = BM, bn = BN;
-    static constexpr bool conv = CONV != 0, pre = SCALED;
+    static constexpr bool conv = CONV != 0, pre = SCALED, window = false;
     static_assert(!SCALED || !CONV, "GEMM rows only");
     static constexpr int VEC = Elem<T>::VEC;
     static constexpr int NT = WAVES * 64;

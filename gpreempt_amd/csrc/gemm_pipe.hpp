@@ -222,9 +222,6 @@ struct PipeKernel {
         const int c_base = cpos ^ (rig >> 1);
         auto chunk_of = [&](int slot) { return c_base ^ ((slot & 1) << 2); };
         const int a_row0 = m0 + wave * A_PW * 8 + rig, b_row0 = n0 + wave * B_PW * 8 + rig;
-        // Pointers with the lane's chunk already added, one per parity of the slot number j: a
-        // load's address is then this plus a wave-uniform offset.
-        const T *a_par[2] = {nullptr, nullptr};  // GEMM: row a_row0 of A
         const T *a_org[CONV ? A_PW : 1];         // CONV: the slot's window origin (may lie outside the image)
         int a_h0[CONV ? A_PW : 1], a_w0[CONV ? A_PW : 1];
         if (CONV) {
@@ -239,30 +236,39 @@ struct PipeKernel {
                 a_h0[j] = ho * g.sh - g.ph; a_w0[j] = wo * g.sw - g.pw;
                 a_org[j] = A + ((long)n * g.H * g.W + (long)a_h0[j] * g.W + a_w0[j]) * g.lda;
             }
-        } else {
-            a_par[0] = A + (long)a_row0 * g.lda + chunk_of(wave * A_PW) * VEC;
-            a_par[1] = A + (long)a_row0 * g.lda + chunk_of(wave * A_PW + 1) * VEC;
         }
-        const T *b_par[2] = {B + (long)b_row0 * g.ldb + chunk_of(wave * B_PW) * VEC,
-                             B + (long)b_row0 * g.ldb + chunk_of(wave * B_PW + 1) * VEC};
+        // GEMM rows of A and B: bytes from the tile's first row, kBufferEnd for a row past the last one; a load is this, the stage's
+        // uniform offset along K and the operand's descriptor.  A wavefront has one instruction stream, and what stands between two of
+        // its MFMAs bounds a K-step here: pointers of 64 bits, advanced per slot and parked on the zero page, took 24 registers and, with a
+        // branch around the K remainder, a dozen instructions and two jumps per load; now it is a compare and a select.  Both builds in
+        // turn: 8192^3 bf16 with checkpoints 981 -> 945 us, 4096^3 fp32 1098 -> 1016, 6000 x 5000 x 2048 fp16 152 -> 146.
+        // (`near`: the tile's rows lie within a descriptor's 2 GB.  Otherwise an address of 64 bits is worked out for every load.)
+        const long far = (long)kBufferEnd / (long)sizeof(T) - g.K;
+        const bool near = (CONV || (long)BM * g.lda <= far) && (long)BN * g.ldb <= far;
+        unsigned a_off[CONV ? 1 : A_PW], b_off[B_PW];
+        if (!CONV) {
+#pragma unroll
+            for (int j = 0; j < (CONV ? 1 : A_PW); ++j)
+                a_off[j] = a_row0 + j * 8 < g.M ? near ? ((unsigned)(a_row0 - m0 + j * 8) * (unsigned)g.lda + (unsigned)(chunk_of(wave * A_PW + j) * VEC)) * (unsigned)sizeof(T) : 0u : kBufferEnd;
+        }
+#pragma unroll
+        for (int j = 0; j < B_PW; ++j)
+            b_off[j] = b_row0 + j * 8 < g.N ? near ? ((unsigned)(b_row0 - n0 + j * 8) * (unsigned)g.ldb + (unsigned)(chunk_of(wave * B_PW + j) * VEC)) * (unsigned)sizeof(T) : 0u : kBufferEnd;
+        const u32x4 rsrc_a = buffer_of(CONV ? A : A + (long)m0 * g.lda), rsrc_b = buffer_of(B + (long)n0 * g.ldb);
         const bool conv_fast = CONV && (g.Cin % BK == 0);  // a K-step never straddles a filter tap
-        const bool k_full = g.K % BK == 0;                 // no K-chunk of any stage lies past K
-        // Running source pointers.  Within one filter tap (conv) or along K (weights, GEMM rows) a
-        // slot's address only advances by BK elements per stage, so it is kept and bumped instead
-        // of rebuilt: a wave has one instruction stream, and twenty address instructions per load
-        // were more issue time than the MFMAs they feed.  `inc` is 0 for a slot parked on the zero
-        // page.  (Only bodies with few slots keep them for the B / GEMM-A side: registers.)
-        constexpr bool INCR = A_PW + B_PW <= 8;
-        const T *a_cur[A_PW], *b_cur[B_PW];
-        int a_inc[A_PW], b_inc[B_PW];
+        // Running source pointers of a convolution's pixels.  Within one filter tap a slot's address only advances by BK elements
+        // per stage, so it is kept and bumped instead of rebuilt: a wave has one instruction stream, and twenty address
+        // instructions per load were more issue time than the MFMAs they feed.  `inc` is 0 for a slot parked on the zero page.
+        const T *a_cur[CONV ? A_PW : 1];
+        int a_inc[CONV ? A_PW : 1];
+        if (CONV) {
 #pragma unroll
-        for (int j = 0; j < A_PW; ++j) { a_cur[j] = zero; a_inc[j] = 0; }
-#pragma unroll
-        for (int j = 0; j < B_PW; ++j) { b_cur[j] = zero; b_inc[j] = 0; }
+            for (int j = 0; j < (CONV ? A_PW : 1); ++j) { a_cur[j] = zero; a_inc[j] = 0; }
+        }
 
         // Loads of one stage: slot l < A_PW is an A slot, the rest are B slots.  `StageAddr` holds
         // the wave-uniform part, computed once per stage.
-        struct StageAddr { unsigned sbase, sbase_poll; int k0, r_u, s_u, tap_off; bool new_tap, first; };
+        struct StageAddr { unsigned sbase, sbase_poll, k_bytes; int k0, r_u, s_u, tap_off; bool new_tap, first; };
         // Stages are fetched in increasing order, so the filter tap (r, s) and channel offset of
         // the next stage advance incrementally instead of being divided out of k every time.
         int nx_r = 0, nx_s = 0, nx_ci = 0;
@@ -277,6 +283,7 @@ struct PipeKernel {
             sa.sbase = lds0 + ((unsigned)kt % STAGES) * STAGE_BYTES;
             sa.sbase_poll = lds0 + (unsigned)RING_BYTES + ((unsigned)kt % STAGES) * WAVES * 256;
             sa.k0 = kt * BK;
+            sa.k_bytes = (unsigned)__builtin_amdgcn_readfirstlane(sa.k0 * (int)sizeof(T));
             sa.r_u = nx_r; sa.s_u = nx_s;
             sa.tap_off = (nx_r * g.W + nx_s) * (int)g.lda + nx_ci;  // elements from the window origin
             sa.first = kt == kt0;                  // first stage fetched for this tile (or its continuation)
@@ -311,8 +318,8 @@ struct PipeKernel {
                 const T *src;
                 if (CONV) {
                     const int jj = CONV ? j : 0;
-                    if (conv_fast) {
-                        if (sa.new_tap) {  // (uniform) rebuild: bounds of the tap, pointer or zero page
+                    if (__builtin_expect(conv_fast, 1)) {
+                        if (__builtin_expect(sa.new_tap, 0)) {  // (uniform) rebuild: bounds of the tap, pointer or zero page
                             const bool ok = (a_row0 + j * 8 < g.M) & ((unsigned)(a_h0[jj] + sa.r_u) < (unsigned)g.H) &
                                             ((unsigned)(a_w0[jj] + sa.s_u) < (unsigned)g.W);
                             a_cur[j] = ok ? a_org[jj] + (sa.tap_off + kc) : zero;
@@ -330,37 +337,26 @@ struct PipeKernel {
                                         ((unsigned)(a_w0[jj] + s2) < (unsigned)g.W);
                         src = ok ? a_org[jj] + off : zero;
                     }
-                } else if (INCR && k_full) {
-                    if (sa.first) {
-                        const bool ok = a_row0 + j * 8 < g.M;
-                        a_cur[j] = ok ? a_par[j & 1] + ((long)(j * 8) * g.lda + sa.k0) : zero;
-                        a_inc[j] = ok ? BK : 0;
-                    } else {
-                        a_cur[j] += a_inc[j];
-                    }
-                    src = a_cur[j];
                 } else {
-                    const bool ok = (a_row0 + j * 8 < g.M) & (k_full | (sa.k0 + kc < g.K));
-                    src = ok ? a_par[j & 1] + ((long)(j * 8) * g.lda + sa.k0) : zero;
+                    const int jj = CONV ? 0 : j;
+                    const bool ok = sa.k0 + kc < g.K;
+                    if (__builtin_expect(near, 1)) {
+                        load_lds16_buffer(rsrc_a, ok ? a_off[jj] : kBufferEnd, sa.k_bytes, sa.sbase + (unsigned)((wave * A_PW + j) * 8 * RB));
+                        return;
+                    }
+                    src = ok && a_off[jj] != kBufferEnd ? A + ((long)(a_row0 + j * 8) * g.lda + (sa.k0 + kc)) : zero;
                 }
                 load_lds16(src, sa.sbase + (unsigned)((wave * A_PW + j) * 8 * RB));
             } else {
                 const int j = l - A_PW;
                 const int kc = chunk_of(wave * B_PW + j) * VEC;
                 const T *src;
-                if (INCR && k_full) {
-                    if (sa.first) {
-                        const bool ok = b_row0 + j * 8 < g.N;
-                        b_cur[j] = ok ? b_par[j & 1] + ((long)(j * 8) * g.ldb + sa.k0) : zero;
-                        b_inc[j] = ok ? BK : 0;
-                    } else {
-                        b_cur[j] += b_inc[j];
-                    }
-                    src = b_cur[j];
-                } else {
-                    const bool ok = (b_row0 + j * 8 < g.N) & (k_full | (sa.k0 + kc < g.K));
-                    src = ok ? b_par[j & 1] + ((long)(j * 8) * g.ldb + sa.k0) : zero;
+                const bool ok = sa.k0 + kc < g.K;
+                if (__builtin_expect(near, 1)) {
+                    load_lds16_buffer(rsrc_b, ok ? b_off[j] : kBufferEnd, sa.k_bytes, sa.sbase + (unsigned)(A_BYTES + (wave * B_PW + j) * 8 * RB));
+                    return;
                 }
+                src = ok && b_off[j] != kBufferEnd ? B + ((long)(b_row0 + j * 8) * g.ldb + (sa.k0 + kc)) : zero;
                 load_lds16(src, sa.sbase + (unsigned)(A_BYTES + (wave * B_PW + j) * 8 * RB));
             }
         };

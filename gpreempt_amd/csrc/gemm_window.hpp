@@ -1,10 +1,12 @@
 // Convolution bodies of the wide kind that keep their input window in LDS.
 //
-// Why: as an implicit GEMM a 3 x 3 layer fetches every input pixel nine times, and for a 64 x 32 tile that is two thirds of what the tile
-// fetches: 1568 x 256 x 2304 (14 x 14 x 256, eight images) 442 KB a workgroup, 88 MB from the L2s in 4.8 us, as much as they give.  At
-// stride 1 and with an output as large as the input, the pixels that a tile's rows read at a tap are consecutive ones (consecutive
-// pixels of the flattened images, moved by the tap), so all taps together read BM + 2 * (ph * W + pw) consecutive pixels: 94 here, 48 KB.
-// They are fetched once, in front of the first stage, and only the weights stream through the ring.
+// Why: as an implicit GEMM a 3 x 3 layer fetches every input pixel nine times, and a row's window has to be worked out in front of its first
+// load.  At stride 1 and with an output as large as the input, the pixels that a tile's rows read at a tap are consecutive ones
+// (consecutive pixels of the flattened images, moved by the tap), so all taps together read BM + 2 * (ph * W + pw) consecutive pixels:
+// 62 for 32 rows of a 14 x 14 image.  They are fetched once, in front of the first stage, only the weights stream through the ring, and
+// the rows' masks are worked out while the loads are under way.  Launches of 32 x 32 tiles: 4 x 14 x 14 x 128 -> 32 channels 7.3 -> 6.3 us,
+// 8 x 7 x 7 x 512 13.1 -> 12.0, 1 x 17 x 17 x 192 7.7 -> 7.2.  Not for 64 x 32 tiles, where the instruction stream of the four
+// multiplying wavefronts bounds a stage and a fragment's address costs more than the ring's: ResNet-152 b8 1530 -> 1560 us with them.
 //
 // Structure: as gemm_wide.hpp (sixteen wavefronts fetch, 0..3 multiply one MFMA k-step each of every block, the same sums in the same
 // order, hence the same bits).  The window lies behind the ring, K-block after K-block of Cin, rows of 128 bytes swizzled like the

@@ -561,8 +561,8 @@ __device__ __forceinline__ void tile_loop_ckpt(const BlpArgs &b, Body &&body) {
     const bool dynamic = b.executed != nullptr;
     const bool leader = (threadIdx.x == 0) & (threadIdx.y == 0) & (threadIdx.z == 0);
     const int grp = wg_group((int)blockIdx.x, b.groups);
-    const int slice_lo = b.groups > 1 ? group_slice_begin(b.total, grp, b.groups, b.grid) : 0;
-    const int slice_n = (b.groups > 1 ? group_slice_begin(b.total, grp + 1, b.groups, b.grid) : b.total) - slice_lo;
+    const int slice_lo = b.groups > 1 ? group_slice_begin(b.total, grp, b.groups, (int)gridDim.x) : 0;
+    const int slice_n = (b.groups > 1 ? group_slice_begin(b.total, grp + 1, b.groups, (int)gridDim.x) : b.total) - slice_lo;
     announce_start(b, leader);
     for (int it = 0;; ++it) {
         int idx, kt0 = 0;
@@ -599,10 +599,10 @@ __device__ __forceinline__ void tile_loop_ckpt(const BlpArgs &b, Body &&body) {
             kt0 = __builtin_amdgcn_readfirstlane(mailbox[it & 1][1]);  // K position stay scalar
         }
         if (idx < 0) { leave_stamped(b); return; }
-        if (body(decode_tile(idx, b.sx, b.sy, b.order, b.inv_sx, b.inv_sy), idx, kt0)) { leave_stamped(b); return; }
+        if (body(decode_tile(idx, b.sx, b.sy, b.order), idx, kt0)) { leave_stamped(b); return; }
         // one claim per workgroup at most (see tile_loop); a relaunch may continue a stored tile and
         // then still owe its slice a claim, so the shortcut holds on the fresh path only
-        if (b.grid >= b.total && kt0 == 0 && !(it == 0 && b.ckpt)) { leave_stamped(b); return; }
+        if ((int)gridDim.x >= b.total && kt0 == 0 && !(it == 0 && b.ckpt)) { leave_stamped(b); return; }
     }
 }
 

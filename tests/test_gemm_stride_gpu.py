@@ -1,0 +1,54 @@
+"""The pipelined bodies fetch through descriptors of 2 GB that begin at a tile's first row, and work out addresses of 64 bits where a
+tile's rows span more.  Rows just inside and just outside of that span, of either operand, give the bits of packed rows, and
+those the oracle's values; K with a remainder, and tiles with rows and columns past the last one."""
+import numpy as np
+import pytest
+
+from helpers import rel_err, sync
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def spread(gp, rows, stride_bytes):
+    """the rows, `stride_bytes` apart"""
+    buf = gp.DevBuf((len(rows) - 1) * stride_bytes + rows[0].nbytes)
+    for i, row in enumerate(rows):
+        gp.check(gp.lib().gp_memcpy_h2d(gp.vp(buf.ptr + i * stride_bytes), row.ctypes.data_as(gp.vp), gp.C.c_size_t(row.nbytes)))
+    return buf
+
+
+@pytest.mark.parametrize("outside", [False, True])
+@pytest.mark.parametrize("dtype_name,tile,variant,K,far_operand", [("bf16", 256, "MAT_PIPE", 200, "A"), ("bf16", 256, "MAT_PIPE", 128, "B"), ("f32", 256, "MAT_PIPE", 68, "A"),
+                                                                   ("f16", 128, "MAT_PIPE", 136, "B"), ("f32", 64, "MAT_PIPE", 36, "A"), ("bf16", 64, "MAT_PIPE_SPLITK", 72, "B")])
+def test_far_rows(gp, dtype_name, tile, variant, K, far_operand, outside):
+    dtype, es, vec = gp.DTYPE_BY_NAME[dtype_name], 4 if dtype_name == "f32" else 2, 4 if dtype_name == "f32" else 8
+    M = N = tile + 4
+    rng = np.random.default_rng(tile + K)
+    A, B = (gp.to_storage(rng.uniform(-1, 1, (s, K)).astype(np.float32), dtype).view(np.uint8).reshape(s, K * es) for s in (M, N))
+    dA, dB, out = gp.DevBuf.from_array(A), gp.DevBuf.from_array(B), gp.DevBuf(M * N * es)
+    p = gp.GemmParams(dtype=dtype, M=M, N=N, K=K, A=dA.ptr, lda=K, B=dB.ptr, ldb=K, b_is_nk=1, C=out.ptr, ldc=N, alpha=1.0, act=gp.ACT_NONE, batch=1,
+                      tile_m=tile, tile_n=tile, variant=getattr(gp, variant))
+    gp.launch("gp_launch_gemm", p)
+    sync(gp)
+    want = out.download().copy()
+    A32, B32 = (gp.from_storage(v.reshape(-1), dtype).reshape(-1, K) for v in (A, B))
+    # fp32 sums of K products, the result rounded to the type: half a unit in its last place
+    assert rel_err(gp.from_storage(want, dtype).reshape(M, N), O.gemm_bias_act(A32, B32, None, None, O.ACT_NONE, b_is_nk=True)) < {"f32": 1e-5, "f16": 1e-3, "bf16": 8e-3}[dtype_name]
+    ld = ((1 << 31) // es - K) // tile // vec * vec + (vec if outside else 0)
+    far = spread(gp, A if far_operand == "A" else B, ld * es)
+    if far_operand == "A":
+        p.A, p.lda = far.ptr, ld
+    else:
+        p.B, p.ldb = far.ptr, ld
+    out.fill32(0x7FC00000)
+    gp.launch("gp_launch_gemm", p)
+    sync(gp)
+    assert np.array_equal(out.download(), want)
+    if variant == "MAT_PIPE":  # and the preemptible form
+        st = gp.BlpState(1, gp.Flag(), 32)
+        st.enable_checkpoints(p)
+        out.fill32(0x7FC00000)
+        gp.launch("gp_launch_gemm", p, st.ctx(fresh=2))
+        sync(gp)
+        assert np.array_equal(out.download(), want)

@@ -60,7 +60,7 @@ template <typename T, int BM, int BN, int BK, int WGM, int WGN, bool CONV, bool 
 using TK = TileKernel<T, BM, BN, BK, WGM, WGN, CONV, B_KN>;
 
 template <class K> struct K_is_ckpt { static constexpr bool value = false; };
-template <typename T, int BM, int BN, int ST, bool CV, int W> struct K_is_ckpt<PipeKernel<T, BM, BN, ST, CV, false, true, W>> { static constexpr bool value = true; };
+template <typename T, int BM, int BN, int ST, int CV, int W> struct K_is_ckpt<PipeKernel<T, BM, BN, ST, CV, false, true, W>> { static constexpr bool value = true; };
 template <class K> struct KernelOf {
     static constexpr auto fn = mat_kernel<K, LOOP_ANY>;
     static constexpr auto plain = mat_kernel<K, LOOP_PLAIN>;
@@ -71,7 +71,7 @@ template <class K> struct KernelOf {
     static constexpr auto looks = mat_kernel<K, K::can_look ? LOOP_LOOKS : LOOP_FIXED>;
 #endif
 };
-template <typename T, int BM, int BN, int ST, bool CV, int W> struct KernelOf<PipeKernel<T, BM, BN, ST, CV, false, true, W>> {
+template <typename T, int BM, int BN, int ST, int CV, int W> struct KernelOf<PipeKernel<T, BM, BN, ST, CV, false, true, W>> {
     static constexpr auto fn = mat_kernel_ckpt<PipeKernel<T, BM, BN, ST, CV, false, true, W>>;
     static constexpr auto plain = fn;
     static constexpr auto fixed = fn;
@@ -162,17 +162,19 @@ template <typename T, bool CK> using BigPipe = PipeKernel<T, GP_BIG_BM, GP_BIG_B
 template <typename T, int TILE, int STAGES, bool SPLITK>
 static int pipe_case(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
     if constexpr (TILE == 64 && !SPLITK)
-        if (pl.pre) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, false, false, false, 4, true>>(pl, ctx, s, info);
-    if (pl.conv) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, true, SPLITK>>(pl, ctx, s, info);
-    return launch_mat<PipeKernel<T, TILE, TILE, STAGES, false, SPLITK>>(pl, ctx, s, info);
+        if (pl.pre) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 0, false, false, 4, true>>(pl, ctx, s, info);
+    if (pl.taps) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 2, SPLITK>>(pl, ctx, s, info);
+    if (pl.conv) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 1, SPLITK>>(pl, ctx, s, info);
+    return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 0, SPLITK>>(pl, ctx, s, info);
 }
 size_t plan_ckpt_bytes(const MatPlan &pl);  // gemm.hip
 // the instantiation that can leave a tile between two K-steps, when the caller brought a workspace big enough for it
 template <typename T, int TILE, int STAGES>
 static int pipe_case_ckpt(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
     if (!(ctx && ctx->ckpt && ctx->ckpt_bytes >= plan_ckpt_bytes(pl))) return pipe_case<T, TILE, STAGES, false>(pl, ctx, s, info);
-    if (pl.conv) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, true, false, true>>(pl, ctx, s, info);
-    return launch_mat<PipeKernel<T, TILE, TILE, STAGES, false, false, true>>(pl, ctx, s, info);
+    if (pl.taps) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 2, false, true>>(pl, ctx, s, info);
+    if (pl.conv) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 1, false, true>>(pl, ctx, s, info);
+    return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 0, false, true>>(pl, ctx, s, info);
 }
 
 // Ring depth of a wide body: three stages, four for the GEMM form of the 32 x 32 tile on 16 wavefronts (a

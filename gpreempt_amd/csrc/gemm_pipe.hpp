@@ -134,12 +134,15 @@ struct NoneAsked { __device__ __forceinline__ void operator()() const {} };
 // NWAVES: wavefronts per workgroup.  With eight (two per SIMD, 128 accumulator registers each) the
 // second wavefront of a SIMD covers the first one's barrier, vmcnt and LDS waits, and each wavefront
 // issues half of a stage's loads: measured 5-8 % faster than four on the 256 x 256 tile.
+// CONV: 1: a convolution; 2: one whose K-steps lie within a filter tap and whose operands fit buffers of 2 GB, of at most 32 taps
+// (a load is then a bit test, a select and the stage's uniform offset, where pointers of 64 bits were rebuilt at every tap and advanced at every
+// step: VGG-16 b16 fp16 1432 -> 1340 us, b8 907 -> 857, ResNet-50 b16 fp16 965 -> 947; 64 x 64 bodies 100 -> 72 registers).
 // PRE: the rows of A go through a scale, shift and ReLU first (gemm_pre.hpp).
-template <typename T, int BM, int BN, int STAGES, bool CONV, bool SPLITK, bool CKPT = false, int NWAVES = 4, bool PRE = false>
+template <typename T, int BM, int BN, int STAGES, int CONV, bool SPLITK, bool CKPT = false, int NWAVES = 4, bool PRE = false>
 struct PipeKernel {
     using elem = T;
     static constexpr int bm = BM, bn = BN;
-    static constexpr bool conv = CONV, pre = PRE, window = false;
+    static constexpr bool conv = CONV != 0, pre = PRE, window = false, TAPS = CONV == 2;
     static_assert(!PRE || (!CONV && !CKPT), "GEMM rows only");
     static constexpr int VEC = Elem<T>::VEC;
     static constexpr int WAVES = NWAVES, NT = WAVES * 64;
@@ -224,6 +227,8 @@ struct PipeKernel {
         const int a_row0 = m0 + wave * A_PW * 8 + rig, b_row0 = n0 + wave * B_PW * 8 + rig;
         const T *a_org[CONV ? A_PW : 1];         // CONV: the slot's window origin (may lie outside the image)
         int a_h0[CONV ? A_PW : 1], a_w0[CONV ? A_PW : 1];
+        unsigned a_off[CONV == 1 ? 1 : A_PW], b_off[B_PW];
+        unsigned a_taps[TAPS ? A_PW : 1];        // bit t: tap t of the slot's window is inside the image
         if (CONV) {
             const int hw = g.Ho * g.Wo;
             const bool small = g.M < kSmallDivLimit;
@@ -234,7 +239,10 @@ struct PipeKernel {
                 int n = small ? small_div(mm, hw, g.rcp_hw) : mm / hw, rem = mm - n * hw;
                 int ho = small ? small_div(rem, g.Wo, g.rcp_wo) : rem / g.Wo, wo = rem - ho * g.Wo;
                 a_h0[j] = ho * g.sh - g.ph; a_w0[j] = wo * g.sw - g.pw;
-                a_org[j] = A + ((long)n * g.H * g.W + (long)a_h0[j] * g.W + a_w0[j]) * g.lda;
+                if constexpr (TAPS) {  // (offsets count from the window of output pixel (0, 0), which lies in front of the image by the padding)
+                    a_off[j] = ((unsigned)((n * g.H + ho * g.sh) * g.W + wo * g.sw) * (unsigned)g.lda + (unsigned)(chunk_of(wave * A_PW + j) * VEC)) * (unsigned)sizeof(T);
+                    a_taps[j] = m < g.M ? window_tap_mask(a_h0[j], a_w0[j], g.H, g.W, g.R, g.S) : 0u;
+                } else a_org[j] = A + ((long)n * g.H * g.W + (long)a_h0[j] * g.W + a_w0[j]) * g.lda;
             }
         }
         // GEMM rows of A and B: bytes from the tile's first row, kBufferEnd for a row past the last one; a load is this, the stage's
@@ -244,8 +252,7 @@ struct PipeKernel {
         // turn: 8192^3 bf16 with checkpoints 981 -> 945 us, 4096^3 fp32 1098 -> 1016, 6000 x 5000 x 2048 fp16 152 -> 146.
         // (`near`: the tile's rows lie within a descriptor's 2 GB.  Otherwise an address of 64 bits is worked out for every load.)
         const long far = (long)kBufferEnd / (long)sizeof(T) - g.K;
-        const bool near = (CONV || (long)BM * g.lda <= far) && (long)BN * g.ldb <= far;
-        unsigned a_off[CONV ? 1 : A_PW], b_off[B_PW];
+        const bool near = TAPS || ((CONV || (long)BM * g.lda <= far) && (long)BN * g.ldb <= far);
         if (!CONV) {
 #pragma unroll
             for (int j = 0; j < (CONV ? 1 : A_PW); ++j)
@@ -254,8 +261,8 @@ struct PipeKernel {
 #pragma unroll
         for (int j = 0; j < B_PW; ++j)
             b_off[j] = b_row0 + j * 8 < g.N ? near ? ((unsigned)(b_row0 - n0 + j * 8) * (unsigned)g.ldb + (unsigned)(chunk_of(wave * B_PW + j) * VEC)) * (unsigned)sizeof(T) : 0u : kBufferEnd;
-        const u32x4 rsrc_a = buffer_of(CONV ? A : A + (long)m0 * g.lda), rsrc_b = buffer_of(B + (long)n0 * g.ldb);
-        const bool conv_fast = CONV && (g.Cin % BK == 0);  // a K-step never straddles a filter tap
+        const u32x4 rsrc_a = buffer_of(CONV ? A - (long)(g.ph * g.W + g.pw) * g.lda : A + (long)m0 * g.lda), rsrc_b = buffer_of(B + (long)n0 * g.ldb);
+        const bool conv_fast = TAPS || (CONV && (g.Cin % BK == 0));  // a K-step never straddles a filter tap
         // Running source pointers of a convolution's pixels.  Within one filter tap a slot's address only advances by BK elements
         // per stage, so it is kept and bumped instead of rebuilt: a wave has one instruction stream, and twenty address
         // instructions per load were more issue time than the MFMAs they feed.  `inc` is 0 for a slot parked on the zero page.
@@ -268,15 +275,16 @@ struct PipeKernel {
 
         // Loads of one stage: slot l < A_PW is an A slot, the rest are B slots.  `StageAddr` holds
         // the wave-uniform part, computed once per stage.
-        struct StageAddr { unsigned sbase, sbase_poll, k_bytes; int k0, r_u, s_u, tap_off; bool new_tap, first; };
+        struct StageAddr { unsigned sbase, sbase_poll, k_bytes, tap_bytes; int k0, tap, r_u, s_u, tap_off; bool new_tap, first; };
         // Stages are fetched in increasing order, so the filter tap (r, s) and channel offset of
         // the next stage advance incrementally instead of being divided out of k every time.
-        int nx_r = 0, nx_s = 0, nx_ci = 0;
+        int nx_r = 0, nx_s = 0, nx_ci = 0, nx_tap = 0;
         if (CKPT && CONV && kt0 > 0 && conv_fast) {  // a tile that is continued starts at K-step kt0
             const int k = kt0 * BK, rs = k / g.Cin;
             nx_ci = k - rs * g.Cin;
             nx_r = rs / g.S;
             nx_s = rs - nx_r * g.S;
+            nx_tap = rs;
         }
         auto stage_addr = [&](int kt) {
             StageAddr sa;
@@ -286,12 +294,14 @@ struct PipeKernel {
             sa.k_bytes = (unsigned)__builtin_amdgcn_readfirstlane(sa.k0 * (int)sizeof(T));
             sa.r_u = nx_r; sa.s_u = nx_s;
             sa.tap_off = (nx_r * g.W + nx_s) * (int)g.lda + nx_ci;  // elements from the window origin
+            if constexpr (TAPS) { sa.tap = nx_tap; sa.tap_bytes = (unsigned)__builtin_amdgcn_readfirstlane(sa.tap_off * (int)sizeof(T)); }
             sa.first = kt == kt0;                  // first stage fetched for this tile (or its continuation)
             sa.new_tap = sa.first || nx_ci == 0;   // the running conv pointers have to be rebuilt
             if (conv_fast) {
                 nx_ci += BK;
                 if (nx_ci >= g.Cin) {
                     nx_ci = 0;
+                    ++nx_tap;
                     if (++nx_s == g.S) { nx_s = 0; ++nx_r; }
                 }
             }
@@ -316,6 +326,10 @@ struct PipeKernel {
                 const int j = l;
                 const int kc = chunk_of(wave * A_PW + j) * VEC;
                 const T *src;
+                if constexpr (TAPS) {
+                    load_lds16_buffer(rsrc_a, a_taps[j] >> sa.tap & 1u ? a_off[j] : kBufferEnd, sa.tap_bytes, sa.sbase + (unsigned)((wave * A_PW + j) * 8 * RB));
+                    return;
+                }
                 if (CONV) {
                     const int jj = CONV ? j : 0;
                     if (__builtin_expect(conv_fast, 1)) {

@@ -52,3 +52,31 @@ def test_far_rows(gp, dtype_name, tile, variant, K, far_operand, outside):
         gp.launch("gp_launch_gemm", p, st.ctx(fresh=2))
         sync(gp)
         assert np.array_equal(out.download(), want)
+
+
+@pytest.mark.parametrize("dtype_name,N,H,W,Cin,Cout,R,stride,pad,tile,variant", [
+    ("f16", 2, 9, 11, 64, 70, 3, 1, 1, 64, "MAT_PIPE"), ("bf16", 3, 8, 7, 128, 133, 3, 2, 1, 128, "MAT_PIPE"), ("f32", 2, 7, 9, 32, 64, 5, 1, 2, 64, "MAT_PIPE"),
+    ("f16", 1, 12, 12, 192, 40, 1, 2, 0, 64, "MAT_PIPE_SPLITK"), ("f16", 2, 9, 5, 128, 36, 3, 1, 0, 32, "MAT_PIPE_SPLITK"), ("f32", 3, 13, 3, 64, 130, 3, 1, 1, 128, "MAT_PIPE")])
+def test_far_pixels(gp, dtype_name, N, H, W, Cin, Cout, R, stride, pad, tile, variant):
+    """a convolution whose K-steps lie within a tap: its form for buffers of 2 GB, and the general one behind pixels that span more"""
+    dtype, es = gp.DTYPE_BY_NAME[dtype_name], 4 if dtype_name == "f32" else 2
+    rng = np.random.default_rng(H * Cin + R)
+    x, w = rng.uniform(-1, 1, (N, H, W, Cin)).astype(np.float32), rng.uniform(-1, 1, (Cout, R, R, Cin)).astype(np.float32)
+    dx, dw, db = (gp.DevBuf.from_array(v, dtype) for v in (x, w, rng.uniform(-1, 1, Cout).astype(np.float32)))
+    Ho, Wo = (H + 2 * pad - R) // stride + 1, (W + 2 * pad - R) // stride + 1
+    out = gp.DevBuf(N * Ho * Wo * Cout * es)
+    p = gp.ConvParams(dtype=dtype, N=N, H=H, W=W, Cin=Cin, Cout=Cout, R=R, S=R, stride_h=stride, stride_w=stride, pad_h=pad, pad_w=pad, in_=dx.ptr, in_pix_stride=Cin,
+                      weight=dw.ptr, bias=db.ptr, out=out.ptr, out_pix_stride=Cout, act=gp.ACT_RELU, tile_m=tile, tile_n=tile, variant=getattr(gp, variant))
+
+    def bits():
+        out.fill32(0x7FC00000)
+        gp.launch("gp_launch_conv2d", p)
+        sync(gp)
+        return out.download().copy()
+
+    packed = bits()
+    stride_elems = ((1 << 31) // es // (N * H * W) // 8 + 1) * 8
+    rows = gp.to_storage(x, dtype).reshape(N * H * W, Cin).view(np.uint8)
+    far = spread(gp, list(rows), stride_elems * es)
+    p.in_, p.in_pix_stride = far.ptr, stride_elems
+    assert np.array_equal(bits(), packed)

@@ -158,8 +158,8 @@ static int choose_body(MatPlan *pl, int tile, int tile_n, int variant) {
     pl->sx = (g.N + tn - 1) / tn;
     pl->sy = (g.M + t - 1) / t;
     pl->lds_bytes = body_lds_bytes(body, pl->dtype);
-    // (what the pipelined bodies' form for whole taps assumes)
-    pl->taps = pl->conv && g.Cin % wide_bk == 0 && wide_ok;
+    // (what the 16-bit pipelined bodies' form for whole taps assumes)
+    pl->taps = pl->conv && pl->dtype != GP_F32 && g.Cin % wide_bk == 0 && wide_ok;
     // A convolution whose tiles' input windows are runs of consecutive pixels that fit in LDS fetches them once (gemm_window.hpp; where the
     // launcher picks the body itself; 16-bit, fp32 being bound by its arithmetic; 32 x 32 tiles: with 64 x 32 the four multiplying wavefronts,
     // which work out where a lane's row lies, are what a stage waits for, 0.76 us for the gather's 0.53, ResNet-152 b8 1530 -> 1560).

@@ -163,7 +163,8 @@ template <typename T, int TILE, int STAGES, bool SPLITK>
 static int pipe_case(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
     if constexpr (TILE == 64 && !SPLITK)
         if (pl.pre) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 0, false, false, 4, true>>(pl, ctx, s, info);
-    if (pl.taps) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 2, SPLITK>>(pl, ctx, s, info);
+    if constexpr (sizeof(T) == 2)
+        if (pl.taps) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 2, SPLITK>>(pl, ctx, s, info);
     if (pl.conv) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 1, SPLITK>>(pl, ctx, s, info);
     return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 0, SPLITK>>(pl, ctx, s, info);
 }
@@ -172,7 +173,8 @@ size_t plan_ckpt_bytes(const MatPlan &pl);  // gemm.hip
 template <typename T, int TILE, int STAGES>
 static int pipe_case_ckpt(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
     if (!(ctx && ctx->ckpt && ctx->ckpt_bytes >= plan_ckpt_bytes(pl))) return pipe_case<T, TILE, STAGES, false>(pl, ctx, s, info);
-    if (pl.taps) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 2, false, true>>(pl, ctx, s, info);
+    if constexpr (sizeof(T) == 2)
+        if (pl.taps) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 2, false, true>>(pl, ctx, s, info);
     if (pl.conv) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 1, false, true>>(pl, ctx, s, info);
     return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 0, false, true>>(pl, ctx, s, info);
 }

@@ -143,7 +143,12 @@ struct PipeKernel {
     using elem = T;
     static constexpr int bm = BM, bn = BN;
     static constexpr bool conv = CONV != 0, pre = PRE, window = false, TAPS = CONV == 2;
-    static_assert(!PRE || (!CONV && !CKPT), "GEMM rows only");
+    // Whether GEMM rows are fetched through descriptors (see `near` below).  Not by the fp32 bodies of 128 x 128 and less: their MFMAs
+    // take eight times as long, a load's instructions hide behind them, and with two workgroups to a compute unit that now advance
+    // in step, a last round of few tiles finds both places of a unit free at once and doubles up there: 5175 x 1833 x 1696
+    // plain 333 -> 428 us, 2048 x 2560 x 4096 preemptible 605 -> 649.  Nor by the 16-bit GEMM of 128 x 128: 3 % faster on 5175 x 1833 x
+    // 1696, but 2048 x 2560 x 4096 preemptible 121 -> 130.
+    static constexpr bool DESC = TAPS || BM == 256 || (sizeof(T) == 2 && BM < 128);
     static constexpr int VEC = Elem<T>::VEC;
     static constexpr int WAVES = NWAVES, NT = WAVES * 64;
     static constexpr int RB = 128;                        // row bytes in LDS
@@ -252,26 +257,37 @@ struct PipeKernel {
         // turn: 8192^3 bf16 with checkpoints 981 -> 945 us, 4096^3 fp32 1098 -> 1016, 6000 x 5000 x 2048 fp16 152 -> 146.
         // (`near`: the tile's rows lie within a descriptor's 2 GB.  Otherwise an address of 64 bits is worked out for every load.)
         const long far = (long)kBufferEnd / (long)sizeof(T) - g.K;
-        const bool near = TAPS || ((CONV || (long)BM * g.lda <= far) && (long)BN * g.ldb <= far);
-        if (!CONV) {
+        const bool near = TAPS || !DESC || ((CONV || (long)BM * g.lda <= far) && (long)BN * g.ldb <= far);
+        if (!CONV && DESC) {
 #pragma unroll
             for (int j = 0; j < (CONV ? 1 : A_PW); ++j)
                 a_off[j] = a_row0 + j * 8 < g.M ? near ? ((unsigned)(a_row0 - m0 + j * 8) * (unsigned)g.lda + (unsigned)(chunk_of(wave * A_PW + j) * VEC)) * (unsigned)sizeof(T) : 0u : kBufferEnd;
         }
 #pragma unroll
-        for (int j = 0; j < B_PW; ++j)
+        for (int j = 0; j < (DESC ? B_PW : 0); ++j)
             b_off[j] = b_row0 + j * 8 < g.N ? near ? ((unsigned)(b_row0 - n0 + j * 8) * (unsigned)g.ldb + (unsigned)(chunk_of(wave * B_PW + j) * VEC)) * (unsigned)sizeof(T) : 0u : kBufferEnd;
         const u32x4 rsrc_a = buffer_of(CONV ? A - (long)(g.ph * g.W + g.pw) * g.lda : A + (long)m0 * g.lda), rsrc_b = buffer_of(B + (long)n0 * g.ldb);
         const bool conv_fast = TAPS || (CONV && (g.Cin % BK == 0));  // a K-step never straddles a filter tap
-        // Running source pointers of a convolution's pixels.  Within one filter tap a slot's address only advances by BK elements
-        // per stage, so it is kept and bumped instead of rebuilt: a wave has one instruction stream, and twenty address
-        // instructions per load were more issue time than the MFMAs they feed.  `inc` is 0 for a slot parked on the zero page.
-        const T *a_cur[CONV ? A_PW : 1];
-        int a_inc[CONV ? A_PW : 1];
-        if (CONV) {
-#pragma unroll
-            for (int j = 0; j < (CONV ? A_PW : 1); ++j) { a_cur[j] = zero; a_inc[j] = 0; }
+        // Pointers with the lane's chunk already added, one per parity of the slot number j: a load's address is this plus a
+        // wave-uniform offset.
+        const T *a_par[2] = {nullptr, nullptr}, *b_par[2] = {nullptr, nullptr};
+        if (!DESC) {
+            if (!CONV)
+                for (int q = 0; q < 2; ++q) a_par[q] = A + (long)a_row0 * g.lda + chunk_of(wave * A_PW + q) * VEC;
+            for (int q = 0; q < 2; ++q) b_par[q] = B + (long)b_row0 * g.ldb + chunk_of(wave * B_PW + q) * VEC;
         }
+        const bool k_full = g.K % BK == 0;                 // no K-chunk of any stage lies past K
+        // Running source pointers.  Within one filter tap (conv) or along K (weights, GEMM rows) a slot's address only advances by
+        // BK elements per stage, so it is kept and bumped instead of rebuilt: a wave has one instruction stream, and twenty
+        // address instructions per load were more issue time than the MFMAs they feed.  `inc` is 0 for a slot parked on the zero
+        // page.  (Only bodies with few slots keep them for the B / GEMM-A side: registers.)
+        constexpr bool INCR = A_PW + B_PW <= 8;
+        const T *a_cur[A_PW], *b_cur[B_PW];
+        int a_inc[A_PW], b_inc[B_PW];
+#pragma unroll
+        for (int j = 0; j < A_PW; ++j) { a_cur[j] = zero; a_inc[j] = 0; }
+#pragma unroll
+        for (int j = 0; j < B_PW; ++j) { b_cur[j] = zero; b_inc[j] = 0; }
 
         // Loads of one stage: slot l < A_PW is an A slot, the rest are B slots.  `StageAddr` holds
         // the wave-uniform part, computed once per stage.
@@ -332,8 +348,8 @@ struct PipeKernel {
                 }
                 if (CONV) {
                     const int jj = CONV ? j : 0;
-                    if (__builtin_expect(conv_fast, 1)) {
-                        if (__builtin_expect(sa.new_tap, 0)) {  // (uniform) rebuild: bounds of the tap, pointer or zero page
+                    if (conv_fast) {
+                        if (sa.new_tap) {  // (uniform) rebuild: bounds of the tap, pointer or zero page
                             const bool ok = (a_row0 + j * 8 < g.M) & ((unsigned)(a_h0[jj] + sa.r_u) < (unsigned)g.H) &
                                             ((unsigned)(a_w0[jj] + sa.s_u) < (unsigned)g.W);
                             a_cur[j] = ok ? a_org[jj] + (sa.tap_off + kc) : zero;
@@ -351,6 +367,18 @@ struct PipeKernel {
                                         ((unsigned)(a_w0[jj] + s2) < (unsigned)g.W);
                         src = ok ? a_org[jj] + off : zero;
                     }
+                } else if (!DESC && INCR && k_full) {
+                    if (sa.first) {
+                        const bool ok = a_row0 + j * 8 < g.M;
+                        a_cur[j] = ok ? a_par[j & 1] + ((long)(j * 8) * g.lda + sa.k0) : zero;
+                        a_inc[j] = ok ? BK : 0;
+                    } else {
+                        a_cur[j] += a_inc[j];
+                    }
+                    src = a_cur[j];
+                } else if (!DESC) {
+                    const bool ok = (a_row0 + j * 8 < g.M) & (k_full | (sa.k0 + kc < g.K));
+                    src = ok ? a_par[j & 1] + ((long)(j * 8) * g.lda + sa.k0) : zero;
                 } else {
                     const int jj = CONV ? 0 : j;
                     const bool ok = sa.k0 + kc < g.K;
@@ -365,12 +393,26 @@ struct PipeKernel {
                 const int j = l - A_PW;
                 const int kc = chunk_of(wave * B_PW + j) * VEC;
                 const T *src;
-                const bool ok = sa.k0 + kc < g.K;
-                if (__builtin_expect(near, 1)) {
-                    load_lds16_buffer(rsrc_b, ok ? b_off[j] : kBufferEnd, sa.k_bytes, sa.sbase + (unsigned)(A_BYTES + (wave * B_PW + j) * 8 * RB));
-                    return;
+                if (!DESC && INCR && k_full) {
+                    if (sa.first) {
+                        const bool ok = b_row0 + j * 8 < g.N;
+                        b_cur[j] = ok ? b_par[j & 1] + ((long)(j * 8) * g.ldb + sa.k0) : zero;
+                        b_inc[j] = ok ? BK : 0;
+                    } else {
+                        b_cur[j] += b_inc[j];
+                    }
+                    src = b_cur[j];
+                } else if (!DESC) {
+                    const bool ok = (b_row0 + j * 8 < g.N) & (k_full | (sa.k0 + kc < g.K));
+                    src = ok ? b_par[j & 1] + ((long)(j * 8) * g.ldb + sa.k0) : zero;
+                } else {
+                    const bool ok = sa.k0 + kc < g.K;
+                    if (__builtin_expect(near, 1)) {
+                        load_lds16_buffer(rsrc_b, ok ? b_off[j] : kBufferEnd, sa.k_bytes, sa.sbase + (unsigned)(A_BYTES + (wave * B_PW + j) * 8 * RB));
+                        return;
+                    }
+                    src = ok && b_off[j] != kBufferEnd ? B + ((long)(b_row0 + j * 8) * g.ldb + (sa.k0 + kc)) : zero;
                 }
-                src = ok && b_off[j] != kBufferEnd ? B + ((long)(b_row0 + j * 8) * g.ldb + (sa.k0 + kc)) : zero;
                 load_lds16(src, sa.sbase + (unsigned)(A_BYTES + (wave * B_PW + j) * 8 * RB));
             }
         };

@@ -1,4 +1,5 @@
-"""The pipelined bodies fetch through descriptors of 2 GB that begin at a tile's first row, and work out addresses of 64 bits where a
+"""The pipelined bodies fetch through descriptors of 2 GB (256 x 256 tiles, 16-bit tiles of 64 x 64 and less, 16-bit convolutions of whole
+taps; the others by pointers) that begin at a tile's first row, and work out addresses of 64 bits where a
 tile's rows span more.  Rows just inside and just outside of that span, of either operand, give the bits of packed rows, and
 those the oracle's values; K with a remainder, and tiles with rows and columns past the last one."""
 import numpy as np

@@ -107,12 +107,13 @@ static int choose_body(MatPlan *pl, int tile, int tile_n, int variant) {
     const MatArgs &g = pl->g;
     auto tiles = [&](int t) { return (long)((g.M + t - 1) / t) * ((g.N + t - 1) / t) * pl->batch; };
     const long cus = device_cus();
-    // both operands K-contiguous; a convolution, whose A operand is gathered, when a K-block never straddles
-    // two filter taps and a bit per tap fits a word
+    // both operands K-contiguous; a convolution, whose A operand is gathered, when a bit per tap fits a word and, where K-blocks
+    // straddle two filter taps, a lane can find its tap by multiplication (inverse_of is 0 from (K + 1) * Cin = 2^32 on)
     const int wide_bk = pl->dtype == GP_F32 ? 32 : 64;
+    const bool whole_taps = pl->conv && g.Cin % wide_bk == 0;
+    const bool wide_taps = !pl->conv || (g.K / g.Cin <= 32 && g.S < 32 && (whole_taps || (g.inv_cin && g.inv_s)));
     // (a caller that asks for a wide body gets one only where no block straddles two taps, as ever)
-    const bool wide_taps = !pl->conv || (g.K / g.Cin <= 32 && g.S < 32 && g.inv_cin && g.inv_s);
-    const bool wide_shape = !pl->b_kn && wide_taps && (!pl->conv || g.Cin % wide_bk == 0);
+    const bool wide_shape = !pl->b_kn && wide_taps && (!pl->conv || whole_taps);
     const bool wide_ok = !pl->b_kn && wide_taps && buffer_ok(g, pl->conv, pl->dtype);
     int body = -1;
     if (g.ln_gamma) body = MB_LNWIDE32x64_16;  // (plan_gemm has checked that the shape fits)
@@ -159,7 +160,7 @@ static int choose_body(MatPlan *pl, int tile, int tile_n, int variant) {
     pl->sy = (g.M + t - 1) / t;
     pl->lds_bytes = body_lds_bytes(body, pl->dtype);
     // (what the 16-bit pipelined bodies' form for whole taps assumes)
-    pl->taps = pl->conv && pl->dtype != GP_F32 && g.Cin % wide_bk == 0 && wide_ok;
+    pl->taps = whole_taps && pl->dtype != GP_F32 && wide_ok;
     // A convolution whose tiles' input windows are runs of consecutive pixels that fit in LDS fetches them once (gemm_window.hpp; where the
     // launcher picks the body itself; 16-bit, fp32 being bound by its arithmetic; 32 x 32 tiles: with 64 x 32 the four multiplying wavefronts,
     // which work out where a lane's row lies, are what a stage waits for, 0.76 us for the gather's 0.53, ResNet-152 b8 1530 -> 1560).

@@ -41,6 +41,17 @@ def test_wide_convolution_over_two_gigabytes_of_images(images, rc):
     assert _rc(p) == rc
 
 
+@pytest.mark.parametrize("dtype", [gp.F32, gp.F16, gp.BF16])
+@pytest.mark.parametrize("channels", [21760, 21888, 65536])
+def test_wide_convolution_of_any_number_of_channels(dtype, channels):
+    """(K + 1) * Cin passes 2^32 between the first two: only blocks that straddle taps divide by the channels"""
+    p = gp.ConvParams(dtype=dtype, N=1, H=5, W=5, Cin=channels, Cout=32, R=3, S=3, stride_h=1, stride_w=1, pad_h=1, pad_w=1, in_=4096, in_pix_stride=channels,
+                      weight=8192, out=12288, out_pix_stride=32, tile_m=32, tile_n=32, variant=gp.MAT_WIDE)
+    assert _rc(p) == gp.SUCC
+    p.Cin = p.in_pix_stride = channels + 8  # blocks that straddle taps: a wide body asked for by name is refused, as ever
+    assert _rc(p) == gp.OUTOFRANGE
+
+
 @pytest.mark.parametrize("ldb", [768, 1 << 22, (1 << 24) - 8])
 def test_layernorm_prologue_over_any_number_of_rows_of_b(ldb):
     """the buffer starts at the tile's first row of B, so only a tile's rows have to fit"""

@@ -12,8 +12,8 @@
 // The scale and shift of all K channels lie behind the ring (pre_table_bytes), fetched in front of the first stage.
 //
 // Same bits as the two launches: the value is rounded to the storage type as it would be on its way through memory, and in
-// between computed as the element-wise kernels do, product and sum rounded one by one.  (In 16 bits the product of two values is
-// exact in fp32, so that one fused multiply-add is the same.)
+// between computed as the element-wise kernels do, product and sum rounded one by one.  (In fp16 the product of two values is
+// exact in fp32, so that one fused multiply-add is the same; the product of two bf16 values can leave fp32's range at either end.)
 #pragma once
 #include "elementwise_bodies.hpp"
 
@@ -25,7 +25,7 @@ inline __host__ __device__ constexpr size_t pre_max_lds(size_t ring) { return ri
 inline __host__ __device__ unsigned pre_table_bytes(int K, unsigned es) { return 2u * (((unsigned)K * es + 1023u) & ~1023u); }
 
 template <typename T> __device__ __forceinline__ out_u32x4 pre_chunk(out_u32x4 x, out_u32x4 scale, out_u32x4 shift, bool relu) {
-#pragma clang fp contract(off)  // (fp32: product and sum are rounded one by one)
+#pragma clang fp contract(off)  // (product and sum are rounded one by one)
     constexpr int VEC = VecIO<T>::VEC;
     float v[VEC], s[VEC], t[VEC];
     VecIO<T>::unpack(x, v);
@@ -33,7 +33,7 @@ template <typename T> __device__ __forceinline__ out_u32x4 pre_chunk(out_u32x4 x
     VecIO<T>::unpack(shift, t);
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
-        if constexpr (sizeof(T) == 2) v[j] = __builtin_fmaf(v[j], s[j], t[j]);
+        if constexpr (__is_same(T, _Float16)) v[j] = __builtin_fmaf(v[j], s[j], t[j]);
         else v[j] = v[j] * s[j] + t[j];
     }
     if (relu) {

@@ -83,6 +83,24 @@ def test_one_launch_has_the_bits_of_two(gp, dt, case):
             assert not info.fixed_claims or st.counters().reshape(32, 16)[:, 0].sum() == info.total_tiles
 
 
+@pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("case", [(1, 9, 72, 36, 96), (4, 14, 1024, 128, 1792)], ids=["64x64", "32x32"])
+def test_products_at_the_ends_of_the_range_round_as_in_two_launches(gp, dt, case):
+    """products beyond the largest float whose sum with the shift is not (bf16, fp32), and ones below the smallest normal float"""
+    e, c, mid, out, keep = setup(gp, dt, case, gp.ACT_NONE)
+    dtype, (images, H, Cin, Cout, wide) = gp.DTYPE_BY_NAME[dt], case
+    big, tiny = (2.0 ** 15, 2.0 ** -24) if dt == "f16" else (2.0 ** 64, 1.5 * 2.0 ** -70)
+    x, scale, shift = np.ones((images * H * H, wide), np.float32), np.ones(Cin, np.float32), np.zeros(Cin, np.float32)
+    x[0::2, 0], x[1::2, 0], scale[0], shift[0] = 1.5 * big, 0.0, big, -1.984375 * 2.0 ** (15 if dt == "f16" else 127)
+    x[:, 2:6], scale[2:6], shift[2:6] = tiny * 1.0078125, tiny * 1.0078125, np.array([0, 1, -1, 8], np.float32) * 2.0 ** (-24 if dt == "f16" else -133)
+    for buf, v in zip(keep, (x, scale, shift, np.eye(Cout, Cin, dtype=np.float32), np.zeros(Cout, np.float32))):
+        buf.upload(gp.to_storage(v, dtype))
+    c.act = gp.ACT_NONE
+    want = two_launches(gp, e, c, mid, out)
+    fused(gp, e, c)
+    assert np.array_equal(out.download(), want)
+
+
 def test_what_one_launch_does_not_take(gp):
     """other activations, an addend, another input, a window, a table that does not fit, a body that does not take it"""
     e, c, mid, out, keep = setup(gp, "f16", (4, 14, 1024, 128, 1792), gp.ACT_RELU)

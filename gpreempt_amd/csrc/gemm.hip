@@ -311,6 +311,7 @@ int plan_eltwise_conv2d(const gp_eltwise_params *e, const gp_conv_params *c, Mat
     GP_REQUIRE(e->scale && e->shift && !e->b && (e->act == GP_ACT_NONE || e->act == GP_ACT_RELU), "eltwise + conv: a scale, a shift and possibly a ReLU");
     GP_REQUIRE(e->dtype == c->dtype && c->in == e->out && c->in_pix_stride == e->out_stride && c->Cin == e->cols && (long)c->N * c->H * c->W == e->rows, "eltwise + conv: the convolution does not read the layer's output");
     GP_REQUIRE(c->out != e->a && c->residual != e->out, "eltwise + conv: overlapping operands");
+    GP_REQUIRE(e->a_stride >= 0, "eltwise + conv: the matrix bodies count a row's bytes from the first one up");
     MatPlan &pl = *out;
     MatArgs alone = pl.g;
     alone.A = e->a; alone.lda = e->a_stride;

@@ -16,6 +16,13 @@ namespace gp {
 void set_error(const char *fmt, ...);
 int device_cus();
 
+// For a question whose answer may be no (gp_*_supported): the text of the last error stays what it was.
+struct KeepLastError {
+    char text[512];
+    KeepLastError() { snprintf(text, sizeof(text), "%s", gp_last_error()); }
+    ~KeepLastError() { set_error("%s", text); }
+};
+
 #define GP_HIP(call)                                                                           \
     do {                                                                                       \
         hipError_t e_ = (call);                                                                \

@@ -209,6 +209,7 @@ extern "C" int gp_gemm_ln_supported(const gp_gemm_params *p) {
     q.ln_gamma = q.ln_beta = nullptr; q.ln_out = nullptr;
     q.tile_m = q.tile_n = q.variant = 0;
     MatPlan pl;
+    KeepLastError keep;
     if (!q.A || !q.B || !q.C || plan_gemm(&q, &pl) != GP_SUCC) return 0;
     return (is_wide_body(pl.body) || pl.body == MB_PIPE64_SK || pl.body == MB_PIPE32_SK) ? 1 : 0;
 }
@@ -348,6 +349,7 @@ using namespace gp;
 
 extern "C" int gp_conv2d_group_supported(const gp_conv_params *p, int n) {
     MatPlan pl[kGroupMax];
+    KeepLastError keep;
     return plan_conv2d_group(p, n, pl) == GP_SUCC ? 1 : 0;
 }
 extern "C" int gp_launch_conv2d_group(const gp_conv_params *p, int n, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
@@ -363,6 +365,7 @@ extern "C" int gp_launch_conv2d_group(const gp_conv_params *p, int n, const gp_p
 
 extern "C" int gp_eltwise_conv2d_supported(const gp_eltwise_params *e, const gp_conv_params *c) {
     MatPlan pl;
+    KeepLastError keep;
     return plan_eltwise_conv2d(e, c, &pl) == GP_SUCC ? 1 : 0;
 }
 extern "C" int gp_launch_eltwise_conv2d(const gp_eltwise_params *e, const gp_conv_params *c, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {

@@ -17,3 +17,22 @@ def _scaled(dtype, a_stride, images=4, H=14, Cin=1024, Cout=128):
 def test_a_scale_and_shift_in_front_of_a_convolution_takes_rows_that_do_not_run_backwards(dtype, a_stride, ok):
     """the element-wise kernel alone takes any distance between rows; the matrix bodies' offsets are unsigned"""
     assert _scaled(dtype, a_stride) == ok
+
+
+def _conv(Cin=1280, Cout=192, H=8, dtype=gp.F16, R=1, S=1):
+    return gp.ConvParams(dtype=dtype, N=1, H=H, W=H, Cin=Cin, Cout=Cout, R=R, S=S, stride_h=1, stride_w=1, pad_h=R // 2, pad_w=S // 2, in_=1 << 30, in_pix_stride=Cin, weight=1 << 16,
+                         out=1 << 31, out_pix_stride=Cout)
+
+
+def test_a_question_leaves_the_last_error_as_it_was():
+    lib = C.CDLL(gp.LIB_PATH)
+    lib.gp_last_error.restype = C.c_char_p
+    assert lib.gp_launch_conv2d(None, None, None, None) == gp.OUTOFRANGE
+    said = lib.gp_last_error()
+    assert said
+    assert _scaled(gp.F16, -1024) == 0
+    two = (gp.ConvParams * 2)(_conv(), _conv(dtype=gp.F32))
+    assert lib.gp_conv2d_group_supported(two, 2) == 0 and lib.gp_conv2d_group_supported(two, 5) == 0
+    g = gp.GemmParams(dtype=gp.F16, M=128, N=768, K=768, A=4096, lda=768, B=8200, ldb=768, b_is_nk=1, C=12288, ldc=768, alpha=1.0, batch=1)
+    assert lib.gp_gemm_ln_supported(C.byref(g)) == 0  # B is not aligned
+    assert lib.gp_last_error() == said

@@ -16,6 +16,7 @@ GROUPS = [
     [(17, 17, 192, 320, 3, 3, 2, 0, 0), (17, 17, 192, 192, 1, 7, 1, 0, 3)],
     [(8, 8, 384, 384, 1, 3, 1, 0, 1), (8, 8, 384, 384, 3, 1, 1, 1, 0)],
     [(9, 9, 104, 50, 3, 3, 1, 1, 1), (9, 9, 1024, 40, 1, 1, 1, 0, 0), (9, 9, 56, 33, 5, 5, 1, 2, 2)],
+    [(7, 7, 8784, 40, 1, 1, 1, 0, 0), (7, 7, 968, 33, 3, 3, 1, 1, 1)],  # the deepest that fp32 takes
 ]
 
 
@@ -89,7 +90,7 @@ def test_a_group_has_the_bits_of_its_members(gp, dt, images, group):
 
 
 def test_the_groups_of_the_test_above_are_groups(gp):
-    for dt, group in (("f16", 0), ("f16", 1), ("f16", 2), ("bf16", 3), ("f32", 4), ("f32", 5)):
+    for dt, group in (("f16", 0), ("f16", 1), ("f16", 2), ("bf16", 3), ("f32", 4), ("f32", 5), ("f32", 6), ("f16", 6)):
         params, outs, keep = members(gp, dt, GROUPS[group])
         assert gp.lib().gp_conv2d_group_supported(params, len(GROUPS[group])) == 1, (dt, group)
     params, outs, keep = members(gp, "f16", GROUPS[2])

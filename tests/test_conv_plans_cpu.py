@@ -1,5 +1,8 @@
 """Which convolutions the planner takes into one launch with others (no GPU: the plan alone)."""
 import ctypes as C
+import os
+import subprocess
+import sys
 
 import pytest
 
@@ -36,3 +39,16 @@ def test_a_question_leaves_the_last_error_as_it_was():
     g = gp.GemmParams(dtype=gp.F16, M=128, N=768, K=768, A=4096, lda=768, B=8200, ldb=768, b_is_nk=1, C=12288, ldc=768, alpha=1.0, batch=1)
     assert lib.gp_gemm_ln_supported(C.byref(g)) == 0  # B is not aligned
     assert lib.gp_last_error() == said
+
+
+@pytest.mark.parametrize("macs,Cin,dtype,ok", [
+    ("", 2048, gp.F16, 1), ("", 17568, gp.F16, 1), ("", 17600, gp.F16, 0),  # 32 x 32 tiles: 1.8e7 from K = 17579 on
+    ("", 2048, gp.F32, 1), ("", 8784, gp.F32, 1), ("", 8800, gp.F32, 0),    # 16 x 16, eight times the weight: from 8790 on
+    ("1000000", 960, gp.F16, 1), ("1000000", 992, gp.F16, 0), ("1000000", 512, gp.F32, 0)])
+def test_a_group_takes_no_layer_whose_tiles_are_given_up_on_a_stop(macs, Cin, dtype, ok):
+    """alone such a layer looks at the stop word inside its tiles, in a group it would not (the variable is read once per process, hence the child)"""
+    code = (f"import sys; sys.path.insert(0, {os.path.dirname(os.path.abspath(__file__))!r}); import ctypes as C, test_conv_plans_cpu as t; from gpreempt_amd import capi as gp; "
+            f"print(C.CDLL(gp.LIB_PATH).gp_conv2d_group_supported((gp.ConvParams * 2)(*[t._conv({Cin}, 64, 7, {dtype})] * 2), 2))")
+    r = subprocess.run([sys.executable, "-c", code], cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))), capture_output=True, text=True, timeout=120,
+                       env={**os.environ, "GPREEMPT_LONG_TILE_MACS": macs})
+    assert r.returncode == 0 and r.stdout.strip() == str(ok), r.stdout + r.stderr

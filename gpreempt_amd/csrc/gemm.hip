@@ -325,17 +325,20 @@ int plan_eltwise_conv2d(const gp_eltwise_params *e, const gp_conv_params *c, Mat
     return GP_SUCC;
 }
 
-// Convolutions that run as one launch (gemm_group.hpp): each with the body it would get alone, which is the same for all, has sixteen
-// wavefronts and tiles too short to be given up (the group's kernel does not look at the stop word inside a tile); together no more tiles than compute units.  (Layers that fill the device alone
-// gain nothing beside each other: with up to two rounds of tiles Inception-v3 b2 fp32 takes 1167 us for 1105, b8 bf16 1227 for 1163.)
+// Convolutions that run as one launch (gemm_group.hpp): each with the body it would get alone, which is the same for all, and tiles
+// too short to be given up (the group's kernel does not look at the stop word inside a tile); together no more tiles than compute
+// units.  (Layers that fill the device alone gain nothing beside each other: with up to two rounds of tiles Inception-v3 b2 fp32 takes 1167 us
+// for 1105, b8 bf16 1227 for 1163.)  That leaves the smallest tiles of either kind: a layer gets the next larger ones (64 x 32, 32 x 16) from
+// more tiles than half of the compute units on, and two of them are too many.
+static int group_body(int dtype) { return dtype == GP_F32 ? MB_NARROW16x16 : MB_WIDE32x32_16; }
 int plan_conv2d_group(const gp_conv_params *p, int n, MatPlan *out) {
     GP_REQUIRE(p && n >= 2 && n <= kGroupMax, "conv group of %d: two to %d", n, kGroupMax);
     long total = 0;
     for (int i = 0; i < n; ++i) {
         if (int rc = plan_conv2d(p + i, out + i)) return rc;
         const MatPlan &pl = out[i];
-        GP_REQUIRE(p[i].tile_m == 0 && p[i].variant == 0 && pl.body == out[0].body && pl.dtype == out[0].dtype &&
-                       (pl.body == MB_WIDE32x32_16 || pl.body == MB_WIDE64x32_16 || is_narrow_body(pl.body)) && !tile_is_long(wide_of(pl.body)->bm, wide_of(pl.body)->bn, pl.g.K, pl.dtype),
+        GP_REQUIRE(p[i].tile_m == 0 && p[i].variant == 0 && pl.dtype == out[0].dtype && pl.body == group_body(pl.dtype) &&
+                       !tile_is_long(wide_of(pl.body)->bm, wide_of(pl.body)->bn, pl.g.K, pl.dtype),
                    "conv group: member %d has no body that runs in a group with the first one's", i);
         total += (long)pl.sx * pl.sy;
     }

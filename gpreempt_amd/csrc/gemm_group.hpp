@@ -5,7 +5,7 @@
 //
 // Structure: the tiles of the members stand one behind the other in the launch's tile order; a workgroup finds the member its tile
 // belongs to and runs that member's own body (one of the forms, GEMM, convolution, convolution whose blocks straddle taps,
-// convolution with its window in LDS, of one wide or narrow tile shape, which is all a kernel can hold), so sums and bits are those of launches of their own.
+// convolution with its window in LDS, of one tile shape, which is all a kernel can hold), so sums and bits are those of launches of their own.
 // Claims, claim counters and the kernel index are the launch's: a stop inside it resumes there.
 #pragma once
 #include "gemm_narrow.hpp"

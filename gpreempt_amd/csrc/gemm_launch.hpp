@@ -273,10 +273,8 @@ template <typename T>
 int launch_group_typed(const MatPlan *pl, int n, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
     if constexpr (sizeof(T) == 4) {
         if (pl[0].body == MB_NARROW16x16) return launch_group<NarrowKernel<16, 3, 0>, NarrowKernel<16, 3, 1>, NarrowKernel<16, 3, 2>>(pl, n, ctx, s, info);
-        if (pl[0].body == MB_NARROW32x16) return launch_group<NarrowKernel<32, 3, 0>, NarrowKernel<32, 3, 1>, NarrowKernel<32, 3, 2>>(pl, n, ctx, s, info);
     } else {
         if (pl[0].body == MB_WIDE32x32_16) return launch_group<WideK<T, 32, 32, 16, 0>, WideK<T, 32, 32, 16, 1>, WideK<T, 32, 32, 16, 2>, WindowKernel<T, 32, 32, 4>>(pl, n, ctx, s, info);
-        if (pl[0].body == MB_WIDE64x32_16) return launch_group<WideK<T, 64, 32, 16, 0>, WideK<T, 64, 32, 16, 1>, WideK<T, 64, 32, 16, 2>>(pl, n, ctx, s, info);
     }
     set_error("matrix kernel body %d does not run in groups", pl[0].body);
     return GP_FAIL;

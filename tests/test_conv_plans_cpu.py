@@ -52,3 +52,14 @@ def test_a_group_takes_no_layer_whose_tiles_are_given_up_on_a_stop(macs, Cin, dt
     r = subprocess.run([sys.executable, "-c", code], cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))), capture_output=True, text=True, timeout=120,
                        env={**os.environ, "GPREEMPT_LONG_TILE_MACS": macs})
     assert r.returncode == 0 and r.stdout.strip() == str(ok), r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("dtype,step", [(gp.F16, 32), (gp.F32, 16)])
+def test_two_layers_of_larger_tiles_are_more_than_a_group_takes(dtype, step):
+    """... whatever their shape, so that a group's kernel needs only the smallest tiles"""
+    lib = C.CDLL(gp.LIB_PATH)
+    for H in range(1, 70):
+        for columns in (1, 2, 3, 5, 8, 16, 40):
+            both = [_conv(1280, step * columns, H, dtype) for _ in range(2)]
+            tiles = -(-H * H // step) * columns  # of one of them
+            assert lib.gp_conv2d_group_supported((gp.ConvParams * 2)(*both), 2) == (1 if 2 * tiles <= 256 else 0), (H, columns)

@@ -259,7 +259,8 @@ void Model::plan_fusions() {
         mm.has_ln_gemm = true;
         ln.fused_away = true;
     }
-    // scale-shift -> pointwise convolution, where nobody else reads (or writes) what lies between the two
+    // scale-shift -> pointwise convolution, where nobody else reads (or writes) what lies between the two and what the layer reads
+    // stays as it is until the pass ends (compute_unread runs it then)
     unread_.assign(storage_infos.size(), SIZE_MAX);
     for (size_t i = 0; i + 1 < kernel_infos.size(); ++i) {
         KernelInfo &el = kernel_infos[i], &cv = kernel_infos[i + 1];
@@ -267,8 +268,10 @@ void Model::plan_fusions() {
         if (el.op != OpKind::Eltwise || cv.op != OpKind::Conv) continue;
         const size_t between = el.args_index[4], from = el.args_index[0];
         bool alone = between != from && between != cv.args_index[4] && from != cv.args_index[4] && storage_infos[between].name != "heads";
+        for (size_t slot = 1; slot < 4; ++slot) alone = alone && el.args_index[slot] != between && cv.args_index[slot] != between;
         for (size_t k = 0; k < kernel_infos.size() && alone; ++k)
             for (size_t st : kernel_infos[k].args_index) alone = alone && (st != between || k == i || k == i + 1);
+        for (size_t k = i + 1; k < kernel_infos.size() && alone; ++k) alone = !writes_operand_of(kernel_infos[k], el);
         if (!alone || gp_eltwise_conv2d_supported(&el.p.eltwise, &cv.p.conv) != 1) continue;
         cv.pre = el.p.eltwise;
         cv.has_pre = true;
@@ -305,9 +308,25 @@ bool Model::run_side_by_side(const KernelInfo &a, const KernelInfo &b) {
         if (a.args_index[slot] == ob || b.args_index[slot] == oa) return false;
     if (oa != ob) return true;
     const gp_conv_params &p = a.p.conv, &q = b.p.conv;
-    const long es = (long)get_stype_size(storage_infos[oa].stype);
-    const long pa = ((char *)p.out - (char *)storages[oa]) / es, pb = ((char *)q.out - (char *)storages[ob]) / es;
-    return p.out_pix_stride == q.out_pix_stride && pa + p.Cout <= p.out_pix_stride && pb + q.Cout <= q.out_pix_stride && (pa + p.Cout <= pb || pb + q.Cout <= pa);
+    return p.out_pix_stride == q.out_pix_stride && slices_apart(oa, p.out, p.Cout, q.out, q.Cout, p.out_pix_stride);
+}
+
+// Whether the channels [a, a + na) and [b, b + nb) of the pixels of one storage, `stride` elements each, lie apart.
+bool Model::slices_apart(size_t storage, const void *a, long na, const void *b, long nb, long stride) {
+    const long es = (long)get_stype_size(storage_infos[storage].stype);
+    const long pa = ((const char *)a - (const char *)storages[storage]) / es, pb = ((const char *)b - (const char *)storages[storage]) / es;
+    return pa + na <= stride && pb + nb <= stride && (pa + na <= pb || pb + nb <= pa);
+}
+
+// Whether kernel w writes what the scale-shift layer el reads.  (A kernel's last slot is its output.  A convolution's output
+// is told channel by channel: in a dense block they all go side by side into the buffer that every layer reads the front of.)
+bool Model::writes_operand_of(const KernelInfo &w, const KernelInfo &el) {
+    const size_t out = w.args_index.back();
+    if (w.op == OpKind::Stencil || out == SIZE_MAX) return true;
+    if (out == el.args_index[2] || out == el.args_index[3]) return true;
+    if (out != el.args_index[0]) return false;
+    const gp_eltwise_params &e = el.p.eltwise;
+    return w.op != OpKind::Conv || w.p.conv.out_pix_stride != e.a_stride || !slices_apart(out, e.a, e.cols, w.p.conv.out, w.p.conv.Cout, e.a_stride);
 }
 
 // The output of a layer that its reader's launch does itself (plan_fusions): computed for a caller that wants to see it.

@@ -240,6 +240,8 @@ private:
     Status allocate_and_bind();
     void plan_fusions();
     bool run_side_by_side(const KernelInfo &a, const KernelInfo &b);
+    bool slices_apart(size_t storage, const void *a, long na, const void *b, long nb, long stride);
+    bool writes_operand_of(const KernelInfo &w, const KernelInfo &el);
     Status compute_unread(size_t idx, GPUstream stream);
     std::vector<size_t> unread_;  // per storage: the kernel that would write it, where plan_fusions found a launch that needs no such storage
     bool fuse_launches_ = true;  // GPREEMPT_FUSE_LN=0 in the environment keeps every launch of the kernel list

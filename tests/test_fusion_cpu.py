@@ -1,0 +1,23 @@
+"""What a caller sees of a model that merges launches, beside one that does not (tests/fusion_check.cpp; no GPU)."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def check(tmp_path_factory):
+    exe, lib = str(tmp_path_factory.mktemp("fusion") / "fusion_check"), os.path.join(ROOT, "gpreempt_amd")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-rdynamic", "-I" + os.path.join(ROOT, "include"), "-o", exe, os.path.join(ROOT, "tests", "fusion_check.cpp"),
+                    "-L" + lib, "-lgpreempt_exec", "-lgpreempt_hip", "-Wl,-rpath," + lib, "-lpthread"], check=True)
+
+    def run(*args):
+        r = subprocess.run([exe, *args], capture_output=True, text=True, timeout=60)
+        assert r.returncode == 0 and r.stdout.startswith("ok "), r.stdout + r.stderr
+    return run
+
+
+def test_a_layer_whose_operand_is_overwritten_later_in_the_pass_is_launched(check):
+    check("writers")

@@ -3,6 +3,7 @@
 #include <atomic>
 #include <ctime>
 #include <mutex>
+#include <unordered_set>
 #include <vector>
 
 namespace gp {
@@ -125,6 +126,13 @@ __global__ void flag_relay_kernel(RelayArgs a) {
 
 using namespace gp;
 
+// what gp_stream_create has made and gp_stream_destroy has not taken back
+struct LiveStreams { std::mutex mu; std::unordered_set<gp_stream> all; };
+static LiveStreams &live_streams() {
+    static LiveStreams *l = new LiveStreams;  // (never destroyed: streams may be, behind the library's statics)
+    return *l;
+}
+
 extern "C" const char *gp_last_error(void) { return g_err; }
 
 extern "C" int gp_init(int device) {
@@ -159,10 +167,23 @@ extern "C" int gp_stream_create(int priority, gp_stream *out) {
     hipStream_t s;
     GP_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
     *out = new gp_stream_s{s, priority};
+    LiveStreams &live = live_streams();
+    std::lock_guard<std::mutex> g(live.mu);
+    live.all.insert(*out);
     return GP_SUCC;
+}
+extern "C" int gp_stream_exists(gp_stream s) {
+    LiveStreams &live = live_streams();
+    std::lock_guard<std::mutex> g(live.mu);
+    return !s || live.all.count(s) ? 1 : 0;
 }
 extern "C" int gp_stream_destroy(gp_stream s) {
     if (!s) return GP_SUCC;
+    {
+        LiveStreams &live = live_streams();
+        std::lock_guard<std::mutex> g(live.mu);
+        live.all.erase(s);
+    }
     hipError_t e = hipStreamDestroy(s->s);
     delete s;
     if (e != hipSuccess) { set_error("hipStreamDestroy: %s", hipGetErrorString(e)); return GP_FAIL; }
@@ -175,6 +196,13 @@ extern "C" int gp_stream_query(gp_stream s, int *idle) {
     if (e == hipErrorNotReady) { if (idle) *idle = 0; return GP_SUCC; }
     set_error("hipStreamQuery: %s", hipGetErrorString(e));
     return GP_FAIL;
+}
+extern "C" int gp_stream_capturing(gp_stream s, int *capturing) {
+    GP_REQUIRE(capturing != nullptr, "null out pointer");
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    GP_HIP(hipStreamIsCapturing(native(s), &st));
+    *capturing = st != hipStreamCaptureStatusNone;
+    return GP_SUCC;
 }
 extern "C" int gp_stream_priority(gp_stream s, int *priority) {
     GP_REQUIRE(s && priority, "null stream");

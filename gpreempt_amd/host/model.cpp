@@ -260,8 +260,15 @@ void Model::plan_fusions() {
         ln.fused_away = true;
     }
     // scale-shift -> pointwise convolution, where nobody else reads (or writes) what lies between the two and what the layer reads
-    // stays as it is until the pass ends (compute_unread runs it then)
-    unread_.assign(storage_infos.size(), SIZE_MAX);
+    // stays as it is until the pass ends (compute_carried runs it then)
+    const size_t kernels = kernel_infos.size();
+    carried_ = std::vector<std::atomic<char>>(kernels);
+    carried_on_ = std::vector<std::atomic<GPUstream>>(kernels);
+    shown_ = std::vector<std::atomic<char>>(kernels);
+    for (size_t i = 0; i < kernels; ++i) { carried_[i] = 0; carried_on_[i] = nullptr; shown_[i] = 0; }
+    merged_.assign(kernels, 0);
+    written_by_scale_.assign(storage_infos.size(), SIZE_MAX);
+    read_by_scale_.assign(storage_infos.size(), {});
     for (size_t i = 0; i + 1 < kernel_infos.size(); ++i) {
         KernelInfo &el = kernel_infos[i], &cv = kernel_infos[i + 1];
         cv.has_pre = false;
@@ -273,10 +280,11 @@ void Model::plan_fusions() {
             for (size_t st : kernel_infos[k].args_index) alone = alone && (st != between || k == i || k == i + 1);
         for (size_t k = i + 1; k < kernel_infos.size() && alone; ++k) alone = !writes_operand_of(kernel_infos[k], el);
         if (!alone || gp_eltwise_conv2d_supported(&el.p.eltwise, &cv.p.conv) != 1) continue;
+        if (!fuse_launches_) continue;
         cv.pre = el.p.eltwise;
         cv.has_pre = true;
-        el.fused_away = true;
-        unread_[between] = i;
+        written_by_scale_[between] = i;
+        for (size_t slot : {0, 2, 3}) read_by_scale_[el.args_index[slot]].push_back(i);
     }
     // convolutions side by side
     for (size_t i = 0; i < kernel_infos.size(); ++i) {
@@ -329,11 +337,56 @@ bool Model::writes_operand_of(const KernelInfo &w, const KernelInfo &el) {
     return w.op != OpKind::Conv || w.p.conv.out_pix_stride != e.a_stride || !slices_apart(out, e.a, e.cols, w.p.conv.out, w.p.conv.Cout, e.a_stride);
 }
 
-// The output of a layer that its reader's launch does itself (plan_fusions): computed for a caller that wants to see it.
-Status Model::compute_unread(size_t idx, GPUstream stream) {
-    if (!fuse_launches_ || idx >= unread_.size() || unread_[idx] == SIZE_MAX) return Status::Succ;
-    CUDA_RETURN_STATUS(gp_launch_eltwise(&kernel_infos[unread_[idx]].p.eltwise, nullptr, stream, nullptr));
+// Runs the layer that writes storage idx, if the convolution behind it did its work so far.
+Status Model::compute_carried(size_t idx, GPUstream stream) {
+    const size_t layer = idx < written_by_scale_.size() ? written_by_scale_[idx] : SIZE_MAX;
+    if (layer == SIZE_MAX || !carried_[layer]) return Status::Succ;
+    CUDA_RETURN_STATUS(gp_launch_eltwise(&kernel_infos[layer].p.eltwise, nullptr, stream, nullptr));
     return Status::Succ;
+}
+
+// Storage idx is about to get another value.
+Status Model::before_set(size_t idx, GPUstream stream) {
+    if (idx >= written_by_scale_.size()) return Status::Succ;
+    for (size_t layer : read_by_scale_[idx]) {
+        RETURN_STATUS(compute_carried(kernel_infos[layer].args_index[4], stream));
+        carried_[layer] = 0;
+    }
+    if (written_by_scale_[idx] != SIZE_MAX) carried_[written_by_scale_[idx]] = 0;
+    return Status::Succ;
+}
+
+// Somebody gets the address of storage idx and may read or write it at any time.
+void Model::show_storage(size_t idx) {
+    if (idx >= written_by_scale_.size()) return;
+    std::vector<size_t> layers = read_by_scale_[idx];
+    if (written_by_scale_[idx] != SIZE_MAX) layers.push_back(written_by_scale_[idx]);
+    for (size_t layer : layers) {
+        shown_[layer] = 1;
+        if (!carried_[layer]) continue;
+        GPUstream on = carried_on_[layer];
+        if (!gp_stream_exists(on)) on = nullptr;  // (destroyed: what ran on it has ended)
+        if (compute_carried(kernel_infos[layer].args_index[4], on) == Status::Succ) carried_[layer] = 0;
+        if (!on) gp_stream_sync(nullptr);  // (the other streams do not wait for this one)
+    }
+}
+
+// Whether the launch of kernel idx also does other kernels' work.  `carried`: it is itself left to the next one's.
+// (A kernel that is launched again with claims made keeps the form of its last launch: the forms need not have the same grid,
+// and the slices that the claim counters stand for follow the grid.)
+bool Model::merges(size_t idx, GPUstream stream, int inject_at, bool &carried) {
+    KernelInfo &k = kernel_infos[idx];
+    const bool again = k.preemptible && idx < launches_.size() && launches_[idx] > 0;
+    if (idx + 1 < kernel_infos.size() && kernel_infos[idx + 1].has_pre) {
+        int capturing = 0;
+        carried = !again && inject_at < 0 && !shown_[idx] && gp_stream_capturing(stream, &capturing) == 0 && !capturing;
+        carried_on_[idx] = stream;
+        carried_[idx] = carried;
+        return false;
+    }
+    if (!k.has_pre && k.group.empty()) return false;
+    if (!again) merged_[idx] = !k.has_pre || carried_[idx - 1];
+    return merged_[idx] != 0;
 }
 
 // A list that is the miniWeather step (x, z, z, x; three stages of halo, fluxes, update) also gets its sweeps.  The state
@@ -385,6 +438,7 @@ Status Model::upload_param(size_t idx, const float *disk, size_t n) {
     size_t es = get_stype_size(info.stype);
     size_t dev_elems = info.size / es;
     if (n < L.disk_elems) return Status::OutOfRange;
+    RETURN_STATUS(before_set(idx, nullptr));
     std::vector<float> dev(dev_elems, 0.f);
     switch (L.kind) {
         case ParamLayout::Plain:
@@ -455,7 +509,7 @@ Status Model::get(size_t idx, void *out, size_t len, GPUstream stream) {
     if (idx >= storages.size()) return Status::OutOfRange;
     size_t size = storage_infos[idx].size;
     if (len < size) return Status::Fail;
-    RETURN_STATUS(compute_unread(idx, stream));
+    RETURN_STATUS(compute_carried(idx, stream));
     CUDA_RETURN_STATUS(gp_memcpy_d2h_async(out, storages[idx], size, stream));
     return Status::Succ;
 }
@@ -469,6 +523,7 @@ Status Model::set(size_t idx, void *value, size_t len, GPUstream stream) {
     if (idx >= storages.size()) return Status::OutOfRange;
     size_t size = storage_infos[idx].size;
     if (len < size) return Status::OutOfRange;
+    RETURN_STATUS(before_set(idx, stream));
     // (through the model's own pinned ring: the value may be gone when this returns)
     {
         std::lock_guard<std::mutex> lock(stage_mu_);
@@ -480,13 +535,14 @@ Status Model::set(size_t idx, void *value, size_t len, GPUstream stream) {
 Status Model::set_pinned(size_t idx, const void *value, size_t len, GPUstream stream) {
     if (idx >= storages.size()) return Status::OutOfRange;
     if (len < storage_infos[idx].size) return Status::OutOfRange;
+    RETURN_STATUS(before_set(idx, stream));
     CUDA_RETURN_STATUS(gp_memcpy_h2d_async(storages[idx], value, storage_infos[idx].size, stream));
     return Status::Succ;
 }
 Status Model::fetch(size_t idx, void *pinned, size_t len, GPUstream stream) {
     if (idx >= storages.size()) return Status::OutOfRange;
     if (len < storage_infos[idx].size) return Status::Fail;
-    RETURN_STATUS(compute_unread(idx, stream));
+    RETURN_STATUS(compute_carried(idx, stream));
     CUDA_RETURN_STATUS(gp_fetch(pinned, storages[idx], storage_infos[idx].size, stream));
     return Status::Succ;
 }
@@ -499,7 +555,10 @@ Status Model::set(const std::string &key, void *value, size_t len, GPUstream str
 size_t Model::get_kernel_num() const { return kernel_infos.size(); }
 size_t Model::get_storage_num() const { return storage_infos.size(); }
 StorageInfo &Model::get_storage_info(size_t idx) { return storage_infos[idx]; }
-GPUdeviceptr Model::get_storage_ptr(size_t idx) { return storages[idx]; }
+GPUdeviceptr Model::get_storage_ptr(size_t idx) {
+    show_storage(idx);
+    return storages[idx];
+}
 size_t Model::get_storage_size(size_t idx) { return storage_infos[idx].size; }
 KernelInfo &Model::get_kernel_info(size_t idx) { return kernel_infos[idx]; }
 
@@ -508,6 +567,7 @@ KernelInfo &Model::get_kernel_info(size_t idx) { return kernel_infos[idx]; }
 Status Model::get_global_ptr(const std::string &name, GPUdeviceptr *ptr) {
     size_t idx;
     if (find_storage_idx(name, idx) != Status::Succ) return Status::NotFound;
+    show_storage(idx);
     *ptr = storages[idx];
     return Status::Succ;
 }
@@ -521,6 +581,7 @@ Status Model::clear() {
     sweep_state_ = nullptr;
     sweeps_.clear();
     storage_infos.clear(); layouts.clear(); kernel_infos.clear(); storages.clear(); storages_idx.clear();
+    carried_.clear(); carried_on_.clear(); shown_.clear(); merged_.clear(); read_by_scale_.clear(); written_by_scale_.clear();
     loaded_ = false;
     return Status::Succ;
 }
@@ -573,14 +634,20 @@ Status Model::launch(size_t idx, GPUstream stream, int inject_at) {
         return Status::Succ;
     }
     const bool fuse = fuse_launches_;
-    if (fuse && k.fused_away) return Status::Succ;  // the next kernel's prologue does this one's work
+    if (fuse && k.fused_away) return Status::Succ;  // the next kernel's prologue does this one's work, or the group's launch in front has done it
+    bool carried = false;
+    const bool merged = fuse && merges(idx, stream, inject_at, carried);
+    if (carried) return Status::Succ;
     gp_preempt_ctx ctx{};
     const gp_preempt_ctx *pc = preempt_ctx(idx, inject_at, ctx) ? &ctx : nullptr;
     gp_launch_info info{};
     int rc = GP_FAIL;
     switch (k.op) {
         case OpKind::Gemm: rc = gp_launch_gemm(fuse && k.has_ln_gemm ? &k.ln_gemm : &k.p.gemm, pc, stream, &info); break;
-        case OpKind::Conv: rc = fuse && !k.group.empty() ? gp_launch_conv2d_group(k.group.data(), (int)k.group.size(), pc, stream, &info) : fuse && k.has_pre ? gp_launch_eltwise_conv2d(&k.pre, &k.p.conv, pc, stream, &info) : gp_launch_conv2d(&k.p.conv, pc, stream, &info); break;
+        case OpKind::Conv:
+            rc = !merged ? gp_launch_conv2d(&k.p.conv, pc, stream, &info) : k.has_pre ? gp_launch_eltwise_conv2d(&k.pre, &k.p.conv, pc, stream, &info)
+                                                                                     : gp_launch_conv2d_group(k.group.data(), (int)k.group.size(), pc, stream, &info);
+            break;
         case OpKind::Layout: rc = gp_launch_nchw_to_nhwc(&k.p.layout, pc, stream, &info); break;
         case OpKind::Pool: rc = gp_launch_pool2d(&k.p.pool, pc, stream, &info); break;
         case OpKind::Eltwise: rc = gp_launch_eltwise(&k.p.eltwise, pc, stream, &info); break;

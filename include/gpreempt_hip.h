@@ -52,6 +52,8 @@ int gp_device_info(int *compute_units, int *clock_khz, char *name, size_t name_l
 int gp_stream_create(int priority, gp_stream *out);
 int gp_stream_destroy(gp_stream s);
 int gp_stream_sync(gp_stream s);
+int gp_stream_exists(gp_stream s); /* 1: the default stream, or one that has not been destroyed */
+int gp_stream_capturing(gp_stream s, int *capturing); /* *capturing = 1 while launches on it are recorded, by whomever */
 int gp_stream_query(gp_stream s, int *idle); /* *idle = 1 when all work has completed */
 int gp_stream_priority(gp_stream s, int *priority);
 /* Replaces the driver call behind set_priority (src/gpreempt.cpp:61-72: the context's timeslice):

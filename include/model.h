@@ -5,6 +5,7 @@
 // TVM-compiled GPU module and two JSON files; here the kernel list is built natively from the
 // workload name and every kernel is an operator of libgpreempt_hip.so.
 #pragma once
+#include <atomic>
 #include <cstdint>
 #include <memory>
 #include <mutex>
@@ -85,13 +86,12 @@ public:
     bool has_ln_gemm = false;
     gp_gemm_params ln_gemm;
     // ... and likewise a scale-shift(-ReLU) layer whose output only the pointwise convolution behind it reads: that one's launch
-    // (gp_launch_eltwise_conv2d) does both, and the layer's output is not written; Model::get and fetch compute it for
-    // whoever asks for it.
+    // (gp_launch_eltwise_conv2d) does both, and the layer's output is not written until somebody asks for it (Model::carried_).
+    bool has_pre = false;
+    gp_eltwise_params pre;
     // ... and convolutions that follow each other in the list without reading each other run as one launch
     // (gp_launch_conv2d_group) under the first one's index.
     std::vector<gp_conv_params> group;
-    bool has_pre = false;
-    gp_eltwise_params pre;
 };
 
 class Model {
@@ -170,8 +170,14 @@ public:
     // until its next launch every kernel is known to have made no claim (gp_preempt_ctx::fresh).
     // `on` = false withdraws that for all kernels (launches that are recorded and replayed).
     void counters_cleared(bool on) { fresh_.assign(kernel_infos.size(), on ? 1 : 0); launches_.assign(kernel_infos.size(), 0); }
-    // every kernel has been launched once more by something else than launch() (a replayed graph)
-    void launched_once_more() { for (int &n : launches_) ++n; }
+    // every kernel has been launched once more by something else than launch() (a replayed graph, in which a scale-shift layer
+    // and its convolution are two launches)
+    void launched_once_more() {
+        for (size_t i = 0; i < launches_.size(); ++i) {
+            ++launches_[i];
+            if (kernel_infos[i].has_pre) merged_[i] = 0;
+        }
+    }
     // counters of the workers that have left, behind the claim counters (gp_preempt_ctx::done): byte distance from `executed`
     void set_done_counters(size_t byte_offset) { done_offset_ = byte_offset; }
     // device-visible address of a host word that a program's last leaving workgroup sets to the
@@ -242,8 +248,22 @@ private:
     bool run_side_by_side(const KernelInfo &a, const KernelInfo &b);
     bool slices_apart(size_t storage, const void *a, long na, const void *b, long nb, long stride);
     bool writes_operand_of(const KernelInfo &w, const KernelInfo &el);
-    Status compute_unread(size_t idx, GPUstream stream);
-    std::vector<size_t> unread_;  // per storage: the kernel that would write it, where plan_fusions found a launch that needs no such storage
+    // A scale-shift layer that its convolution's launch does (KernelInfo::has_pre) leaves its output storage behind: it holds what it held
+    // before.  carried_[kernel] says that it does, i.e. that the layer was launched last by being left to the convolution.  Whoever
+    // could tell gets the layer run after all: a read of the storage, a new value for what the layer reads, and (show_storage) a
+    // pointer to either, after which the layer is launched like any other; a value for the storage itself stands, and the
+    // convolution alone then reads it.  What cannot be had again is the output of the pass before, once kernels in front
+    // of the layer have written its operand anew.  Launches that are recorded into a graph are not merged: a replay asks nobody.
+    std::vector<std::atomic<char>> carried_;
+    std::vector<std::atomic<GPUstream>> carried_on_;   // where it would have been launched
+    std::vector<std::atomic<char>> shown_;             // by kernel: somebody has a pointer, it is always launched
+    std::vector<char> merged_;                         // by kernel: its last launch did other kernels' work too
+    std::vector<std::vector<size_t>> read_by_scale_;   // by storage: the scale-shift layers that read it and that a convolution can do
+    std::vector<size_t> written_by_scale_;             // by storage: the layer that writes it, or SIZE_MAX
+    Status compute_carried(size_t idx, GPUstream stream);
+    Status before_set(size_t idx, GPUstream stream);
+    void show_storage(size_t idx);
+    bool merges(size_t idx, GPUstream stream, int inject_at, bool &carried);
     bool fuse_launches_ = true;  // GPREEMPT_FUSE_LN=0 in the environment keeps every launch of the kernel list
     bool eager_tiles_ = true;    // first launches start their tiles before the stop index has come back (gp_preempt_ctx::fresh = 2); GPREEMPT_EAGER_TILES=0 makes them wait for it
     Status upload_param(size_t idx, const float *disk, size_t n);

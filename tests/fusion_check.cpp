@@ -18,6 +18,9 @@ using foo::Model;
 using foo::Tensor;
 
 static int g_merged = 0, g_launches = 0;  // launches that did the work of several kernels, and all
+static int g_capturing = 0;
+static gp_stream g_scaled_on = nullptr;  // where the last scale-shift layer was launched
+static std::vector<gp_stream> g_gone;
 
 static uint32_t mix(uint32_t a, uint32_t b) { return (a ^ (b + 0x9E3779B9u + (a << 6) + (a >> 2))) * 0x85EBCA6Bu; }
 static uint32_t hash(const void *p, long n, uint32_t h = 1) {
@@ -48,13 +51,16 @@ int gp_memcpy_d2h_async(void *h, const void *d, size_t n, gp_stream) { std::memc
 int gp_fetch(void *h, const void *d, size_t n, gp_stream) { std::memcpy(h, d, n); return 0; }
 int gp_fill32_async(void *, uint32_t, size_t, gp_stream) { return 0; }
 int gp_stream_sync(gp_stream) { return 0; }
+int gp_stream_capturing(gp_stream, int *capturing) { *capturing = g_capturing; return 0; }
+int gp_stream_exists(gp_stream s) { for (gp_stream g : g_gone) if (g == s) return 0; return 1; }
 int gp_stage_create(gp_stage *out) { *out = (gp_stage)std::malloc(1); return 0; }
 int gp_stage_destroy(gp_stage st) { std::free(st); return 0; }
 int gp_stage_upload_async(gp_stage, void *d, const void *h, size_t n, gp_stream) { std::memcpy(d, h, n); return 0; }
 int gp_launch_nchw_to_nhwc(const gp_layout_params *p, const gp_preempt_ctx *x, gp_stream, gp_launch_info *i) { put(p->out, p->c_pad, hash(p->in, p->C)); return done(x, i); }
 int gp_launch_pool2d(const gp_pool_params *p, const gp_preempt_ctx *x, gp_stream, gp_launch_info *i) { put(p->out, p->C, hash(p->in, p->C)); return done(x, i); }
 int gp_launch_softmax(const gp_softmax_params *p, const gp_preempt_ctx *x, gp_stream, gp_launch_info *i) { put(p->out, p->cols, hash(p->x, p->cols)); return done(x, i); }
-int gp_launch_eltwise(const gp_eltwise_params *e, const gp_preempt_ctx *x, gp_stream, gp_launch_info *info) {
+int gp_launch_eltwise(const gp_eltwise_params *e, const gp_preempt_ctx *x, gp_stream s, gp_launch_info *info) {
+    g_scaled_on = s;
     for (long i = 0; i < e->cols; ++i) ((uint32_t *)e->out)[i] = scaled(e, i);
     return done(x, info);
 }
@@ -91,7 +97,8 @@ Status foo::zoo_build(Model &m, const std::string &name) {
     Tensor c2 = b.conv("conv2", n2, 32, 1, 1, 0, GP_ACT_RELU, is("residual") ? &n2 : nullptr);
     if (is("rewritten")) b.pool("over", c2, 1, 1, 0, 0, &c1);
     if (is("beside")) b.conv("grow", c2, 32, 3, 1, 1, GP_ACT_NONE, nullptr, &next);
-    Tensor n3 = b.eltwise("norm3", c2, nullptr, "norm3", GP_ACT_NONE);
+    Tensor mid = b.pool("mid", c2, 1, 1, 0, 0);
+    Tensor n3 = b.eltwise("norm3", mid, nullptr, "norm3", GP_ACT_NONE);
     Tensor c3 = b.conv("conv3", n3, 32, 1, 1, 0, GP_ACT_RELU);
     size_t heads = b.add_storage("heads", 32, "float32");
     b.softmax(c3.st, heads, 1, 32, 1.f);
@@ -121,11 +128,25 @@ struct Pair {
         if (m.find_storage_idx(name, idx) != Status::Succ) { std::printf("no storage %s\n", name); std::exit(1); }
         return idx;
     }
-    void pass() {
-        each([](Model &m) {
-            for (size_t i = 0; i < m.get_kernel_num(); ++i)
-                if (m.launch(i, nullptr) != Status::Succ) { std::printf("kernel %zu\n", i); std::exit(1); }
-        });
+    static void launch(Model &m, size_t from, size_t to, gp_stream s = nullptr) {
+        for (size_t i = from; i < to; ++i)
+            if (m.launch(i, s) != Status::Succ) { std::printf("kernel %zu\n", i); std::exit(1); }
+    }
+    void pass(gp_stream s = nullptr) {
+        each([&](Model &m) { launch(m, 0, m.get_kernel_num(), s); });
+    }
+    // `f` on both, then the same in every storage, before and after another pass, and on another pair from fresh values
+    void then(const char *when, const std::function<void(Model &)> &f) {
+        each(f);
+        same(when);
+        pass();
+        same(when);
+    }
+    // what a pointer of before shows
+    void same_at(GPUdeviceptr a, GPUdeviceptr b, size_t bytes, const char *when) {
+        if (std::memcmp(a, b, bytes) == 0) return;
+        std::printf("%s: the memory differs\n", when);
+        std::exit(1);
     }
     // both models show the same in every storage
     void same(const char *when) {
@@ -149,6 +170,109 @@ static void passes_merge(const char *name, int merged) {
     }
 }
 
+// kernels of "plain": 0 layout, 1 stem, 2 norm1, 3 conv1, 4 norm2, 5 conv2, 6 pool, 7 norm3, 8 conv3, 9 softmax
+static void storages() {
+    auto index = [](Model &m, const char *key) { return Pair::at(m, key); };
+    for (const char *key : {"norm2.out", "conv1.out", "norm2.scale", "norm2.shift", "block", "conv2.out", "data"}) {
+        Pair p("plain");
+        p.pass();
+        p.then((std::string("set ") + key).c_str(), [&](Model &m) { Pair::fill(m, index(m, key), 21); });
+        p.then("set twice", [&](Model &m) { Pair::fill(m, index(m, key), 22); Pair::fill(m, index(m, key), 23); });
+        // ... and the convolution alone, which reads what was set
+        p.then("the convolution alone", [&](Model &m) { Pair::fill(m, index(m, key), 24); Pair::launch(m, 5, 6); });
+        p.then("the layer alone", [&](Model &m) { Pair::launch(m, 4, 5); });
+        p.then("the layer, a value, the convolution", [&](Model &m) { Pair::launch(m, 4, 5); Pair::fill(m, index(m, key), 25); Pair::launch(m, 5, 6); });
+        p.then("pinned", [&](Model &m) {
+            std::vector<uint32_t> v(m.get_storage_size(index(m, key)) / 4, 26);
+            if (m.set_pinned(index(m, key), v.data(), v.size() * 4, nullptr) != Status::Succ) std::exit(1);
+            Pair::launch(m, 5, 6);
+        });
+        g_merged = 0;
+        p.pass();
+        if (g_merged != 3) { std::printf("set %s: %d launches merged afterwards\n", key, g_merged); std::exit(1); }
+    }
+    // the convolution alone, before any pass: the layer has not run
+    Pair fresh("plain");
+    fresh.then("the convolution first", [](Model &m) { Pair::launch(m, 5, 6); });
+    // pointers, to the layer's output and to what it reads, taken before the first pass or behind one
+    for (const char *key : {"norm2.out", "conv1.out", "norm2.scale"})
+        for (int passes = 0; passes < 2; ++passes)
+            for (int by_name = 0; by_name < 2; ++by_name) {
+                Pair p("plain");
+                const size_t out = index(p.merged, "norm2.out"), bytes = p.merged.get_storage_size(out), at = index(p.merged, key);
+                for (int i = 0; i < passes; ++i) p.pass((gp_stream)64);
+                g_scaled_on = nullptr;
+                GPUdeviceptr a = nullptr, b = nullptr;
+                if (by_name) {
+                    if (p.apart.get_global_ptr(key, &a) != Status::Succ || p.merged.get_global_ptr(key, &b) != Status::Succ) std::exit(1);
+                } else { a = p.apart.get_storage_ptr(at); b = p.merged.get_storage_ptr(at); }
+                if (passes && g_scaled_on != (gp_stream)64) { std::printf("not on the stream of the pass\n"); std::exit(1); }
+                for (int i = 0; i < 2; ++i) {
+                    p.same_at(a, b, p.merged.get_storage_size(at), "a pointer");
+                    p.same("a pointer");
+                    put(a, 4, 31 + (uint32_t)i);  // the caller writes through it
+                    put(b, 4, 31 + (uint32_t)i);
+                    p.same("a value through a pointer");
+                    p.each([](Model &m) { Pair::launch(m, 5, 6); });
+                    p.same("a value through a pointer, and the convolution");
+                    p.pass();
+                }
+                p.same_at(p.apart.get_storage_ptr(out), p.merged.get_storage_ptr(out), bytes, "the output");
+            }
+    // the stream of the pass is gone
+    Pair p("plain");
+    p.pass((gp_stream)64);
+    g_gone = {(gp_stream)64};
+    p.same_at(p.apart.get_storage_ptr(Pair::at(p.apart, "norm2.out")), p.merged.get_storage_ptr(Pair::at(p.merged, "norm2.out")), 32 * 4, "a stream that is gone");
+    if (g_scaled_on != nullptr) { std::printf("on a stream that is gone\n"); std::exit(1); }
+    g_gone.clear();
+}
+
+// a recorded pass writes everything, since its replays cannot be followed
+static void recorded() {
+    Pair p("plain");
+    p.pass();
+    g_capturing = 1;
+    g_merged = 0;
+    p.pass();
+    if (g_merged) { std::printf("%d recorded launches merged\n", g_merged); std::exit(1); }
+    g_capturing = 0;
+    p.each([](Model &m) { Pair::fill(m, Pair::at(m, "norm2.scale"), 41); });
+    p.same("recorded");
+}
+
+// A kernel that is stopped and launched again has the form of its first launch, whatever has been asked for in between.
+static void stopped() {
+    for (int first_merged = 0; first_merged < 2; ++first_merged) {
+        Pair p("plain");
+        static int counters[10 * 32 * 16], flag, stop;
+        GPUdeviceptr pf = &flag, ps = &stop;
+        Model &m = p.merged;
+        m.batchAddParam(&pf);
+        m.batchAddParam(&ps);
+        if (m.add_block_preemption_param(counters, 32) != Status::Succ) std::exit(1);
+        m.counters_cleared(true);
+        g_capturing = !first_merged;
+        Pair::launch(m, 0, 6);
+        g_capturing = 0;
+        g_merged = g_launches = 0;
+        if (first_merged) m.get_storage_ptr(Pair::at(m, "norm2.out"));  // (runs the layer)
+        else if (m.launch(2, nullptr) != Status::Succ) std::exit(1);    // (resumes a layer that was launched itself)
+        const int layers = g_launches;
+        Pair::launch(m, 5, 6);
+        if (g_merged != first_merged || layers != 1) { std::printf("%d layers, %d of %d merged when launched again\n", layers, g_merged, first_merged); std::exit(1); }
+        m.counters_cleared(true);
+        g_merged = 0;
+        Pair::launch(m, 0, m.get_kernel_num());
+        if (g_merged != (first_merged ? 2 : 3)) { std::printf("%d merged in a fresh run\n", g_merged); std::exit(1); }
+        // a replayed graph has launched every kernel by itself
+        m.launched_once_more();
+        g_merged = 0;
+        Pair::launch(m, 3, 4);
+        if (g_merged) { std::printf("merged behind a replay\n"); std::exit(1); }
+    }
+}
+
 int main(int argc, char **argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "writers") {
@@ -156,6 +280,9 @@ int main(int argc, char **argv) {
         passes_merge("beside", 3);
         passes_merge("rewritten", 2);
         passes_merge("residual", 2);
-    } else return 1;
+    } else if (what == "storages") storages();
+    else if (what == "recorded") recorded();
+    else if (what == "stopped") stopped();
+    else return 1;
     std::printf("ok %s\n", what.c_str());
 }

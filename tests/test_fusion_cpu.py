@@ -21,3 +21,16 @@ def check(tmp_path_factory):
 
 def test_a_layer_whose_operand_is_overwritten_later_in_the_pass_is_launched(check):
     check("writers")
+
+
+def test_storages_show_what_they_would_if_every_kernel_were_launched(check):
+    """values set before, between and behind the launches, and pointers handed out"""
+    check("storages")
+
+
+def test_a_recorded_pass_writes_every_storage(check):
+    check("recorded")
+
+
+def test_a_kernel_launched_again_keeps_the_form_of_its_first_launch(check):
+    check("stopped")

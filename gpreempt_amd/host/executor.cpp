@@ -167,6 +167,7 @@ void Executor::capture_graph(GPUstream stream) {
     }
     graph_exec = g;
     use_cuda_graph = true;
+    model->launches_recorded();
 }
 
 BaseExecutor::BaseExecutor() {}
@@ -246,6 +247,7 @@ Status BLPExecutor::init(std::string workload) {
 
 Status BLPExecutor::launch_kernel(size_t kernel_offset, GPUstream stream) {
     model->set_poll_every(poll_every);
+    model->keep_apart(inject_kernel);
     int inject = ((int)kernel_offset == inject_kernel) ? inject_claim : -1;
     return model->launch(kernel_offset, stream, inject);
 }

@@ -267,6 +267,8 @@ void Model::plan_fusions() {
     shown_ = std::vector<std::atomic<char>>(kernels);
     for (size_t i = 0; i < kernels; ++i) { carried_[i] = 0; carried_on_[i] = nullptr; shown_[i] = 0; }
     merged_.assign(kernels, 0);
+    recorded_.assign(kernels, 0);
+    in_groups_at_.assign(storage_infos.size(), {});
     written_by_scale_.assign(storage_infos.size(), SIZE_MAX);
     read_by_scale_.assign(storage_infos.size(), {});
     for (size_t i = 0; i + 1 < kernel_infos.size(); ++i) {
@@ -290,7 +292,9 @@ void Model::plan_fusions() {
     for (size_t i = 0; i < kernel_infos.size(); ++i) {
         KernelInfo &first = kernel_infos[i];
         first.group.clear();
-        if (first.op != OpKind::Conv || first.fused_away || first.has_pre) continue;
+        first.in_group = false;
+        if (!fuse_launches_) continue;
+        if (first.op != OpKind::Conv || first.has_pre) continue;
         std::vector<gp_conv_params> group = {first.p.conv};
         size_t end = i + 1;
         for (; end < kernel_infos.size(); ++end) {
@@ -302,7 +306,12 @@ void Model::plan_fusions() {
             if (gp_conv2d_group_supported(group.data(), (int)group.size()) != 1) { group.pop_back(); break; }
         }
         if (group.size() < 2) continue;
-        for (size_t m = i + 1; m < end; ++m) kernel_infos[m].fused_away = true;
+        for (size_t m = i + 1; m < end; ++m) {
+            kernel_infos[m].group.clear();
+            kernel_infos[m].in_group = true;
+            for (size_t st : kernel_infos[m].args_index)
+                if (st != SIZE_MAX) in_groups_at_[st].push_back(m);
+        }
         first.group = std::move(group);
         i = end - 1;
     }
@@ -353,6 +362,7 @@ Status Model::before_set(size_t idx, GPUstream stream) {
         carried_[layer] = 0;
     }
     if (written_by_scale_[idx] != SIZE_MAX) carried_[written_by_scale_[idx]] = 0;
+    for (size_t conv : in_groups_at_[idx]) carried_[conv] = 0;
     return Status::Succ;
 }
 
@@ -371,7 +381,7 @@ void Model::show_storage(size_t idx) {
     }
 }
 
-// Whether the launch of kernel idx also does other kernels' work.  `carried`: it is itself left to the next one's.
+// Whether the launch of kernel idx also does other kernels' work.  `carried`: it is itself left to the next one's, or a group's has done it.
 // (A kernel that is launched again with claims made keeps the form of its last launch: the forms need not have the same grid,
 // and the slices that the claim counters stand for follow the grid.)
 bool Model::merges(size_t idx, GPUstream stream, int inject_at, bool &carried) {
@@ -384,8 +394,12 @@ bool Model::merges(size_t idx, GPUstream stream, int inject_at, bool &carried) {
         carried_[idx] = carried;
         return false;
     }
+    if (k.in_group) {
+        carried = carried_[idx].exchange(0) != 0;
+        return false;
+    }
     if (!k.has_pre && k.group.empty()) return false;
-    if (!again) merged_[idx] = !k.has_pre || carried_[idx - 1];
+    if (!again) merged_[idx] = k.has_pre ? carried_[idx - 1] != 0 : apart_ <= (int)idx || apart_ >= (int)(idx + k.group.size());
     return merged_[idx] != 0;
 }
 
@@ -581,7 +595,7 @@ Status Model::clear() {
     sweep_state_ = nullptr;
     sweeps_.clear();
     storage_infos.clear(); layouts.clear(); kernel_infos.clear(); storages.clear(); storages_idx.clear();
-    carried_.clear(); carried_on_.clear(); shown_.clear(); merged_.clear(); read_by_scale_.clear(); written_by_scale_.clear();
+    carried_.clear(); carried_on_.clear(); shown_.clear(); merged_.clear(); read_by_scale_.clear(); written_by_scale_.clear(); in_groups_at_.clear();
     loaded_ = false;
     return Status::Succ;
 }
@@ -634,7 +648,7 @@ Status Model::launch(size_t idx, GPUstream stream, int inject_at) {
         return Status::Succ;
     }
     const bool fuse = fuse_launches_;
-    if (fuse && k.fused_away) return Status::Succ;  // the next kernel's prologue does this one's work, or the group's launch in front has done it
+    if (fuse && k.fused_away) return Status::Succ;  // the next kernel's prologue does this one's work
     bool carried = false;
     const bool merged = fuse && merges(idx, stream, inject_at, carried);
     if (carried) return Status::Succ;
@@ -660,6 +674,8 @@ Status Model::launch(size_t idx, GPUstream stream, int inject_at) {
     }
     if (idx < fresh_.size()) fresh_[idx] = 0;  // launched (or refused): from here on only its counters know
     CUDA_RETURN_STATUS(rc);
+    if (merged)
+        for (size_t m = 1; m < k.group.size(); ++m) carried_[idx + m] = 1;
     launched(idx, pc != nullptr, info);
     return Status::Succ;
 }

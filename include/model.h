@@ -90,8 +90,9 @@ public:
     bool has_pre = false;
     gp_eltwise_params pre;
     // ... and convolutions that follow each other in the list without reading each other run as one launch
-    // (gp_launch_conv2d_group) under the first one's index.
+    // (gp_launch_conv2d_group) under the first one's index; the launches of the others behind it have nothing left to do.
     std::vector<gp_conv_params> group;
+    bool in_group = false;  // one of the others
 };
 
 class Model {
@@ -169,15 +170,21 @@ public:
     // The claim counters have just been cleared (or are about to be, earlier on the same stream):
     // until its next launch every kernel is known to have made no claim (gp_preempt_ctx::fresh).
     // `on` = false withdraws that for all kernels (launches that are recorded and replayed).
-    void counters_cleared(bool on) { fresh_.assign(kernel_infos.size(), on ? 1 : 0); launches_.assign(kernel_infos.size(), 0); }
-    // every kernel has been launched once more by something else than launch() (a replayed graph, in which a scale-shift layer
-    // and its convolution are two launches)
-    void launched_once_more() {
-        for (size_t i = 0; i < launches_.size(); ++i) {
-            ++launches_[i];
-            if (kernel_infos[i].has_pre) merged_[i] = 0;
-        }
+    void counters_cleared(bool on) {
+        fresh_.assign(kernel_infos.size(), on ? 1 : 0);
+        launches_.assign(kernel_infos.size(), 0);
+        for (size_t i = 0; i < kernel_infos.size(); ++i)
+            if (kernel_infos[i].in_group) carried_[i] = 0;
     }
+    // the launches since counters_cleared() have been recorded ...
+    void launches_recorded() { recorded_ = merged_; }
+    // ... and every kernel has been launched once more by a replay of the recording
+    void launched_once_more() {
+        for (int &n : launches_) ++n;
+        merged_ = recorded_;
+    }
+    // kernel `kernel` (-1: none) is launched by itself, not in a group of convolutions
+    void keep_apart(int kernel) { apart_ = kernel; }
     // counters of the workers that have left, behind the claim counters (gp_preempt_ctx::done): byte distance from `executed`
     void set_done_counters(size_t byte_offset) { done_offset_ = byte_offset; }
     // device-visible address of a host word that a program's last leaving workgroup sets to the
@@ -252,14 +259,17 @@ private:
     // before.  carried_[kernel] says that it does, i.e. that the layer was launched last by being left to the convolution.  Whoever
     // could tell gets the layer run after all: a read of the storage, a new value for what the layer reads, and (show_storage) a
     // pointer to either, after which the layer is launched like any other; a value for the storage itself stands, and the
-    // convolution alone then reads it.  What cannot be had again is the output of the pass before, once kernels in front
+    // convolution alone then reads it.  (For a convolution of a group: that the group's launch has done it.  Its own launch clears
+    // that, and so does a new value for what it reads or writes: launched then, it runs.)  What cannot be had again is the output of the pass before, once kernels in front
     // of the layer have written its operand anew.  Launches that are recorded into a graph are not merged: a replay asks nobody.
     std::vector<std::atomic<char>> carried_;
     std::vector<std::atomic<GPUstream>> carried_on_;   // where it would have been launched
     std::vector<std::atomic<char>> shown_;             // by kernel: somebody has a pointer, it is always launched
-    std::vector<char> merged_;                         // by kernel: its last launch did other kernels' work too
+    std::vector<char> merged_, recorded_;              // by kernel: its last launch (the recorded one) did other kernels' work too
+    int apart_ = -1;                                   // see keep_apart
     std::vector<std::vector<size_t>> read_by_scale_;   // by storage: the scale-shift layers that read it and that a convolution can do
     std::vector<size_t> written_by_scale_;             // by storage: the layer that writes it, or SIZE_MAX
+    std::vector<std::vector<size_t>> in_groups_at_;    // by storage: the convolutions in a group's launch that read or write it
     Status compute_carried(size_t idx, GPUstream stream);
     Status before_set(size_t idx, GPUstream stream);
     void show_storage(size_t idx);

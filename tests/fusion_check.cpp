@@ -35,7 +35,9 @@ static uint32_t scaled(const gp_eltwise_params *e, long i) {
     return mix(mix(((const uint32_t *)e->a)[i], ((const uint32_t *)e->scale)[i]), ((const uint32_t *)e->shift)[i]);
 }
 static void conv(const gp_conv_params *c, uint32_t in) { put(c->out, c->Cout, mix(mix(hash(c->weight, c->Cin), hash(c->bias, c->Cout)), mix(in, hash(c->residual, c->Cout)))); }
-static int done(const gp_preempt_ctx *, gp_launch_info *info) {
+static std::vector<int> g_at;  // the kernel of each launch that a preemption was injected into
+static int done(const gp_preempt_ctx *ctx, gp_launch_info *info) {
+    if (ctx && ctx->inject_at >= 0) g_at.push_back(ctx->kernel_id);
     if (info) std::memset(info, 0, sizeof(*info));
     ++g_launches;
     return 0;
@@ -82,12 +84,22 @@ int gp_launch_conv2d_group(const gp_conv_params *p, int n, const gp_preempt_ctx 
 }
 }
 
-// Three scale-shift layers in front of pointwise convolutions, the way DenseNet has them; "group": two convolutions side by side;
+// Three scale-shift layers in front of pointwise convolutions, the way DenseNet has them; "group": three convolutions side by side;
 // "rewritten": what the second layer reads is overwritten by a kernel behind its convolution; "beside": by one that writes the
 // channels next to those; "residual": the second convolution also adds the second layer's output.
 Status foo::zoo_build(Model &m, const std::string &name) {
     GraphBuilder b(m, "f32");
     auto is = [&](const char *s) { return name == s; };
+    if (is("group")) {  // kernels: 0 layout, 1 stem, 2 left, 3 middle, 4 right (side by side), 5 join, 6 softmax
+        Tensor t = b.conv("stem", b.input_nchw(1, 8, 2, 2), 512, 1, 1, 0, GP_ACT_RELU);
+        Tensor left = b.conv("left", t, 512, 1, 1, 0, GP_ACT_RELU);
+        b.conv("middle", t, 32, 3, 1, 1, GP_ACT_RELU);
+        Tensor right = b.conv("right", t, 512, 1, 1, 0, GP_ACT_RELU);
+        Tensor join = b.conv("join", left, 512, 1, 1, 0, GP_ACT_RELU, &right);
+        size_t heads = b.add_storage("heads", 512, "float32");
+        b.softmax(join.st, heads, 1, 512, 1.f);
+        return Status::Succ;
+    }
     Tensor t = b.input_nchw(1, 8, 2, 2);
     Tensor block = b.activation("block", 1, 2, 2, 64), first = GraphBuilder::slice(block, 0, 32), next = GraphBuilder::slice(block, 32, 32);
     b.conv("stem", t, 32, 1, 1, 0, GP_ACT_RELU, nullptr, &first);
@@ -273,6 +285,64 @@ static void stopped() {
     }
 }
 
+static void groups() {
+    passes_merge("group", 1);
+    Pair p("group");
+    p.pass();
+    // a member alone, behind a pass and from new values, in front of any launch of the group
+    for (size_t k = 2; k < 5; ++k)
+        for (const char *key : {"stem.out", "left.weight", "middle.weight", "middle.out", "right.bias", "left.out"}) {
+            p.then("a new value, a member alone", [&](Model &m) { Pair::fill(m, Pair::at(m, key), 50 + (uint32_t)k); Pair::launch(m, k, k + 1); if (k == 2) Pair::launch(m, 3, 5); });
+            p.then("a new value between the members", [&](Model &m) { Pair::launch(m, 2, 3); Pair::fill(m, Pair::at(m, key), 60 + (uint32_t)k); Pair::launch(m, 3, 5); });
+        }
+    Pair fresh("group");
+    fresh.then("a member first", [](Model &m) { Pair::launch(m, 3, 4); });
+    g_launches = 0;
+    Pair::launch(p.merged, 0, p.merged.get_kernel_num());
+    if (g_launches != 5) { std::printf("%d launches of seven kernels, three of them side by side\n", g_launches); std::exit(1); }
+
+    // a preemption injected at a member is launched with that member, and the kernels launched again keep their form
+    static int counters[7 * 32 * 16], flag, stop;
+    GPUdeviceptr pf = &flag, ps = &stop;
+    Model &m = p.merged;
+    m.batchAddParam(&pf);
+    m.batchAddParam(&ps);
+    if (m.add_block_preemption_param(counters, 32) != Status::Succ) std::exit(1);
+    auto run = [&](size_t from, int inject) {
+        g_merged = g_launches = 0;
+        g_at.clear();
+        m.keep_apart(inject);
+        for (size_t i = from; i < 7; ++i)
+            if (m.launch(i, nullptr, (int)i == inject ? 0 : -1) != Status::Succ) std::exit(1);
+    };
+    for (int inject = 0; inject < 7; ++inject) {
+        const int apart = inject == 3 || inject == 4;
+        m.counters_cleared(true);
+        run(0, inject);
+        if (g_at != std::vector<int>{inject} || g_merged != !apart) { std::printf("injected at %d: %zu launches, %d merged\n", inject, g_at.size(), g_merged); std::exit(1); }
+        if (inject > 4) continue;
+        run(apart ? 2 : (size_t)(inject < 2 ? inject : 2), -1);  // resumed at or in front of the group
+        if (g_merged != !apart) { std::printf("injected at %d and resumed: %d merged\n", inject, g_merged); std::exit(1); }
+    }
+    // recorded in a group, launched apart since, replayed, resumed: in a group
+    m.counters_cleared(false);
+    run(0, -1);
+    m.launches_recorded();
+    m.counters_cleared(true);
+    run(0, 3);
+    m.counters_cleared(false);
+    m.launched_once_more();
+    run(2, -1);
+    if (g_merged != 1) { std::printf("a replay resumed: %d merged\n", g_merged); std::exit(1); }
+    // a run given up behind the group's first kernel: the next one's members are launched
+    m.counters_cleared(true);
+    Pair::launch(m, 2, 3);
+    m.counters_cleared(true);
+    g_launches = 0;
+    Pair::launch(m, 3, 4);
+    if (g_launches != 1) { std::printf("a member of a run given up is not launched\n"); std::exit(1); }
+}
+
 int main(int argc, char **argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "writers") {
@@ -281,6 +351,7 @@ int main(int argc, char **argv) {
         passes_merge("rewritten", 2);
         passes_merge("residual", 2);
     } else if (what == "storages") storages();
+    else if (what == "groups") groups();
     else if (what == "recorded") recorded();
     else if (what == "stopped") stopped();
     else return 1;

@@ -34,3 +34,7 @@ def test_a_recorded_pass_writes_every_storage(check):
 
 def test_a_kernel_launched_again_keeps_the_form_of_its_first_launch(check):
     check("stopped")
+
+
+def test_members_of_a_group_launched_alone_set_and_injected_into(check):
+    check("groups")

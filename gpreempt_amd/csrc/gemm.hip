@@ -435,6 +435,17 @@ extern "C" int gp_gemm_ckpt_bytes(const gp_gemm_params *p, size_t *bytes) {
     *bytes = plan_ckpt_bytes(pl);
     return GP_SUCC;
 }
+extern "C" int gp_conv2d_body(const gp_conv_params *p, char *name, size_t len) {
+    GP_REQUIRE(name && len, "null name");
+    MatPlan pl;
+    if (int rc = plan_conv2d(p, &pl)) return rc;
+    static const char *const names[] = {"pipe128", "pipe64", "pipe64_splitk", "pipe32_splitk", "staged128", "staged64", "pipe256", "wide32x32_16", "wide32x32_8", "wide64x32_16",
+                                        "wide64x64_8", "lnwide32x64_16", "narrow16x16", "narrow32x16"};
+    static_assert(MB_PIPE128 == 0 && MB_PIPE64 == 1 && MB_PIPE64_SK == 2 && MB_PIPE32_SK == 3 && MB_STAGED128 == 4 && MB_STAGED64 == 5 && MB_PIPE256 == 6 && MB_NARROW32x16 == 13, "names");
+    const bool blocks_straddle = pl.conv && pl.g.Cin % (pl.dtype == GP_F32 ? 32 : 64) != 0;
+    snprintf(name, len, "%s%s", names[pl.body], !pl.conv ? "" : pl.window ? " window" : blocks_straddle ? " straddling" : pl.taps ? " taps" : " gathered");
+    return GP_SUCC;
+}
 extern "C" int gp_conv_ckpt_bytes(const gp_conv_params *p, size_t *bytes) {
     GP_REQUIRE(bytes != nullptr, "null bytes");
     MatPlan pl;

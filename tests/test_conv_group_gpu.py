@@ -81,6 +81,17 @@ def test_a_group_has_the_bits_of_its_members(gp, dt, images, group):
         check()
         launch(gp, params, st.ctx())  # all made: nothing runs
         check()
+    # the general loop: one claim counter, and fewer workgroups than tiles, each running members of different forms in turn
+    for groups, workgroups in ((1, 0), (1, 3), (4, 4)):
+        for inject in (-1, sum(tiles) // 2):
+            st = gp.BlpState(1, flag, groups)
+            wipe()
+            info = launch(gp, params, st.ctx(inject_at=inject, max_workgroups=workgroups, poll_every=1))
+            assert not info.fixed_claims or sum(tiles) <= 4
+            flag.set(0)
+            st.stop.upload(np.array([-1], np.int32))
+            launch(gp, params, st.ctx(max_workgroups=workgroups))
+            check()
     # a launch behind a stop leaves without writing
     st = gp.BlpState(1, flag, 32)
     st.stop.upload(np.array([0], np.int32))

@@ -1,5 +1,7 @@
 """Convolutions that keep their input window in LDS (gemm_window.hpp): the bits of the body that gathers every tap, plain, preempted
 and resumed."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -38,6 +40,9 @@ def test_a_window_gives_the_bits_of_the_gather(gp, dt, N, H, W, Cin, Cout, R, S,
     want = out.download().copy()
     assert np.isfinite(gp.from_storage(want[:N * H * W * Cout * 2].copy(), dtype)).all()
     p.tile_m = p.tile_n = p.variant = 0
+    name = C.create_string_buffer(64)
+    gp.check(gp.lib().gp_conv2d_body(C.byref(p), name, C.c_size_t(len(name))))
+    assert name.value == (b"wide64x32_16 taps" if tile == 64 else b"wide32x32_16 taps" if (H, W) == (9, 40) else b"wide32x32_16 window")
     flag = gp.Flag()
     for ctx_of in (None, lambda st: st.ctx(fresh=2), lambda st: st.ctx(inject_at=0), lambda st: st.ctx(max_workgroups=8)):
         st = gp.BlpState(1, flag, 32)
@@ -51,3 +56,4 @@ def test_a_window_gives_the_bits_of_the_gather(gp, dt, N, H, W, Cin, Cout, R, S,
             gp.launch("gp_launch_conv2d", p, st.ctx())
             sync(gp)
         assert np.array_equal(out.download(), want)
+

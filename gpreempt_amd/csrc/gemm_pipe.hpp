@@ -7,8 +7,9 @@
 // load writes lane i's 16 bytes at (wave-uniform base) + 16*i, i.e. one instruction fills 8
 // consecutive rows; the swizzle is applied on the global-address side (lane i fetches the chunk
 // that belongs at its slot), which keeps the later 16-byte MFMA-operand reads spread over the
-// banks.  Rows outside M/N, K-chunks past K and convolution taps outside the image are fetched
-// from a zero page instead of being predicated.
+// banks.  Rows outside M/N, K-chunks past K and convolution taps outside the image are not
+// predicated: where operands are fetched through buffer descriptors (DESC and TAPS below) such a lane's offset lies beyond the
+// descriptor's end, which reads as zeros; where through pointers, they point at a page of zeros.
 //
 // SPLITK = false: the 4 waves tile the BM x BN block 2 x 2.
 // SPLITK = true : every wave computes the whole BM x BN block for one quarter of each K-step

@@ -426,8 +426,8 @@ __device__ __forceinline__ void unclaim_fixed(const BlpArgs &b) {
 // with the first operands, stands in for the look in front of the claim.  The bit and the count go
 // out without waiting for their old values and are withdrawn like any claim if the body finds the
 // stop recorded.  They go out behind the body's first loads (late_claim), from the last wavefront: the claim's code is 0.4 us that
-// stood in front of the first load of every launch, and in the bodies whose first four wavefronts multiply, the last one only
-// fetches.  One thread makes the claim and withdraws it, so that the two cannot pass each other.  A launch saves the wait for the stop index that way (0.2 us of a 10 us
+// stood in front of the first load of every launch, and in the bodies of eight and sixteen wavefronts, whose first four multiply, the last one
+// only fetches (in those of four it multiplies like the others, and the claim still hides behind its first loads).  One thread makes the claim and withdraws it, so that the two cannot pass each other.  A launch saves the wait for the stop index that way (0.2 us of a 10 us
 // convolution); a kernel queued behind a stop leaves a first operand fetch later than it would
 // have, which adds 4 us to the drain of a chunk of launches.  That trade is the caller's.
 // Everything the body is handed is computed from kernel arguments and the workgroup's number alone:

@@ -269,6 +269,8 @@ void Model::plan_fusions() {
     merged_.assign(kernels, 0);
     recorded_.assign(kernels, 0);
     in_groups_at_.assign(storage_infos.size(), {});
+    in_groups_.clear();
+    roles_.assign(kernels, Alone);
     written_by_scale_.assign(storage_infos.size(), SIZE_MAX);
     read_by_scale_.assign(storage_infos.size(), {});
     for (size_t i = 0; i + 1 < kernel_infos.size(); ++i) {
@@ -285,6 +287,8 @@ void Model::plan_fusions() {
         if (!fuse_launches_) continue;
         cv.pre = el.p.eltwise;
         cv.has_pre = true;
+        roles_[i] = LeftToConv;
+        roles_[i + 1] = WithScale;
         written_by_scale_[between] = i;
         for (size_t slot : {0, 2, 3}) read_by_scale_[el.args_index[slot]].push_back(i);
     }
@@ -292,7 +296,6 @@ void Model::plan_fusions() {
     for (size_t i = 0; i < kernel_infos.size(); ++i) {
         KernelInfo &first = kernel_infos[i];
         first.group.clear();
-        first.in_group = false;
         if (!fuse_launches_) continue;
         if (first.op != OpKind::Conv || first.has_pre) continue;
         std::vector<gp_conv_params> group = {first.p.conv};
@@ -308,11 +311,13 @@ void Model::plan_fusions() {
         if (group.size() < 2) continue;
         for (size_t m = i + 1; m < end; ++m) {
             kernel_infos[m].group.clear();
-            kernel_infos[m].in_group = true;
+            roles_[m] = InGroup;
+            in_groups_.push_back(m);
             for (size_t st : kernel_infos[m].args_index)
                 if (st != SIZE_MAX) in_groups_at_[st].push_back(m);
         }
         first.group = std::move(group);
+        roles_[i] = HeadsGroup;
         i = end - 1;
     }
 }
@@ -385,22 +390,26 @@ void Model::show_storage(size_t idx) {
 // (A kernel that is launched again with claims made keeps the form of its last launch: the forms need not have the same grid,
 // and the slices that the claim counters stand for follow the grid.)
 bool Model::merges(size_t idx, GPUstream stream, int inject_at, bool &carried) {
-    KernelInfo &k = kernel_infos[idx];
+    const KernelInfo &k = kernel_infos[idx];
     const bool again = k.preemptible && idx < launches_.size() && launches_[idx] > 0;
-    if (idx + 1 < kernel_infos.size() && kernel_infos[idx + 1].has_pre) {
-        int capturing = 0;
-        carried = !again && inject_at < 0 && !shown_[idx] && gp_stream_capturing(stream, &capturing) == 0 && !capturing;
-        carried_on_[idx] = stream;
-        carried_[idx] = carried;
-        return false;
+    switch (roles_[idx]) {
+        case LeftToConv: {
+            int capturing = 0;
+            carried = !again && inject_at < 0 && !shown_[idx] && gp_stream_capturing(stream, &capturing) == 0 && !capturing;
+            carried_on_[idx] = stream;
+            carried_[idx] = carried;
+            return false;
+        }
+        case InGroup: carried = carried_[idx].exchange(0) != 0; return false;
+        case WithScale:
+            if (!again) merged_[idx] = carried_[idx - 1] != 0;
+            return merged_[idx] != 0;
+        case HeadsGroup:
+            if (!again) merged_[idx] = apart_ <= (int)idx || apart_ >= (int)(idx + k.group.size());
+            return merged_[idx] != 0;
+        case Alone: break;
     }
-    if (k.in_group) {
-        carried = carried_[idx].exchange(0) != 0;
-        return false;
-    }
-    if (!k.has_pre && k.group.empty()) return false;
-    if (!again) merged_[idx] = k.has_pre ? carried_[idx - 1] != 0 : apart_ <= (int)idx || apart_ >= (int)(idx + k.group.size());
-    return merged_[idx] != 0;
+    return false;
 }
 
 // A list that is the miniWeather step (x, z, z, x; three stages of halo, fluxes, update) also gets its sweeps.  The state
@@ -595,7 +604,7 @@ Status Model::clear() {
     sweep_state_ = nullptr;
     sweeps_.clear();
     storage_infos.clear(); layouts.clear(); kernel_infos.clear(); storages.clear(); storages_idx.clear();
-    carried_.clear(); carried_on_.clear(); shown_.clear(); merged_.clear(); read_by_scale_.clear(); written_by_scale_.clear(); in_groups_at_.clear();
+    carried_.clear(); carried_on_.clear(); shown_.clear(); merged_.clear(); read_by_scale_.clear(); written_by_scale_.clear(); in_groups_at_.clear(); in_groups_.clear(); roles_.clear();
     loaded_ = false;
     return Status::Succ;
 }
@@ -650,7 +659,7 @@ Status Model::launch(size_t idx, GPUstream stream, int inject_at) {
     const bool fuse = fuse_launches_;
     if (fuse && k.fused_away) return Status::Succ;  // the next kernel's prologue does this one's work
     bool carried = false;
-    const bool merged = fuse && merges(idx, stream, inject_at, carried);
+    const bool merged = fuse && roles_[idx] != Alone && merges(idx, stream, inject_at, carried);
     if (carried) return Status::Succ;
     gp_preempt_ctx ctx{};
     const gp_preempt_ctx *pc = preempt_ctx(idx, inject_at, ctx) ? &ctx : nullptr;

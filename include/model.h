@@ -92,7 +92,6 @@ public:
     // ... and convolutions that follow each other in the list without reading each other run as one launch
     // (gp_launch_conv2d_group) under the first one's index; the launches of the others behind it have nothing left to do.
     std::vector<gp_conv_params> group;
-    bool in_group = false;  // one of the others
 };
 
 class Model {
@@ -173,8 +172,7 @@ public:
     void counters_cleared(bool on) {
         fresh_.assign(kernel_infos.size(), on ? 1 : 0);
         launches_.assign(kernel_infos.size(), 0);
-        for (size_t i = 0; i < kernel_infos.size(); ++i)
-            if (kernel_infos[i].in_group) carried_[i] = 0;
+        for (size_t conv : in_groups_) carried_[conv] = 0;
     }
     // the launches since counters_cleared() have been recorded ...
     void launches_recorded() { recorded_ = merged_; }
@@ -270,6 +268,9 @@ private:
     std::vector<std::vector<size_t>> read_by_scale_;   // by storage: the scale-shift layers that read it and that a convolution can do
     std::vector<size_t> written_by_scale_;             // by storage: the layer that writes it, or SIZE_MAX
     std::vector<std::vector<size_t>> in_groups_at_;    // by storage: the convolutions in a group's launch that read or write it
+    std::vector<size_t> in_groups_;                    // all of those
+    enum Role : char { Alone, LeftToConv, WithScale, HeadsGroup, InGroup };
+    std::vector<Role> roles_;                          // by kernel (a byte: looked at in front of every launch)
     Status compute_carried(size_t idx, GPUstream stream);
     Status before_set(size_t idx, GPUstream stream);
     void show_storage(size_t idx);

@@ -255,7 +255,7 @@ struct PipeKernel {
         // uniform offset along K and the operand's descriptor.  A wavefront has one instruction stream, and what stands between two of
         // its MFMAs bounds a K-step here: pointers of 64 bits, advanced per slot and parked on the zero page, took 24 registers and, with a
         // branch around the K remainder, a dozen instructions and two jumps per load; now it is a compare and a select.  Both builds in
-        // turn: 8192^3 bf16 with checkpoints 981 -> 945 us, 4096^3 fp32 1098 -> 1016, 6000 x 5000 x 2048 fp16 152 -> 146.
+        // turn: 8192^3 bf16 with checkpoints, its clears included, 970 -> 951 us, 4096^3 fp32 1098 -> 1016, 6000 x 5000 x 2048 fp16 152 -> 146.
         // (`near`: the tile's rows lie within a descriptor's 2 GB.  Otherwise an address of 64 bits is worked out for every load.)
         const long far = (long)kBufferEnd / (long)sizeof(T) - g.K;
         const bool near = TAPS || !DESC || ((CONV || (long)BM * g.lda <= far) && (long)BN * g.ldb <= far);

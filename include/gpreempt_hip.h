@@ -302,8 +302,8 @@ typedef struct gp_conv_params {
 int gp_launch_conv2d(const gp_conv_params *p, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info);
 /* No counterpart in the reference (TVM launches operators one by one): n convolutions, two to four, as one launch, with one set of claim
  * counters.  None may read or overwrite what another writes.  The results have the bits of n launches.  Only for what
- * gp_conv2d_group_supported accepts (1): each would get the same one of the sixteen-wavefront bodies alone (layers of few
- * tiles), and together they have at most one tile per compute unit. */
+ * gp_conv2d_group_supported accepts (1): each would get 32 x 32 (fp32: 16 x 16) tiles on sixteen wavefronts alone (layers of few
+ * tiles), none of them long enough to be given up on a stop, and together they have at most one tile per compute unit. */
 int gp_conv2d_group_supported(const gp_conv_params *p, int n);
 int gp_launch_conv2d_group(const gp_conv_params *p, int n, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info);
 /* For diagnosis: the tile body a convolution would be launched with and how it fetches its input, as text ("wide32x32_16 window",
@@ -348,7 +348,7 @@ int gp_launch_eltwise(const gp_eltwise_params *p, const gp_preempt_ctx *ctx, gp_
  * out = act(conv(relu?(a * scale + shift))) in one launch, where `e` is a per-channel scale and shift with an optional
  * ReLU (no addend) and `c` a pointwise convolution (1 x 1, stride 1) of its output.  e->out is not written.  The result has
  * the bits of gp_launch_eltwise followed by gp_launch_conv2d.  Only for what gp_eltwise_conv2d_supported accepts (1): the
- * convolution reads exactly the layer's output, and a matrix body that takes a scale and shift serves its shape;
+ * convolution reads exactly the layer's output, a matrix body that takes a scale and shift serves its shape, and e->a_stride >= 0;
  * c->out must not overlap e->a. */
 int gp_eltwise_conv2d_supported(const gp_eltwise_params *e, const gp_conv_params *c);
 int gp_launch_eltwise_conv2d(const gp_eltwise_params *e, const gp_conv_params *c, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info);

@@ -138,30 +138,3 @@ def test_inception_in_groups_has_the_bits_of_inception_kernel_by_kernel(gp, monk
             ex.resume(stream)
             got.append(ex.get_output("heads", stream))
     assert all(np.array_equal(g, got[0]) for g in got)
-
-
-def test_a_preemption_injected_at_a_member_fires_and_a_member_launched_alone_runs(gp):
-    from gpreempt_amd import executor as ex_mod
-    x = gp.to_storage(np.random.default_rng(4).standard_normal((1, 3, 139, 139), np.float32), gp.F16)
-    ex = ex_mod.Executor("inception@b=1,hw=139,dtype=f16", blp=True)
-    stream, flag = gp.Stream(1), gp.Flag()
-    ex.set_flag(flag)
-    ex.set_running(True)
-    ex.set_input("data", x, stream)
-    ex.execute(stream)
-    want = ex.get_output("heads", stream)
-    members = [i for i, n in enumerate(ex.counters()) if n == 0]
-    assert len(members) > 20
-    for kernel in members[::6] + [members[0] - 1]:
-        ex.inject_preempt(kernel, 0)
-        ex.execute(stream)
-        stream.sync()
-        assert flag.get() == 1, kernel
-        flag.set(0)
-        ex.inject_preempt(-1, -1)
-        ex.resume(stream)
-        assert ex.last_stop_index() >= kernel and np.array_equal(ex.get_output("heads", stream), want)
-        ex.reset_counters(stream)
-        ex.launch_kernel(kernel, stream)
-        stream.sync()
-        assert ex.counters()[kernel] > 0

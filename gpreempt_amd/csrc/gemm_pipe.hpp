@@ -41,13 +41,18 @@ __device__ __forceinline__ void load_lds16(const void *gptr, unsigned lds_byte) 
 
 // The same through a buffer descriptor: lane i reads 16 bytes at the descriptor's base + off + soff.  A lane whose `off`
 // is kBufferEnd reads zeros (the descriptor's range ends there, and soff is not negative).
+// The four wait states behind M0: a vector instruction that writes a scalar register has to be five wait states ahead of a vector-memory
+// instruction that reads it, nothing in the hardware sees to that, and the compiler, which does for its own instructions, does not
+// look into inline assembly.  Such writes are v_readlane, by which a kernel short of scalar registers gets a descriptor's word or an offset back
+// right in front of the load: with one wait state 110 loads of the whole-model program and 30 of the general forms of three matrix
+// bodies could read the register's old content.
 constexpr unsigned kBufferEnd = 0x80000000u;
 __device__ __forceinline__ u32x4 buffer_of(const void *base, unsigned bytes = kBufferEnd) {  // (a raw buffer of 2 GB: what the planners allow an operand to span)
     const unsigned long long a = (unsigned long long)base;
     return u32x4{(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)a), (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(a >> 32)), bytes, 0x00027000u};
 }
 __device__ __forceinline__ void load_lds16_buffer(u32x4 rsrc, unsigned off, unsigned soff, unsigned lds_byte) {
-    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 3\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
                  :
                  : "v"(off), "s"(rsrc), "s"(soff), "s"(lds_byte)
                  : "memory", "m0");

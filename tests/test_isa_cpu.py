@@ -1,0 +1,59 @@
+"""What the compiler cannot see in the matrix kernels' hand-written loads, checked in the code that it made of them (the device code of the
+in-tree library, disassembled; no GPU)."""
+import glob
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+from gpreempt_amd import capi as gp
+
+OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
+pytestmark = pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="no disassembler")
+WORD = re.compile(r"^\s+([a-z]\S*)\s*(.*?)\s*// ([0-9A-F]+):(.*)$")
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    """{name: [(address, mnemonic, operands, branch target or None)]} of every kernel that loads to LDS"""
+    work = tmp_path_factory.mktemp("isa")
+    lib = shutil.copy(gp.LIB_PATH, work)
+    subprocess.run([OBJDUMP, "--offloading", os.path.basename(lib)], cwd=work, check=True, capture_output=True)
+    found = {}
+    for part in glob.glob(os.path.join(work, "*gfx950*")):
+        name, code = None, []
+        for line in subprocess.run([OBJDUMP, "-d", part], check=True, capture_output=True, text=True).stdout.splitlines():
+            if line.endswith(">:") and not line.startswith(" "):
+                name, code = line[line.index("<") + 1:-2], []
+                found[os.path.basename(part) + name] = code
+                continue
+            m = WORD.match(line)
+            if m and name:
+                to = re.search(r"\+0x([0-9a-f]+)>$", m.group(4)) if m.group(1).startswith(("s_branch", "s_cbranch")) else None
+                code.append((int(m.group(3), 16), m.group(1), m.group(2), int(to.group(1), 16) if to else None))
+    found = {k: v for k, v in found.items() if any((op.startswith("buffer_load") and args.endswith(" lds")) or op.startswith("global_load_lds") for _, op, args, _ in v)}
+    assert len(found) > 400
+    return found
+
+
+def scalars(operand):
+    m = re.match(r"^s(?:\[(\d+):(\d+)\]|(\d+))$", operand)
+    return range(int(m.group(1) or m.group(3)), int(m.group(2) or m.group(3)) + 1) if m else ()
+
+
+def test_a_scalar_written_by_a_vector_instruction_is_read_by_a_load_five_wait_states_later(kernels):
+    """... or later: the hardware does not wait, and the compiler does not look into the loads, which are inline assembly"""
+    bad = []
+    for name, code in kernels.items():
+        at, written = 0, {}  # wait states so far; scalar -> when it was last written
+        for _, op, args, _ in code:
+            parts = [p for p in re.split(r"[,\s]+", args) if p]
+            if op.startswith(("buffer_", "global_", "scratch_")):
+                bad += [(name, op, args) for p in parts for s in scalars(p) if at - written.get(s, -9) - 1 < 5]
+            elif op.startswith("v_") and parts:
+                for s in scalars(parts[0]):
+                    written[s] = at
+            at += int(parts[0], 0) + 1 if op == "s_nop" else 1
+    assert not bad, (len(bad), bad[:4])

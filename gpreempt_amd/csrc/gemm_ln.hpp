@@ -182,7 +182,7 @@ struct LnWideKernel {
             if (s == 0) wait_stages<LPW>((NS < PRE ? NS : PRE) - 1);
             else if (s + STAGES - 2 < NS) wait_vmcnt<(STAGES - 2) * LPW>();
             else wait_vmcnt<0>();
-            __syncthreads();  // stage s of B (and, the first time, the rows of A) visible; the buffer of stage s-1 is free
+            stage_barrier();  // stage s of B (and, the first time, the rows of A) visible; the buffer of stage s-1 is free
             if (s == 0) GP_PROBE(2);
             if (s == 0 && early && __builtin_amdgcn_readfirstlane(read_lds_word(early_slot)) != -1) {
                 wait_vmcnt<0>();  // loads still landing in LDS must not outlive the workgroup

@@ -110,6 +110,16 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// The barrier at the top of a stage: behind it the buffer of the stage before is loaded into again, so a wavefront that comes to it must
+// have its fragments of that stage in registers.  __syncthreads() alone does not see to that: the loads to LDS are inline assembly, nothing that
+// the compiler knows writes the buffer, and in the forms with a loop in the loop it leaves the reads outstanding across the barrier.  A
+// wavefront held up long enough (its compute unit shared with a front workgroup) then read the stage four K-steps on: in one launch of 150 a few rows
+// of 1024 x 1024 x 8192 in 64 x 64 tiles came out wrong.
+__device__ __forceinline__ void stage_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __syncthreads();
+}
+
 // four consecutive output elements
 template <typename T> struct __attribute__((aligned(4 * sizeof(T)))) Vec4 { T v[4]; };
 template <typename T> __device__ __forceinline__ void st_vec4(T *p, Vec4<T> o) {
@@ -530,12 +540,12 @@ struct PipeKernel {
             else wait_vmcnt<0>();
             int stop_word = -1, flag_word = 0;
             if constexpr (PRE) {
-                if (kt == kt0) __syncthreads();  // everyone's part of the table
+                if (kt == kt0) stage_barrier();  // everyone's part of the table
                 char *mine = (char *)lds_t + (size_t)((unsigned)kt % STAGES) * STAGE_BYTES + (size_t)wave * A_PW * 8 * RB + lane * 16;
 #pragma unroll
                 for (int j = 0; j < A_PW; ++j) pre_apply<T>(g, mine + j * 8 * RB, lds_c + LDS_BYTES, kt * BK + chunk_of(wave * A_PW + j) * VEC);
             }
-            __syncthreads();  // everyone's part of stage kt is visible; stage kt-1's buffer is free
+            stage_barrier();  // everyone's part of stage kt is visible; stage kt-1's buffer is free
             if (kt == 0) GP_PROBE(2);
             if constexpr (LOOKS && !ISSUE)
                 if (looking && kt == KT - 1 && kt > kt0) announce();

@@ -329,7 +329,7 @@ struct WideKernel {
             else if (s + STAGES - 2 < NS) wait_vmcnt<(STAGES - 2) * LPW>();
             else wait_vmcnt<0>();
             if constexpr (SCALED) {
-                if (s == 0) __syncthreads();  // everyone's part of the table
+                if (s == 0) stage_barrier();  // everyone's part of the table
                 const int k0 = (s * KB + kb) * BK;
                 char *blk = (char *)lds_t + (size_t)((unsigned)s % STAGES) * STAGE_BYTES + (size_t)kb * BLK_BYTES + lane * 16;
                 if (k0 < g.K) {
@@ -337,7 +337,7 @@ struct WideKernel {
                     for (int j = 0; j < LPW_A; ++j) pre_apply<T>(g, blk + group_of(wv, j) * 8 * RB, lds_c + LDS_BYTES, k0 + kc[j]);
                 }
             }
-            __syncthreads();  // everyone's part of stage s is visible; the buffer of stage s-1 is free
+            stage_barrier();  // everyone's part of stage s is visible; the buffer of stage s-1 is free
             if (s == 0) GP_PROBE(2);
             if (((s == 0 && early) || (looking && s > 0 && (s & (LOOK_EVERY - 1)) == 0)) && __builtin_amdgcn_readfirstlane(read_lds_word(early_slot)) != -1) {
                 wait_vmcnt<0>();  // loads still landing in LDS must not outlive the workgroup

@@ -116,7 +116,7 @@ struct WindowKernel {
             if (s == 0) wait_stages<LPW>((NS < STAGES - 1 ? NS : STAGES - 1) - 1);
             else if (s + STAGES - 2 < NS) wait_vmcnt<(STAGES - 2) * LPW>();
             else wait_vmcnt<0>();
-            __syncthreads();  // everyone's part of stage s (and, the first time, of the window) is visible; the buffer of stage s-1 is free
+            stage_barrier();  // everyone's part of stage s (and, the first time, of the window) is visible; the buffer of stage s-1 is free
             if (s == 0) GP_PROBE(2);
             if (((s == 0 && early) || (looking && s > 0 && (s & (LOOK_EVERY - 1)) == 0)) && __builtin_amdgcn_readfirstlane(read_lds_word(early_slot)) != -1) {
                 wait_vmcnt<0>();  // loads still landing in LDS must not outlive the workgroup

@@ -57,3 +57,32 @@ def test_a_scalar_written_by_a_vector_instruction_is_read_by_a_load_five_wait_st
                     written[s] = at
             at += int(parts[0], 0) + 1 if op == "s_nop" else 1
     assert not bad, (len(bad), bad[:4])
+
+
+def test_no_barrier_is_reached_with_lds_reads_outstanding(kernels):
+    """behind a stage's barrier the buffer that they read is loaded into again, which the compiler does not know"""
+    bad = []
+    for name, code in kernels.items():
+        index = {a: i for i, (a, *_) in enumerate(code)}
+        most, work = [-1] * len(code), [(0, 0)]  # reads and writes outstanding in front of an instruction, on the worst way there
+        while work:
+            i, n = work.pop()
+            while i < len(code) and n > most[i]:
+                most[i] = n
+                a, op, args, to = code[i]
+                if op.startswith("ds_"):
+                    n = min(n + 1, 15)
+                elif op == "s_waitcnt" and "lgkmcnt" in args:
+                    n = min(n, int(re.search(r"lgkmcnt\((\d+)\)", args).group(1)))
+                elif op == "s_barrier" and n:
+                    bad.append((name, hex(a), n))
+                elif op == "s_endpgm":
+                    break
+                if to is not None:
+                    j = index[code[0][0] + to]
+                    if op == "s_branch":
+                        i = j
+                        continue
+                    work.append((j, n))
+                i += 1
+    assert not bad, (len(bad), bad[:4])

@@ -89,7 +89,7 @@ struct LnWideKernel {
             const unsigned sbase = lds0 + ((unsigned)s % STAGES) * STAGE_BYTES + (unsigned)kb * B_BLK_BYTES;
 #pragma unroll
             for (int j = 0; j < LPW; ++j)  // (whole blocks past the last one, when the stage is not full: zeros)
-                load_lds16_buffer(rsrc_b, k0 < g.K ? off[j] : kBufferEnd, (unsigned)k0 * (unsigned)sizeof(T), sbase + (unsigned)((wv * LPW + j) * 8 * RB));
+                load_lds16_buffer<SINGLE>(rsrc_b, k0 < g.K ? off[j] : kBufferEnd, (unsigned)k0 * (unsigned)sizeof(T), sbase + (unsigned)((wv * LPW + j) * 8 * RB));
         };
 
         if (!SINGLE) __syncthreads();  // the previous tile of this workgroup may still be reading LDS
@@ -182,7 +182,7 @@ struct LnWideKernel {
             if (s == 0) wait_stages<LPW>((NS < PRE ? NS : PRE) - 1);
             else if (s + STAGES - 2 < NS) wait_vmcnt<(STAGES - 2) * LPW>();
             else wait_vmcnt<0>();
-            stage_barrier();  // stage s of B (and, the first time, the rows of A) visible; the buffer of stage s-1 is free
+            __syncthreads();  // stage s of B (and, the first time, the rows of A) visible; the buffer of stage s-1 is free
             if (s == 0) GP_PROBE(2);
             if (s == 0 && early && __builtin_amdgcn_readfirstlane(read_lds_word(early_slot)) != -1) {
                 wait_vmcnt<0>();  // loads still landing in LDS must not outlive the workgroup

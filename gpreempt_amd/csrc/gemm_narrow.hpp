@@ -112,9 +112,9 @@ struct NarrowKernel {
                 if (CONV && j < LPW_A && straddles) {
                     const int k = k0 + kc[j], tap = (int)__umulhi((unsigned)k + 1u, g.inv_cin), ci = k - tap * g.Cin, r = (int)__umulhi((unsigned)tap + 1u, g.inv_s), s2 = tap - r * g.S;
                     const unsigned at = row[CONV ? j : 0] + (unsigned)((r * g.W + s2) * (int)g.lda + ci) * 4u;
-                    load_lds16_buffer(rsrc_a, k < g.K && (taps[CONV ? j : 0] >> tap & 1u) ? at : kBufferEnd, 0u, to);
-                } else if (CONV && j < LPW_A) load_lds16_buffer(rsrc_a, (taps[CONV ? j : 0] & tap_bit) ? off[j] : kBufferEnd, tap_off, to);
-                else load_lds16_buffer(j < LPW_A ? rsrc_a : rsrc_b, whole || k0 + kc[j] < g.K ? off[j] : kBufferEnd, (unsigned)k0 * 4u, to);
+                    load_lds16_buffer<SINGLE>(rsrc_a, k < g.K && (taps[CONV ? j : 0] >> tap & 1u) ? at : kBufferEnd, 0u, to);
+                } else if (CONV && j < LPW_A) load_lds16_buffer<SINGLE>(rsrc_a, (taps[CONV ? j : 0] & tap_bit) ? off[j] : kBufferEnd, tap_off, to);
+                else load_lds16_buffer<SINGLE>(j < LPW_A ? rsrc_a : rsrc_b, whole || k0 + kc[j] < g.K ? off[j] : kBufferEnd, (unsigned)k0 * 4u, to);
             }
             if (CONV && last == LPW_A) advance(KB * BK);
         };
@@ -162,7 +162,7 @@ struct NarrowKernel {
             else if (s + STAGES - 2 < NS) wait_vmcnt<(STAGES - 2) * LPW>();
             else wait_vmcnt<0>();
             if constexpr (SCALED) {
-                if (s == 0) stage_barrier();  // everyone's part of the table
+                if (s == 0) __syncthreads();  // everyone's part of the table
                 const int k0 = (s * KB + kb) * BK;
                 char *blk = (char *)lds_t + (size_t)((unsigned)s % STAGES) * STAGE_BYTES + (size_t)kb * BLK_BYTES + lane * 16;
                 if (k0 < g.K) {
@@ -170,7 +170,7 @@ struct NarrowKernel {
                     for (int j = 0; j < LPW_A; ++j) pre_apply<T>(g, blk + group_of(j) * 8 * RB, lds_c + LDS_BYTES, k0 + kc[j]);
                 }
             }
-            stage_barrier();  // everyone's part of stage s is visible; the buffer of stage s-1 is free
+            __syncthreads();  // everyone's part of stage s is visible; the buffer of stage s-1 is free
             if (s == 0) GP_PROBE(2);
             if (((s == 0 && early) || (looking && s > 0 && (s & (LOOK_EVERY - 1)) == 0)) && __builtin_amdgcn_readfirstlane(read_lds_word(early_slot)) != -1) {
                 wait_vmcnt<0>();  // loads still landing in LDS must not outlive the workgroup

@@ -41,20 +41,22 @@ __device__ __forceinline__ void load_lds16(const void *gptr, unsigned lds_byte) 
 
 // The same through a buffer descriptor: lane i reads 16 bytes at the descriptor's base + off + soff.  A lane whose `off`
 // is kBufferEnd reads zeros (the descriptor's range ends there, and soff is not negative).
-// The four wait states behind M0: a vector instruction that writes a scalar register has to be five wait states ahead of a vector-memory
-// instruction that reads it, nothing in the hardware sees to that, and the compiler, which does for its own instructions, does not
-// look into inline assembly.  Such writes are v_readlane, by which a kernel short of scalar registers gets a descriptor's word or an offset back
-// right in front of the load: with one wait state 110 loads of the whole-model program and 30 of the general forms of three matrix
-// bodies could read the register's old content.
 constexpr unsigned kBufferEnd = 0x80000000u;
 __device__ __forceinline__ u32x4 buffer_of(const void *base, unsigned bytes = kBufferEnd) {  // (a raw buffer of 2 GB: what the planners allow an operand to span)
     const unsigned long long a = (unsigned long long)base;
     return u32x4{(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)a), (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(a >> 32)), bytes, 0x00027000u};
 }
+// A vector instruction that writes a scalar register has to be five wait states ahead of a vector-memory instruction that reads it; nothing in
+// the hardware sees to that, and the compiler, which does for its own instructions, does not look into inline assembly.  Such writes are
+// v_readlane, by which a kernel short of scalar registers gets a descriptor's word or an offset back right in front of the load.  So the load
+// brings the wait states along.  TIGHT is for the kernels that run one tile or checkpoint: they have their descriptors and offsets in scalar
+// registers well ahead, and a load costs the one wait state that M0 wants (the others in every load: DenseNet-201 b4 fp16 1637 -> 1662 us, 8192^3 bf16
+// 976 -> 991; the offset through a scalar copy instead: BERT b1 465 -> 469).  tests/test_isa_cpu.py looks at every load of the library.
+template <bool TIGHT = false>
 __device__ __forceinline__ void load_lds16_buffer(u32x4 rsrc, unsigned off, unsigned soff, unsigned lds_byte) {
-    asm volatile("s_mov_b32 m0, %3\n\ts_nop 3\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop %4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
                  :
-                 : "v"(off), "s"(rsrc), "s"(soff), "s"(lds_byte)
+                 : "v"(off), "s"(rsrc), "s"(soff), "s"(lds_byte), "n"(TIGHT ? 0 : 3)
                  : "memory", "m0");
 }
 
@@ -114,7 +116,8 @@ template <int N> __device__ __forceinline__ void wait_vmcnt() {
 // have its fragments of that stage in registers.  __syncthreads() alone does not see to that: the loads to LDS are inline assembly, nothing that
 // the compiler knows writes the buffer, and in the forms with a loop in the loop it leaves the reads outstanding across the barrier.  A
 // wavefront held up long enough (its compute unit shared with a front workgroup) then read the stage four K-steps on: in one launch of 150 a few rows
-// of 1024 x 1024 x 8192 in 64 x 64 tiles came out wrong.
+// of 1024 x 1024 x 8192 in 64 x 64 tiles came out wrong.  (The wide bodies multiply what they have read before they come to a barrier.
+// tests/test_isa_cpu.py follows the reads to every barrier, theirs included.)
 __device__ __forceinline__ void stage_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __syncthreads();
@@ -359,7 +362,7 @@ struct PipeKernel {
                 const int kc = chunk_of(wave * A_PW + j) * VEC;
                 const T *src;
                 if constexpr (TAPS) {
-                    load_lds16_buffer(rsrc_a, a_taps[j] >> sa.tap & 1u ? a_off[j] : kBufferEnd, sa.tap_bytes, sa.sbase + (unsigned)((wave * A_PW + j) * 8 * RB));
+                    load_lds16_buffer<SINGLE || CKPT>(rsrc_a, a_taps[j] >> sa.tap & 1u ? a_off[j] : kBufferEnd, sa.tap_bytes, sa.sbase + (unsigned)((wave * A_PW + j) * 8 * RB));
                     return;
                 }
                 if (CONV) {
@@ -399,7 +402,7 @@ struct PipeKernel {
                     const int jj = CONV ? 0 : j;
                     const bool ok = sa.k0 + kc < g.K;
                     if (__builtin_expect(near, 1)) {
-                        load_lds16_buffer(rsrc_a, ok ? a_off[jj] : kBufferEnd, sa.k_bytes, sa.sbase + (unsigned)((wave * A_PW + j) * 8 * RB));
+                        load_lds16_buffer<SINGLE || CKPT>(rsrc_a, ok ? a_off[jj] : kBufferEnd, sa.k_bytes, sa.sbase + (unsigned)((wave * A_PW + j) * 8 * RB));
                         return;
                     }
                     src = ok && a_off[jj] != kBufferEnd ? A + ((long)(a_row0 + j * 8) * g.lda + (sa.k0 + kc)) : zero;
@@ -424,7 +427,7 @@ struct PipeKernel {
                 } else {
                     const bool ok = sa.k0 + kc < g.K;
                     if (__builtin_expect(near, 1)) {
-                        load_lds16_buffer(rsrc_b, ok ? b_off[j] : kBufferEnd, sa.k_bytes, sa.sbase + (unsigned)(A_BYTES + (wave * B_PW + j) * 8 * RB));
+                        load_lds16_buffer<SINGLE || CKPT>(rsrc_b, ok ? b_off[j] : kBufferEnd, sa.k_bytes, sa.sbase + (unsigned)(A_BYTES + (wave * B_PW + j) * 8 * RB));
                         return;
                     }
                     src = ok && b_off[j] != kBufferEnd ? B + ((long)(b_row0 + j * 8) * g.ldb + (sa.k0 + kc)) : zero;

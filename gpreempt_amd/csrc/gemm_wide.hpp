@@ -273,15 +273,15 @@ struct WideKernel {
                 if (CONV && j < LPW_A && straddles) {
                     const int k = k0 + kc[j], tap = (int)__umulhi((unsigned)k + 1u, g.inv_cin), ci = k - tap * g.Cin, r = (int)__umulhi((unsigned)tap + 1u, g.inv_s), s2 = tap - r * g.S;
                     const unsigned at = row[CONV ? j : 0] + (unsigned)((r * g.W + s2) * (int)g.lda + ci) * (unsigned)sizeof(T);
-                    load_lds16_buffer(rsrc_a, k < g.K && (taps[CONV ? j : 0] >> tap & 1u) ? at : kBufferEnd, 0u, sbase + (unsigned)(gi * 8 * RB));
+                    load_lds16_buffer<SINGLE>(rsrc_a, k < g.K && (taps[CONV ? j : 0] >> tap & 1u) ? at : kBufferEnd, 0u, sbase + (unsigned)(gi * 8 * RB));
                 } else if (CONV && j < LPW_A) {
                     // taps outside the image, rows outside the problem and blocks past K have nothing to fetch
-                    load_lds16_buffer(rsrc_a, (taps[CONV ? j : 0] & tap_bit) ? off[j] : kBufferEnd, tap_off, sbase + (unsigned)(gi * 8 * RB));
+                    load_lds16_buffer<SINGLE>(rsrc_a, (taps[CONV ? j : 0] & tap_bit) ? off[j] : kBufferEnd, tap_off, sbase + (unsigned)(gi * 8 * RB));
                 } else {
                     // (nor have rows outside the problem and K-chunks past K, also whole blocks past the last one when
                     // the stage is not full)
                     const unsigned at = whole || k0 + kc[j] < g.K ? off[j] : kBufferEnd;
-                    load_lds16_buffer(j < LPW_A ? rsrc_a : rsrc_b, at, (unsigned)k0 * (unsigned)sizeof(T), sbase + (unsigned)(gi * 8 * RB));
+                    load_lds16_buffer<SINGLE>(j < LPW_A ? rsrc_a : rsrc_b, at, (unsigned)k0 * (unsigned)sizeof(T), sbase + (unsigned)(gi * 8 * RB));
                 }
             }
             if (CONV && last == LPW_A) advance(KB * BK);
@@ -329,7 +329,7 @@ struct WideKernel {
             else if (s + STAGES - 2 < NS) wait_vmcnt<(STAGES - 2) * LPW>();
             else wait_vmcnt<0>();
             if constexpr (SCALED) {
-                if (s == 0) stage_barrier();  // everyone's part of the table
+                if (s == 0) __syncthreads();  // everyone's part of the table
                 const int k0 = (s * KB + kb) * BK;
                 char *blk = (char *)lds_t + (size_t)((unsigned)s % STAGES) * STAGE_BYTES + (size_t)kb * BLK_BYTES + lane * 16;
                 if (k0 < g.K) {
@@ -337,7 +337,7 @@ struct WideKernel {
                     for (int j = 0; j < LPW_A; ++j) pre_apply<T>(g, blk + group_of(wv, j) * 8 * RB, lds_c + LDS_BYTES, k0 + kc[j]);
                 }
             }
-            stage_barrier();  // everyone's part of stage s is visible; the buffer of stage s-1 is free
+            __syncthreads();  // everyone's part of stage s is visible; the buffer of stage s-1 is free
             if (s == 0) GP_PROBE(2);
             if (((s == 0 && early) || (looking && s > 0 && (s & (LOOK_EVERY - 1)) == 0)) && __builtin_amdgcn_readfirstlane(read_lds_word(early_slot)) != -1) {
                 wait_vmcnt<0>();  // loads still landing in LDS must not outlive the workgroup

@@ -73,7 +73,7 @@ struct WindowKernel {
             const unsigned sbase = lds0 + ((unsigned)s % STAGES) * STAGE_BYTES + (unsigned)kb * BLK_BYTES;
 #pragma unroll
             for (int j = 0; j < LPW; ++j)  // (whole blocks past the last one, when the stage is not full: zeros)
-                load_lds16_buffer(rsrc_b, k0 < g.K ? off[j] : kBufferEnd, (unsigned)k0 * (unsigned)sizeof(T), sbase + (unsigned)((wv * LPW + j) * 8 * RB));
+                load_lds16_buffer<SINGLE>(rsrc_b, k0 < g.K ? off[j] : kBufferEnd, (unsigned)k0 * (unsigned)sizeof(T), sbase + (unsigned)((wv * LPW + j) * 8 * RB));
         };
 
         if (!SINGLE) __syncthreads();  // the previous tile of this workgroup may still be reading LDS
@@ -84,7 +84,7 @@ struct WindowKernel {
             if (blk >= blocks) break;
             const int r = gi * 8 + rig, pixel = origin + r;
             const unsigned at = ((unsigned)pixel * (unsigned)g.lda + (unsigned)((cpos ^ ((r >> 1) & 7)) * VEC)) * (unsigned)sizeof(T);
-            load_lds16_buffer(rsrc_a, (unsigned)pixel < (unsigned)g.M ? at : kBufferEnd, (unsigned)(blk * RB), lds0 + win + (unsigned)((blk * rows + gi * 8) * RB));
+            load_lds16_buffer<SINGLE>(rsrc_a, (unsigned)pixel < (unsigned)g.M ? at : kBufferEnd, (unsigned)(blk * RB), lds0 + win + (unsigned)((blk * rows + gi * 8) * RB));
         }
 #pragma unroll
         for (int s = 0; s < STAGES - 1; ++s) {
@@ -116,7 +116,7 @@ struct WindowKernel {
             if (s == 0) wait_stages<LPW>((NS < STAGES - 1 ? NS : STAGES - 1) - 1);
             else if (s + STAGES - 2 < NS) wait_vmcnt<(STAGES - 2) * LPW>();
             else wait_vmcnt<0>();
-            stage_barrier();  // everyone's part of stage s (and, the first time, of the window) is visible; the buffer of stage s-1 is free
+            __syncthreads();  // everyone's part of stage s (and, the first time, of the window) is visible; the buffer of stage s-1 is free
             if (s == 0) GP_PROBE(2);
             if (((s == 0 && early) || (looking && s > 0 && (s & (LOOK_EVERY - 1)) == 0)) && __builtin_amdgcn_readfirstlane(read_lds_word(early_slot)) != -1) {
                 wait_vmcnt<0>();  // loads still landing in LDS must not outlive the workgroup

@@ -82,3 +82,38 @@ def test_a_preemption_injected_at_a_member_fires_and_a_member_launched_alone_run
         ex.launch_kernel(kernel, stream)
         stream.sync()
         assert ex.counters()[kernel] > 0
+
+
+def test_inception_in_a_graph_stopped_and_resumed_kernel_by_kernel(gp, monkeypatch):
+    """the recorded launches are the groups', and so are the relaunches, also when the model has been launched apart in between"""
+    from gpreempt_amd import executor as ex_mod
+    monkeypatch.setenv("GPREEMPT_USE_HIPGRAPH", "1")
+    inputs = [gp.to_storage(np.random.default_rng(s).standard_normal((1, 3, 139, 139), np.float32), gp.F16) for s in range(2)]
+    ex = ex_mod.Executor("inception@b=1,hw=139,dtype=f16", blp=True)
+    stream, flag = gp.Stream(1), gp.Flag()
+    ex.set_flag(flag)
+    ex.set_running(True)
+
+    def see(x):
+        ex.set_input("data", x, stream)
+        ex.execute(stream)
+        return ex.get_output("heads", stream).tobytes()
+
+    want = [see(x) for x in inputs]
+    members = [i for i, n in enumerate(ex.counters()) if n == 0]
+    ex.capture_graph(stream)
+    assert not ex.uses_program()
+    for k in range(6):
+        assert [see(x) for x in inputs] == want
+        ex.reset_counters(stream)  # kernel by kernel, one group apart
+        ex.inject_preempt(members[5 * k], 1 << 20)
+        for i in range(ex.kernel_num()):
+            ex.launch_kernel(i, stream)
+        ex.inject_preempt(-1, -1)
+        assert ex.get_output("heads", stream).tobytes() == want[1]
+        ex.execute(stream)
+        flag.set(1)
+        stream.sync()
+        flag.set(0)
+        ex.resume(stream)
+        assert ex.get_output("heads", stream).tobytes() == want[1]

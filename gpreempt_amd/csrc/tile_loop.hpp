@@ -259,6 +259,11 @@ __device__ __forceinline__ bool spare_workgroup(const BlpArgs &b, bool fixed, bo
 // The first one stays: one lane reads the flag about every microsecond and records the stop, until a stop is
 // recorded, or every claim of the launch has been made (from then on no workgroup starts that a stop could hold
 // back), or its bounded number of looks is used up.  The others leave at once.  Returns true in a front workgroup.
+// Between two reads of the flag the first wavefront pauses for about two microseconds, in which it only looks whether it is time to go: a read of
+// host memory under way makes every load of that XCD come back later, and the launch lasts until its slowest XCD is done.  VGG-16 b16
+// 1332 -> 1282 us, ResNet-152 b8 1547 -> 1537, Inception-v3 b1 stopped and resumed level (860 -> 850); three times the pause: VGG 1300,
+// Inception 864 (a stop is seen later).
+constexpr int FRONT_PAUSE = 10;  // sleeps of 256 cycles
 __device__ __forceinline__ bool front_workgroup(const BlpArgs &b, bool leader) {
     announce_start(b, leader);  // (here because every dispatcher loop comes through here first)
     if (b.front == 0 || (int)blockIdx.x >= b.front) return false;
@@ -293,7 +298,7 @@ __device__ __forceinline__ bool front_workgroup(const BlpArgs &b, bool leader) {
         return __builtin_amdgcn_readfirstlane(stop) != -1 || __builtin_amdgcn_readfirstlane(n) >= target;
     };
     if (tid < 64) {
-        for (int look = 0; look < (1 << 17); ++look) {  // 1-2 us per look: at most about a quarter of a second
+        for (int look = 0; look < (1 << 17); ++look) {  // 3-4 us per look: at most about half a second
             int flag = 0;
             if (tid == 0) flag = __hip_atomic_load(b.flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             if (__builtin_amdgcn_readfirstlane(flag) != 0) {
@@ -301,7 +306,8 @@ __device__ __forceinline__ bool front_workgroup(const BlpArgs &b, bool leader) {
                 break;
             }
             if (two ? told() : device_look(tid)) break;
-            __builtin_amdgcn_s_sleep(4);
+#pragma unroll 1
+            for (int pause = 0; pause < FRONT_PAUSE && !(two && told()); ++pause) __builtin_amdgcn_s_sleep(4);
         }
         if (tid == 0) tell();
     } else if (two && tid < 128) {

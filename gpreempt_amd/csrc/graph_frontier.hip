@@ -130,6 +130,31 @@ __device__ __forceinline__ bool gf_walk(const u32x4 *ids, unsigned begin, unsign
     return false;
 }
 
+// The words in which the workgroups say how the iteration goes: a set of them, in lines of its own, per XCD where the caller has
+// room for that (gp_graph_iter_params::sets).  In one set, the stores of all wavefronts go through eight L2s to a line that moves from
+// one to the other, and with it what else it holds: in a line with claim counters or with the words that the launch's
+// workgroups read first, every second pull over 2^20 vertices took 56 us for 46.  PageRank at 2^20 vertices of degree 16
+// 3600 -> 3385 us, at 2^17 of degree 4 441 -> 392 (one set, in a line of its own: 3400 and 435).
+constexpr unsigned kSetInts = 32;
+static_assert(GP_GRAPH_SETS == kXcds, "a set per XCD");
+__device__ __forceinline__ unsigned *own_words(const gp_graph_iter_params &p) { return p.changed + (p.sets ? blockIdx.x % kXcds * kSetInts : 0u); }
+// What the launch before said: lane 8 * w + x reads word w of set x, for the first five words.
+struct WordsBefore {
+    unsigned mine = 0;
+    __device__ __forceinline__ explicit WordsBefore(const gp_graph_iter_params &p) {
+        const unsigned lane = threadIdx.x & 63, word = lane / kXcds, set = lane % kXcds;
+        if (p.prev_changed && word < 5 && (p.sets || set == 0)) mine = p.prev_changed[set * kSetInts + word];
+    }
+    __device__ __forceinline__ bool any(unsigned word) const { return (__builtin_amdgcn_ballot_w64(mine != 0) >> word * kXcds & 0xFF) != 0; }
+    // f over a word of all sets, the same in every lane
+    template <class F> __device__ __forceinline__ unsigned fold(unsigned word, F &&f) const {
+        unsigned x = mine;
+#pragma unroll
+        for (int d = 1; d < kXcds; d <<= 1) x = f(x, (unsigned)__shfl_xor((int)x, d));
+        return (unsigned)__builtin_amdgcn_readlane((int)x, (int)(word * kXcds));
+    }
+};
+
 __device__ __forceinline__ void raise_changed(unsigned *word, bool mine) {
     if (__builtin_amdgcn_ballot_w64(mine) && (threadIdx.x & 63) == 0) *word = 1;
 }
@@ -180,8 +205,9 @@ __device__ __forceinline__ float pr_share(const gp_graph_iter_params &p, unsigne
 __device__ __forceinline__ void pr_report(const gp_graph_iter_params &p, int tile, bool up) {
     const unsigned long long ups = __builtin_amdgcn_ballot_w64(up);
     if (ups == 0 || (threadIdx.x & 63) != 0) return;
-    *p.changed = 1;
-    if (tile % GP_GRAPH_SAMPLED == 0) atomicAdd(p.changed + 1, (unsigned)__builtin_popcountll(ups));
+    unsigned *words = own_words(p);
+    words[0] = 1;
+    if (tile % GP_GRAPH_SAMPLED == 0) atomicAdd(words + 1, (unsigned)__builtin_popcountll(ups));
 }
 __device__ __forceinline__ void pr_push(const gp_graph_iter_params &p, const u32x4 *ids, unsigned v, float share) {
     if (!__builtin_amdgcn_ballot_w64(share != 0.f)) return;
@@ -207,8 +233,8 @@ __device__ __forceinline__ void pr_push(const gp_graph_iter_params &p, const u32
 __device__ __forceinline__ void sssp_lowest(const gp_graph_iter_params &p, unsigned cost) {
     for (int d = 32; d; d >>= 1) cost = min(cost, (unsigned)__shfl_xor((int)cost, d));
     // (a look first: it may be an old one, which is a higher cost; an atomic on one address takes 40 ns of everybody's time)
-    if (cost != GF_INF && (threadIdx.x & 63) == 0 && __hip_atomic_load(p.changed + 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < ~cost)
-        atomicMax(p.changed + 4, ~cost);
+    if (cost != GF_INF && (threadIdx.x & 63) == 0 && __hip_atomic_load(own_words(p) + 4, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < ~cost)
+        atomicMax(own_words(p) + 4, ~cost);
 }
 
 // What a tile is looked through for (the vertices on the frontier): read for several tiles at a time, and before the
@@ -249,7 +275,7 @@ __device__ __forceinline__ bool gf_tile(const gp_graph_iter_params &p, int tile,
             for (int j = 0; j < 4; ++j)
                 if (p.label[i[j]] == GF_INF) { p.label[i[j]] = p.level + 1; mine = true; }
         });
-        raise_changed(p.changed, mine);
+        raise_changed(own_words(p), mine);
         return left;
     } else if constexpr (KIND == GP_GRAPH_IT_SSSP) {
         bool on = key != 0;
@@ -264,7 +290,7 @@ __device__ __forceinline__ bool gf_tile(const gp_graph_iter_params &p, int tile,
             if (far) p.next_active[v] = 1;  // its turn comes with a later limit
         }
         if (find) sssp_lowest(p, far ? cost : GF_INF);
-        else raise_changed(p.changed + 3, on);
+        else raise_changed(own_words(p) + 3, on);
         if (on) { begin = p.row[v]; end = p.row[v + 1]; }
         bool mine = far, near = false;
         const u32x4 *weights = reinterpret_cast<const u32x4 *>(p.weights);
@@ -282,13 +308,14 @@ __device__ __forceinline__ bool gf_tile(const gp_graph_iter_params &p, int tile,
             }
         });
         if (left && on) p.active[v] = 1;  // its turn again when the tile is done again
-        raise_changed(p.changed, mine);
-        raise_changed(p.changed + 1, near);
+        raise_changed(own_words(p), mine);
+        raise_changed(own_words(p) + 1, near);
         return left;
     } else if constexpr (KIND == GP_GRAPH_IT_PR) {
         unsigned begin = 0, end = 0;
-        float r = 0.f;
-        if (in) { begin = p.row[v]; end = p.row[v + 1]; r = p.residual[v]; }
+        float r = 0.f, value = 0.f, degree = 0.f;
+        // (value and degree are wanted at the end; asked for there, they were one more trip to memory: 5000 vertices of degree 8, 338 -> 325 us a run)
+        if (in) { begin = p.row[v]; end = p.row[v + 1]; r = p.residual[v]; value = p.value[v]; degree = p.degree[v]; }
         const unsigned sub = threadIdx.x & 3, none = p.row_end;
         const bool is_long = end - begin > kLongRow;
         const unsigned stop = is_long ? begin : end;
@@ -330,10 +357,10 @@ __device__ __forceinline__ bool gf_tile(const gp_graph_iter_params &p, int tile,
         }
         const bool up = in && r > p.tolerance;
         if (in) {
-            __builtin_nontemporal_store(up ? pr_share(p, v, r) : 0.f, p.next_share + v);
+            __builtin_nontemporal_store(up && degree > 0.f ? r * p.alpha / degree : 0.f, p.next_share + v);
             __builtin_nontemporal_store(up ? 0.f : r, p.residual + v);
         }
-        if (up) __builtin_nontemporal_store(p.value[v] + r, p.value + v);
+        if (up) __builtin_nontemporal_store(value + r, p.value + v);
         pr_report(p, tile, up);
     } else if constexpr (KIND == GP_GRAPH_IT_PR_PUSH) {
         const float share = in ? p.share[v] : 0.f;
@@ -402,15 +429,16 @@ __device__ __forceinline__ bool gf_tile(const gp_graph_iter_params &p, int tile,
     return false;
 }
 
-__device__ __forceinline__ unsigned sssp_limit(const gp_graph_iter_params &p, bool *find) {
+__device__ __forceinline__ unsigned sssp_limit(const gp_graph_iter_params &p, const WordsBefore &before, bool *find) {
     unsigned limit = p.step;
     *find = false;
     if (p.prev_changed) {
         auto above = [&](unsigned x) { return x + p.step < x ? GF_INF : x + p.step; };
-        limit = p.prev_changed[2];
-        if (p.prev_changed[4]) limit = above(~p.prev_changed[4]);
-        else if (!p.prev_changed[1] && p.prev_changed[3]) limit = above(limit);
-        else *find = !p.prev_changed[1];
+        limit = (unsigned)__builtin_amdgcn_readlane((int)before.mine, 2 * kXcds);  // (set 0 has it: workgroup 0 wrote it)
+        const bool near = before.any(1);
+        if (before.any(4)) limit = above(~before.fold(4, [](unsigned a, unsigned b) { return max(a, b); }));
+        else if (!near && before.any(3)) limit = above(limit);
+        else *find = !near;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) p.changed[2] = limit;
     return limit;
@@ -418,10 +446,12 @@ __device__ __forceinline__ unsigned sssp_limit(const gp_graph_iter_params &p, bo
 
 // The launch tells the host that it has started, and how the iteration before it went (gp_graph_iter_params::started).
 // One store to host memory that nobody waits for; the next launch is queued while this one works.
-__device__ __forceinline__ void report_start(const gp_graph_iter_params &p, const BlpArgs &blp) {
-    if (!p.started || blockIdx.x != 0 || threadIdx.x != 0) return;
+__device__ __forceinline__ void report_start(const gp_graph_iter_params &p, const WordsBefore &before, const BlpArgs &blp) {
+    if (!p.started || blockIdx.x != 0 || threadIdx.x >= 64) return;
+    const unsigned count = before.fold(1, [](unsigned a, unsigned b) { return a + b; });
     unsigned low = GP_GRAPH_START_CHANGED;
-    if (p.prev_changed) low = p.prev_changed[0] ? GP_GRAPH_START_CHANGED | min(p.prev_changed[1], GP_GRAPH_START_COUNT) : 0u;
+    if (p.prev_changed) low = before.any(0) ? GP_GRAPH_START_CHANGED | min(count, GP_GRAPH_START_COUNT) : 0u;
+    if (threadIdx.x != 0) return;
     const int stop = blp.stop_index ? __hip_atomic_load(blp.stop_index, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : -1;
     if (stop != -1) low = GP_GRAPH_START_STOPPED | (unsigned)stop;
     __hip_atomic_store(p.started, (unsigned long long)p.seq << 32 | low, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -434,11 +464,12 @@ __device__ __forceinline__ void report_start(const gp_graph_iter_params &p, cons
 // sssp 39 / 71 (118 / 256 without), pagerank 32 / 57 (51 / 120), connected components 48 / 134 (278 / 598, linked at once).
 template <int KIND, int LOOP = LOOP_ANY>
 __global__ __launch_bounds__(GF_TILE) void graph_iter_kernel(gp_graph_iter_params p, int per, BlpArgs blp) {
-    report_start(p, blp);
-    if (p.prev_changed && *p.prev_changed == 0) return;  // converged before this iteration (the same answer for every workgroup)
+    const WordsBefore before(p);
+    report_start(p, before, blp);
+    if (p.prev_changed && !before.any(0)) return;  // converged before this iteration (the same answer for every workgroup)
     unsigned limit = 0;
     bool find = false;
-    if constexpr (KIND == GP_GRAPH_IT_SSSP) limit = sssp_limit(p, &find);
+    if constexpr (KIND == GP_GRAPH_IT_SSSP) limit = sssp_limit(p, before, &find);
     unsigned key[4];  // of the next tiles
     auto look = [&](int first, int count) {
 #pragma unroll

@@ -327,9 +327,9 @@ Status Workload::run_kernels(const std::vector<int> &kernels, GPUstream stream, 
 }
 
 // A launch's slot: its words, the claim counters and as many counters of the workgroups that have left it
-// (gp_preempt_ctx::done).  Behind the slots, gp_graph_iter_params::relay.
+// (gp_preempt_ctx::done), each in lines of 128 bytes of its own.  Behind the slots, gp_graph_iter_params::relay.
 static size_t per_kernel_ints(const PreemptEnv *env) { return (size_t)env->counter_groups * env->counter_stride; }
-constexpr size_t kWords = 16, kRelayInts = GP_GRAPH_RELAYS * 32;
+constexpr size_t kWords = GP_GRAPH_SETS * 32, kRelayInts = GP_GRAPH_RELAYS * 32;
 
 Status Workload::launch_slot(int i, bool fresh, GPUstream stream, const PreemptEnv *env) {
     gp_graph_iter_params p = queued_[i % kRing];
@@ -337,6 +337,7 @@ Status Workload::launch_slot(int i, bool fresh, GPUstream stream, const PreemptE
     p.changed = (unsigned *)slot;
     if (p.prev_changed) p.prev_changed = (const unsigned *)((int *)ring_ + slot_ints_ * ((i - (int)(uintptr_t)p.prev_changed) % kRing));
     p.started = (unsigned long long *)starts_dev_ + i % kRing;
+    p.sets = 1;
     p.seq = seq_of_[i % kRing] = ++seq_;
     gp_preempt_ctx ctx;
     if (env) {
@@ -488,9 +489,10 @@ Status Workload::compute(GPUstream stream, const PreemptEnv *env) {
             if (next & 1) std::swap(p.active, p.next_active);
             p.prev_changed = next ? (const unsigned *)(uintptr_t)1 : nullptr;  // (how many launches back that word is; launch_slot makes it an address)
             first_of.push_back(submitted_);
-            // (2^20 vertices of degree 16: 45-55 us for the pull, as much for atomics from one vertex in twenty-five.  The
-            // push begins a little below that, because going over to it takes a launch.)
-            if (pagerank) push = symmetric_ && sampled < n_ / GP_GRAPH_SAMPLED / (push ? 25 : 32);
+            // (2^20 vertices of degree 16: 46 us for the pull, as much for atomics from one vertex in thirty-five, and the count is
+            // two launches old while the vertices become more by an eighth per iteration.  The push begins a little below that,
+            // because going over to it takes a launch.  From one in twenty-five and back to it below one in 32: 1-2 % slower.)
+            if (pagerank) push = symmetric_ && sampled < n_ / GP_GRAPH_SAMPLED / (push ? 32 : 36);
             if (pagerank && pushing) {
                 p.kernel = GP_GRAPH_IT_PR_STEP;
                 p.gained = gained;

@@ -401,3 +401,64 @@ def test_pagerank_of_a_generated_graph_pushes(gp, ex_mod, tmp_path, n, deg, blp)
             launches.append(info["kernels_launched"] - before - info["iterations"])
     if n >= 30000:  # (going over to the push takes a launch; a small graph's sample of its vertices may miss the moment)
         assert min(launches[:2]) > max(launches[2:]), launches
+
+
+class IterParams(C.Structure):
+    vp = C.c_void_p
+    _fields_ = [("kernel", C.c_int), ("level", C.c_uint), ("vertex_count", C.c_uint), ("row_end", C.c_uint)] + [(n, C.c_void_p) for n in (
+        "row", "ids", "weights", "label", "cost", "parent", "active", "next_active", "comp", "share", "degree", "next_share", "residual",
+        "value", "gained", "next_gained")] + [("alpha", C.c_float), ("tolerance", C.c_float), ("step", C.c_uint), ("changed", C.c_void_p),
+        ("prev_changed", C.c_void_p), ("started", C.c_void_p), ("seq", C.c_uint), ("relay", C.c_void_p), ("sets", C.c_uint)]
+
+
+@pytest.mark.parametrize("sets", [0, 1])
+@pytest.mark.parametrize("gap", [1, 1000])
+def test_progress_words_in_one_set_and_in_eight(gp, sets, gap):
+    """Shortest paths over 3000 vertices (twelve workgroups) launch by launch through the C ABI: the words of an iteration say how the
+    next one goes on, whether they come in one set or in one per XCD.  gap: the weight of the one edge in the middle of the path
+    behind the random part, so that the limit has to be looked for where it is large."""
+    rng = np.random.default_rng(11)
+    n, random_part = 3000, 2900
+    edges = [(int(u), int(v), int(w)) for u, v, w in zip(rng.integers(0, random_part, 6000), rng.integers(0, random_part, 6000), rng.integers(1, 9, 6000)) if u != v]
+    edges += [(v - 1, v, gap if v == 2950 else 1) for v in range(1, n)]
+    edges += [(v, u, w) for u, v, w in edges]
+    lists = [[] for _ in range(n)]
+    for u, v, w in edges:
+        lists[u].append((v, w))
+    row, ids, weights = [0], [], []
+    for l in lists:
+        l = l + [(n, 0)] * (-len(l) % 4)
+        ids += [v for v, _ in l]
+        weights += [w for _, w in l]
+        row.append(len(ids) // 4)
+    ids += [n] * 4
+
+    def dev(x):
+        d = gp.DevBuf(x.nbytes)
+        d.upload(x)
+        return d
+
+    d_row, d_ids, d_w = dev(np.array(row, np.uint32)), dev(np.array(ids, np.uint32)), dev(np.array(weights + [0] * 4, np.uint32))
+    cost, active, next_active = dev(np.zeros(n + 1, np.uint32)), dev(np.zeros(n + 8, np.uint8)), dev(np.zeros(n + 8, np.uint8))
+    slot = 8 * 32 if sets else 32
+    rounds = 400
+    words = dev(np.zeros((rounds, slot), np.uint32))
+    s = gp.Stream(0)
+    p = IterParams(kernel=3, vertex_count=n, row_end=row[-1], row=d_row.ptr, ids=d_ids.ptr, weights=d_w.ptr, cost=cost.ptr, active=active.ptr,
+                   next_active=next_active.ptr, step=5, changed=words.ptr, sets=sets)
+    gp.launch("gp_launch_graph_iter", p, None, s)
+    p.kernel = 2
+    for i in range(rounds):
+        p.changed = words.ptr + 4 * slot * i
+        p.prev_changed = words.ptr + 4 * slot * (i - 1) if i else None
+        p.active, p.next_active = (active.ptr, next_active.ptr) if i % 2 == 0 else (next_active.ptr, active.ptr)
+        gp.launch("gp_launch_graph_iter", p, None, s)
+    s.sync()
+    said = words.download(np_dtype=np.uint8).view(np.uint32).reshape(rounds, -1, 32)
+    ran = said[:, :, 0].any(axis=1)
+    assert ran[0] and not ran[-1] and not ran[int(np.argmin(ran)):].any()  # it converged, and nothing ran behind that
+    assert (said[:int(np.argmin(ran)), 1:, :5].any() if sets else True)    # (the other sets are used)
+    indptr = np.cumsum([0] + [len(l) for l in lists])
+    indices = np.array([v for l in lists for v, _ in l])
+    want = G.sssp(indptr, indices, np.array([w for l in lists for _, w in l], np.uint32))[0]
+    assert np.array_equal(cost.download(np_dtype=np.uint8).view(np.uint32)[:n], want)

@@ -637,9 +637,9 @@ __global__ __launch_bounds__(NT) void softmax_kernel(gp_softmax_params p, BlpArg
 // is, and every kernel that normalises rows goes through this function, so that a row gets the same
 // bits wherever it is computed.
 // Sum over the 64 lanes, every lane getting the total.  The first four steps (partners 1, 2, 4 and 8 lanes
-// apart, inside a row of 16) are DPP moves, which run in the vector ALU; only the last two cross rows
-// and go through the LDS crossbar.  (Six crossbar shuffles per sum, from the sixteen wavefronts of a
-// workgroup that all normalise rows, made the layer-norm prologue of gemm_ln.hpp wait for the LDS pipe.)
+// apart, inside a row of 16) are DPP moves, the last two swaps of rows and halves: all run in the vector ALU.  (Shuffles go
+// through the LDS crossbar, and six per sum, from the sixteen wavefronts of a workgroup that all normalise rows, made the
+// layer-norm prologue of gemm_ln.hpp wait for the LDS pipe.)
 template <int CTRL> __device__ __forceinline__ float dpp_mov(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
@@ -656,13 +656,20 @@ __device__ __forceinline__ void wave_sum_rows(float (&s)[R]) {
     for (int q = 0; q < R; ++q) s[q] += dpp_mov<0x141>(s[q]);
 #pragma unroll
     for (int q = 0; q < R; ++q) s[q] += dpp_mov<0x140>(s[q]);
+    // (both results of a swap of a register with itself: one half or row of the pair, and the other)
 #pragma unroll
-    for (int o = 16; o <= 32; o <<= 1) {
-        float t[R];
+    for (int q = 0; q < R; ++q) {
+        const unsigned v = __builtin_bit_cast(unsigned, s[q]);
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        const unsigned a = r[0], b = r[1];
+        s[q] = __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
+    }
 #pragma unroll
-        for (int q = 0; q < R; ++q) t[q] = __shfl_xor(s[q], o, 64);
-#pragma unroll
-        for (int q = 0; q < R; ++q) s[q] += t[q];
+    for (int q = 0; q < R; ++q) {
+        const unsigned v = __builtin_bit_cast(unsigned, s[q]);
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        const unsigned a = r[0], b = r[1];
+        s[q] = __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
     }
 }
 // PRE: gamma and beta come as the lane's raw chunks (chunk lane + 64 i in slot i), fetched by the caller when

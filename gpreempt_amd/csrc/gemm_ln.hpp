@@ -16,10 +16,98 @@
 // the main loop and the reduction are those of WideKernel (wavefront w multiplies MFMA k-step w of
 // every K-block, partial tiles summed in wavefront order).
 #pragma once
+#include <type_traits>
 #include "elementwise_bodies.hpp"
 #include "gemm_wide.hpp"
 
 namespace gp {
+
+// Two rows of 65 to 96 chunks by one wavefront, with the bits of ln_rows_math.  There a lane holds chunks l and l + 64 of each row, and at 96
+// chunks every second instruction runs for half of the lanes.  Sixteen wavefronts, four to a SIMD, normalise the rows of a tile, and the
+// prologue's time is the number of vector instructions: so the chunks behind the 64th share a register, row 0's in the lower half of the
+// wavefront and row 1's in the upper.  A lane adds up its chunk l first and its chunk l + 64 behind it, as there: the upper half's sums of row 0
+// and the lower half's of row 1 change places in between.  430 -> 240 vector instructions with f16; BERT-base b1 s128 fp16 467 -> 456 us,
+// b2 s211 bf16 level (its conversions are instructions of their own, and its launches have more tiles than compute units).
+__device__ __forceinline__ void swap_halves(float &row0, float &row1) {  // row 0's upper half <-> row 1's lower half
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, row0), __builtin_bit_cast(unsigned, row1), false, false);
+    const unsigned lo = r[0], hi = r[1];
+    row0 = __builtin_bit_cast(float, lo);
+    row1 = __builtin_bit_cast(float, hi);
+}
+// x + the value in a half of `word`, and with f16 no conversion of its own (exact, so the sum is rounded once either way)
+template <typename T, int HALF> __device__ __forceinline__ float add_half(unsigned word, float x) {
+    if constexpr (std::is_same<T, _Float16>::value) {
+        float y;
+        if constexpr (HALF == 0) asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(y) : "v"(word), "v"(x));
+        else asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(y) : "v"(word), "v"(x));
+        return y;
+    } else {
+        return __builtin_bit_cast(float, HALF ? word & 0xFFFF0000u : word << 16) + x;
+    }
+}
+template <typename T> __device__ __forceinline__ void ln_pair_math(const out_u32x4 (&x)[3], int tail, int lane, int cols, float eps,
+                                                                   const out_u32x4 (&gamma)[2], const out_u32x4 (&beta)[2], out_u32x4 (&y)[3]) {
+    static_assert(sizeof(T) == 2, "two values to a word");
+    const bool behind = (lane & 31) < tail;  // this lane has a chunk behind the 64th
+    float sum[2], sq[2];
+    auto add_chunk = [](const out_u32x4 &c, float s) {
+#pragma unroll
+        for (int w = 0; w < 4; ++w) s = add_half<T, 1>(c[w], add_half<T, 0>(c[w], s));
+        return s;
+    };
+    sum[0] = add_chunk(x[0], 0.f);
+    sum[1] = add_chunk(x[1], 0.f);
+    swap_halves(sum[0], sum[1]);
+    sum[0] = add_chunk(x[2], sum[0]);  // (zeros where there is no chunk)
+    swap_halves(sum[0], sum[1]);
+    wave_sum_rows<2>(sum);
+    // x / cols with the bits of the division, in three instructions for ten, from the rounded reciprocal: its product, corrected by the exact
+    // remainder (Markstein).  With f16 only, whose sums of squares cannot overflow: of an infinity the remainder makes NaN.
+    const float n = (float)cols, c = 1.0f / n;
+    auto over_cols = [&](float v) {
+        if constexpr (!std::is_same<T, _Float16>::value) return v / n;
+        const float q = v * c;
+        return __builtin_fmaf(__builtin_fmaf(-q, n, v), c, q);
+    };
+    const float mean[2] = {over_cols(sum[0]), over_cols(sum[1])};
+    const float mean_behind = lane < 32 ? mean[0] : mean[1];
+    float d[3][8];
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const float m = c < 2 ? mean[c] : mean_behind;
+            d[c][2 * w] = add_half<T, 0>(x[c][w], -m);
+            d[c][2 * w + 1] = add_half<T, 1>(x[c][w], -m);
+        }
+    // (the first product of a row is the fused one and its second the rounded one, as the compiler pairs them there)
+    auto first_squares = [](const float (&v)[8]) {
+        float s = __builtin_fmaf(v[0], v[0], v[1] * v[1]);
+#pragma unroll
+        for (int j = 2; j < 8; ++j) s = __builtin_fmaf(v[j], v[j], s);
+        return s;
+    };
+    sq[0] = first_squares(d[0]);
+    sq[1] = first_squares(d[1]);
+    swap_halves(sq[0], sq[1]);
+    float with = sq[0];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) with = __builtin_fmaf(d[2][j], d[2][j], with);
+    sq[0] = behind ? with : sq[0];
+    swap_halves(sq[0], sq[1]);
+    wave_sum_rows<2>(sq);
+    const float inv[2] = {rsqrtf(over_cols(sq[0]) + eps), rsqrtf(over_cols(sq[1]) + eps)};
+    const float inv_behind = lane < 32 ? inv[0] : inv[1];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        float ga[8], be[8], o[8];
+        VecIO<T>::unpack(gamma[c / 2], ga);
+        VecIO<T>::unpack(beta[c / 2], be);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o[j] = __builtin_fmaf(d[c][j] * (c < 2 ? inv[c] : inv_behind), ga[j], be[j]);
+        y[c] = VecIO<T>::pack(o);
+    }
+}
 
 template <typename T, int BM, int BN, int WAVES, int STAGES>
 struct LnWideKernel {
@@ -95,13 +183,47 @@ struct LnWideKernel {
         if (!SINGLE) __syncthreads();  // the previous tile of this workgroup may still be reading LDS
 
         // ---- the rows of A: normalise, keep in LDS, store once -------------------------------------
-        // wavefront w takes rows w, w + WAVES, ...; lane l holds chunks l and l + 64 of a row.  The rows are
-        // asked for first and B only once they are here: the wait for them would otherwise also wait for
-        // B (the counter of outstanding loads does not tell them apart), and B's way from memory is then
-        // covered by the arithmetic on the rows.
-        {
-            constexpr int RPW = BM / WAVES;
-            const int chunks = g.K / VEC;
+        // wavefront w takes rows w, w + WAVES, ...; lane l holds chunks l and l + 64 of a row.  B is asked for behind the rows, so that the
+        // arithmetic on them covers its way from memory.  (It takes longer than that: 128 x 2304 x 768 spends 5000 ticks until the rows
+        // and the first stage are there, and 1900 more on the rows; 3300 more before ln_pair_math.)
+        constexpr int RPW = BM / WAVES;
+        const int chunks = g.K / VEC, tail = chunks - 64;
+        auto first_stages = [&]() {
+#pragma unroll
+            for (int s = 0; s < PRE; ++s) {
+                if (s < NS) issue(s);
+                if (s == 0 && early && wave == 0) load_lds4(cc.stop_index, (unsigned)(size_t)(__attribute__((address_space(3))) void *)early_slot);
+            }
+            asked();
+        };
+        // chunk ch of row r is chunk ch % 8 of K-block ch / 8, at the swizzled position
+        auto keep = [&](int r, int ch, const out_u32x4 &y) {
+            *(out_u32x4 *)(a_res + (size_t)(ch >> 3) * A_BLK_BYTES + r * RB + ((ch & 7) ^ ((r >> 1) & 7)) * 16) = y;
+        };
+        if (RPW == 2 && tail > 0 && tail <= 32) {
+            // (no branch stands around these loads and what is computed from them, so the wait for the rows leaves B, asked for behind them, alone)
+            const int m = m0 + wave, over = lane >> 5, ch = 64 + (lane & 31);
+            const int r0 = m < g.M ? m : g.M - 1, r1 = m + WAVES < g.M ? m + WAVES : g.M - 1;
+            const bool behind = (lane & 31) < tail;
+            const int at = behind ? ch : 0;  // (a chunk of the row for the lanes that have none)
+            const T *a0 = A + (long)r0 * g.lda, *a1 = A + (long)r1 * g.lda;
+            out_u32x4 x[3] = {*(const out_u32x4 *)(a0 + lane * VEC), *(const out_u32x4 *)(a1 + lane * VEC), *(const out_u32x4 *)((over ? a1 : a0) + at * VEC)};
+            const T *ga = (const T *)g.ln_gamma, *be = (const T *)g.ln_beta;
+            const out_u32x4 gamma[2] = {*(const out_u32x4 *)(ga + lane * VEC), *(const out_u32x4 *)(ga + at * VEC)};
+            const out_u32x4 beta[2] = {*(const out_u32x4 *)(be + lane * VEC), *(const out_u32x4 *)(be + at * VEC)};
+            __builtin_amdgcn_sched_barrier(0);
+            first_stages();
+            __builtin_amdgcn_sched_barrier(0);
+            if (tail < 32) {
+#pragma unroll
+                for (int w = 0; w < 4; ++w) x[2][w] = behind ? x[2][w] : 0u;
+            }
+            out_u32x4 y[3];
+            ln_pair_math<T>(x, tail, lane, g.K, g.ln_eps, gamma, beta, y);
+            keep(wave, lane, y[0]);
+            keep(wave + WAVES, lane, y[1]);
+            if (behind) keep(wave + over * WAVES, ch, y[2]);
+        } else {  // (the waits stand inside branches here, and the compiler's for the rows would be one for B too: B is asked for when they are there)
             out_u32x4 rx[RPW][MAXC];
 #pragma unroll
             for (int q = 0; q < RPW; ++q) {
@@ -131,12 +253,7 @@ struct LnWideKernel {
                 for (int q = 0; q < RPW; ++q) asm volatile("" : "+v"(rx[q][i]) :: "memory");  // the rows have arrived
                 asm volatile("" : "+v"(graw[i]), "+v"(braw[i]) :: "memory");
             }
-#pragma unroll
-            for (int s = 0; s < PRE; ++s) {
-                if (s < NS) issue(s);
-                if (s == 0 && early && wave == 0) load_lds4(cc.stop_index, (unsigned)(size_t)(__attribute__((address_space(3))) void *)early_slot);
-            }
-            asked();
+            first_stages();
             float v[RPW][MAXC][VEC];
 #pragma unroll
             for (int q = 0; q < RPW; ++q)
@@ -149,15 +266,11 @@ struct LnWideKernel {
             ln_rows_math<T, MAXC, RPW, true>(v, chunks, lane, g.K, g.ln_eps, (const T *)g.ln_gamma, (const T *)g.ln_beta, graw, braw, y);
 #pragma unroll
             for (int q = 0; q < RPW; ++q) {
-                const int r = wave + q * WAVES, m = m0 + r;
+                const int r = wave + q * WAVES;
 #pragma unroll
                 for (int i = 0; i < MAXC; ++i) {
                     const int ch = lane + i * 64;
-                    if (ch < chunks) {
-                        // chunk ch of the row is chunk ch % 8 of K-block ch / 8, at the swizzled position
-                        const int blk = ch >> 3, phys = (ch & 7) ^ ((r >> 1) & 7);
-                        *(out_u32x4 *)(a_res + (size_t)blk * A_BLK_BYTES + r * RB + phys * 16) = y[q][i];
-                    }
+                    if (ch < chunks) keep(r, ch, y[q][i]);
                 }
             }
         }
@@ -192,7 +305,6 @@ struct LnWideKernel {
             // eagerly behind a stopped kernel normalised rows of an incomplete x, and must leave (above) without
             // having written anything.  Every wavefront stores the rows it normalised, from their copy in LDS.
             if (s == 0 && t.x == 0) {
-                const int chunks = g.K / VEC;
 #pragma unroll
                 for (int q = 0; q < BM / WAVES; ++q) {
                     const int r = wave + q * WAVES, m = m0 + r;

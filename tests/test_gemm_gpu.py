@@ -773,6 +773,32 @@ def test_gemm_with_layernorm_prologue_has_the_bits_of_two_launches(gp, dt, M, N,
             assert np.array_equal(dLN.download(), ln_two) and np.array_equal(dC.download(), c_two), (groups, frac)
 
 
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("K", [512, 576, 704, 768, 832])
+def test_layernorm_prologue_rows_of_every_length(gp, dt, K):
+    """The normalised rows of the one launch and of gp_launch_layernorm, bit for bit, where a row has 64 chunks, up to 96 (two rows of a
+    wavefront share the registers of what is behind the 64th) and more, for subnormal, large and infinite values and NaN; the
+    last tile has one row."""
+    rng = np.random.default_rng(K)
+    dtype, M, N = gp.DTYPE_BY_NAME[dt], 33 + 64, 64
+    X = rng.normal(0.3, 1, (M, K)).astype(np.float32)
+    X[:32] *= np.float32(2.0) ** -np.arange(32, dtype=np.float32)[:, None]
+    X[40] = 60000.0 * rng.choice([-1, 1], K)
+    X[41, 3], X[42, K - 1], X[43, K - 8] = np.inf, -np.inf, np.nan
+    X[44] = 0
+    X = O.round_to(X, dt)
+    arrays = [O.round_to(a.astype(np.float32), dt) for a in (X, rng.uniform(-1, 1, (N, K)), rng.uniform(0.5, 1.5, K), rng.normal(0, 0.2, K))]
+    dX, dB, dg, dbeta = (gp.DevBuf.from_array(a, dtype) for a in arrays)
+    two, one, dC = gp.DevBuf(M * K * 2), gp.DevBuf(M * K * 2), gp.DevBuf(M * N * 2)
+    gp.launch("gp_launch_layernorm", gp.LayernormParams(dtype, M, K, dX.ptr, None, dg.ptr, dbeta.ptr, two.ptr, 1e-12))
+    gp.launch("gp_launch_gemm", gp.GemmParams(dtype=dtype, M=M, N=N, K=K, A=dX.ptr, lda=K, B=dB.ptr, ldb=K, b_is_nk=1, C=dC.ptr, ldc=N, alpha=1.0, act=0,
+                                              batch=1, ln_gamma=dg.ptr, ln_beta=dbeta.ptr, ln_out=one.ptr, ln_eps=1e-12))
+    gp.check(gp.lib().gp_stream_sync(None))
+    a, b = two.download(dtype, (M, K)), one.download(dtype, (M, K))
+    assert np.isnan(a[41:44]).all() and np.isfinite(a[:41]).all()
+    assert np.array_equal(a, b, equal_nan=True)
+
+
 def test_layernorm_prologue_is_refused_where_it_does_not_fit(gp):
     dA = gp.DevBuf(1 << 20)
     def params(**kw):

@@ -190,6 +190,8 @@ struct PipeKernel {
     // The stop words are fetched with every stage (so that every wave issues the same number of
     // loads) but looked at every POLL_EVERY-th K-step: about every 2.5 us for either tile size.
     static constexpr int POLL_EVERY = BM >= 256 ? 2 : 4;
+    // 16-bit GEMM tiles of 256 x 256 take a K-step in four phases (see the loop)
+    static constexpr bool PHASED = BM == 256 && BN == 256 && WAVES == 8 && STAGES == 2 && sizeof(T) == 2 && !CONV && !SPLITK && !PRE;
     static_assert(!CKPT || !SPLITK, "checkpointing is built for the bodies without split K");
     static_assert(WAVES == 4 || (WAVES == 8 && !SPLITK), "4 wavefronts, or 8 without split K");
     static_assert(BM % 32 == 0 && BN % 32 == 0 && A_PW >= 1 && B_PW >= 1, "tile shape");
@@ -249,6 +251,9 @@ struct PipeKernel {
         const int c_base = cpos ^ (rig >> 1);
         auto chunk_of = [&](int slot) { return c_base ^ ((slot & 1) << 2); };
         const int a_row0 = m0 + wave * A_PW * 8 + rig, b_row0 = n0 + wave * B_PW * 8 + rig;
+        // a slot's first row in the tile.  PHASED: slots 0 and 1 in the rows of A that the first two phases read, or of B that the first and the last do
+        auto a_at = [&](int j) { return PHASED ? (wave >> 2) * 128 + (j >> 1) * 64 + (2 * wave + (j & 1)) % 8 * 8 : (wave * A_PW + j) * 8; };
+        auto b_at = [&](int j) { return PHASED ? (wave >> 1) * 64 + (j >> 1) * 32 + (2 * wave + (j & 1)) % 4 * 8 : (wave * B_PW + j) * 8; };
         const T *a_org[CONV ? A_PW : 1];         // CONV: the slot's window origin (may lie outside the image)
         int a_h0[CONV ? A_PW : 1], a_w0[CONV ? A_PW : 1];
         unsigned a_off[CONV == 1 ? 1 : A_PW], b_off[B_PW];
@@ -276,15 +281,15 @@ struct PipeKernel {
         // turn: 8192^3 bf16 with checkpoints, its clears included, 970 -> 951 us, 4096^3 fp32 1098 -> 1016, 6000 x 5000 x 2048 fp16 152 -> 146.
         // (`near`: the tile's rows lie within a descriptor's 2 GB.  Otherwise an address of 64 bits is worked out for every load.)
         const long far = (long)kBufferEnd / (long)sizeof(T) - g.K;
-        const bool near = TAPS || !DESC || ((CONV || (long)BM * g.lda <= far) && (long)BN * g.ldb <= far);
+        const bool near = TAPS || !DESC || PHASED || ((CONV || (long)BM * g.lda <= far) && (long)BN * g.ldb <= far);
         if (!CONV && DESC) {
 #pragma unroll
             for (int j = 0; j < (CONV ? 1 : A_PW); ++j)
-                a_off[j] = a_row0 + j * 8 < g.M ? near ? ((unsigned)(a_row0 - m0 + j * 8) * (unsigned)g.lda + (unsigned)(chunk_of(wave * A_PW + j) * VEC)) * (unsigned)sizeof(T) : 0u : kBufferEnd;
+                a_off[j] = m0 + a_at(j) + rig < g.M ? near ? ((unsigned)(a_at(j) + rig) * (unsigned)g.lda + (unsigned)(chunk_of(wave * A_PW + j) * VEC)) * (unsigned)sizeof(T) : 0u : kBufferEnd;
         }
 #pragma unroll
         for (int j = 0; j < (DESC ? B_PW : 0); ++j)
-            b_off[j] = b_row0 + j * 8 < g.N ? near ? ((unsigned)(b_row0 - n0 + j * 8) * (unsigned)g.ldb + (unsigned)(chunk_of(wave * B_PW + j) * VEC)) * (unsigned)sizeof(T) : 0u : kBufferEnd;
+            b_off[j] = n0 + b_at(j) + rig < g.N ? near ? ((unsigned)(b_at(j) + rig) * (unsigned)g.ldb + (unsigned)(chunk_of(wave * B_PW + j) * VEC)) * (unsigned)sizeof(T) : 0u : kBufferEnd;
         const u32x4 rsrc_a = buffer_of(CONV ? A - (long)(g.ph * g.W + g.pw) * g.lda : A + (long)m0 * g.lda), rsrc_b = buffer_of(B + (long)n0 * g.ldb);
         const bool conv_fast = TAPS || (CONV && (g.Cin % BK == 0));  // a K-step never straddles a filter tap
         // Pointers with the lane's chunk already added, one per parity of the slot number j: a load's address is this plus a
@@ -402,12 +407,12 @@ struct PipeKernel {
                     const int jj = CONV ? 0 : j;
                     const bool ok = sa.k0 + kc < g.K;
                     if (__builtin_expect(near, 1)) {
-                        load_lds16_buffer<SINGLE || CKPT>(rsrc_a, ok ? a_off[jj] : kBufferEnd, sa.k_bytes, sa.sbase + (unsigned)((wave * A_PW + j) * 8 * RB));
+                        load_lds16_buffer<SINGLE || CKPT>(rsrc_a, ok ? a_off[jj] : kBufferEnd, sa.k_bytes, sa.sbase + (unsigned)(a_at(j) * RB));
                         return;
                     }
-                    src = ok && a_off[jj] != kBufferEnd ? A + ((long)(a_row0 + j * 8) * g.lda + (sa.k0 + kc)) : zero;
+                    src = ok && a_off[jj] != kBufferEnd ? A + ((long)(m0 + a_at(j) + rig) * g.lda + (sa.k0 + kc)) : zero;
                 }
-                load_lds16(src, sa.sbase + (unsigned)((wave * A_PW + j) * 8 * RB));
+                load_lds16(src, sa.sbase + (unsigned)(a_at(j) * RB));
             } else {
                 const int j = l - A_PW;
                 const int kc = chunk_of(wave * B_PW + j) * VEC;
@@ -427,12 +432,12 @@ struct PipeKernel {
                 } else {
                     const bool ok = sa.k0 + kc < g.K;
                     if (__builtin_expect(near, 1)) {
-                        load_lds16_buffer<SINGLE || CKPT>(rsrc_b, ok ? b_off[j] : kBufferEnd, sa.k_bytes, sa.sbase + (unsigned)(A_BYTES + (wave * B_PW + j) * 8 * RB));
+                        load_lds16_buffer<SINGLE || CKPT>(rsrc_b, ok ? b_off[j] : kBufferEnd, sa.k_bytes, sa.sbase + (unsigned)(A_BYTES + b_at(j) * RB));
                         return;
                     }
-                    src = ok && b_off[j] != kBufferEnd ? B + ((long)(b_row0 + j * 8) * g.ldb + (sa.k0 + kc)) : zero;
+                    src = ok && b_off[j] != kBufferEnd ? B + ((long)(n0 + b_at(j) + rig) * g.ldb + (sa.k0 + kc)) : zero;
                 }
-                load_lds16(src, sa.sbase + (unsigned)(A_BYTES + (wave * B_PW + j) * 8 * RB));
+                load_lds16(src, sa.sbase + (unsigned)(A_BYTES + b_at(j) * RB));
             }
         };
         auto issue = [&](int kt) {
@@ -622,6 +627,123 @@ struct PipeKernel {
         GP_PROBE(1);
         if (!SINGLE) __syncthreads();  // the previous tile of this workgroup may still be reading LDS
         if constexpr (PRE) pre_fetch_table<T, WAVES>(g, lds0 + (unsigned)LDS_BYTES, wave, lane);  // (older than the first stage: the wait for that covers it)
+        int kt = kt0, stopped = 0;
+        if constexpr (PHASED) {
+            // A K-step in four phases of eight MFMAs, each a quarter of the wavefront's block over the whole depth of the K-step, so that
+            // parts of a stage's buffer are free long before the stage is done: A's first half (the wavefront's rows 0-63) with B's first
+            // (its columns 0-31), A's first with B's second, A's second with B's second, A's second with B's first.  Stage kt + 2 follows into the
+            // place of stage kt half by half: A's and B's first behind the barrier in front of the second phase, the others behind the one in
+            // front of the last.  So a load has one to one and a half K-steps to arrive in; in the loop below, which fetches a stage while
+            // the one before it is multiplied, the last of its loads has half a K-step, and the wait for it is where the matrix cores stood idle.
+            // (The waits count the loads behind the ones that are needed, and every K-step issues the same ones: what lies past K is fetched from
+            // beyond the descriptor's end.)  8192^3 bf16 in turn with the loop below, its clears included: with checkpoints 953 -> 889 us, plain
+            // 888 -> 835.  What bounds it now: LDS, read and written for about as many cycles as the MFMAs take, and the power the
+            // multipliers draw.  (The reads spread evenly over the phases, with the second barrier a phase earlier: plain 848 -> 875.)
+            // Wavefront 0 asks for the stop index with every second stage, and wavefront 1 for the flag when it is the workgroup's turn (see
+            // issue_one).  Nobody else asks for anything in their place: the waits below count the operand loads, and a wavefront that has
+            // asked for a word as well waits a load longer than it has to.  (Reads past the caches of one address come back one per 11 ns; with
+            // eight wavefronts of 256 workgroups reading a word with every stage, six of them zeros, 8192^3 bf16 took 908 us for 893.)
+            auto ask = [&](int stage) {
+                if (!can_ckpt || (stage & (POLL_EVERY - 1)) != 0) return;
+                const unsigned to = lds0 + (unsigned)RING_BYTES + (unsigned)wave * 256;
+                if (wave == 0) load_lds4(cc.stop_index, to);
+                else if (blockIdx.x < 8 && cc.flag && (int)((wall_clock64() >> 9) & 7) == (int)blockIdx.x) load_lds4(cc.flag, to);
+            };
+            if (CKPT && tid == 64) pollw[64] = 0;
+            // A wavefront at its MFMAs goes before the other one of its SIMD, which is fetching or waiting: plain 848 -> 835 us; with checkpoints 893 -> 901.
+            auto ahead = [&](auto level) { if constexpr (!CKPT) __builtin_amdgcn_s_setprio(decltype(level)::value); };
+            auto issue_near = [&](const StageAddr &sa, int l) {  // (issue_one without what operands beyond a descriptor's 2 GB take)
+                const int j = l < A_PW ? l : l - A_PW;
+                const unsigned at = chunk_of(j) * VEC < g.K - sa.k0 ? l < A_PW ? a_off[CONV == 1 ? 0 : j] : b_off[j] : kBufferEnd;
+                load_lds16_buffer<SINGLE || CKPT>(l < A_PW ? rsrc_a : rsrc_b, at, sa.k_bytes, sa.sbase + (unsigned)(l < A_PW ? a_at(j) * RB : A_BYTES + b_at(j) * RB));
+            };
+            u32x4 fa0[2][KSTEPS], fa1[2][KSTEPS], fb0[KSTEPS], fb1[KSTEPS];
+            auto read_a = [&](u32x4 (&f)[2][KSTEPS], int stage, int first, int ks) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) f[i][ks] = frag(stage, 0, wm * WM + (first + i) * 32 + l32, ks * 2 + half);
+            };
+            auto read_b = [&](u32x4 (&f)[KSTEPS], int stage, int j, int ks) { f[ks] = frag(stage, A_BYTES, wn * WN + j * 32 + l32, ks * 2 + half); };
+            static_for<0, 2>([&](auto sc) {
+                const StageAddr sa = stage_addr(kt0 + decltype(sc)::value);
+                issue_near(sa, 0); issue_near(sa, 1); issue_near(sa, 4); issue_near(sa, 5);
+                if (CKPT && wave < 2) ask(kt0 + decltype(sc)::value);
+                issue_near(sa, 6); issue_near(sa, 7); issue_near(sa, 2); issue_near(sa, 3);
+                if (!CKPT && decltype(sc)::value == 0 && early && wave == 0) load_lds4(cc.stop_index, (unsigned)(size_t)(__attribute__((address_space(3))) void *)early_slot);
+            });
+            asked();
+            wait_vmcnt<2 + LPS>();  // all of the first stage but A's second half
+            stage_barrier();
+            static_for<0, KSTEPS>([&](auto kc) { read_a(fa0, kt0 & 1, 0, decltype(kc)::value); read_b(fb0, kt0 & 1, 0, decltype(kc)::value); });
+            for (; kt < KT; ++kt) {
+                const int stage = kt & 1;
+                static_for<0, KSTEPS>([&](auto kc) { read_b(fb1, stage, 1, decltype(kc)::value); });
+                __builtin_amdgcn_sched_barrier(0);
+                ahead(IntC<1>{});
+                static_for<0, 2 * KSTEPS>([&](auto qc) {
+                    constexpr int ks = decltype(qc)::value / 2, i = decltype(qc)::value % 2;
+                    Elem<T>::mma(fa0[i][ks], fb0[ks], acc[i][0]);
+                });
+                ahead(IntC<0>{});
+                __builtin_amdgcn_sched_barrier(0);
+                wait_vmcnt<LPS>();  // this stage's second half of A (behind it: a stage less A's and B's first halves, and those of the next)
+                stage_barrier();       // A's and B's first halves have been read by everybody
+                if constexpr (!CKPT) {
+                    bool leave = early && kt == kt0 && __builtin_amdgcn_readfirstlane(read_lds_word(early_slot)) != -1;
+                    if constexpr (LOOKS) {
+                        if (looking && ((kt - kt0) & (LOOK_EVERY - 1)) == LOOK_EVERY / 2) leave = __builtin_amdgcn_readfirstlane(read_lds_word(early_slot + 64)) != -1;
+                        if (looking && ((kt - kt0) & (LOOK_EVERY - 1)) == 0 && wave == 0)
+                            load_lds4(cc.stop_index, (unsigned)(size_t)(__attribute__((address_space(3))) void *)(early_slot + 64));
+                    }
+                    if (leave) { stopped = 1; break; }
+                    if constexpr (LOOKS) if (looking && kt == KT - 1) announce();
+                }
+                const StageAddr sa = stage_addr(kt + 2);
+                static_for<0, KSTEPS>([&](auto kc) { read_a(fa1, stage, 2, decltype(kc)::value); });
+                __builtin_amdgcn_sched_barrier(0);
+                ahead(IntC<1>{});
+                static_for<0, 2 * KSTEPS>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value, ks = q / 2, i = q % 2;
+                    Elem<T>::mma(fa0[i][ks], fb1[ks], acc[i][1]);
+                    if constexpr (q % 4 == 0) issue_near(sa, q / 4);
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+                static_for<0, 2 * KSTEPS>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value, ks = q / 2, i = q % 2;
+                    Elem<T>::mma(fa1[i][ks], fb1[ks], acc[2 + i][1]);
+                    if constexpr (q % 4 == 0) issue_near(sa, 4 + q / 4);
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+                ahead(IntC<0>{});
+                wait_vmcnt<6>();  // the next stage but for its second half of A (behind it: that, and four loads of this K-step)
+                stage_barrier();  // the second halves have been read by everybody
+                int stop_word = -1, flag_word = 0;
+                if constexpr (CKPT) {
+                    if (can_ckpt && ((kt + 1) & (POLL_EVERY - 1)) == 0) {  // what was asked for with stage kt + 1
+                        stop_word = pollw[0];
+                        flag_word = pollw[64];
+                    }
+                    if (wave < 2) ask(kt + 2);
+                }
+                ahead(IntC<1>{});
+                static_for<0, KSTEPS>([&](auto kc) {
+                    constexpr int ks = decltype(kc)::value;
+                    Elem<T>::mma(fa1[0][ks], fb0[ks], acc[2][0]);
+                    read_a(fa0, stage ^ 1, 0, ks);
+                    issue_near(sa, ks < 2 ? 6 + ks : ks);
+                    Elem<T>::mma(fa1[1][ks], fb0[ks], acc[3][0]);
+                    read_b(fb0, stage ^ 1, 0, ks);
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+                ahead(IntC<0>{});
+                if constexpr (CKPT) {
+                    const int sw = __builtin_amdgcn_readfirstlane(stop_word), fw = __builtin_amdgcn_readfirstlane(flag_word);
+                    if (fw != 0 && tid == 0) record_stop(cc.stop_index, cc.kernel_id, cc.stamps);  // pass the host flag on
+                    if (((sw != -1) | (fw != 0)) && kt + 1 < KT) { stopped = 1; break; }
+                }
+            }
+            wait_vmcnt<0>();  // what was fetched beyond the last K-step lands in LDS as well
+            if (!CKPT && stopped) return true;
+        } else {
 #pragma unroll
         for (int s = 0; s < STAGES - 1; ++s) {
             if (kt0 + s < KT) issue(kt0 + s);
@@ -631,7 +753,6 @@ struct PipeKernel {
                 load_lds4(cc.stop_index, (unsigned)(size_t)(__attribute__((address_space(3))) void *)early_slot);
         }
         asked();
-        int kt = kt0, stopped = 0;
         // Later looks: after the first K-step the tile goes on in runs of LOOK_EVERY K-steps, as many as fit in front
         // of the last STAGES-1 K-steps.  Wavefront 0 fetches the word in front of a run, everybody reads it behind
         // the run (the waits and barriers of the K-steps between have made it land and be seen), and the runs take two
@@ -666,7 +787,8 @@ struct PipeKernel {
             wait_vmcnt<0>();  // operand loads still landing in LDS must not outlive the workgroup
             return true;
         }
-        if (!SPLITK && KT > kt0) mma_all((KSTEPS - 1) & 1);
+            if (!SPLITK && KT > kt0) mma_all((KSTEPS - 1) & 1);
+        }
         GP_PROBE(3);
         // When `stopped` (CKPT only), K-steps kt0..kt are in the accumulators and the "epilogue" below
         // writes them to the checkpoint slot instead of finishing the tile.  The loads of step kt+1

@@ -81,3 +81,31 @@ def test_far_pixels(gp, dtype_name, N, H, W, Cin, Cout, R, stride, pad, tile, va
     far = spread(gp, list(rows), stride_elems * es)
     p.in_, p.in_pix_stride = far.ptr, stride_elems
     assert np.array_equal(bits(), packed)
+
+
+@pytest.mark.parametrize("form", ["plain", "claims", "checkpoints"])
+@pytest.mark.parametrize("dtype_name", ["f16", "bf16"])
+def test_256_tiles_of_few_k_steps(gp, dtype_name, form):
+    """The 16-bit 256 x 256 body asks for two K-steps ahead of the one it multiplies, also where there are fewer: from a part of one
+    K-step to five, with and without a remainder, give the bits of 128 x 128 tiles (the same products in the same order); tiles with one row
+    and one column of the problem."""
+    dtype = gp.DTYPE_BY_NAME[dtype_name]
+    for M, N, K in [(256, 256, 8), (257, 260, 64), (300, 520, 72), (256, 512, 128), (513, 256, 136), (260, 257, 192), (256, 256, 256), (300, 300, 328)]:
+        rng = np.random.default_rng(M + N + K)
+        dA, dB, dbias = (gp.DevBuf.from_array(O.round_to(rng.uniform(-1, 1, s).astype(np.float32), dtype_name), dtype) for s in ((M, K), (N, K), (N,)))
+        outs = []
+        for tile in (128, 256):
+            out = gp.DevBuf(M * N * 2)
+            out.fill32(0x7E007E00)
+            p = gp.GemmParams(dtype=dtype, M=M, N=N, K=K, A=dA.ptr, lda=K, B=dB.ptr, ldb=K, b_is_nk=1, C=out.ptr, ldc=N, bias=dbias.ptr, alpha=0.5, act=gp.ACT_RELU,
+                              batch=1, tile_m=tile, tile_n=tile, variant=gp.MAT_PIPE)
+            ctx = None
+            if form != "plain":
+                blp = gp.BlpState(1, gp.Flag(), 32)
+                if form == "checkpoints":
+                    blp.enable_checkpoints(p)
+                ctx = blp.ctx()
+            gp.launch("gp_launch_gemm", p, ctx)
+            sync(gp)
+            outs.append(out.download().copy())
+        assert np.array_equal(*outs), (M, N, K)

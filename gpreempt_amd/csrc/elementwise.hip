@@ -135,9 +135,8 @@ int plan_attention(const gp_attention_params *p, EltPlan *out) {
     GP_REQUIRE(al16(p->q) && al16(p->k) && al16(p->v), "attention: 16-byte alignment");
     *out = EltPlan{};
     out->op = OP_ATTENTION; out->dtype = p->dtype;
-    const int qb = attention_queries_per_tile(p->seq);
-    out->sx = (p->seq + qb - 1) / qb; out->sy = p->batch * p->heads;
-    out->lds_bytes = attention_class_lds_bytes(p->seq);
+    out->sx = (p->seq + ATT_QB - 1) / ATT_QB; out->sy = p->batch * p->heads;
+    out->lds_bytes = attention_lds_bytes(attention_nb_class(p->seq));
     out->u.attn = AttnArgs{*p};
     if (out->u.attn.p.scale == 0.f) out->u.attn.p.scale = 1.f;
     return GP_SUCC;
@@ -181,8 +180,8 @@ int launch_elt_plan(const EltPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, g
         case OP_ATTENTION:
             switch (attention_nb_class(pl.u.attn.p.seq) * 2 + (pl.dtype == GP_F16)) {
 #define GP_ATT(NB)                                                                                                            \
-    case NB * 2 + 1: return launch_tiles(GP_KSET(attention_kernel<_Float16, NB), pl.sx, pl.sy, ctx, s, info, pl.u.attn, pl.lds_bytes); \
-    case NB * 2: return launch_tiles(GP_KSET(attention_kernel<__bf16, NB), pl.sx, pl.sy, ctx, s, info, pl.u.attn, pl.lds_bytes);
+    case NB * 2 + 1: return launch_tiles(GP_KSET(attention_kernel<_Float16, NB), pl.sx, pl.sy, ctx, s, info, pl.u.attn, pl.lds_bytes, 16, attention_threads(NB)); \
+    case NB * 2: return launch_tiles(GP_KSET(attention_kernel<__bf16, NB), pl.sx, pl.sy, ctx, s, info, pl.u.attn, pl.lds_bytes, 16, attention_threads(NB));
                 GP_ATT(4) GP_ATT(8) GP_ATT(12) GP_ATT(16)
 #undef GP_ATT
             }

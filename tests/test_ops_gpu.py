@@ -431,6 +431,51 @@ def test_fused_attention_preempt_resume_bit_exact(gp):
     assert np.array_equal(do.download(), want)
 
 
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (2, 2, 31), (1, 2, 65), (1, 2, 192), (2, 1, 256), (1, 2, 289), (1, 2, 511), (12, 12, 300)])
+def test_fused_attention_parts_without_keys_and_rows_off_16_bytes(gp, dt, shape):
+    """Sequences that leave some of the wavefronts sharing the keys without any, peaked scores of both signs, rows of the output that do not
+    start on 16 bytes: against fp64; and a launch stopped and resumed has the bits of the plain one.  The probabilities are rounded once to the
+    type, relative to the largest of their part, and the result once more: two roundings of half a unit."""
+    B, Hh, S = shape
+    d, Hd = 64, Hh * 64
+    rng = np.random.default_rng(S + 1000 * Hh)
+    qkv = rnd(rng, (B * S, 3 * Hd), dt, -4, 4)
+    dtype = gp.DTYPE_BY_NAME[dt]
+    es = gp.DTYPE_SIZE[dtype]
+    dq = gp.DevBuf.from_array(qkv, dtype)
+    ld = Hd + 4
+    do = gp.DevBuf(B * S * ld * es)
+    do.fill32(0)
+    p = gp.AttentionParams(dtype=dtype, batch=B, heads=Hh, seq=S, head_dim=d, q=dq.ptr, k=dq.ptr + Hd * es, v=dq.ptr + 2 * Hd * es,
+                           ld_qkv=3 * Hd, out=do.ptr, ld_out=ld, scale=-0.125)
+    gp.launch("gp_launch_attention", p)
+    sync(gp)
+    want = do.download().copy()
+    got = gp.from_storage(want, dtype).reshape(B, S, ld)
+    assert not got[:, :, Hd:].any()
+    x = qkv.astype(np.float64).reshape(B, S, 3, Hh, d)
+    q, k, v = (x[:, :, i].transpose(0, 2, 1, 3) for i in range(3))
+    sc = q @ k.transpose(0, 1, 3, 2) * -0.125
+    pr = np.exp(sc - sc.max(-1, keepdims=True))
+    pr /= pr.sum(-1, keepdims=True)
+    ref = (pr @ v).transpose(0, 2, 1, 3).reshape(B, S, Hd)
+    eps = 2.0 ** (-11 if dt == "f16" else -8)
+    assert np.abs(got[:, :, :Hd] - ref).max() <= 2 * eps * np.abs(qkv).max() + 1e-3 * eps
+
+    flag = gp.Flag()
+    st = gp.BlpState(1, flag)
+    do.fill32(0)
+    gp.launch("gp_launch_attention", p, st.ctx(inject_at=0, max_workgroups=2))
+    sync(gp)
+    assert flag.get() == 1
+    flag.set(0)
+    st.clear_stop()
+    gp.launch("gp_launch_attention", p, st.ctx(max_workgroups=2))
+    sync(gp)
+    assert np.array_equal(do.download(), want)
+
+
 def test_deep_preemptible_convolution_takes_small_tiles_with_the_same_bits(gp):
     """A preemptible launch finishes the tiles it holds before it leaves: where the rule would run 128 x 128 tiles
     over K >= 2304 (VGG-16's 256 -> 256 layers at 56 x 56), a launch with claim counters takes 64 x 64 tiles,

@@ -164,6 +164,8 @@ static int choose_body(MatPlan *pl, int tile, int tile_n, int variant) {
     pl->lds_bytes = body_lds_bytes(body, pl->dtype);
     // (what the 16-bit pipelined bodies' form for whole taps assumes)
     pl->taps = whole_taps && pl->dtype != GP_F32 && wide_ok;
+    // (... and their form for K-steps that straddle taps: inverses, and factors of 24 bits)
+    pl->straddles = pl->conv && !whole_taps && g.inv_cin && g.inv_s && g.K + 64 < (1 << 24) && (double)(g.R + 64) * g.W < 16777216.0 && buffer_ok(g, true, pl->dtype);
     // A convolution whose tiles' input windows are runs of consecutive pixels that fit in LDS fetches them once (gemm_window.hpp; where the
     // launcher picks the body itself; 16-bit, fp32 being bound by its arithmetic; 32 x 32 tiles: with 64 x 32 the four multiplying wavefronts,
     // which work out where a lane's row lies, are what a stage waits for, 0.76 us for the gather's 0.53, ResNet-152 b8 1530 -> 1560).

@@ -20,19 +20,23 @@ namespace gp {
 
 // Asks for the arguments that stand in front of a tile's first load, and for those of its epilogue, in one go.  Left to itself
 // the compiler reads them where they are used, in four or five batches one behind the other, each a trip of 0.2 us.
-template <bool CONV> __device__ __forceinline__ void read_args(const MatArgs &g, const BlpArgs &b) {
+// (INVERSES: of the channels and window columns too, for the form that finds its taps by them.)
+template <bool CONV, bool INVERSES> __device__ __forceinline__ void read_args(const MatArgs &g, const BlpArgs &b) {
     asm volatile("" ::"s"(b.total), "s"(b.sx), "s"(b.sy), "s"(b.order), "s"(b.inv_sx), "s"(b.inv_sy), "s"(b.grid), "s"(b.front), "s"(b.executed), "s"(b.stop_index), "s"(g.M), "s"(g.N), "s"(g.K),
                  "s"(g.A), "s"(g.lda), "s"(g.B), "s"(g.ldb), "s"(g.batch_inner), "s"(g.C), "s"(g.ldc), "s"(g.bias), "s"(g.alpha), "s"(g.act));
     if (CONV) asm volatile("" ::"s"(g.H), "s"(g.W), "s"(g.Cin), "s"(g.S), "s"(g.Ho), "s"(g.Wo), "s"(g.sh), "s"(g.sw), "s"(g.ph), "s"(g.pw), "s"(g.R), "s"(g.rcp_hw), "s"(g.rcp_wo));
+    if (INVERSES) asm volatile("" ::"s"(g.inv_cin), "s"(g.inv_s));
 }
 
+template <class K> struct K_divides { static constexpr bool value = false; };
+template <typename T, int BM, int BN, int ST> struct K_divides<PipeKernel<T, BM, BN, ST, 3, false>> { static constexpr bool value = true; };
 // LOOP: which dispatcher loop the instantiation is built around (tile_loop.hpp)
 constexpr int LOOP_LOOKS = 3;
 template <class TK, int LOOP>
 __global__ __launch_bounds__(TK::NT) void mat_kernel(MatArgs g, BlpArgs blp) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
     auto *lds = reinterpret_cast<typename TK::elem *>(lds_raw);
-    if constexpr (LOOP != LOOP_ANY) read_args<TK::conv>(g, blp);
+    if constexpr (LOOP != LOOP_ANY) read_args<TK::conv, K_divides<TK>::value>(g, blp);
     if constexpr (LOOP == LOOP_LOOKS)  // long tiles: fixed claims, and the body looks at the stop word every few K-stages
         tile_fixed_early<TK::NT, true>(blp, [&](TileIdx t, int *stop) {
             CkptCtx cc{stop, nullptr, nullptr, 0};
@@ -169,6 +173,8 @@ static int pipe_case(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, 
         if (pl.pre) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 0, false, false, 4, true>>(pl, ctx, s, info);
     if constexpr (sizeof(T) == 2)
         if (pl.taps) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 2, SPLITK>>(pl, ctx, s, info);
+    if constexpr (TILE >= 64 && !SPLITK)
+        if (pl.straddles) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 3, false>>(pl, ctx, s, info);
     if (pl.conv) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 1, SPLITK>>(pl, ctx, s, info);
     return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 0, SPLITK>>(pl, ctx, s, info);
 }

@@ -156,18 +156,22 @@ struct NoneAsked { __device__ __forceinline__ void operator()() const {} };
 // CONV: 1: a convolution; 2: one whose K-steps lie within a filter tap and whose operands fit buffers of 2 GB, of at most 32 taps
 // (a load is then a bit test, a select and the stage's uniform offset, where pointers of 64 bits were rebuilt at every tap and advanced at every
 // step: VGG-16 b16 fp16 1432 -> 1340 us, b8 907 -> 857, ResNet-50 b16 fp16 965 -> 947; 64 x 64 bodies 100 -> 72 registers).
+// 3: one whose K-steps straddle taps, through descriptors: a lane finds the tap of its chunk by two multiplications.  (1 divides, twice for every load, and a
+// K-step waits for that.  A preemptible launch, fp16: 7 x 7 over 8 channels at 224 x 224, stride 2, batch 8 27.0 -> 21.2 us, batch 1 10.8 -> 7.8; 5 x 5 over 48 at
+// 35 x 35, batch 16 20.6 -> 13.8; 3 x 3 over 80 at 73 x 73, batch 16, in 128 x 128 tiles 85 -> 60.  fp32, 7 x 7 over 4 channels, batch 1 14.1 -> 12.0.  What bounds
+// the first layers now is the way from the claim to the store of a tile with two to seven K-steps.)
 // PRE: the rows of A go through a scale, shift and ReLU first (gemm_pre.hpp).
 template <typename T, int BM, int BN, int STAGES, int CONV, bool SPLITK, bool CKPT = false, int NWAVES = 4, bool PRE = false>
 struct PipeKernel {
     using elem = T;
     static constexpr int bm = BM, bn = BN;
-    static constexpr bool conv = CONV != 0, pre = PRE, window = false, TAPS = CONV == 2;
+    static constexpr bool conv = CONV != 0, pre = PRE, window = false, TAPS = CONV == 2, STRADDLES = CONV == 3;
     // Whether GEMM rows are fetched through descriptors (see `near` below).  Not by the fp32 bodies of 128 x 128 and less: their MFMAs
     // take eight times as long, a load's instructions hide behind them, and with two workgroups to a compute unit that now advance
     // in step, a last round of few tiles finds both places of a unit free at once and doubles up there: 5175 x 1833 x 1696
     // plain 333 -> 428 us, 2048 x 2560 x 4096 preemptible 605 -> 649.  Nor by the 16-bit GEMM of 128 x 128: 3 % faster on 5175 x 1833 x
     // 1696, but 2048 x 2560 x 4096 preemptible 121 -> 130.
-    static constexpr bool DESC = TAPS || BM == 256 || (sizeof(T) == 2 && BM < 128);
+    static constexpr bool DESC = TAPS || STRADDLES || BM == 256 || (sizeof(T) == 2 && BM < 128);
     static constexpr int VEC = Elem<T>::VEC;
     static constexpr int WAVES = NWAVES, NT = WAVES * 64;
     static constexpr int RB = 128;                        // row bytes in LDS
@@ -271,6 +275,9 @@ struct PipeKernel {
                 if constexpr (TAPS) {  // (offsets count from the window of output pixel (0, 0), which lies in front of the image by the padding)
                     a_off[j] = ((unsigned)((n * g.H + ho * g.sh) * g.W + wo * g.sw) * (unsigned)g.lda + (unsigned)(chunk_of(wave * A_PW + j) * VEC)) * (unsigned)sizeof(T);
                     a_taps[j] = m < g.M ? window_tap_mask(a_h0[j], a_w0[j], g.H, g.W, g.R, g.S) : 0u;
+                } else if constexpr (STRADDLES) {
+                    a_off[j] = (unsigned)((n * g.H + ho * g.sh) * g.W + wo * g.sw) * (unsigned)g.lda * (unsigned)sizeof(T);
+                    if (m >= g.M) a_h0[j] = g.H;  // no tap inside the image
                 } else a_org[j] = A + ((long)n * g.H * g.W + (long)a_h0[j] * g.W + a_w0[j]) * g.lda;
             }
         }
@@ -281,7 +288,7 @@ struct PipeKernel {
         // turn: 8192^3 bf16 with checkpoints, its clears included, 970 -> 951 us, 4096^3 fp32 1098 -> 1016, 6000 x 5000 x 2048 fp16 152 -> 146.
         // (`near`: the tile's rows lie within a descriptor's 2 GB.  Otherwise an address of 64 bits is worked out for every load.)
         const long far = (long)kBufferEnd / (long)sizeof(T) - g.K;
-        const bool near = TAPS || !DESC || PHASED || ((CONV || (long)BM * g.lda <= far) && (long)BN * g.ldb <= far);
+        const bool near = TAPS || STRADDLES || !DESC || PHASED || ((CONV || (long)BM * g.lda <= far) && (long)BN * g.ldb <= far);
         if (!CONV && DESC) {
 #pragma unroll
             for (int j = 0; j < (CONV ? 1 : A_PW); ++j)
@@ -291,7 +298,7 @@ struct PipeKernel {
         for (int j = 0; j < (DESC ? B_PW : 0); ++j)
             b_off[j] = n0 + b_at(j) + rig < g.N ? near ? ((unsigned)(b_at(j) + rig) * (unsigned)g.ldb + (unsigned)(chunk_of(wave * B_PW + j) * VEC)) * (unsigned)sizeof(T) : 0u : kBufferEnd;
         const u32x4 rsrc_a = buffer_of(CONV ? A - (long)(g.ph * g.W + g.pw) * g.lda : A + (long)m0 * g.lda), rsrc_b = buffer_of(B + (long)n0 * g.ldb);
-        const bool conv_fast = TAPS || (CONV && (g.Cin % BK == 0));  // a K-step never straddles a filter tap
+        const bool conv_fast = TAPS || (CONV == 1 && (g.Cin % BK == 0));  // a K-step never straddles a filter tap
         // Pointers with the lane's chunk already added, one per parity of the slot number j: a load's address is this plus a
         // wave-uniform offset.
         const T *a_par[2] = {nullptr, nullptr}, *b_par[2] = {nullptr, nullptr};
@@ -368,6 +375,14 @@ struct PipeKernel {
                 const T *src;
                 if constexpr (TAPS) {
                     load_lds16_buffer<SINGLE || CKPT>(rsrc_a, a_taps[j] >> sa.tap & 1u ? a_off[j] : kBufferEnd, sa.tap_bytes, sa.sbase + (unsigned)((wave * A_PW + j) * 8 * RB));
+                    return;
+                }
+                if constexpr (STRADDLES) {  // (the planner's limits keep the factors of the 24-bit products below 2^24)
+                    const unsigned k = (unsigned)(sa.k0 + kc), rs = __umulhi(k + 1, g.inv_cin), r = __umulhi(rs + 1, g.inv_s);
+                    const unsigned ci = k - __umul24(rs, (unsigned)g.Cin), s2 = rs - __umul24(r, (unsigned)g.S);
+                    const bool ok = (k < (unsigned)g.K) & ((unsigned)(a_h0[j] + (int)r) < (unsigned)g.H) & ((unsigned)(a_w0[j] + (int)s2) < (unsigned)g.W);
+                    const unsigned off = (__umul24(r, (unsigned)g.W) + s2) * ((unsigned)g.lda * (unsigned)sizeof(T)) + ci * (unsigned)sizeof(T);
+                    load_lds16_buffer<SINGLE || CKPT>(rsrc_a, ok ? a_off[j] + off : kBufferEnd, 0u, sa.sbase + (unsigned)((wave * A_PW + j) * 8 * RB));
                     return;
                 }
                 if (CONV) {

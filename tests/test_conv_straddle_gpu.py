@@ -53,3 +53,48 @@ def test_blocks_that_straddle_taps(gp, dt, N, H, W, Cin, Cout, R, S, stride, ph,
             p.variant = variant
             with pytest.raises(gp.GpError):
                 gp.launch("gp_launch_conv2d", p)
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("N,H,W,Cin,Cout,R,S,stride,ph,pw,tile", [
+    (1, 20, 20, 8, 64, 3, 3, 1, 1, 1, 64),    # a first layer: two K-steps, the second one mostly past K
+    (1, 41, 39, 8, 64, 7, 7, 2, 3, 3, 64),    # 49 taps
+    (2, 13, 9, 40, 24, 1, 7, 1, 0, 3, 64),
+    (1, 12, 10, 24, 33, 5, 6, 1, 4, 5, 64),   # windows mostly outside the image, ragged columns
+    (2, 15, 15, 104, 136, 3, 3, 1, 1, 1, 128),
+])
+def test_pipelined_bodies_that_straddle_taps(gp, dt, N, H, W, Cin, Cout, R, S, stride, ph, pw, tile):
+    """Against fp64, plain and stopped and resumed.  The largest error is that of K
+    products summed in fp32 (K roundings of half a unit of the sum of their magnitudes at most) and one rounding to the type."""
+    import torch
+    dtype = gp.DTYPE_BY_NAME[dt]
+    rng = np.random.default_rng(H + Cin + Cout)
+    Ho, Wo = (H + 2 * ph - R) // stride + 1, (W + 2 * pw - S) // stride + 1
+    x, w, b = rng.uniform(-1, 1, (N, H, W, Cin + 8)).astype(np.float32), rng.uniform(-1, 1, (Cout, R, S, Cin)).astype(np.float32), rng.uniform(-1, 1, Cout).astype(np.float32)
+    dx, dw, db = (gp.DevBuf.from_array(v, dtype) for v in (x, w, b))
+    x, w, b = (torch.from_numpy(v.download(dtype, a.shape)).double() for v, a in ((dx, x), (dw, w), (db, b)))
+    x = x[..., :Cin].permute(0, 3, 1, 2)
+    conv = lambda x, w, b: torch.nn.functional.conv2d(x, w.permute(0, 3, 1, 2), b, stride, (ph, pw)).permute(0, 2, 3, 1).numpy()
+    ref, size = conv(x, w, b), conv(x.abs(), w.abs(), b.abs())
+    out = gp.DevBuf((N * Ho * Wo * Cout * gp.DTYPE_SIZE[dtype] + 3) // 4 * 4)
+    p = gp.ConvParams(dtype=dtype, N=N, H=H, W=W, Cin=Cin, Cout=Cout, R=R, S=S, stride_h=stride, stride_w=stride, pad_h=ph, pad_w=pw, in_=dx.ptr, in_pix_stride=Cin + 8,
+                      weight=dw.ptr, bias=db.ptr, out=out.ptr, out_pix_stride=Cout, act=gp.ACT_NONE, tile_m=tile, tile_n=tile, variant=gp.MAT_PIPE)
+    out.fill32(0x7E007E00)
+    info = gp.launch("gp_launch_conv2d", p)
+    sync(gp)
+    want = out.download().copy()
+    rows = N * Ho * Wo
+    assert info.total_tiles == -(-rows // tile) * -(-Cout // tile)
+    got = out.download(dtype)[: rows * Cout].reshape(ref.shape)
+    eps = {"f32": 0.0, "f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dt]
+    assert (np.abs(got - ref) <= R * S * Cin * 2.0 ** -24 * size * 2 + eps * np.abs(ref) * 1.01).all()
+    flag = gp.Flag()
+    st = gp.BlpState(1, flag, 32)
+    out.fill32(0x7E007E00)
+    gp.launch("gp_launch_conv2d", p, st.ctx(inject_at=0))
+    sync(gp)
+    flag.set(0)
+    st.clear_stop()
+    gp.launch("gp_launch_conv2d", p, st.ctx())
+    sync(gp)
+    assert np.array_equal(out.download(), want)

@@ -179,6 +179,14 @@ static int choose_body(MatPlan *pl, int tile, int tile_n, int variant) {
     // a stop its workgroups still have to start and leave, about a microsecond per thousand.  (fp32, whose tiles take eight times as long and
     // wait no longer: 3136 tiles there 150 us either way.)
     if (tile == 0 && variant == GP_MAT_AUTO && body == MB_PIPE64 && g.K <= 640) pl->rounds = 20;
+    // Layers of at most 64 channels over many pixels (the first ones of a VGG) in tiles of 128 x 64: half the workgroups, each of which takes about as
+    // long from its claim to its first operands and from its last to its store, and half the weights through LDS.  Preemptible, fp16, batch 16 at
+    // 224 x 224: 8 -> 64 channels 75 -> 65 us, 64 -> 64 138 -> 120; batch 8 72 -> 64.  From sixteen tiles of 64 x 64 to a compute unit on: batch 4,
+    // twelve, is level.
+    if (pl->ring == 2 && body == MB_PIPE64 && pl->dtype != GP_F32 && (pl->taps || pl->straddles) && g.N > 32 && g.N <= 64 && g.K <= 640 && tiles(64) >= 16 * cus) {
+        pl->tall = true;
+        pl->sy = (g.M + 127) / 128;
+    }
     // Each XCD works on a contiguous eighth of the tile order (util/slice_map.h).  With x fastest
     // that is a band of tile rows: every XCD fetches its share of A and all of B; with y fastest
     // it is a band of tile columns: all of A and a share of B.  Take the cheaper one.

@@ -171,6 +171,10 @@ template <typename T, int TILE, int STAGES, bool SPLITK>
 static int pipe_case(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
     if constexpr (TILE == 64 && !SPLITK)
         if (pl.pre) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 0, false, false, 4, true>>(pl, ctx, s, info);
+    if constexpr (sizeof(T) == 2 && TILE == 64 && STAGES == 2) {
+        if (pl.tall && pl.taps) return launch_mat<PipeKernel<T, 128, 64, 2, 2, false>>(pl, ctx, s, info);
+        if (pl.tall) return launch_mat<PipeKernel<T, 128, 64, 2, 3, false>>(pl, ctx, s, info);
+    }
     if constexpr (sizeof(T) == 2)
         if (pl.taps) return launch_mat<PipeKernel<T, TILE, TILE, STAGES, 2, SPLITK>>(pl, ctx, s, info);
     if constexpr (TILE >= 64 && !SPLITK)

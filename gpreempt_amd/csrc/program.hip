@@ -317,8 +317,8 @@ static int push_mat(gp_program pr, const MatPlan &pl) {
     GP_REQUIRE(ok, "matrix kernel body %d is not available inside a program", pl.body);
     LayerDesc d{};
     d.op = OP_MAT; d.dtype = pl.dtype; d.body = pl.body; d.conv = pl.conv; d.b_kn = pl.b_kn;
-    d.sx = pl.sx; d.sy = pl.sy;
-    long total = (long)pl.sx * pl.sy * pl.batch;
+    d.sx = pl.sx; d.sy = pl.tall ? (pl.g.M + 63) / 64 : pl.sy;  // (the program keeps tiles of 64 x 64)
+    long total = (long)d.sx * d.sy * pl.batch;
     GP_REQUIRE(total > 0 && total < (1L << 31), "tile count %ld out of range", total);
     d.total = (int)total;
     d.u.mat = pl.g;

@@ -62,9 +62,11 @@ def test_blocks_that_straddle_taps(gp, dt, N, H, W, Cin, Cout, R, S, stride, ph,
     (2, 13, 9, 40, 24, 1, 7, 1, 0, 3, 64),
     (1, 12, 10, 24, 33, 5, 6, 1, 4, 5, 64),   # windows mostly outside the image, ragged columns
     (2, 15, 15, 104, 136, 3, 3, 1, 1, 1, 128),
+    (1, 517, 523, 8, 64, 3, 3, 1, 1, 1, 0),   # tiles of 128 x 64, the last one partly past the rows
+    (1, 519, 521, 64, 40, 3, 3, 1, 1, 1, 0),  # ... whose K-steps lie within a tap, ragged columns
 ])
-def test_pipelined_bodies_that_straddle_taps(gp, dt, N, H, W, Cin, Cout, R, S, stride, ph, pw, tile):
-    """Against fp64, plain and stopped and resumed.  The largest error is that of K
+def test_pipelined_bodies_that_straddle_taps_or_take_tall_tiles(gp, dt, N, H, W, Cin, Cout, R, S, stride, ph, pw, tile):
+    """Against fp64, plain and stopped and resumed; where the launcher picks, with the bits of 64 x 64 tiles.  The largest error is that of K
     products summed in fp32 (K roundings of half a unit of the sum of their magnitudes at most) and one rounding to the type."""
     import torch
     dtype = gp.DTYPE_BY_NAME[dt]
@@ -78,13 +80,13 @@ def test_pipelined_bodies_that_straddle_taps(gp, dt, N, H, W, Cin, Cout, R, S, s
     ref, size = conv(x, w, b), conv(x.abs(), w.abs(), b.abs())
     out = gp.DevBuf((N * Ho * Wo * Cout * gp.DTYPE_SIZE[dtype] + 3) // 4 * 4)
     p = gp.ConvParams(dtype=dtype, N=N, H=H, W=W, Cin=Cin, Cout=Cout, R=R, S=S, stride_h=stride, stride_w=stride, pad_h=ph, pad_w=pw, in_=dx.ptr, in_pix_stride=Cin + 8,
-                      weight=dw.ptr, bias=db.ptr, out=out.ptr, out_pix_stride=Cout, act=gp.ACT_NONE, tile_m=tile, tile_n=tile, variant=gp.MAT_PIPE)
+                      weight=dw.ptr, bias=db.ptr, out=out.ptr, out_pix_stride=Cout, act=gp.ACT_NONE, tile_m=tile, tile_n=tile, variant=gp.MAT_PIPE if tile else 0)
     out.fill32(0x7E007E00)
     info = gp.launch("gp_launch_conv2d", p)
     sync(gp)
     want = out.download().copy()
     rows = N * Ho * Wo
-    assert info.total_tiles == -(-rows // tile) * -(-Cout // tile)
+    assert info.total_tiles == -(-rows // (tile or (64 if dt == "f32" else 128))) * -(-Cout // (tile or 64))
     got = out.download(dtype)[: rows * Cout].reshape(ref.shape)
     eps = {"f32": 0.0, "f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dt]
     assert (np.abs(got - ref) <= R * S * Cin * 2.0 ** -24 * size * 2 + eps * np.abs(ref) * 1.01).all()
@@ -98,3 +100,10 @@ def test_pipelined_bodies_that_straddle_taps(gp, dt, N, H, W, Cin, Cout, R, S, s
     gp.launch("gp_launch_conv2d", p, st.ctx())
     sync(gp)
     assert np.array_equal(out.download(), want)
+    if not tile:
+        p.tile_m = p.tile_n = 64
+        p.variant = gp.MAT_PIPE
+        out.fill32(0x7E007E00)
+        gp.launch("gp_launch_conv2d", p)
+        sync(gp)
+        assert np.array_equal(out.download(), want)

@@ -45,6 +45,9 @@ __host__ __device__ inline size_t attention_lds_bytes(int nb) { return attention
 // 16 x 512 x 64 472 -> 255 (270 TFLOP/s; bound by the vector instructions of the softmax), 12 x 256 x 64 64 -> 54.
 template <typename T, int NB>
 __device__ __forceinline__ void attention_tile(const AttnArgs &a, TileIdx t, T *lds) {
+    // (products and sums are contracted where the code says so and nowhere else, so that the kernels and the whole-model program, which are built around
+    // this body, give the same bits)
+#pragma clang fp contract(off)
     constexpr int PARTS = attention_parts(NB), NBW = NB / PARTS, THREADS = attention_threads(NB);
     static_assert(NB % PARTS == 0, "key blocks are shared evenly");
     const gp_attention_params &p = a.p;
@@ -183,7 +186,7 @@ __device__ __forceinline__ void attention_tile(const AttnArgs &a, TileIdx t, T *
 #pragma unroll
         for (int i = 0; i < PARTS; ++i) {
             f[i] = ms[i][0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms[i][0] - M);
-            den += f[i] * ms[i][1];
+            den = __builtin_fmaf(f[i], ms[i][1], den);
         }
         f32x4 x[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
@@ -193,14 +196,18 @@ __device__ __forceinline__ void attention_tile(const AttnArgs &a, TileIdx t, T *
             for (int h = 0; h < 2; ++h) {
                 const f32x4 y = *(const f32x4 *)(partial + (i * ATT_QB + r) * ATT_OP + d8 + 4 * h);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) x[h][e] += w * y[e];
+                for (int e = 0; e < 4; ++e) x[h][e] = __builtin_fmaf(w, y[e], x[h][e]);
             }
         }
         if (t.x * ATT_QB + r >= S) continue;
         T *dst = O + (long)(t.x * ATT_QB + r) * p.ld_out + d8;
         T out[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) out[e] = Elem<T>::from_f(x[e / 4][e % 4]);
+        for (int e = 0; e < 8; ++e) {
+            float r32 = x[e / 4][e % 4];
+            asm("" : "+v"(r32));  // (rounded to fp32 first: the compiler makes one operation with a single rounding of the last sum and the conversion, for some of them)
+            out[e] = Elem<T>::from_f(r32);
+        }
         if (vec_out) st_out128(dst, *(const out_u32x4 *)out);
         else {
 #pragma unroll

@@ -11,6 +11,7 @@ import pytest
 from gpreempt_amd import capi as gp
 
 OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
+READELF = "/opt/rocm/llvm/bin/llvm-readelf"
 pytestmark = pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="no disassembler")
 WORD = re.compile(r"^\s+([a-z]\S*)\s*(.*?)\s*// ([0-9A-F]+):(.*)$")
 
@@ -86,3 +87,26 @@ def test_no_barrier_is_reached_with_lds_reads_outstanding(kernels):
                     work.append((j, n))
                 i += 1
     assert not bad, (len(bad), bad[:4])
+
+
+@pytest.fixture(scope="module")
+def spilled(tmp_path_factory):
+    """{name: vector registers that the compiler spilled} of the kernels that run one tile of 256 x 256: the forms without claims (1), with fixed claims (2), and with looks (3)"""
+    work = tmp_path_factory.mktemp("notes")
+    lib = shutil.copy(gp.LIB_PATH, work)
+    subprocess.run([OBJDUMP, "--offloading", os.path.basename(lib)], cwd=work, check=True, capture_output=True)
+    found = {}
+    for part in glob.glob(os.path.join(work, "*gfx950*")):
+        notes = subprocess.run([READELF, "--notes", part], check=True, capture_output=True, text=True).stdout
+        for kernel in re.split(r"\n\s+- \.agpr_count:", notes)[1:]:
+            name = re.search(r"\.name:\s+(\S+)", kernel).group(1)
+            if "mat_kernelINS_10PipeKernelI" in name and "Li256ELi256ELi2E" in name and re.findall(r"Li(\d+)E", name)[-1] in "123":
+                found[name] = int(re.search(r"\.vgpr_spill_count:\s+(\d+)", kernel).group(1))
+    assert len(found) == 9
+    return found
+
+
+def test_tiles_of_256_keep_to_their_registers(spilled):
+    """... all but the nine addresses that the fp32 form with looks parks across its main loop"""
+    bad = {k: n for k, n in spilled.items() if n > (9 if "IfLi" in k and k.split("ELi")[-1].startswith("3") else 0)}
+    assert not bad, bad

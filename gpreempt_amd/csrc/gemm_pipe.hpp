@@ -322,7 +322,7 @@ struct PipeKernel {
 
         // Loads of one stage: slot l < A_PW is an A slot, the rest are B slots.  `StageAddr` holds
         // the wave-uniform part, computed once per stage.
-        struct StageAddr { unsigned sbase, sbase_poll, k_bytes, tap_bytes; int k0, tap, r_u, s_u, tap_off; bool new_tap, first; };
+        struct StageAddr { unsigned sbase, sbase_poll, k_bytes, tap_bytes; int k0, tap, r_u, s_u, tap_off, chunk; bool new_tap, first; };
         // Stages are fetched in increasing order, so the filter tap (r, s) and channel offset of
         // the next stage advance incrementally instead of being divided out of k every time.
         int nx_r = 0, nx_s = 0, nx_ci = 0, nx_tap = 0;
@@ -339,6 +339,13 @@ struct PipeKernel {
             sa.sbase_poll = lds0 + (unsigned)RING_BYTES + ((unsigned)kt % STAGES) * WAVES * 256;
             sa.k0 = kt * BK;
             sa.k_bytes = (unsigned)__builtin_amdgcn_readfirstlane(sa.k0 * (int)sizeof(T));
+            if constexpr (PHASED && CKPT) {
+                // (the lane's chunk, worked out for every stage: kept, it was one register more than there are, and came back from scratch memory
+                // in front of a stage's first load, behind a wait of the compiler's for everything that was on its way to LDS)
+                unsigned me;
+                asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(me));
+                sa.chunk = (int)((me & 7) ^ (me >> 4));
+            } else sa.chunk = c_base;
             sa.r_u = nx_r; sa.s_u = nx_s;
             sa.tap_off = (nx_r * g.W + nx_s) * (int)g.lda + nx_ci;  // elements from the window origin
             if constexpr (TAPS) { sa.tap = nx_tap; sa.tap_bytes = (unsigned)__builtin_amdgcn_readfirstlane(sa.tap_off * (int)sizeof(T)); }
@@ -462,12 +469,14 @@ struct PipeKernel {
         };
 
         f32x16 acc[MI][NI];
+        float nought = 0.f;
+        if constexpr (CKPT && PHASED) asm volatile("" : "+v"(nought));  // (a tile's own zeros: those of all tiles were sixteen registers, kept across the K loop in scratch memory)
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int j = 0; j < NI; ++j)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+                for (int v = 0; v < 16; ++v) acc[i][j][v] = nought;
         // checkpointing state
         f32x4 *slot = nullptr;       // this wave's part of the workgroup's checkpoint slot
         // landing slots of the stop-word loads, behind the ring: [stage][wave][64 dwords]
@@ -650,12 +659,12 @@ struct PipeKernel {
             // parts of a stage's buffer are free long before the stage is done: A's first half (the wavefront's rows 0-63) with B's first
             // (its columns 0-31), A's first with B's second, A's second with B's second, A's second with B's first.  Stage kt + 2 follows into the
             // place of stage kt half by half: A's and B's first behind the barrier in front of the second phase, the others behind the one in
-            // front of the last.  So a load has one to one and a half K-steps to arrive in; in the loop below, which fetches a stage while
-            // the one before it is multiplied, the last of its loads has half a K-step, and the wait for it is where the matrix cores stood idle.
-            // (The waits count the loads behind the ones that are needed, and every K-step issues the same ones: what lies past K is fetched from
-            // beyond the descriptor's end.)  8192^3 bf16 in turn with the loop below, its clears included: with checkpoints 953 -> 889 us, plain
-            // 888 -> 835.  What bounds it now: LDS, read and written for about as many cycles as the MFMAs take, and the power the
-            // multipliers draw.  (The reads spread evenly over the phases, with the second barrier a phase earlier: plain 848 -> 875.)
+            // front of the last.  So a load has nine tenths of a K-step to arrive in (B's second half) to one and a half (A's first); in the loop
+            // below, which fetches a stage while the one before it is multiplied, the last of its loads has half a K-step, and the wait for it is
+            // where the matrix cores stood idle.  (The waits count the loads behind the ones that are needed, and every K-step issues the same ones:
+            // what lies past K is fetched from beyond the descriptor's end.)  8192^3 bf16, its clears included, in turn with the form whose K-steps
+            // drained all loads behind a register from scratch memory: with checkpoints 923 -> 890 us (f16 975 -> 950); plain 833 either way.
+            // (The reads spread evenly over the phases, with the second barrier a phase earlier: plain 848 -> 875.)
             // Wavefront 0 asks for the stop index with every second stage, and wavefront 1 for the flag when it is the workgroup's turn (see
             // issue_one).  Nobody else asks for anything in their place: the waits below count the operand loads, and a wavefront that has
             // asked for a word as well waits a load longer than it has to.  (Reads past the caches of one address come back one per 11 ns; with
@@ -671,7 +680,7 @@ struct PipeKernel {
             auto ahead = [&](auto level) { if constexpr (!CKPT) __builtin_amdgcn_s_setprio(decltype(level)::value); };
             auto issue_near = [&](const StageAddr &sa, int l) {  // (issue_one without what operands beyond a descriptor's 2 GB take)
                 const int j = l < A_PW ? l : l - A_PW;
-                const unsigned at = chunk_of(j) * VEC < g.K - sa.k0 ? l < A_PW ? a_off[CONV == 1 ? 0 : j] : b_off[j] : kBufferEnd;
+                const unsigned at = (sa.chunk ^ ((j & 1) << 2)) * VEC < g.K - sa.k0 ? l < A_PW ? a_off[CONV == 1 ? 0 : j] : b_off[j] : kBufferEnd;
                 load_lds16_buffer<SINGLE || CKPT>(l < A_PW ? rsrc_a : rsrc_b, at, sa.k_bytes, sa.sbase + (unsigned)(l < A_PW ? a_at(j) * RB : A_BYTES + b_at(j) * RB));
             };
             u32x4 fa0[2][KSTEPS], fa1[2][KSTEPS], fb0[KSTEPS], fb1[KSTEPS];
@@ -691,6 +700,7 @@ struct PipeKernel {
             wait_vmcnt<2 + LPS>();  // all of the first stage but A's second half
             stage_barrier();
             static_for<0, KSTEPS>([&](auto kc) { read_a(fa0, kt0 & 1, 0, decltype(kc)::value); read_b(fb0, kt0 & 1, 0, decltype(kc)::value); });
+            int raised = 0;
             for (; kt < KT; ++kt) {
                 const int stage = kt & 1;
                 static_for<0, KSTEPS>([&](auto kc) { read_b(fb1, stage, 1, decltype(kc)::value); });
@@ -702,7 +712,7 @@ struct PipeKernel {
                 });
                 ahead(IntC<0>{});
                 __builtin_amdgcn_sched_barrier(0);
-                wait_vmcnt<LPS>();  // this stage's second half of A (behind it: a stage less A's and B's first halves, and those of the next)
+                wait_vmcnt<LPS>();  // this stage's second half of A (behind it: the eight loads of the next stage)
                 stage_barrier();       // A's and B's first halves have been read by everybody
                 if constexpr (!CKPT) {
                     bool leave = early && kt == kt0 && __builtin_amdgcn_readfirstlane(read_lds_word(early_slot)) != -1;
@@ -754,10 +764,12 @@ struct PipeKernel {
                 ahead(IntC<0>{});
                 if constexpr (CKPT) {
                     const int sw = __builtin_amdgcn_readfirstlane(stop_word), fw = __builtin_amdgcn_readfirstlane(flag_word);
-                    if (fw != 0 && tid == 0) record_stop(cc.stop_index, cc.kernel_id, cc.stamps);  // pass the host flag on
+                    raised = fw;
                     if (((sw != -1) | (fw != 0)) && kt + 1 < KT) { stopped = 1; break; }
                 }
             }
+            // (behind the loop: its pointers and its compare-and-swap took scalar registers away from every K-step)
+            if (CKPT && raised != 0 && tid == 0) record_stop(cc.stop_index, cc.kernel_id, cc.stamps);  // pass the host flag on
             wait_vmcnt<0>();  // what was fetched beyond the last K-step lands in LDS as well
             if (!CKPT && stopped) return true;
         }

@@ -89,6 +89,27 @@ def test_no_barrier_is_reached_with_lds_reads_outstanding(kernels):
     assert not bad, (len(bad), bad[:4])
 
 
+def loops_of(code, mfmas):
+    """the innermost ways back over that many matrix instructions"""
+    index = {a: i for i, (a, *_) in enumerate(code)}
+    before = [0]
+    for _, op, _, _ in code:
+        before.append(before[-1] + op.startswith("v_mfma"))
+    back = [(index[code[0][0] + to], i) for i, (_, _, _, to) in enumerate(code) if to is not None and index[code[0][0] + to] <= i]
+    back = [(j, i) for j, i in back if before[i + 1] - before[j] == mfmas]
+    return [code[j:i + 1] for j, i in back if not any((a, b) != (j, i) and j <= a and b <= i for a, b in back)]
+
+
+def test_the_loop_of_256_tiles_in_phases_waits_for_nothing_it_need_not(kernels):
+    """Operands are asked for two K-steps ahead: no wait for everything that is on its way stands in the loop, and no register comes back from
+    scratch memory, behind which the compiler puts one"""
+    loops = {k: loops_of(v, 32) for k, v in kernels.items() if "PipeKernelIDF16" in k and "Li256ELi256ELi2E" in k}
+    assert len(loops) == 10 and all(loops.values())
+    for name, loop in ((k, l) for k, ls in loops.items() for l in ls):
+        assert not [op for _, op, _, _ in loop if op.startswith("scratch_")], name
+        assert [a for _, op, a, _ in loop if op == "s_waitcnt" and "vmcnt" in a] == ["vmcnt(8)", "vmcnt(6)"], name
+
+
 @pytest.fixture(scope="module")
 def spilled(tmp_path_factory):
     """{name: vector registers that the compiler spilled} of the kernels that run one tile of 256 x 256: the forms without claims (1), with fixed claims (2), and with looks (3)"""

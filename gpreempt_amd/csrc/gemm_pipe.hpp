@@ -555,7 +555,8 @@ struct PipeKernel {
         };
         const int KT = (g.K + BK - 1) / BK;
         // A tile that is being finished counts its workgroup in cc.announce at the top of its last K-step, behind that step's
-        // wait for its operands: nothing the wavefront issues later is waited for before the epilogue.  (Counted at the last
+        // wait for its operands (in phases: behind the loop and the wait for what it fetched beyond K): nothing the wavefront issues later
+        // is waited for before the epilogue.  (Counted at the last
         // look instead, several K-steps from the end, the atomic stood in wavefront 0's queue in front of operand loads: the
         // counts that the waits of the next K-steps rely on go down in the order of issue, so the whole workgroup waited for
         // the atomic to be acknowledged, 6 us a tile with 512 workgroups resident.)
@@ -722,7 +723,6 @@ struct PipeKernel {
                             load_lds4(cc.stop_index, (unsigned)(size_t)(__attribute__((address_space(3))) void *)(early_slot + 64));
                     }
                     if (leave) { stopped = 1; break; }
-                    if constexpr (LOOKS) if (looking && kt == KT - 1) announce();
                 }
                 const StageAddr sa = stage_addr(kt + 2);
                 static_for<0, KSTEPS>([&](auto kc) { read_a(fa1, stage, 2, decltype(kc)::value); });
@@ -772,6 +772,7 @@ struct PipeKernel {
             if (CKPT && raised != 0 && tid == 0) record_stop(cc.stop_index, cc.kernel_id, cc.stamps);  // pass the host flag on
             wait_vmcnt<0>();  // what was fetched beyond the last K-step lands in LDS as well
             if (!CKPT && stopped) return true;
+            if constexpr (LOOKS) if (looking) announce();
         }
         // The loop of all other bodies.  (Conditions on its statements, not the branch of an `else`: in a scope of its own the compiler spilled 147
         // registers of the fp32 256 x 256 form with fixed claims, where it spills none now, and 112 for 9 of the one that looks.)

@@ -456,7 +456,10 @@ extern "C" int gp_conv2d_body(const gp_conv_params *p, char *name, size_t len) {
                                         "wide64x64_8", "lnwide32x64_16", "narrow16x16", "narrow32x16"};
     static_assert(MB_PIPE128 == 0 && MB_PIPE64 == 1 && MB_PIPE64_SK == 2 && MB_PIPE32_SK == 3 && MB_STAGED128 == 4 && MB_STAGED64 == 5 && MB_PIPE256 == 6 && MB_NARROW32x16 == 13, "names");
     const bool blocks_straddle = pl.conv && pl.g.Cin % (pl.dtype == GP_F32 ? 32 : 64) != 0;
-    snprintf(name, len, "%s%s", names[pl.body], !pl.conv ? "" : pl.window ? " window" : blocks_straddle ? " straddling" : pl.taps ? " taps" : " gathered");
+    // (the wide bodies multiply as well; those of four wavefronts do where the launcher takes that form of them, gemm_launch.hpp)
+    const bool divides = !is_wide_body(pl.body) && !((pl.body == MB_PIPE64 || pl.body == MB_PIPE128) && pl.straddles);
+    snprintf(name, len, "%s%s", pl.tall ? "pipe128x64" : names[pl.body],
+             !pl.conv ? "" : pl.window ? " window" : blocks_straddle ? divides ? " divided" : " straddling" : pl.taps ? " taps" : " gathered");
     return GP_SUCC;
 }
 extern "C" int gp_conv_ckpt_bytes(const gp_conv_params *p, size_t *bytes) {

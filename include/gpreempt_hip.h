@@ -307,7 +307,8 @@ int gp_launch_conv2d(const gp_conv_params *p, const gp_preempt_ctx *ctx, gp_stre
 int gp_conv2d_group_supported(const gp_conv_params *p, int n);
 int gp_launch_conv2d_group(const gp_conv_params *p, int n, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info);
 /* For diagnosis: the tile body a convolution would be launched with and how it fetches its input, as text ("wide32x32_16 window",
- * "pipe64 taps"; no second word for a pointwise one, which is a GEMM).  Needs no GPU. */
+ * "pipe64 taps", "pipe128x64 taps"; "straddling" where K-steps straddle filter taps that a lane finds by multiplication, "divided" where it
+ * divides; no second word for a pointwise one, which is a GEMM).  Needs no GPU. */
 int gp_conv2d_body(const gp_conv_params *p, char *name, size_t len);
 /* As gp_gemm_ckpt_bytes, for a convolution (0 unless it runs on the 128 x 128 body). */
 int gp_conv_ckpt_bytes(const gp_conv_params *p, size_t *bytes);

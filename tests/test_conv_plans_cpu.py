@@ -63,3 +63,18 @@ def test_two_layers_of_larger_tiles_are_more_than_a_group_takes(dtype, step):
             both = [_conv(1280, step * columns, H, dtype) for _ in range(2)]
             tiles = -(-H * H // step) * columns  # of one of them
             assert lib.gp_conv2d_group_supported((gp.ConvParams * 2)(*both), 2) == (1 if 2 * tiles <= 256 else 0), (H, columns)
+
+
+@pytest.mark.parametrize("dt,N,H,Cin,Cout,R,stride,tile,variant,want", [
+    ("f16", 16, 224, 64, 64, 3, 1, 0, "MAT_AUTO", "pipe128x64 taps"), ("bf16", 16, 224, 8, 64, 3, 1, 0, "MAT_AUTO", "pipe128x64 straddling"),
+    ("f16", 4, 224, 64, 64, 3, 1, 0, "MAT_AUTO", "pipe64 taps"), ("f32", 16, 224, 64, 64, 3, 1, 0, "MAT_AUTO", "pipe64 gathered"),
+    ("f16", 16, 224, 64, 64, 3, 1, 64, "MAT_PIPE", "pipe64 taps"), ("f32", 16, 73, 80, 192, 3, 1, 0, "MAT_AUTO", "pipe128 straddling"),
+    ("f16", 1, 35, 48, 64, 5, 1, 0, "MAT_AUTO", "wide32x32_16 straddling"), ("f16", 1, 35, 48, 64, 5, 1, 64, "MAT_PIPE_SPLITK", "pipe64_splitk divided"),
+    ("f16", 3, 9, 23176, 64, 9, 1, 64, "MAT_PIPE", "pipe64 divided"),  # (too deep for the inverse of the channels)
+    ("f16", 1, 56, 64, 256, 1, 1, 0, "MAT_AUTO", "pipe64")])
+def test_the_body_that_is_named_is_the_one_that_runs(dt, N, H, Cin, Cout, R, stride, tile, variant, want):
+    p = gp.ConvParams(dtype=gp.DTYPE_BY_NAME[dt], N=N, H=H, W=H, Cin=Cin, Cout=Cout, R=R, S=R, stride_h=stride, stride_w=stride, pad_h=R // 2, pad_w=R // 2, in_=4096,
+                      in_pix_stride=Cin, weight=8192, bias=12288, out=16384, out_pix_stride=Cout, tile_m=tile, tile_n=tile, variant=getattr(gp, variant))
+    name = C.create_string_buffer(64)
+    assert C.CDLL(gp.LIB_PATH).gp_conv2d_body(C.byref(p), name, C.c_size_t(64)) == gp.SUCC
+    assert name.value.decode() == want

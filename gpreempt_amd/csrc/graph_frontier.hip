@@ -137,13 +137,13 @@ __device__ __forceinline__ bool gf_walk(const u32x4 *ids, unsigned begin, unsign
 // 3600 -> 3385 us, at 2^17 of degree 4 441 -> 392 (one set, in a line of its own: 3400 and 435).
 constexpr unsigned kSetInts = 32;
 static_assert(GP_GRAPH_SETS == kXcds, "a set per XCD");
-__device__ __forceinline__ unsigned *own_words(const gp_graph_iter_params &p) { return p.changed + (p.sets ? blockIdx.x % kXcds * kSetInts : 0u); }
+__device__ __forceinline__ unsigned *own_words(const gp_graph_iter_params &p) { return p.changed + (p.sets == GP_GRAPH_IN_SETS ? blockIdx.x % kXcds * kSetInts : 0u); }
 // What the launch before said: lane 8 * w + x reads word w of set x, for the first five words.
 struct WordsBefore {
     unsigned mine = 0;
     __device__ __forceinline__ explicit WordsBefore(const gp_graph_iter_params &p) {
         const unsigned lane = threadIdx.x & 63, word = lane / kXcds, set = lane % kXcds;
-        if (p.prev_changed && word < 5 && (p.sets || set == 0)) mine = p.prev_changed[set * kSetInts + word];
+        if (p.prev_changed && word < 5 && (p.sets == GP_GRAPH_IN_SETS || set == 0)) mine = p.prev_changed[set * kSetInts + word];
     }
     __device__ __forceinline__ bool any(unsigned word) const { return (__builtin_amdgcn_ballot_w64(mine != 0) >> word * kXcds & 0xFF) != 0; }
     // f over a word of all sets, the same in every lane

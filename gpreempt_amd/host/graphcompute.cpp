@@ -337,7 +337,7 @@ Status Workload::launch_slot(int i, bool fresh, GPUstream stream, const PreemptE
     p.changed = (unsigned *)slot;
     if (p.prev_changed) p.prev_changed = (const unsigned *)((int *)ring_ + slot_ints_ * ((i - (int)(uintptr_t)p.prev_changed) % kRing));
     p.started = (unsigned long long *)starts_dev_ + i % kRing;
-    p.sets = 1;
+    p.sets = GP_GRAPH_IN_SETS;
     p.seq = seq_of_[i % kRing] = ++seq_;
     gp_preempt_ctx ctx;
     if (env) {

@@ -486,14 +486,16 @@ int gp_launch_graph(const gp_graph_params *p, const gp_preempt_ctx *ctx, gp_stre
  * started, if given, is a device-visible word of host memory (gp_host_alloc_coherent) in which the launch stores, when it
  * starts, seq in the upper half and in the lower one what is known then: GP_GRAPH_START_STOPPED | the stop index if a stop
  * is recorded, else GP_GRAPH_START_CHANGED unless *prev_changed is 0, and prev_changed[1] (at most GP_GRAPH_START_COUNT).
- * With `sets` nonzero, changed and prev_changed are each GP_GRAPH_SETS sets of these words, 128 bytes apart: an XCD's workgroups
- * use a set of their own, and what a launch is told is all of them together.
+ * With `sets` == GP_GRAPH_IN_SETS, changed and prev_changed are each GP_GRAPH_SETS sets of these words, 128 bytes apart: an XCD's workgroups
+ * use a set of their own, and what a launch is told is all of them together.  (Any other value: one set.  The word stands where the
+ * structure had a gap, so that callers built before there was one hand over what they always did.)
  * A preemptible launch over a million edges and more that comes with gp_preempt_ctx::done counters (done_launches 0: cleared
  * before every launch) and with relay (GP_GRAPH_RELAYS words 128 bytes apart, cleared before the launch that follows a
  * stop) gives the claims back that it is in when a stop is recorded, where the kernel allows it (BFS, SSSP, CC_LINK,
  * PR_STEP with next_gained); the relaunch does them again. */
 #define GP_GRAPH_RELAYS 64
 #define GP_GRAPH_SETS 8
+#define GP_GRAPH_IN_SETS 0x53455453u
 #define GP_GRAPH_START_STOPPED 0x80000000u
 #define GP_GRAPH_START_CHANGED 0x40000000u
 #define GP_GRAPH_START_COUNT 0x3FFFFFFFu
@@ -516,8 +518,8 @@ typedef struct gp_graph_iter_params {
     const unsigned int *prev_changed;
     unsigned long long *started;             /* may be NULL */
     unsigned int seq;
+    unsigned int sets;                       /* GP_GRAPH_IN_SETS, or one set of words */
     unsigned int *relay;                     /* may be NULL */
-    unsigned int sets;                       /* 0: one set of words */
 } gp_graph_iter_params;
 int gp_launch_graph_iter(const gp_graph_iter_params *p, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info);
 /* fills ids (4 * row_end + 4 of them: a last vector of vertex_count lies behind the lists) and weights of that layout from

@@ -53,6 +53,15 @@ def test_struct_sizes_match_header():
     assert sizes == [C.sizeof(m) for m in mirrors]
 
 
+def test_a_graph_iteration_takes_no_more_memory_than_callers_have_handed_over_before(tmp_path):
+    """gp_graph_iter_params ended with `relay`, with a gap in front of it, when programs were first built against it: what has come since lies in the gap"""
+    import subprocess
+    src = '#include <stddef.h>\n#include "gpreempt_hip.h"\n' \
+          '_Static_assert(sizeof(gp_graph_iter_params) == 200 && offsetof(gp_graph_iter_params, seq) == 184 && offsetof(gp_graph_iter_params, relay) == 192, "layout");'
+    (tmp_path / "s.c").write_text(src)
+    subprocess.check_call(["gcc", "-fsyntax-only", "-I", os.path.join(ROOT, "include"), str(tmp_path / "s.c")])
+
+
 def test_param_file_round_trip_and_malformed(tmp_path):
     from gpreempt_amd import executor
     lib = executor.lib()

@@ -678,6 +678,8 @@ template <typename T, int MAXC, int R, bool PRE>
 __device__ __forceinline__ void ln_rows_math(const float (&v)[R][MAXC][VecIO<T>::VEC], int chunks, int lane, int cols, float eps,
                                              const T *gamma_p, const T *beta_p, const out_u32x4 (&gamma)[PRE ? MAXC : 1],
                                              const out_u32x4 (&beta)[PRE ? MAXC : 1], out_u32x4 (&y)[R][MAXC]) {
+    // (which products are fused with a sum is written out: ln_pair_math of gemm_ln.hpp gives the same bits, whatever is compiled around either)
+#pragma clang fp contract(off)
     constexpr int VEC = VecIO<T>::VEC;
     float sum[R], mean[R], sq[R], inv[R];
 #pragma unroll
@@ -702,7 +704,12 @@ __device__ __forceinline__ void ln_rows_math(const float (&v)[R][MAXC][VecIO<T>:
             const int ch = lane + i * 64;
             if (ch < chunks) {
 #pragma unroll
-                for (int j = 0; j < VEC; ++j) { float d = v[q][i][j] - mean[q]; sq[q] += d * d; }
+                for (int j = 0; j < VEC; ++j) {
+                    const float d = v[q][i][j] - mean[q];
+                    if (i == 0 && j == 0) continue;
+                    if (i == 0 && j == 1) { const float d0 = v[q][0][0] - mean[q]; sq[q] = __builtin_fmaf(d0, d0, d * d); }
+                    else sq[q] = __builtin_fmaf(d, d, sq[q]);
+                }
             }
         }
     }
@@ -725,7 +732,7 @@ __device__ __forceinline__ void ln_rows_math(const float (&v)[R][MAXC][VecIO<T>:
             for (int q = 0; q < R; ++q) {
                 float o[VEC];
 #pragma unroll
-                for (int j = 0; j < VEC; ++j) o[j] = (v[q][i][j] - mean[q]) * inv[q] * ga[j] + be[j];
+                for (int j = 0; j < VEC; ++j) o[j] = __builtin_fmaf((v[q][i][j] - mean[q]) * inv[q], ga[j], be[j]);
                 y[q][i] = VecIO<T>::pack(o);
             }
         }

@@ -47,6 +47,7 @@ template <typename T, int HALF> __device__ __forceinline__ float add_half(unsign
 }
 template <typename T> __device__ __forceinline__ void ln_pair_math(const out_u32x4 (&x)[3], int tail, int lane, int cols, float eps,
                                                                    const out_u32x4 (&gamma)[2], const out_u32x4 (&beta)[2], out_u32x4 (&y)[3]) {
+#pragma clang fp contract(off)
     static_assert(sizeof(T) == 2, "two values to a word");
     const bool behind = (lane & 31) < tail;  // this lane has a chunk behind the 64th
     float sum[2], sq[2];
@@ -80,7 +81,7 @@ template <typename T> __device__ __forceinline__ void ln_pair_math(const out_u32
             d[c][2 * w] = add_half<T, 0>(x[c][w], -m);
             d[c][2 * w + 1] = add_half<T, 1>(x[c][w], -m);
         }
-    // (the first product of a row is the fused one and its second the rounded one, as the compiler pairs them there)
+    // (the first product of a row is the fused one and its second the rounded one, as there)
     auto first_squares = [](const float (&v)[8]) {
         float s = __builtin_fmaf(v[0], v[0], v[1] * v[1]);
 #pragma unroll

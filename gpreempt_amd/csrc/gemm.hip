@@ -151,9 +151,8 @@ static int choose_body(MatPlan *pl, int tile, int tile_n, int variant) {
         set_error("no matrix kernel for tile %d x %d with variant %d (tiles: 256, 128, 64; 64, 32 with split K; wide: 32x32, 64x32, 64x64, N x K operands; convolutions with Cin a multiple of the K-block and at most 32 taps)", tile, tile_n ? tile_n : tile, variant);
         return GP_OUTOFRANGE;
     }
-    // The 16-bit body of 256 x 256 fetches through descriptors of 2 GB that begin at a tile's first row, and has no registers left for addresses
-    // of 64 bits; where a tile's rows span more, tiles of 128 x 128 (the same sums in the same order).
-    if (body == MB_PIPE256 && pl->dtype != GP_F32 && 256.0 * (double)std::max(g.lda, g.ldb) + g.K >= 1073741823.0) body = MB_PIPE128;
+    // (the phases of the 16-bit body of 256 x 256 have no registers left for addresses of 64 bits)
+    pl->near = body == MB_PIPE256 && pl->dtype != GP_F32 && 256.0 * (double)std::max(g.lda, g.ldb) + g.K < 1073741823.0;
     int t = body == MB_PIPE256 ? GP_BIG_BM : (body == MB_PIPE128 || body == MB_STAGED128) ? 128 : (body == MB_PIPE32_SK ? 32 : 64);
     int tn = body == MB_PIPE256 ? GP_BIG_BN : t;
     if (const WideChoice *w = wide_of(body)) { t = w->bm; tn = w->bn; }

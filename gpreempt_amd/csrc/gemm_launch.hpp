@@ -78,7 +78,7 @@ template <typename T, int BM, int BN, int BK, int WGM, int WGN, bool CONV, bool 
 using TK = TileKernel<T, BM, BN, BK, WGM, WGN, CONV, B_KN>;
 
 template <class K> struct K_is_ckpt { static constexpr bool value = false; };
-template <typename T, int BM, int BN, int ST, int CV, int W> struct K_is_ckpt<PipeKernel<T, BM, BN, ST, CV, false, true, W>> { static constexpr bool value = true; };
+template <typename T, int BM, int BN, int ST, int CV, int W, bool PH> struct K_is_ckpt<PipeKernel<T, BM, BN, ST, CV, false, true, W, false, PH>> { static constexpr bool value = true; };
 template <class K> struct KernelOf {
     static constexpr auto fn = mat_kernel<K, LOOP_ANY>;
     static constexpr auto plain = mat_kernel<K, LOOP_PLAIN>;
@@ -89,8 +89,8 @@ template <class K> struct KernelOf {
     static constexpr auto looks = mat_kernel<K, K::can_look ? LOOP_LOOKS : LOOP_FIXED>;
 #endif
 };
-template <typename T, int BM, int BN, int ST, int CV, int W> struct KernelOf<PipeKernel<T, BM, BN, ST, CV, false, true, W>> {
-    static constexpr auto fn = mat_kernel_ckpt<PipeKernel<T, BM, BN, ST, CV, false, true, W>>;
+template <typename T, int BM, int BN, int ST, int CV, int W, bool PH> struct KernelOf<PipeKernel<T, BM, BN, ST, CV, false, true, W, false, PH>> {
+    static constexpr auto fn = mat_kernel_ckpt<PipeKernel<T, BM, BN, ST, CV, false, true, W, false, PH>>;
     static constexpr auto plain = fn;
     static constexpr auto fixed = fn;
     static constexpr auto looks = fn;
@@ -166,7 +166,14 @@ static int launch_mat(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s,
 #define GP_BIG_BN 256
 #define GP_BIG_STAGES 2
 #endif
-template <typename T, bool CK> using BigPipe = PipeKernel<T, GP_BIG_BM, GP_BIG_BN, GP_BIG_STAGES, false, false, CK, GP_W256>;
+template <typename T, bool CK, bool PHASED = false> using BigPipe = PipeKernel<T, GP_BIG_BM, GP_BIG_BN, GP_BIG_STAGES, false, false, CK, GP_W256, false, PHASED>;
+// From which K on 16-bit tiles of 256 x 256 take a K-step in four phases.  Those fetch two K-steps ahead, and so two beyond the last one, and take
+// longer to begin and to end.  Stage by stage -> in phases, f16, us, plain: 8192 x 8192 x 256 81.9 -> 88.5, x 512 107.3 -> 110.7, x 896 148.8 -> 150.1, x 1024
+// 161.1 -> 162.0, x 2048 266.5 -> 264.6, x 8192 928 -> 894; 2600 x 8000 x 640 50.8 -> 51.1, x 1024 67.0 -> 66.1; with claim counters 5000 x 6000 x 512 61.5 -> 63.0, x 1024
+// 85.7 -> 86.1, x 2048 138.4 -> 137.3; 4096 x 4096 x 256 24.9 -> 25.1, x 1024 44.3 -> 43.8.  Later with checkpoints, where more of a tile's state goes through scratch memory
+// around the loop: 8192 x 8192 x 256 95.6 -> 109.5, x 1280 209.1 -> 210.3, x 1792 268.5 -> 265.8, x 2560 358.8 -> 350.8; 4096 x 4096 x 1024 54.4 -> 56.2,
+// x 1792 77.0 -> 77.4, x 4096 144.1 -> 140.6.
+constexpr int kPhasedK = 1024, kPhasedCkptK = 1792;
 template <typename T, int TILE, int STAGES, bool SPLITK>
 static int pipe_case(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, gp_launch_info *info) {
     if constexpr (TILE == 64 && !SPLITK)
@@ -225,6 +232,10 @@ int launch_typed(const MatPlan &pl, const gp_preempt_ctx *ctx, gp_stream s, gp_l
     constexpr int SBK = sizeof(T) == 4 ? 16 : 32;
     switch (pl.body) {
         case MB_PIPE256:  // GEMM only: the gathered A operand of a convolution does not fit its register budget
+            if constexpr (sizeof(T) == 2) {
+                if (pl.near && ctx && ctx->ckpt && pl.g.K >= kPhasedCkptK) return launch_mat<BigPipe<T, true, true>>(pl, ctx, s, info);
+                if (pl.near && !(ctx && ctx->ckpt) && pl.g.K >= kPhasedK) return launch_mat<BigPipe<T, false, true>>(pl, ctx, s, info);
+            }
             if (ctx && ctx->ckpt) return launch_mat<BigPipe<T, true>>(pl, ctx, s, info);
             return launch_mat<BigPipe<T, false>>(pl, ctx, s, info);
         // The depth of the ring decides how many workgroups a compute unit holds (160 KB of LDS).  A launch that gives it

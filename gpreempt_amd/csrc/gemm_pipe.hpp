@@ -161,7 +161,8 @@ struct NoneAsked { __device__ __forceinline__ void operator()() const {} };
 // 35 x 35, batch 16 20.6 -> 13.8; 3 x 3 over 80 at 73 x 73, batch 16, in 128 x 128 tiles 85 -> 60.  fp32, 7 x 7 over 4 channels, batch 1 14.1 -> 12.0.  What bounds
 // the first layers now is the way from the claim to the store of a tile with two to seven K-steps.)
 // PRE: the rows of A go through a scale, shift and ReLU first (gemm_pre.hpp).
-template <typename T, int BM, int BN, int STAGES, int CONV, bool SPLITK, bool CKPT = false, int NWAVES = 4, bool PRE = false>
+// PHASED: 16-bit GEMM tiles of 256 x 256 that take a K-step in four phases (see the loop), for rows within a descriptor's 2 GB.
+template <typename T, int BM, int BN, int STAGES, int CONV, bool SPLITK, bool CKPT = false, int NWAVES = 4, bool PRE = false, bool PHASED = false>
 struct PipeKernel {
     using elem = T;
     static constexpr int bm = BM, bn = BN;
@@ -194,8 +195,7 @@ struct PipeKernel {
     // The stop words are fetched with every stage (so that every wave issues the same number of
     // loads) but looked at every POLL_EVERY-th K-step: about every 2.5 us for either tile size.
     static constexpr int POLL_EVERY = BM >= 256 ? 2 : 4;
-    // 16-bit GEMM tiles of 256 x 256 take a K-step in four phases (see the loop)
-    static constexpr bool PHASED = BM == 256 && BN == 256 && WAVES == 8 && STAGES == 2 && sizeof(T) == 2 && !CONV && !SPLITK && !PRE;
+    static_assert(!PHASED || (BM == 256 && BN == 256 && WAVES == 8 && STAGES == 2 && sizeof(T) == 2 && !CONV && !SPLITK && !PRE), "what the phases' quarters and waits count on");
     static_assert(!CKPT || !SPLITK, "checkpointing is built for the bodies without split K");
     static_assert(WAVES == 4 || (WAVES == 8 && !SPLITK), "4 wavefronts, or 8 without split K");
     static_assert(BM % 32 == 0 && BN % 32 == 0 && A_PW >= 1 && B_PW >= 1, "tile shape");

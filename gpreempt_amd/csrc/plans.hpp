@@ -31,6 +31,7 @@ struct MatPlan {
     bool taps = false;    // a 16-bit convolution whose K-steps lie within a filter tap, of at most 32, with operands in buffers of 2 GB
     bool straddles = false;  // a convolution whose K-steps straddle filter taps, with operands in buffers of 2 GB and its tap found by multiplication
     bool tall = false;    // MB_PIPE64 in tiles of 128 x 64
+    bool near = false;    // MB_PIPE256 in 16 bits, a tile's rows within the 2 GB of a buffer
     bool pre;          // the rows of A go through g.pre_* first
     int rounds;        // rounds of workgroups a preemptible launch may take with a workgroup per claim; 0: the launcher's own number
 };

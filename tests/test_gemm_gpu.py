@@ -1026,7 +1026,7 @@ flag = gp.Flag()
 cases = 0
 for variant, tm, tn, M, N, ks in ((gp.MAT_PIPE, 64, 64, 256, 256, (64, 128, 192, 256, 320, 704, 768, 832, 1280)),
                                   (gp.MAT_PIPE, 128, 128, 256, 256, (64, 192, 256, 704, 1216)),
-                                  (gp.MAT_PIPE, 256, 256, 512, 512, (64, 128, 256, 320, 512, 576, 768, 1280)),
+                                  (gp.MAT_PIPE, 256, 256, 512, 512, (64, 128, 256, 320, 512, 576, 768, 1024, 1032, 1088, 1280, 1344, 1536, 1600)),
                                   (gp.MAT_WIDE, 32, 32, 64, 128, (1024, 2048, 3072, 5120, 9216))):
     for K in ks:
         A = rng.uniform(-1, 1, (M, K)).astype(np.float16)
@@ -1069,7 +1069,7 @@ print("OK", cases)
 
 def test_looks_at_every_count_of_k_steps(gp):
     """The instantiation that looks again during a tile, on tiles of 1 to 20 K-steps (no run of 8, exactly one, one and
-    a rest, two; fewer K-steps than stages; 256 x 256: the word asked for in every eighth and read four later, the last K-step on either) and on split-K tiles of 4 to 36 stages: the bits of the plain launch, every
+    a rest, two; fewer K-steps than stages; 256 x 256 over K >= 1024: the word asked for in every eighth and read four later, the last K-step on either) and on split-K tiles of 4 to 36 stages: the bits of the plain launch, every
     worker counted once in gp_preempt_ctx::done whether it finished its tile or gave it up, and a launch that finds
     the flag up leaves its tiles unwritten for the relaunch.  The threshold that selects the instantiation is read
     once per process, hence the child process with GPREEMPT_LONG_TILE_MACS=1."""
@@ -1079,7 +1079,7 @@ def test_looks_at_every_count_of_k_steps(gp):
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     out = subprocess.run([sys.executable, "-c", _LOOKS_SWEEP, root], capture_output=True, text=True, timeout=110,
                          env={**os.environ, "GPREEMPT_LONG_TILE_MACS": "1"})
-    assert out.returncode == 0 and out.stdout.strip().startswith("OK 27"), (out.stdout[-300:], out.stderr[-1500:])
+    assert out.returncode == 0 and out.stdout.strip().startswith("OK 33"), (out.stdout[-300:], out.stderr[-1500:])
 
 
 _RINGS = [(4096, 1920, 1152), (4096, 2200, 1160), (2048, 1600, 4608), (2000, 1580, 4640), (4096, 2048, 2048)]

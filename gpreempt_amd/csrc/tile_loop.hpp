@@ -74,7 +74,7 @@ struct BlpArgs {
 // The first workgroup tells the host that this launch has reached the GPU, i.e. that everything submitted before it on
 // the stream has left (a store to host memory: nobody waits for it).
 __device__ __forceinline__ void announce_start(const BlpArgs &b, bool leader) {
-    if (__builtin_expect(b.started && blockIdx.x == 0, 0) && leader) __hip_atomic_store(b.started, b.started_seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (b.started && blockIdx.x == 0 && leader) __hip_atomic_store(b.started, b.started_seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // a worker's number among the workers of the launch, and how many there are
@@ -256,18 +256,20 @@ __device__ __forceinline__ bool spare_workgroup(const BlpArgs &b, bool fixed, bo
 // retire) looks at the flag only when a workgroup starts, and those start in bursts, a tile's length apart: with
 // 40 us tiles (VGG-16's 512-channel 3 x 3 layers at batch 16) a stop took up to 43 us to be so much as recorded.
 // Such a launch gets `front` workgroups ahead of its workers (a multiple of 8, so that the workers keep their XCDs).
-// The first one stays: one lane reads the flag about every microsecond and records the stop, until a stop is
+// The first one stays: one lane reads the flag every two to three microseconds and records the stop, until a stop is
 // recorded, or every claim of the launch has been made (from then on no workgroup starts that a stop could hold
 // back), or its bounded number of looks is used up.  The others leave at once.  Returns true in a front workgroup.
 // (The ways out of the common path are marked as unlikely, here and below, so that their code does not stand between a kernel's entry and its first
-// load, where it is fetched and jumped over: with the pause 1024^3 fp32 had become 21.8 -> 22.0 us, now 21.7; ResNet-50 b1 fp32 578 -> 570.)
-// Between two reads of the flag the first wavefront pauses for about two microseconds, in which it only looks whether it is time to go: a read of
+// load, where it is fetched and jumped over: with the pause 1024^3 fp32 had become 21.8 -> 22.0 us, now 21.7.  Not in front of tiles with checkpoints, whose
+// loop has no such ways: 8192 x 8192 x 256 f16 94.5 us with the mark, 92.2 without, 4096 x 4096 x 256 33.1 and 32.7.)
+// Between two reads of the flag the first wavefront pauses for a good microsecond, in which it only looks whether the second one has told it to go
+// (a wavefront alone just pauses): a read of
 // host memory under way makes every load of that XCD come back later, and the launch lasts until its slowest XCD is done.  VGG-16 b16
 // 1332 -> 1282 us, ResNet-152 b8 1547 -> 1537, Inception-v3 b1 stopped and resumed level (860 -> 850); three times the pause: VGG 1300,
 // Inception 864 (a stop is seen later).
 constexpr int FRONT_PAUSE = 10;  // sleeps of 256 cycles
 __device__ __forceinline__ bool front_workgroup(const BlpArgs &b, bool leader) {
-    announce_start(b, leader);  // (here because every dispatcher loop comes through here first)
+    if (__builtin_expect(b.started && blockIdx.x == 0, 0)) announce_start(b, leader);  // (here because every other dispatcher loop comes through here first)
     if (__builtin_expect(b.front == 0 || (int)blockIdx.x >= b.front, 1)) return false;
     const int tid = (int)(threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z));
     if (blockIdx.x != 0 || !b.flag) return true;
@@ -300,7 +302,7 @@ __device__ __forceinline__ bool front_workgroup(const BlpArgs &b, bool leader) {
         return __builtin_amdgcn_readfirstlane(stop) != -1 || __builtin_amdgcn_readfirstlane(n) >= target;
     };
     if (tid < 64) {
-        for (int look = 0; look < (1 << 17); ++look) {  // 3-4 us per look: at most about half a second
+        for (int look = 0; look < (1 << 17); ++look) {  // 2-3 us per look; the second wavefront's bound, about a quarter of a second, is reached first
             int flag = 0;
             if (tid == 0) flag = __hip_atomic_load(b.flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             if (__builtin_amdgcn_readfirstlane(flag) != 0) {
@@ -313,7 +315,7 @@ __device__ __forceinline__ bool front_workgroup(const BlpArgs &b, bool leader) {
         }
         if (tid == 0) tell();
     } else if (two && tid < 128) {
-        for (int look = 0; look < (1 << 19); ++look) {  // about half a microsecond per look
+        for (int look = 0; look < (1 << 19); ++look) {  // about half a microsecond per look: a quarter of a second
             if (device_look(tid - 64) || told()) break;
             __builtin_amdgcn_s_sleep(4);
         }

@@ -75,6 +75,7 @@ static int g_stop_at_level = -1;  // the iteration that finds the flag up, once
 static std::vector<int> g_ran;    // levels in the order in which they ran
 static std::atomic<int> g_in_flight{0};  // launches submitted and not done
 static int g_left = 0;            // launches that left because of a recorded stop
+static std::atomic<size_t> g_cleared{0};  // words
 static void pause_us(int us) { if (us) std::this_thread::sleep_for(std::chrono::microseconds(us)); }
 
 extern "C" {
@@ -91,6 +92,7 @@ int gp_fetch(void *h, const void *d, size_t n, gp_stream s) { gp_stream_sync(s);
 int gp_stream_sync(gp_stream s) { while (of(s)->pending) std::this_thread::yield(); return 0; }
 int gp_stream_query(gp_stream s, int *idle) { *idle = of(s)->pending == 0; return 0; }
 int gp_fill32_async(void *p, uint32_t v, size_t n, gp_stream s) {
+    g_cleared += n;
     of(s)->submit([=] { for (size_t i = 0; i < n; ++i) ((uint32_t *)p)[i] = v; });
     return 0;
 }
@@ -208,10 +210,24 @@ static void check_long_run_keeps_nothing() {
     CHECK(g_peak - before < 256 << 10, "%ld bytes more in use during %d iterations", g_peak.load() - before, iterations);
 }
 
+// connected components is a handful of launches, and what it clears in front of them counts: half a ring of claim counters, and a line of words each
+static void check_what_cc_clears() {
+    auto w = GraphCompute::Workload::create("cc", path_graph(64));
+    const GraphCompute::PreemptEnv env = env_of();
+    gp_stream_s s;
+    for (int i = 0; i < 2; ++i) {
+        g_cleared = 0;
+        CHECK(w->compute(&s, &env) == Status::Succ, "cc");
+    }
+    const size_t counters = 2 * (size_t)env.counter_groups * env.counter_stride;
+    CHECK(g_cleared <= 32 * (counters + 32), "%zu words cleared, with %zu words of counters to a launch", g_cleared.load(), counters);
+}
+
 int main(int argc, char **argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "blocking") check_nothing_left_behind();
     else if (what == "stops") check_stops();
+    else if (what == "clears") check_what_cc_clears();
     else if (what == "memory") check_long_run_keeps_nothing();
     else return 2;
     std::printf("ok %s\n", what.c_str());

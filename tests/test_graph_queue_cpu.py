@@ -30,3 +30,7 @@ def test_a_long_run_keeps_nothing_per_launch(check):
 
 def test_a_stop_waits_for_few_launches(check):
     check("stops")
+
+
+def test_what_connected_components_clears(check):
+    check("clears")

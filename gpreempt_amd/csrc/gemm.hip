@@ -181,7 +181,7 @@ static int choose_body(MatPlan *pl, int tile, int tile_n, int variant) {
     // Layers of at most 64 channels over many pixels (the first ones of a VGG) in tiles of 128 x 64: half the workgroups, each of which takes about as
     // long from its claim to its first operands and from its last to its store, and half the weights through LDS.  Preemptible, fp16, batch 16 at
     // 224 x 224: 8 -> 64 channels 75 -> 65 us, 64 -> 64 138 -> 120; batch 8 72 -> 64.  From sixteen tiles of 64 x 64 to a compute unit on: batch 4,
-    // twelve, is level.
+    // twelve, is level.  (bf16 125 -> 109; plain, f16 and bf16: 64 -> 64 115 -> 103 and 111 -> 100, batch 8 60 -> 56 and 56 -> 55.)
     if (pl->ring == 2 && body == MB_PIPE64 && pl->dtype != GP_F32 && (pl->taps || pl->straddles) && g.N > 32 && g.N <= 64 && g.K <= 640 && tiles(64) >= 16 * cus) {
         pl->tall = true;
         pl->sy = (g.M + 127) / 128;

@@ -202,7 +202,9 @@ struct LnWideKernel {
             *(out_u32x4 *)(a_res + (size_t)(ch >> 3) * A_BLK_BYTES + r * RB + ((ch & 7) ^ ((r >> 1) & 7)) * 16) = y;
         };
         if (RPW == 2 && tail > 0 && tail <= 32) {
-            // (no branch stands around these loads and what is computed from them, so the wait for the rows leaves B, asked for behind them, alone)
+            // No branch stands around these loads and what is computed from them, so the compiler waits for each where it is used.  It counts the seven loads here
+            // and not B's, which come behind them: its wait for the rows, four loads of gamma and beta outstanding, lets four of B be on their way, which is
+            // all of them where two stages are asked for.  Those for gamma and beta let two and none, so B has landed before the first row is kept.
             const int m = m0 + wave, over = lane >> 5, ch = 64 + (lane & 31);
             const int r0 = m < g.M ? m : g.M - 1, r1 = m + WAVES < g.M ? m + WAVES : g.M - 1;
             const bool behind = (lane & 31) < tail;

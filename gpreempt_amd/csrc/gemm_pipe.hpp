@@ -170,7 +170,9 @@ struct PipeKernel {
     // Whether GEMM rows are fetched through descriptors (see `near` below).  Not by the fp32 bodies of 128 x 128 and less: their MFMAs
     // take eight times as long, a load's instructions hide behind them, and with two workgroups to a compute unit that now advance
     // in step, a last round of few tiles finds both places of a unit free at once and doubles up there: 5175 x 1833 x 1696
-    // plain 333 -> 428 us, 2048 x 2560 x 4096 preemptible 605 -> 649.  Nor by the 16-bit GEMM of 128 x 128: 3 % faster on 5175 x 1833 x
+    // plain 333 -> 428 us, 2048 x 2560 x 4096 preemptible 605 -> 649.  (Where K-steps straddle taps they do: what a load saves there is two
+    // divisions.  fp32 in 128 x 128 tiles, plain and with claims: 3 x 3 over 80 at 73 x 73, batch 16 348 -> 299 and 361 -> 303; over 48 at 56 x 56 79 -> 67 and 80 -> 68;
+    // over 200 at 61 x 61, batch 3 282 -> 237 and 282 -> 238.)  Nor by the 16-bit GEMM of 128 x 128: 3 % faster on 5175 x 1833 x
     // 1696, but 2048 x 2560 x 4096 preemptible 121 -> 130.
     static constexpr bool DESC = TAPS || STRADDLES || BM == 256 || (sizeof(T) == 2 && BM < 128);
     static constexpr int VEC = Elem<T>::VEC;

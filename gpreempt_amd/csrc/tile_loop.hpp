@@ -265,8 +265,9 @@ __device__ __forceinline__ bool spare_workgroup(const BlpArgs &b, bool fixed, bo
 // Between two reads of the flag the first wavefront pauses for a good microsecond, in which it only looks whether the second one has told it to go
 // (a wavefront alone just pauses): a read of
 // host memory under way makes every load of that XCD come back later, and the launch lasts until its slowest XCD is done.  VGG-16 b16
-// 1332 -> 1282 us, ResNet-152 b8 1547 -> 1537, Inception-v3 b1 stopped and resumed level (860 -> 850); three times the pause: VGG 1300,
-// Inception 864 (a stop is seen later).
+// 1332 -> 1282 us, ResNet-152 b8, DenseNet-201 b4, ResNet-50 b1 and Inception-v3 b1 stopped and resumed level; three times the pause: VGG 1300,
+// Inception 864 (a stop is seen later).  The price: from a flag raised somewhere in a pass to an idle stream, VGG 85.7 -> 87.2 us, ResNet-152 181 -> 183,
+// DenseNet 149 -> 152, ResNet-50 57.5 -> 58.6.  (Half the pause: VGG between the two; no pause in a launch's first eight looks: as with it.)
 constexpr int FRONT_PAUSE = 10;  // sleeps of 256 cycles
 __device__ __forceinline__ bool front_workgroup(const BlpArgs &b, bool leader) {
     if (__builtin_expect(b.started && blockIdx.x == 0, 0)) announce_start(b, leader);  // (here because every other dispatcher loop comes through here first)
